@@ -4,6 +4,7 @@ The library is the only compute path of this package: if it is missing the
 import of any operator fails loudly instead of falling back to PyTorch.
 """
 import ctypes
+import importlib
 import os
 from typing import Optional
 
@@ -82,6 +83,7 @@ _SIGNATURES = {
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lib: Optional[ctypes.CDLL] = None
+_native = None
 
 
 def load() -> ctypes.CDLL:
@@ -100,6 +102,20 @@ def load() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+def native():
+    """The extension module of the native host path (csrc/native.cpp), imported on first use so
+    that the package can be imported - and built - before the module exists."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            _native = importlib.import_module('sparta_amd._native')
+        except ImportError as exc:
+            raise RuntimeError(f'sparta_amd._native could not be imported ({exc}): the extension has not been built. '
+                               'Run `python -m sparta_amd.build` (needs hipcc and g++); there is no fallback path.') from exc
+    return _native
 
 
 def last_error() -> str:

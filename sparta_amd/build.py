@@ -1,7 +1,9 @@
-"""Ahead-of-time build of libsparta_hip.so for gfx950 with hipcc.
+"""Ahead-of-time build of libsparta_hip.so for gfx950 with hipcc, and of the native host path.
 
 Every ``csrc/*.hip`` translation unit is compiled to an object (in parallel) and
-linked into ``sparta_amd/lib/libsparta_hip.so``.  Run as
+linked into ``sparta_amd/lib/libsparta_hip.so``; ``csrc/native.cpp`` (host code only, the
+Python extension module ``sparta_amd._native``) is compiled with the host compiler against
+torch's headers and linked against that library.  Run as
 ``python -m sparta_amd.build`` or through ``__graft_entry__.build()``.
 """
 import concurrent.futures
@@ -17,6 +19,8 @@ CSRC = os.path.join(ROOT, 'csrc')
 OBJ = os.path.join(ROOT, 'build', 'obj')
 LIB_DIR = os.path.join(ROOT, 'lib')
 LIB = os.path.join(LIB_DIR, 'libsparta_hip.so')
+NATIVE_SRC = os.path.join(CSRC, 'native.cpp')
+NATIVE = os.path.join(ROOT, '_native.so')
 
 HIPCC_FLAGS = [
     '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC',
@@ -301,18 +305,51 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
+def _compile_native(force: bool) -> str:
+    """csrc/native.cpp -> object file."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    obj = os.path.join(OBJ, 'native.o')
+    deps = [NATIVE_SRC, os.path.join(ROOT, '..', 'include', 'sparta_hip.h')]
+    if not force and os.path.exists(obj) and os.path.getmtime(obj) >= max(os.path.getmtime(d) for d in deps):
+        return obj
+    cmd = [shutil.which('g++') or 'c++', '-O2', '-std=c++17', '-fPIC', '-fvisibility=hidden', '-c', NATIVE_SRC, '-o', obj,
+           '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1', '-DTORCH_EXTENSION_NAME=_native',
+           '-isystem', sysconfig.get_paths()['include'], '-isystem', '/opt/rocm/include']
+    for path in cpp_extension.include_paths():
+        cmd += ['-isystem', path]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f'compiling {NATIVE_SRC} failed:\n{proc.stderr}')
+    return obj
+
+
+def _link_native(obj: str) -> None:
+    from torch.utils import cpp_extension
+    tmp = NATIVE + '.tmp'   # moved into place: a process may have the old module loaded
+    cmd = [shutil.which('g++') or 'c++', '-shared', '-o', tmp, obj, '-L' + LIB_DIR, '-lsparta_hip', '-Wl,-rpath,$ORIGIN/lib']
+    cmd += ['-L' + path for path in cpp_extension.library_paths()]
+    cmd += ['-ltorch_python', '-ltorch', '-ltorch_cpu', '-ltorch_hip', '-lc10', '-lc10_hip']
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f'linking {NATIVE} failed:\n{proc.stderr}')
+    os.replace(tmp, NATIVE)
+
+
 def build(force: bool = True, jobs: int = 8, verbose: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     sources = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith('.hip'))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        native = pool.submit(_compile_native, force)
         objs = list(pool.map(lambda s: _compile(s, force), sources))
     cmd = [_hipcc(), '--offload-arch=gfx950', '-shared', '-fPIC', '-o', LIB, *objs]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f'link failed:\n{proc.stderr}')
+    _link_native(native.result())
     if verbose:
-        print(f'built {LIB} from {len(sources)} translation units')
+        print(f'built {LIB} from {len(sources)} translation units, and {NATIVE}')
     return LIB
 
 

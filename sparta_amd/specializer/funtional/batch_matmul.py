@@ -7,6 +7,7 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
+from sparta_amd import _lib
 from sparta_amd.specializer.kernels import SparTASparseMatMulKernel, OpenAISparseMatMulKernel
 from sparta_amd.specializer.funtional.sparse_ctx_base import SparseCtxBase, KernelPlaceholder
 
@@ -35,8 +36,11 @@ def _tile_dims(mode: str, trans_A: bool, trans_B: bool) -> Tuple[str, str]:
 
 class SparseBatchMatMulCtx(SparseCtxBase):
 
-    def __init__(self, mode: str, transpose_A: bool, transpose_B: bool, biased: bool, compressed: bool):
+    def __init__(self, mode: str, transpose_A: bool, transpose_B: bool, biased: bool, compressed: bool,
+                 drop_batch: bool = False):
+        """`drop_batch`: the result comes without its batch axis (of one entry)."""
         super().__init__()
+        self._drop_batch = drop_batch
         self._mode = mode
         self._transpose_A = transpose_A
         self._transpose_B = transpose_B
@@ -77,18 +81,22 @@ class SparseBatchMatMulCtx(SparseCtxBase):
         fwd = self._kernels['forward:C'].active_kernel()
         if fwd is not None:
             fwd.set_epilogue(activation)
+            if fwd.ready:
+                self._bind_operator()
+
+    def _bind_operator(self):
+        """The native operator object: the active kernels' launch objects and the autograd node
+        that connects them."""
+        launch = [None if k.active_kernel() is None else k.active_kernel()._func
+                  for k in (self._kernels[name] for name in ('forward:C', 'backward:A', 'backward:B'))]
+        self.apply = _lib.native().MatmulOp(*launch, self._transpose_A, self._transpose_B,
+                                      self._activation == 'relu', self._drop_batch)
 
     def build(self, config: Dict[str, Dict[str, Any]]):
         super().build(config)
         fwd = self._kernels['forward:C'].active_kernel()
         if fwd is not None:
             fwd.set_epilogue(self._activation)
-            self.forward_C = (lambda A, B, bias: fwd(A, B, bias)) if self._biased else (lambda A, B: fwd(A, B))
-            if self._mode == 'dds' and self._compressed:
-                kernel = fwd
-                self.backward_bias = lambda grad_C: kernel.ports['C'].indexes.sum(grad_C, axis=-2)
-            else:
-                self.backward_bias = lambda grad_C: grad_C.sum(-2)
         bwd_A = self._kernels['backward:A'].active_kernel()
         if bwd_A is not None:
             if self._transpose_A:
@@ -101,6 +109,8 @@ class SparseBatchMatMulCtx(SparseCtxBase):
                 self.backward_B = lambda grad_C, A: bwd_B(grad_C, A)
             else:
                 self.backward_B = lambda grad_C, A: bwd_B(A, grad_C)
+        if fwd is not None:
+            self._bind_operator()
 
     def set_sample_inputs(self, sample_inputs: List[torch.Tensor],
                           sample_grads: Optional[List[torch.Tensor]] = None):
@@ -127,32 +137,11 @@ class SparseBatchMatMulCtx(SparseCtxBase):
         return self._kernels['forward:C'].dense_func(*args)
 
 
-class SparseBatchMatMulFunc(torch.autograd.Function):
+class SparseBatchMatMulFunc:
+    """C = op(A) op(B) (+ bias) with its gradients: the autograd node is part of the native
+    operator object that the context holds once it is built."""
 
     @staticmethod
-    def forward(ctx, sparta_ctx: SparseBatchMatMulCtx, input: torch.Tensor, weight: torch.Tensor,
-                bias: Optional[torch.Tensor] = None):
-        input, weight = input.detach(), weight.detach()
-        ctx.sparta_ctx = sparta_ctx
-        if bias is None:
-            output = sparta_ctx.forward_C(input, weight)
-        else:
-            output = sparta_ctx.forward_C(input, weight, bias.detach())
-        # a fused relu: the gradient passes where the output is positive
-        ctx.save_for_backward(input, weight, bias, output if sparta_ctx._activation == 'relu' else None)
-        return output
-
-    @staticmethod
-    def backward(ctx, grad_output: torch.Tensor):
-        input, weight, bias, gate = ctx.saved_tensors
-        grad_output = grad_output.detach().contiguous()
-        if gate is not None:
-            grad_output = grad_output * (gate > 0)
-        grad_input = grad_weight = grad_bias = None
-        if ctx.needs_input_grad[1]:
-            grad_input = ctx.sparta_ctx.backward_A(grad_output, weight)
-        if ctx.needs_input_grad[2]:
-            grad_weight = ctx.sparta_ctx.backward_B(grad_output, input)
-        if bias is not None and ctx.needs_input_grad[3]:
-            grad_bias = ctx.sparta_ctx.backward_bias(grad_output)
-        return None, grad_input, grad_weight, grad_bias
+    def apply(sparta_ctx: SparseBatchMatMulCtx, input: torch.Tensor, weight: torch.Tensor,
+              bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+        return sparta_ctx.apply(input, weight, bias)

@@ -82,7 +82,7 @@ def check_shared_block_shapes(placeholders: Dict[str, KernelPlaceholder], built)
             raise AssertionError(
                 f'kernel {name} takes {want[0]}x{want[1]} blocks of its sparse tensor, the kernels it shares '
                 f'that tensor with take {port._block_H}x{port._block_W}')
-        kernel.ready = False
+        kernel.switch_off()
         placeholder.ready = False
 
 

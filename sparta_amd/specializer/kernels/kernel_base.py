@@ -3,7 +3,7 @@ filtering, self-test.
 
 Interface of sparta/specializer/kernels/kernel_base.py:24-220.  There is no
 code generation here: `compile()` validates a configuration, fixes the block
-sizes (which triggers the index build of the sparse port) and binds a closure
+sizes (which triggers the index build of the sparse port) and binds the callable
 that launches the ahead-of-time compiled HIP kernel through the C ABI.
 """
 from __future__ import annotations
@@ -243,11 +243,22 @@ class KernelBase(abc.ABC):
         target = self.reference(*sample)
         targets = list(target) if isinstance(target, tuple) else [target]
         self._convert_data(sample, targets)
-        self._tile_strict = True
+        self._set_tile_strict(True)
         try:
             return profile(self, sample, targets, num_warmups, num_iters, cuda)
         finally:
-            self._tile_strict = False
+            self._set_tile_strict(False)
+
+    def _set_tile_strict(self, strict: bool):
+        self._tile_strict = strict
+        if hasattr(self._func, 'set_strict'):   # a native launch object
+            self._func.set_strict(strict)
+
+    def switch_off(self):
+        """Calls raise until the kernel is compiled again."""
+        self.ready = False
+        if hasattr(self._func, 'unbind'):
+            self._func.unbind()
 
     def __call__(self, *args) -> torch.Tensor:
         if not self.ready:

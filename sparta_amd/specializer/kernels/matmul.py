@@ -1,5 +1,5 @@
 """Block-sparse matmul kernels: which operand is sparse, which block sizes tile
-it, the search space, and the launch closure around spx_matmul.
+it, the search space, and the binding of the native launch object around spx_matmul.
 
 Interface of sparta/specializer/kernels/matmul.py:21-331.  The mode letters name
 A, B, C in that order ('sdd' = sparse A, 'dsd' = sparse B, 'dds' = sparse C).
@@ -15,7 +15,7 @@ import torch
 from sparta_amd import _lib
 from sparta_amd.common.tuning import TunableItemCfg
 from sparta_amd.specializer.kernels.kernel_base import KernelBase, PortConfig
-from sparta_amd.specializer.kernels.operand_sizes import matmul_extent, check_matmul_operands
+from sparta_amd.specializer.kernels.operand_sizes import matmul_extent
 
 # mode / transpose -> (sparse port, tile height param, tile width param, index format)
 _SPARSE_LAYOUT = {
@@ -55,6 +55,7 @@ class SparseMatMulKernel(KernelBase):
             self._tesa_vars = self._tesa_vars[1:]
         self._epilogue = 0
         super().__init__()
+        self._func = _lib.native().MatmulKernel()
 
     def set_epilogue(self, activation: Optional[str]):
         """Activation applied by the kernel's own epilogue (an extension: the reference runs a
@@ -129,78 +130,35 @@ class SparseMatMulKernel(KernelBase):
     def threads_per_block(self):
         return (256, 1, 1)
 
-    # ---- launch closure ---------------------------------------------------------------
+    # ---- launch object ----------------------------------------------------------------
     def update_func(self):
+        """Bind the native launch object to the current shape and index.  It checks what it is
+        handed against what the kernel walks (a compressed operand laid out by another index is
+        refused before the launch), and gives a configured tile variant that the library
+        refuses for these shapes up for the library's own choice (but for tuner trials)."""
         batch_size, M, K, N = self.get_shape()
-        BM, BK, BN = self.get_block_shape()
-        indexes = self.ports[self._sparse_port].indexes
-        mode_code = _lib.MODE_CODE[self._mode]
-        tA, tB = int(self._transpose_A), int(self._transpose_B)
-        compressed = int(self._compressed)
-        biased = self._biased
-        tile_cfg = int(self.get_parameter('TILE_CFG') or 0) | self._epilogue
-        tile_elems = self.get_parameter(self._sparse_block_H) * self.get_parameter(self._sparse_block_W)
-        lib = _lib.load()
-
+        port = self.ports[self._sparse_port]
+        indexes = port.indexes
+        # Only a compressed operand / a sparse output need the live block count on the
+        # host; a port in at-capacity mode leaves it on the device.
+        dds = self._mode == 'dds'
+        nnz_dev = None
+        if port.at_capacity:
+            nnz, nnz_dev = indexes.capacity, indexes.nnz_dev
+        else:
+            nnz = indexes.block_nnz if (self._compressed or dds) else 0
         if self._bcs_mode == 'BCSR':
             ptr, idx, idx_kind = indexes.row_ptr, indexes._bcsr_buf, _lib.IDX_BCSR_I32
         else:
             ptr, idx = indexes.col_ptr, indexes._bcsc_buf
             idx_kind = _lib.IDX_BCSC_I64 if idx.dtype == torch.int64 else _lib.IDX_BCSC_I32
-        dds = self._mode == 'dds'
         sched = None if dds else indexes.launch_order('row' if self._bcs_mode == 'BCSR' else 'col')
-        sched_p = _lib.dev_ptr(sched)
-        # Only a compressed operand / a sparse output need the live block count on the
-        # host; a port in at-capacity mode leaves it on the device.
-        at_capacity = self.ports[self._sparse_port].at_capacity
-        nnz_dev_p = None
-        if at_capacity:
-            nnz = indexes.capacity
-            nnz_dev_p = _lib.dev_ptr(indexes.nnz_dev)
-        else:
-            nnz = indexes.block_nnz if (compressed or dds) else 0
-        sparse_stride = nnz * tile_elems
-        if dds and compressed:
-            C_shape = (batch_size, nnz * BM * BN)
-        else:
-            C_shape = (batch_size, M, N)
-        # A dense sparse-output result keeps zeros in dead tiles; every other result is
-        # fully overwritten by the kernel.
-        alloc = torch.zeros if (dds and not compressed) else torch.empty
-        ptr_p, idx_p = _lib.dev_ptr(ptr), _lib.dev_ptr(idx)
-        # what this closure's kernel walks behind each pointer: a compressed operand laid out
-        # by another index (other block shape, other mask) is refused before the launch
-        extent = matmul_extent(self._mode, bool(compressed), batch_size, M, K, N, sparse_stride)
-        tile = [tile_cfg]   # tile variant (low 16 bits) | epilogue flags; see the retry below
-
-        def matmul_func(A: torch.Tensor, B: torch.Tensor, bias: torch.Tensor = None,
-                        _keepalive=(indexes, ptr, idx, sched)):
-            assert A.dtype == B.dtype, f'operand dtypes differ: {A.dtype} vs {B.dtype}'
-            check_matmul_operands(extent, A, B, bias, biased)
-            C = alloc(C_shape, dtype=A.dtype, device=A.device)
-            if bias is not None:
-                bias = bias.to(A.dtype).contiguous()
-            A, B = A.contiguous(), B.contiguous()
-            cfg = tile[0]
-            while True:
-                rc = lib.spx_matmul(
-                    mode_code, _lib.dtype_code(A.dtype), tA, tB, compressed,
-                    _lib.dev_ptr(A), _lib.dev_ptr(B), _lib.dev_ptr(bias), _lib.dev_ptr(C),
-                    ptr_p, idx_p, idx_kind, sched_p, nnz, nnz_dev_p, sparse_stride,
-                    batch_size, M, K, N, BM, BK, BN, cfg, _lib.current_stream(A.device))
-                if rc == _lib.E_CONFIG and cfg & 0xffff and not self._tile_strict:
-                    # the configured tile variant does not take these shapes (nothing was
-                    # launched): the library's own choice from here on
-                    cfg = tile[0] = cfg & ~0xffff
-                    continue
-                break
-            _lib.check(rc, 'spx_matmul')
-            return C
-
-        if biased:
-            self._func = lambda A, B, bias: matmul_func(A, B, bias)
-        else:
-            self._func = lambda A, B: matmul_func(A, B)
+        stride = nnz * indexes.block_H * indexes.block_W
+        extent = matmul_extent(self._mode, self._compressed, batch_size, M, K, N, stride)
+        self._func.bind(
+            _lib.MODE_CODE[self._mode], self._transpose_A, self._transpose_B, self._compressed, self._biased,
+            batch_size, M, K, N, *self.get_block_shape(), ptr, idx, idx_kind, sched, nnz, nnz_dev,
+            stride, extent.A, extent.B, int(self.get_parameter('TILE_CFG') or 0) | self._epilogue)
 
     # ---- self test ------------------------------------------------------------------------
     def _convert_data(self, inputs: List[torch.Tensor], outputs: List[torch.Tensor]):

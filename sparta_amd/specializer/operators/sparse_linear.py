@@ -54,14 +54,14 @@ class SparseLinear(OperatorBase):
         self.bias = raw_module.bias
         M = None
         if input_mask is not None:
-            self._sparse_ctx = SparseBatchMatMulCtx('sdd', False, True, biased, False)
+            self._sparse_ctx = SparseBatchMatMulCtx('sdd', False, True, biased, False, drop_batch=True)
             M = input_mask.shape[0]
         elif weight_mask is not None:
             # dynamic: the kernels read the live blocks out of the dense weight through the
             # index, so a new mask costs an index rebuild and nothing else
-            self._sparse_ctx = SparseBatchMatMulCtx('dsd', False, True, biased, not dynamic)
+            self._sparse_ctx = SparseBatchMatMulCtx('dsd', False, True, biased, not dynamic, drop_batch=True)
         elif output_mask is not None:
-            self._sparse_ctx = SparseBatchMatMulCtx('dds', False, True, biased, False)
+            self._sparse_ctx = SparseBatchMatMulCtx('dds', False, True, biased, False, drop_batch=True)
             M = output_mask.shape[0]
         else:
             raise ValueError('expected a sparse mask on input / weight / output')
@@ -129,10 +129,7 @@ class SparseLinear(OperatorBase):
         return torch.relu(out) if self._activation == 'relu' else out
 
     def _sparse_forward(self, input_tensor: torch.Tensor):
-        args = [self._sparse_ctx, input_tensor, self.weight]
-        if self.bias is not None:
-            args.append(self.bias)
-        return self.__sparse_func__.apply(*args).squeeze(0)
+        return self._sparse_ctx.apply(input_tensor, self.weight, self.bias)
 
     def set_sample_inputs(self, sample_inputs: List[torch.Tensor],
                           sample_grads: Optional[List[torch.Tensor]] = None):
