@@ -214,6 +214,24 @@ int spx_matmul(int mode, int dtype, int transA, int transB, int compressed,
                int batch, int M, int K, int N, int BM, int BK, int BN,
                int tile_cfg, spx_stream_t stream);
 
+/* SPX_DDS with the reduction over k split over workgroups, and optionally the sums of op(A)
+ * over k from the same launches: the weight gradient of a linear layer and its bias gradient
+ * (A = grad_y stored [K = tokens, M = out], transA; B = x stored [K, N = in]).  The reference
+ * launches its sparse_matmul_dds template and torch.sum (batch_matmul.py:145-179).
+ *
+ * slices     0: chosen from the sizes; 1: not split; 2, 4 or 8: that many ranges of k, whose fp32
+ *            partial blocks are added in order by a second kernel.
+ * a_colsum   optional, [batch, M] of `dtype`: sum over k of op(A) (fp32 accumulate); needs transA.
+ * workspace  device memory, 16-byte aligned, spx_matmul_split_workspace_bytes() bytes (0: may be NULL).
+ * The other arguments as for spx_matmul with mode SPX_DDS (BCSR index, nnz on the host). */
+size_t spx_matmul_split_workspace_bytes(int dtype, int transA, int transB, int nnz, int batch, int M, int K, int N,
+                                        int BM, int BN, int slices, int with_colsum);
+int spx_matmul_split(int dtype, int transA, int transB, int compressed,
+                     const void* A, const void* B, void* C, void* a_colsum,
+                     const int32_t* row_ptr, const int32_t* idx, int nnz, int64_t sparse_batch_stride,
+                     int batch, int M, int K, int N, int BM, int BN, int slices,
+                     void* workspace, size_t workspace_bytes, spx_stream_t stream);
+
 /* ------------------------------------------------------------------------ *
  * Masked block-sparse softmax over the last axis.
  * Replaces SparseSoftmaxForwardKernel.update_func / BackwardKernel.update_func

@@ -63,6 +63,8 @@ _SIGNATURES = {
     'spx_bcs_schedule': (_I, [_P, _I, _P, _P]),
     'spx_matmul': (_I, [_I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _L,
                         _I, _I, _I, _I, _I, _I, _I, _I, _P]),
+    'spx_matmul_split_workspace_bytes': (_Z, [_I] * 12),
+    'spx_matmul_split': (_I, [_I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _L, _I, _I, _I, _I, _I, _I, _I, _P, _Z, _P]),
     'spx_softmax_forward': (_I, [_I, _I, _P, _P, _P, _P, _P, _F, _I, _I, _I, _I, _I, _L, _I, _P]),
     'spx_softmax_backward': (_I, [_I, _I, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _I, _I, _L, _I, _P]),
     'spx_attention_forward': (_I, [_I, _P, _P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _I, _I, _I, _I, _P]),

@@ -2,6 +2,7 @@
 // compressed) onto the two kernel families.
 #include "matmul_spmm.hpp"
 #include "matmul_dds.hpp"
+#include "matmul_dds_split.hpp"
 
 namespace spx {
 
@@ -128,5 +129,70 @@ extern "C" int spx_matmul(int mode, int dtype, int transA, int transB, int compr
         default:
             return run_matmul<bf16_t>(mode, transA, transB, compressed, A, B, bias, C, ptr, idx, idx_kind, sched, nnz_bound,
                                       nnz_dev, sparse_batch_stride, batch, M, K, N, BM, BK, BN, tile_cfg, st);
+    }
+}
+
+namespace spx {
+
+static int split_slices(int dtype, int transA, int transB, int nnz, int batch, int K, int BM, int BN, int slices) {
+    return slices ? slices : dds_split_slices(dtype_bytes(dtype), !transA && transB, nnz, batch, K, BM, BN);
+}
+static size_t split_partial_bytes(int slices, int nnz, int batch, int BM, int BN) {
+    return slices > 1 ? (size_t)batch * slices * nnz * BM * BN * sizeof(float) : 0;
+}
+
+}  // namespace spx
+
+extern "C" size_t spx_matmul_split_workspace_bytes(int dtype, int transA, int transB, int nnz, int batch, int M, int K, int N,
+                                                   int BM, int BN, int slices, int with_colsum) {
+    using namespace spx;
+    (void)N;
+    return split_partial_bytes(split_slices(dtype, transA, transB, nnz, batch, K, BM, BN, slices), nnz, batch, BM, BN) +
+           (with_colsum ? (size_t)batch * kColsumSlices * M * sizeof(float) : 0);
+}
+
+extern "C" int spx_matmul_split(int dtype, int transA, int transB, int compressed, const void* A, const void* B, void* C,
+                                void* a_colsum, const int32_t* row_ptr, const int32_t* idx, int nnz, int64_t sparse_batch_stride,
+                                int batch, int M, int K, int N, int BM, int BN, int slices, void* workspace,
+                                size_t workspace_bytes, spx_stream_t stream) {
+    using namespace spx;
+    SPX_REQUIRE(dtype == SPX_F32 || dtype == SPX_F16 || dtype == SPX_BF16, SPX_E_DTYPE, "unknown dtype %d", dtype);
+    SPX_REQUIRE(nnz >= 0 && batch >= 0 && batch <= 65535 && M > 0 && K > 0 && N > 0, SPX_E_SHAPE, "bad sizes");
+    SPX_REQUIRE((BM == 16 || BM == 32 || BM == 64) && (BN == 16 || BN == 32 || BN == 64), SPX_E_CONFIG,
+                "output block (%d,%d) not in {16,32,64}^2", BM, BN);
+    SPX_REQUIRE(M % BM == 0 && N % BN == 0, SPX_E_SHAPE, "%d x %d is not a multiple of the block (%d,%d)", M, N, BM, BN);
+    SPX_REQUIRE(K % 16 == 0, SPX_E_SHAPE, "K=%d must be a multiple of 16", K);
+    SPX_REQUIRE(!a_colsum || transA, SPX_E_CONFIG, "the column sums need a transposed A");
+    SPX_REQUIRE(A && B && (C || nnz == 0) && (idx || nnz == 0), SPX_E_NULL, "a required buffer is NULL");
+    const int es = dtype_bytes(dtype);
+    SPX_REQUIRE(aligned(A, 16) && aligned(B, 16) && aligned(C, 16) && aligned(workspace, 16), SPX_E_ALIGN, "buffers must be 16-byte aligned");
+    SPX_REQUIRE(!compressed || (sparse_batch_stride * es) % 16 == 0, SPX_E_ALIGN, "sparse batch stride must keep blocks 16-byte aligned");
+    DdsSplit s;
+    SPX_REQUIRE(slices == 0 || slices == 1 || slices == 2 || slices == 4 || slices == 8, SPX_E_CONFIG, "slices=%d not in {0,1,2,4,8}", slices);
+    s.slices = split_slices(dtype, transA, transB, nnz, batch, K, BM, BN, slices);
+    s.k_slice = 0;
+    s.nnz = nnz;
+    s.n_product = 0;
+    const size_t part = split_partial_bytes(s.slices, nnz, batch, BM, BN);
+    s.partial = reinterpret_cast<float*>(workspace);
+    s.colsum = a_colsum ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + part) : nullptr;
+    const size_t need = part + (a_colsum ? (size_t)batch * kColsumSlices * M * sizeof(float) : 0);
+    SPX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), SPX_E_WORKSPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, need);
+    if (batch == 0) return 0;
+    DdsParams p;
+    p.A = A; p.B = B; p.bias = nullptr; p.C = C;
+    p.idx = idx; p.row_ptr = row_ptr; p.nnz_dev = nullptr;
+    p.M = M; p.K = K; p.N = N;
+    p.a_kcontig = !transA; p.a_ld = transA ? M : K;
+    p.b_kcontig = transB;  p.b_ld = transB ? K : N;
+    p.compressed = compressed;
+    p.a_batch = (int64_t)M * K; p.b_batch = (int64_t)K * N;
+    p.c_batch = compressed ? sparse_batch_stride : (int64_t)M * N;
+    p.bias_batch = N;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    switch (dtype) {
+        case SPX_F32: return launch_dds_split<float>(p, s, a_colsum, BM, BN, batch, st);
+        case SPX_F16: return launch_dds_split<_Float16>(p, s, a_colsum, BM, BN, batch, st);
+        default: return launch_dds_split<bf16_t>(p, s, a_colsum, BM, BN, batch, st);
     }
 }

@@ -1,0 +1,12 @@
+// bf16 instantiations of the k-split sparse-output matmul kernel.
+#include "matmul_dds_split.hpp"
+namespace spx {
+template <>
+int launch_dds_split<bf16_t>(const DdsParams& p, const DdsSplit& s, void* colsum, int BM, int BN, int batch, hipStream_t st) {
+    return launch_dds_split_impl<bf16_t>(p, s, colsum, BM, BN, batch, st);
+}
+template <>
+int launch_dds_unsliced<bf16_t>(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, hipStream_t st) {
+    return launch_dds_split<bf16_t>(p, DdsSplit{1, 0, nnz_bound, 0, nullptr, nullptr}, nullptr, BM, BN, batch, st);
+}
+}  // namespace spx

@@ -1,0 +1,12 @@
+// f32 instantiations of the k-split sparse-output matmul kernel.
+#include "matmul_dds_split.hpp"
+namespace spx {
+template <>
+int launch_dds_split<float>(const DdsParams& p, const DdsSplit& s, void* colsum, int BM, int BN, int batch, hipStream_t st) {
+    return launch_dds_split_impl<float>(p, s, colsum, BM, BN, batch, st);
+}
+template <>
+int launch_dds_unsliced<float>(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, hipStream_t st) {
+    return launch_dds_split<float>(p, DdsSplit{1, 0, nnz_bound, 0, nullptr, nullptr}, nullptr, BM, BN, batch, st);
+}
+}  // namespace spx

@@ -140,6 +140,10 @@ struct MatmulPlan {
         if (bias_in && bias_in->defined()) bias = bias_in->to(a.scalar_type()).contiguous();
         void *pa = device_ptr(a), *pb = device_ptr(b);
         void* pbias = bias.defined() ? device_ptr(bias) : nullptr;
+        if (mode == SPX_DDS) {
+            const size_t ws_bytes = split_workspace(code, false);
+            if (ws_bytes > 0) return run_split(code, a, b, nullptr, ws_bytes, out_shape);
+        }
         // a dense sparse-output result keeps zeros in dead tiles; every other result is fully
         // overwritten by the kernel
         Tensor c = mode == SPX_DDS && !compressed ? at::zeros(out_shape, a.options()) : at::empty(out_shape, a.options());
@@ -161,6 +165,36 @@ struct MatmulPlan {
         check_rc(rc, "spx_matmul");
         return c;
     }
+
+    // A sparse-output product may be split along k (spx_matmul_split); the bytes that takes, 0: not split.
+    size_t split_workspace(int code, bool colsum) const {
+        const int cfg = tile_cfg.load(std::memory_order_relaxed) & 0xffff;
+        if (nnz_dev.has_value() || biased || (cfg != 0 && !colsum)) return 0;
+        // the whole reduction is one or two stages deep: the block-row kernels of spx_matmul
+        if (!trans_a && trans_b && K * (code == SPX_F32 ? 4 : 2) <= 256) return 0;
+        return spx_matmul_split_workspace_bytes(code, trans_a, trans_b, nnz, batch, M, K, N, BM, BN, 0, colsum);
+    }
+    // `colsum` (may be null) receives the sums of op(A) over k.  Contiguous operands.
+    Tensor run_split(int code, const Tensor& a, const Tensor& b, Tensor* colsum, size_t ws_bytes, at::IntArrayRef out_shape) const {
+        Tensor c = compressed ? at::empty(out_shape, a.options()) : at::zeros(out_shape, a.options());
+        Tensor ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+        check_rc(spx_matmul_split(code, trans_a, trans_b, compressed, device_ptr(a), device_ptr(b), c.data_ptr(),
+                                  colsum ? device_ptr(*colsum) : nullptr, (const int32_t*)device_ptr(ptr),
+                                  (const int32_t*)device_ptr(idx), nnz, sparse_stride, batch, M, K, N, BM, BN, 0,
+                                  ws.data_ptr(), ws_bytes, stream_of(a)), "spx_matmul_split");
+        return c;
+    }
+    // The weight gradient together with the sums of its first operand over k (the bias gradient).
+    Tensor run_with_colsum(const Tensor& a, const Tensor& b, at::IntArrayRef out_shape, Tensor* colsum) const {
+        if (a.scalar_type() != b.scalar_type()) assertion("operand dtypes differ: ", a.dtype(), " vs ", b.dtype());
+        require_numel("spx_matmul_split", "A", a, numel_a);
+        require_numel("spx_matmul_split", "B", b, numel_b);
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        const int code = dtype_code(a);
+        *colsum = at::empty({batch, M}, a.options());
+        return run_split(code, a.contiguous(), b.contiguous(), colsum, split_workspace(code, true), out_shape);
+    }
+    bool gives_colsum() const { return mode == SPX_DDS && trans_a && !nnz_dev.has_value(); }
 
     c10::SmallVector<int64_t, 3> shape() const {
         if (sparse_out()) return {batch, sparse_stride};
@@ -238,6 +272,12 @@ struct MatmulBackward : public Node {
             }
             if (task_should_compute_output(1)) {
                 require_built(have_b, bwd_b, "backward_B");
+                if (num_outputs() > 2 && task_should_compute_output(2) && trans_b && !fwd->sparse_out() && bwd_b->gives_colsum()) {
+                    Tensor bias_grad;
+                    out[1] = bwd_b->run_with_colsum(grad, A, B.sizes(), &bias_grad);
+                    out[2] = bias_grad.view(bias_shape);
+                    return out;
+                }
                 out[1] = trans_b ? bwd_b->run(grad, A, nullptr, B.sizes()) : bwd_b->run(A, grad, nullptr, B.sizes());
             }
             if (num_outputs() > 2 && task_should_compute_output(2)) out[2] = fwd->bias_grad(grad, bias_shape);
