@@ -171,6 +171,15 @@ __device__ __forceinline__ void lds_direct_load16(const void* g, uint32_t lds_wa
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_wave_base), "v"(g) : "memory", "m0");
 }
 
+// The same from a wave-uniform base plus a 32-bit byte offset per lane.
+__device__ __forceinline__ void lds_direct_load16_at(const void* base, uint32_t offset, uint32_t lds_wave_base) {
+    const uint64_t v = (uint64_t)base;
+    // (readfirstlane gives a signed int: each half is made unsigned before they meet in 64 bits)
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    const uint64_t s = ((uint64_t)hi << 32) | lo;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_wave_base), "v"(offset), "s"(s) : "memory", "m0");
+}
+
 // 16-byte accesses for data that is streamed once: the non-temporal hint keeps it from
 // displacing operands that other workgroups re-read from L2.
 __device__ __forceinline__ vec16 load16_stream(const void* p) {

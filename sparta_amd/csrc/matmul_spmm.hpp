@@ -217,6 +217,16 @@ int launch_spmm_stream(const SpmmParams& p, int BN, int batch, hipStream_t st);
 template <typename T>
 int launch_spmm_ksplit(const SpmmParams& p, int BN, int batch, hipStream_t st);
 template <typename T>
+int launch_spmm_ring(const SpmmParams& p, int BN, int batch, int rows, hipStream_t st);
+// What the LDS-ring kernel takes: 64-byte block rows, and a dense operand that can be read in 16-byte pieces.
+template <typename T>
+bool spmm_ring_supported(const SpmmParams& p, int BN) {
+    constexpr int VE = 16 / (int)sizeof(T);
+    return (p.BK * (int)sizeof(T)) % 64 == 0 && (BN == 16 || BN == 32 || BN == 64) &&
+           (p.d_kcontig || (p.Mc % VE == 0 && p.d_ld % VE == 0)) && (p.out_ncontig || p.Mc % VE == 0) &&
+           p.d_ld * 128 + p.K < (int64_t)1 << 29 && (p.compressed || p.s_ld * 64 + p.K < (int64_t)1 << 29);   // byte offsets in 32 bits
+}
+template <typename T>
 bool spmm_thin_supported(const SpmmParams& p, int BN);
 template <typename T>
 int launch_spmm_thin(const SpmmParams& p, int batch, hipStream_t st);
@@ -234,6 +244,8 @@ int launch_spmm_thin(const SpmmParams& p, int batch, hipStream_t st);
 //          types, 64-wide k-contiguous sparse blocks): one workgroup per block-column.
 //   10     persistent form of 7 for a k-contiguous dense operand: a workgroup walks the
 //          tiles of its XCD as one stream of steps (matmul_spmm_stream.hpp).
+//   11 / 12  ring of LDS stages filled by a loader wavefront, 64 / 128-row tiles, any layout with
+//          64-byte block rows (matmul_spmm_ring.hpp).
 template <typename T>
 int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipStream_t st) {
     const bool kcontig = p.d_kcontig && p.s_kcontig;
@@ -242,41 +254,65 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
     // ... and reads a dense operand stored with m contiguous through LDS transpose reads
     const bool panel7_ok = (p.BK * (int)sizeof(T)) % 64 == 0 &&
                            (p.d_kcontig || (p.Mc % (16 / (int)sizeof(T)) == 0 && p.d_ld % (16 / (int)sizeof(T)) == 0));
-    if (tile_cfg < 0 || tile_cfg > 10) return fail(SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
+    if (tile_cfg < 0 || tile_cfg > 12) return fail(SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
     const bool stream_ok = p.d_kcontig && (p.BK * (int)sizeof(T)) % 64 == 0 && p.d_ld * 256 + 64 < (int64_t)0x7fffffff / (int)sizeof(T);
     const bool ksplit_ok = panel_ok && BN <= 32;
     const bool thin_ok = spmm_thin_supported<T>(p, BN);
-    if (tile_cfg == 0 && thin_ok) tile_cfg = 9;
+    // one workgroup per block-column only where every one of them has a long walk over a sparse operand
+    // that streams from HBM (96 x 4096 x 4096: 82 us against 106 through the ring); below, the ring kernel
+    // is ahead (1 x 3072 x 4096 x 64 at 20 %: 15.3 / 9.3, 48 x 1024 x 1024 x 64 at 10 %: 8.2 / 7.8)
+    if (tile_cfg == 0 && thin_ok && (int64_t)batch * p.K * p.Nc >= 500000000) tile_cfg = 9;
     if (tile_cfg == 9) {
         if (!thin_ok) return fail(SPX_E_CONFIG, "tile config 9 needs a 16-bit dense operand with 64 or 128 contiguous m and 64-wide k-contiguous blocks of depth 32 / 64");
         return launch_spmm_thin<T>(p, batch, st);
     }
+    const bool ring_ok = spmm_ring_supported<T>(p, BN);
     if (tile_cfg == 0) {
         // 256-row tiles only when they still give every CU a few workgroups; small
         // problems are latency-bound and want more, shorter workgroups.
-        const int64_t big_tiles = (int64_t)((p.Mc + 255) / 256) * (p.Nc / BN) * batch;
+        const int nb = p.Nc / BN, cols = p.K / p.BK;
+        const int64_t big_tiles = (int64_t)((p.Mc + 255) / 256) * nb * batch;
+        const int64_t tiles128 = (int64_t)((p.Mc + 127) / 128) * nb * batch;
         const bool fill = big_tiles >= 512;
+        // 128-row tiles halve the traffic of the sparse blocks and want a few rounds of workgroups to
+        // even out (fp32 spends longer on a tile: more of them)
+        const int ring = tiles128 >= (sizeof(T) == 4 ? 2048 : BN == 64 ? 1024 : 768) ? 12 : 11;
+        // The ring kernel, where it was measured ahead (rows x K x N; us of the best other kernel / ring):
+        //   * operands that are not both k-contiguous: sdd 4096 x 3072 x 768 fp32 at 20 % 110 / 38, fp16 26 / 14,
+        //     dsd 400 x 3072 x 768 fp32 at 15 % 38 / 10, bf16 14 / 10 - but for large fp32 problems in blocks
+        //     of depth 16, whose stages hold two blocks each (4096 x 768 x 3072: 46 / 55);
+        //   * k-contiguous fp32 and 16-bit blocks of depth 64: 4096 x 3072 x 768 fp32 at 10 % 33 / 22, bf16
+        //     64 x 64 at 20 % 25 / 14, 200 x 768 x 3072 7 / 5;
+        //   * 16-bit blocks of depth 32 (two to a stage) while the result is narrow: 8192 x 1024 x 1024
+        //     at 10 % 16.5 / 13.5; wide results (tiles of one or two stages) stay with the 256-row
+        //     kernels: 8192 x 768 x 3072 at 10 % 23 / 28, 4096^3 at 5 % 25.5 / 31.
+        const bool two_blocks = p.BK * (int)sizeof(T) == 64;
+        bool use_ring = ring_ok;
+        if (two_blocks && sizeof(T) == 4) use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
+        else if (two_blocks && kcontig) {
+            if (fill) use_ring = ring_ok && p.Nc < 2048 && cols >= 32;
+            else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32);
+        }
         // the persistent form when its 8 * (N / BN) slots fill the device four times over, every
         // slot walks at least two 256-row tiles and the block-columns are long: 28.4 - 28.7 us
         // against 29.9 - 30.0 us for 7 on the 4096^3 problem (alternating runs on three
         // machines); with fewer slots or tiles it loses (C4 layers: 28 / 34 against 20 / 21 us)
-        const int nb = p.Nc / BN;
-        if (stream_ok && panel_ok && batch == 1 && 8 * nb >= 1024 && p.Mc >= 16 * 256 && p.K / p.BK >= 32 &&
-            (BN == 16 || BN == 32 || BN == 64))
+        if (stream_ok && panel_ok && batch == 1 && 8 * nb >= 1024 && p.Mc >= 16 * 256 && cols >= 32 && two_blocks &&
+            sizeof(T) == 2 && (BN == 16 || BN == 32 || BN == 64))
             tile_cfg = 10;
+        else if (use_ring) tile_cfg = ring;
         else if (panel_ok && p.Mc >= 512 && fill) tile_cfg = p.Mc >= 1024 ? 7 : 5;
-        else if (ksplit_ok && !fill && p.K / p.BK >= 8) tile_cfg = 8;  // few tiles, long block-columns
-        // operands that are not both k-contiguous (input gradients, transposed layouts) have only
-        // the LDS-staged kernel besides 7, which 7 beats two- to threefold at every size measured
-        // (64 to 8192 rows, 10 to 99 % sparsity)
-        // (fp32 with an m-contiguous dense operand builds its fragments from 4-byte LDS reads and
-        // only pays on large problems: 1024^3 29.7 against 17.5 us)
-        else if (panel7_ok && ((!kcontig && (sizeof(T) == 2 || p.d_kcontig)) || (p.Mc >= 512 && fill))) tile_cfg = 7;
-        // sparse blocks wider than the K-split kernel takes: the register-direct kernel only while
-        // the problem is small and its block-columns short (measured 2 - 3x behind 5 otherwise)
-        else if (panel_ok && !ksplit_ok && (big_tiles >= 128 || (big_tiles >= 64 && p.K / p.BK >= 64))) tile_cfg = 5;
+        // few rows and short columns: no barrier and no shared block pays (64 x 768 x 3072 bf16: 3.9 us
+        // against 4.4 with the columns split and 5.2 through the ring)
+        else if (kcontig && (p.Mc <= 16 ? cols <= 128 : p.Mc <= 256 && cols <= 32)) tile_cfg = 3;
+        else if (ksplit_ok && !fill && cols >= 8) tile_cfg = 8;  // few tiles, long block-columns
+        else if (panel7_ok && p.Mc >= 512 && fill) tile_cfg = 7;
         else if (kcontig) tile_cfg = p.Mc >= 1024 && fill ? 4 : 3;
         else tile_cfg = p.Mc >= 1024 && fill ? 2 : 1;
+    }
+    if (tile_cfg >= 11) {
+        if (!ring_ok) return fail(SPX_E_CONFIG, "tile config %d needs 64-byte block rows and 16-byte pieces of the dense operand", tile_cfg);
+        return launch_spmm_ring<T>(p, BN, batch, tile_cfg == 11 ? 64 : 128, st);
     }
     if (tile_cfg == 10) {
         if (!stream_ok) return fail(SPX_E_CONFIG, "tile config 10 needs a k-contiguous dense operand and 64-byte block rows");

@@ -39,12 +39,14 @@ __global__ __launch_bounds__(256) void spmm_direct_kernel(SpmmParams p, int n_mt
     constexpr int TM = 64 * WM;
     constexpr int CH = DM::CH, KC = DM::KC, LK = DM::LK;
 
-    // XCD-aware numbering: L -> (xcd, sequence); a row panel stays on one XCD.
+    // XCD-aware numbering: L -> (xcd, sequence); a row panel stays on one XCD.  Fewer panels than XCDs are
+    // dealt out column by column instead (in the first numbering one panel would leave seven of
+    // the eight XCDs idle).
     const int nb = p.Nc / BN;
     const int L = blockIdx.x;
-    const int xcd = L % kNumXcd;
-    const int seq = L / kNumXcd;
-    const int mt = (seq / nb) * kNumXcd + xcd;
+    const bool few = n_mtiles < kNumXcd;
+    const int seq = few ? L : L / kNumXcd;
+    const int mt = few ? seq / nb : (seq / nb) * kNumXcd + L % kNumXcd;
     const int j = p.sched ? p.sched[seq % nb] : seq % nb;
     if (mt >= n_mtiles) return;
     const int64_t b = blockIdx.y;
@@ -176,8 +178,8 @@ static int launch_spmm_direct_inst(const SpmmParams& p, int batch, hipStream_t s
     constexpr int TM = 64 * WM;
     const int n_mtiles = (p.Mc + TM - 1) / TM;
     const int nb = p.Nc / BN;
-    const int64_t groups = (n_mtiles + kNumXcd - 1) / kNumXcd;
-    const int64_t nblocks = groups * kNumXcd * nb;
+    const int64_t panels = n_mtiles < kNumXcd ? n_mtiles : (n_mtiles + kNumXcd - 1) / kNumXcd * kNumXcd;
+    const int64_t nblocks = panels * nb;
     if (nblocks > 0x7fffffffLL) return fail(SPX_E_SHAPE, "problem too large for one launch");
     hipLaunchKernelGGL((spmm_direct_kernel<T, BN, BK, WM, SWAP>), dim3((unsigned)nblocks, batch, 1), dim3(256), 0, st,
                        p, n_mtiles);

@@ -29,11 +29,14 @@ __global__ __launch_bounds__(256) void spmm_ksplit_kernel(SpmmParams p, int n_mt
     static_assert(BK % KC == 0, "block depth must be a multiple of the step");
     __shared__ __align__(16) char lds_all[STAGE_BYTES > PART_BYTES ? STAGE_BYTES : PART_BYTES];
 
+    // XCD-aware numbering: L -> (xcd, sequence); a row panel stays on one XCD.  Fewer panels than XCDs are
+    // dealt out column by column instead (in the first numbering one panel would leave seven of
+    // the eight XCDs idle).
     const int nb = p.Nc / BN;
     const int L = blockIdx.x;
-    const int xcd = L % kPanelXcd;
-    const int seq = L / kPanelXcd;
-    const int mt = (seq / nb) * kPanelXcd + xcd;   // 64-row tile; neighbours in m share an XCD's L2
+    const bool few = n_mtiles < kPanelXcd;
+    const int seq = few ? L : L / kPanelXcd;
+    const int mt = few ? seq / nb : (seq / nb) * kPanelXcd + L % kPanelXcd;
     const int j = p.sched ? p.sched[seq % nb] : seq % nb;
     if (mt >= n_mtiles) return;
     const int64_t b = blockIdx.y;
@@ -252,8 +255,8 @@ template <typename T, int BN, int BK, bool SWAP>
 static int launch_spmm_ksplit_inst(const SpmmParams& p, int batch, hipStream_t st) {
     const int n_mtiles = (p.Mc + 63) / 64;
     const int nb = p.Nc / BN;
-    const int64_t groups = (n_mtiles + kPanelXcd - 1) / kPanelXcd;
-    const int64_t nblocks = groups * kPanelXcd * nb;
+    const int64_t panels = n_mtiles < kPanelXcd ? n_mtiles : (n_mtiles + kPanelXcd - 1) / kPanelXcd * kPanelXcd;
+    const int64_t nblocks = panels * nb;
     if (nblocks > 0x7fffffffLL) return fail(SPX_E_SHAPE, "problem too large for one launch");
     hipLaunchKernelGGL((spmm_ksplit_kernel<T, BN, BK, SWAP>), dim3((unsigned)nblocks, batch, 1), dim3(256), 0, st,
                        p, n_mtiles);

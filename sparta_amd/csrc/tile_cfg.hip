@@ -21,6 +21,8 @@ static const spx_tile_cfg kSpmmCfgs[] = {
     {8, 64, 0, 4, 2, 16, 7, "panel-64-ksplit"},
     {9, 64, 0, 4, 2, 64, 6, "thin-dense-operand"},
     {10, 256, 0, 4, 2, 16, 7, "panel-256-persistent"},
+    {11, 64, 0, 5, 3, 16, 7, "ring-64"},
+    {12, 128, 0, 5, 3, 16, 7, "ring-128"},
 };
 static const spx_tile_cfg kDdsCfgs[] = {
     {0, 0, 0, 4, 1, 16, 7, "auto"},
