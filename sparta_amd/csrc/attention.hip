@@ -511,18 +511,10 @@ static int launch_attention_v2_inst(const AttnParams& p, int batch, hipStream_t 
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
     if (p.mask) {
-        if (smem > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_kernel_v2<T, BW, E, WAVES, true>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_kernel_v2)");
-        }
+        SPX_GRANT_LDS((attention_kernel_v2<T, BW, E, WAVES, true>), smem, "attention_kernel_v2");
         hipLaunchKernelGGL((attention_kernel_v2<T, BW, E, WAVES, true>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, batch);
     } else {
-        if (smem > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_kernel_v2<T, BW, E, WAVES, false>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_kernel_v2)");
-        }
+        SPX_GRANT_LDS((attention_kernel_v2<T, BW, E, WAVES, false>), smem, "attention_kernel_v2");
         hipLaunchKernelGGL((attention_kernel_v2<T, BW, E, WAVES, false>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, batch);
     }
     SPX_LAUNCH_CHECK("attention_kernel_v2");
@@ -537,11 +529,7 @@ static int launch_attention_v2_seq_inst(const AttnParams& p, int batch, hipStrea
     const int nbr = p.Nt / TB;
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_kernel_v2<T, TB, E, TB / 16, true, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_kernel_v2)");
-    }
+    SPX_GRANT_LDS((attention_kernel_v2<T, TB, E, TB / 16, true, true>), smem, "attention_kernel_v2");
     hipLaunchKernelGGL((attention_kernel_v2<T, TB, E, TB / 16, true, true>), dim3((unsigned)groups), dim3(4 * TB), smem, st, p, nbr, batch);
     SPX_LAUNCH_CHECK("attention_kernel_v2 (sequence lengths)");
     return 0;
@@ -861,18 +849,10 @@ static int launch_attention_train_inst(const AttnParams& p, int batch, hipStream
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
     if (p.mask) {
-        if (smem > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_train_kernel<T, BW, E, WAVES, true>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_train_kernel)");
-        }
+        SPX_GRANT_LDS((attention_train_kernel<T, BW, E, WAVES, true>), smem, "attention_train_kernel");
         hipLaunchKernelGGL((attention_train_kernel<T, BW, E, WAVES, true>), dim3((unsigned)groups), dim3(64 * (WAVES + 1)), smem, st, p, nbr, batch);
     } else {
-        if (smem > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_train_kernel<T, BW, E, WAVES, false>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_train_kernel)");
-        }
+        SPX_GRANT_LDS((attention_train_kernel<T, BW, E, WAVES, false>), smem, "attention_train_kernel");
         hipLaunchKernelGGL((attention_train_kernel<T, BW, E, WAVES, false>), dim3((unsigned)groups), dim3(64 * (WAVES + 1)), smem, st, p, nbr, batch);
     }
     SPX_LAUNCH_CHECK("attention_train_kernel");
@@ -1144,11 +1124,7 @@ static int launch_attention_bwd_row_inst(const AttnParams& p, int batch, hipStre
     const int nbr = p.Nt / p.BH;
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_bwd_row_kernel<T, BW, E, WAVES>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_bwd_row_kernel)");
-    }
+    SPX_GRANT_LDS((attention_bwd_row_kernel<T, BW, E, WAVES>), smem, "attention_bwd_row_kernel");
     hipLaunchKernelGGL((attention_bwd_row_kernel<T, BW, E, WAVES>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, batch);
     SPX_LAUNCH_CHECK("attention_bwd_row_kernel");
     return 0;
@@ -1377,11 +1353,7 @@ static int launch_attention_bwd_row_rc_inst(const AttnParams& p, int batch, hipS
     const int nbr = p.Nt / p.BH;
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_bwd_row_rc_kernel<T, BW, E, WAVES>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_bwd_row_rc_kernel)");
-    }
+    SPX_GRANT_LDS((attention_bwd_row_rc_kernel<T, BW, E, WAVES>), smem, "attention_bwd_row_rc_kernel");
     hipLaunchKernelGGL((attention_bwd_row_rc_kernel<T, BW, E, WAVES>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, batch);
     SPX_LAUNCH_CHECK("attention_bwd_row_rc_kernel");
     return 0;
@@ -1792,11 +1764,7 @@ static int launch_attention_bwd_col_inst(const AttnParams& p, int batch, hipStre
     const int nbc = p.Ns / (16 * WAVES);
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbc;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_bwd_col_kernel<T, BH, E, WAVES>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_bwd_col_kernel)");
-    }
+    SPX_GRANT_LDS((attention_bwd_col_kernel<T, BH, E, WAVES>), smem, "attention_bwd_col_kernel");
     hipLaunchKernelGGL((attention_bwd_col_kernel<T, BH, E, WAVES>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbc, batch);
     SPX_LAUNCH_CHECK("attention_bwd_col_kernel");
     return 0;
@@ -1827,11 +1795,7 @@ static int launch_attention_bwd_col_rc_inst(const AttnParams& p, int batch, hipS
     const int nbc = p.Ns / (16 * WAVES);
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbc;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_bwd_col_rc_kernel<T, BH, E, WAVES>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_bwd_col_rc_kernel)");
-    }
+    SPX_GRANT_LDS((attention_bwd_col_rc_kernel<T, BH, E, WAVES>), smem, "attention_bwd_col_rc_kernel");
     hipLaunchKernelGGL((attention_bwd_col_rc_kernel<T, BH, E, WAVES>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbc, batch);
     SPX_LAUNCH_CHECK("attention_bwd_col_rc_kernel");
     return 0;
@@ -2053,18 +2017,10 @@ static int launch_attention_v3_inst(const AttnParams& p, int batch, hipStream_t 
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
     if (p.mask) {
-        if (smem > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_kernel_v3<T, BW, E, WAVES, true>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_kernel_v3)");
-        }
+        SPX_GRANT_LDS((attention_kernel_v3<T, BW, E, WAVES, true>), smem, "attention_kernel_v3");
         hipLaunchKernelGGL((attention_kernel_v3<T, BW, E, WAVES, true>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, batch);
     } else {
-        if (smem > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_kernel_v3<T, BW, E, WAVES, false>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_kernel_v3)");
-        }
+        SPX_GRANT_LDS((attention_kernel_v3<T, BW, E, WAVES, false>), smem, "attention_kernel_v3");
         hipLaunchKernelGGL((attention_kernel_v3<T, BW, E, WAVES, false>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, batch);
     }
     SPX_LAUNCH_CHECK("attention_kernel_v3");
@@ -2091,11 +2047,7 @@ template <typename T, int BW, int E>
 static int launch_attention_inst(const AttnParams& p, int batch, hipStream_t st) {
     const int waves = p.BH / 16;
     const size_t smem = ((size_t)BW * (E + 8) + (size_t)E * (BW + 8)) * sizeof(T);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_kernel<T, BW, E>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_kernel)");
-    }
+    SPX_GRANT_LDS((attention_kernel<T, BW, E>), smem, "attention_kernel");
     hipLaunchKernelGGL((attention_kernel<T, BW, E>), dim3(p.Nt / p.BH, batch, 1), dim3(64 * waves), smem, st, p);
     SPX_LAUNCH_CHECK("attention_kernel");
     return 0;
@@ -2257,11 +2209,7 @@ template <typename T, int TB, int E>
 static int launch_attention_seqlen_inst(const SeqlenParams& p, int batch_heads, hipStream_t st) {
     constexpr int VE = 16 / (int)sizeof(T);
     const size_t smem = ((size_t)TB * (E + VE) + (size_t)E * (TB + VE)) * sizeof(T);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_seqlen_kernel<T, TB, E>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attention_seqlen_kernel)");
-    }
+    SPX_GRANT_LDS((attention_seqlen_kernel<T, TB, E>), smem, "attention_seqlen_kernel");
     hipLaunchKernelGGL((attention_seqlen_kernel<T, TB, E>), dim3(p.N / TB, batch_heads, 1), dim3(TB * 4), smem, st, p);
     SPX_LAUNCH_CHECK("attention_seqlen_kernel");
     return 0;

@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <atomic>
+
 #include "../../include/sparta_hip.h"
 
 namespace spx {
@@ -28,6 +30,33 @@ inline int hip_fail(hipError_t e, const char* what) {
 #define SPX_LAUNCH_CHECK(name) \
     do { hipError_t e__ = hipGetLastError(); \
          if (e__ != hipSuccess) return ::spx::hip_fail(e__, name); } while (0)
+
+// Dynamic LDS above 48 KB has to be granted to a kernel first.  The grant lasts for the process,
+// so each instantiation asks the runtime once per device and not at every launch.
+class LdsGrant {
+public:
+    int ensure(const void* kernel, int bytes, const char* name) {
+        if (bytes <= 48 * 1024) return 0;
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return hip_fail(e, name);
+        const bool known = dev >= 0 && dev < kDevices;
+        if (known && granted_[dev].load(std::memory_order_acquire) >= bytes) return 0;
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e != hipSuccess) return hip_fail(e, name);
+        if (known) granted_[dev].store(bytes, std::memory_order_release);
+        return 0;
+    }
+
+private:
+    static constexpr int kDevices = 32;
+    std::atomic<int> granted_[kDevices] = {};
+};
+// `kernel` in parentheses (template arguments contain commas); returns from the caller on failure
+#define SPX_GRANT_LDS(kernel, bytes, name) \
+    do { static ::spx::LdsGrant grant__; \
+         if (const int rc__ = grant__.ensure(reinterpret_cast<const void*>(&kernel), (int)(bytes), "hipFuncSetAttribute(" name ")")) \
+             return rc__; } while (0)
 
 inline bool is_pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
 inline int ilog2(int x) { int l = 0; while ((1 << l) < x) ++l; return l; }

@@ -358,11 +358,7 @@ static int launch_dds_pipe_inst(const DdsParams& p, int nnz_bound, int batch, hi
     size_t smem = 2 * (size_t)(BM + BN) * (KT + VE) * sizeof(T);
     size_t epi = (size_t)G::KS * BM * (BN + 4) * sizeof(float);
     if (epi > smem) smem = epi;
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dds_pipe_kernel<T, BM, BN, NST>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(dds_pipe_kernel)");
-    }
+    SPX_GRANT_LDS((dds_pipe_kernel<T, BM, BN, NST>), smem, "dds_pipe_kernel");
     hipLaunchKernelGGL((dds_pipe_kernel<T, BM, BN, NST>), dim3(nnz_bound, batch, 1), dim3(256), smem, st, p);
     SPX_LAUNCH_CHECK("dds_pipe_kernel");
     return 0;
@@ -482,11 +478,7 @@ static int launch_dds_row_inst(const DdsParams& p, int batch, hipStream_t st) {
     constexpr int K = KB / (int)sizeof(T);
     typedef DdsWaveGrid<BM / 16, BN / 16> G;
     const size_t smem = (size_t)(BM + 2 * BN) * (K + VE) * sizeof(T) + (size_t)G::KS * BM * (BN + 4) * sizeof(float);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dds_row_kernel<T, BM, BN, KB>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(dds_row_kernel)");
-    }
+    SPX_GRANT_LDS((dds_row_kernel<T, BM, BN, KB>), smem, "dds_row_kernel");
     hipLaunchKernelGGL((dds_row_kernel<T, BM, BN, KB>), dim3(p.M / BM, batch, 1), dim3(256), smem, st, p);
     SPX_LAUNCH_CHECK("dds_row_kernel");
     return 0;
@@ -621,14 +613,8 @@ static int launch_dds_rowq_inst(const DdsParams& p, int batch, hipStream_t st) {
     const size_t smem = (size_t)3 * BN * K * 2 + (size_t)WAVES * 16 * (BN * 2 + 16);
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * (p.M / (16 * WAVES));
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dds_rowq_kernel<T, BN, K, WAVES, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dds_rowq_kernel<T, BN, K, WAVES, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(dds_rowq_kernel)");
-    }
+    SPX_GRANT_LDS((dds_rowq_kernel<T, BN, K, WAVES, true>), smem, "dds_rowq_kernel");
+    SPX_GRANT_LDS((dds_rowq_kernel<T, BN, K, WAVES, false>), smem, "dds_rowq_kernel");
     if (p.bias) hipLaunchKernelGGL((dds_rowq_kernel<T, BN, K, WAVES, true>), dim3((unsigned)groups), dim3(64 * (WAVES + 1)), smem, st, p, batch);
     else hipLaunchKernelGGL((dds_rowq_kernel<T, BN, K, WAVES, false>), dim3((unsigned)groups), dim3(64 * (WAVES + 1)), smem, st, p, batch);
     SPX_LAUNCH_CHECK("dds_rowq_kernel");

@@ -402,11 +402,7 @@ static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, i
     if (n_product + cs_groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)(n_product + cs_groups));
     if (n_product + cs_groups == 0) return 0;
     s.n_product = (int)n_product;
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dds_split_kernel<T, BM, BN, AT, BT>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(dds_split_kernel)");
-    }
+    SPX_GRANT_LDS((dds_split_kernel<T, BM, BN, AT, BT>), smem, "dds_split_kernel");
     hipLaunchKernelGGL((dds_split_kernel<T, BM, BN, AT, BT>), dim3((unsigned)(n_product + cs_groups), batch, 1), dim3(256), smem, st, p, s);
     SPX_LAUNCH_CHECK("dds_split_kernel");
     const int n_blocks = s.slices > 1 ? (int)(((int64_t)s.nnz * BM * BN / 4 + 255) / 256) : 0;

@@ -449,11 +449,7 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
     const int n_list = ((l.n_mtiles * l.parts + 7) / 8) * l.cols;   // the longest of the eight lists
     int n_pos = 32 * per_cu / batch;
     n_pos = n_pos < 1 ? 1 : n_pos > n_list ? n_list : n_pos;
-    if (smem > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-        if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(spmm_ring_kernel)");
-    }
+    SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>), smem, "spmm_ring_kernel");
     hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>), dim3(8 * n_pos, batch, 1), dim3(kRingThreads), smem, st, p, l);
     SPX_LAUNCH_CHECK("spmm_ring_kernel");
     return 0;

@@ -976,9 +976,7 @@ static int launch_moe_direct_inst(const MoeParams& p, hipStream_t st) {
     // the epilogue stages every wavefront's (TM / WGM) x 64 output tile as rows of 128 bytes
     const int epi = sizeof(T) == 2 ? WAVES * (TM / WGM) * 128 : 0;
     const int smem = NBUF * (TM + TN) * KTB > epi ? NBUF * (TM + TN) * KTB : epi;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_gemm_direct_kernel<T, TM, TN, WAVES, WGM, NBUF, KTB, BKN, XS>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(moe_gemm_direct_kernel)");
+    SPX_GRANT_LDS((moe_gemm_direct_kernel<T, TM, TN, WAVES, WGM, NBUF, KTB, BKN, XS>), smem, "moe_gemm_direct_kernel");
     hipLaunchKernelGGL((moe_gemm_direct_kernel<T, TM, TN, WAVES, WGM, NBUF, KTB, BKN, XS>), dim3((p.N + TN - 1) / TN, tiles, 1), dim3(64 * WAVES), smem, st, p);
     SPX_LAUNCH_CHECK("moe_gemm_direct_kernel");
     return 0;

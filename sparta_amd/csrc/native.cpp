@@ -339,6 +339,355 @@ private:
     bool trans_a_, trans_b_, relu_, drop_batch_;
 };
 
+// ---- masked block softmax ----------------------------------------------------------------------
+struct SoftmaxPlan {
+    bool backward;
+    int compressed, batch, H, W, BH, BW;
+    int64_t stride;
+    Tensor row_ptr, idx;
+    std::optional<Tensor> mask;
+    mutable std::atomic<int> tile_cfg;
+    mutable std::atomic<bool> strict{false};
+
+    const char* what() const { return backward ? "spx_softmax_backward" : "spx_softmax_forward"; }
+
+    // forward: a = x; backward: a = gradient of y, y
+    Tensor run(const Tensor& a_in, const Tensor* y_in, double T, at::IntArrayRef out_shape) const {
+        require_numel(what(), backward ? "grad_y" : "x", a_in, batch * stride);
+        if (backward) {
+            require_numel(what(), "y", *y_in, batch * stride);
+            if (a_in.scalar_type() != y_in->scalar_type())
+                assertion("operand dtypes differ: ", a_in.dtype(), " vs ", y_in->dtype());
+        }
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        Tensor out = compressed ? at::empty(out_shape, a_in.options()) : at::zeros(out_shape, a_in.options());
+        if (out.numel() == 0) return out;   // no live block: nothing to compute
+        const int code = dtype_code(a_in);
+        const Tensor a = a_in.contiguous();
+        const Tensor y = backward ? y_in->contiguous() : Tensor();
+        const int32_t *rp = (const int32_t*)device_ptr(row_ptr), *ix = (const int32_t*)device_ptr(idx);
+        const uint8_t* m = (const uint8_t*)device_ptr(mask);
+        int cfg = tile_cfg.load(std::memory_order_relaxed), rc;
+        while (true) {
+            rc = backward ? spx_softmax_backward(code, compressed, device_ptr(a), device_ptr(y), out.data_ptr(), rp, ix, m, (float)T,
+                                                 batch, H, W, BH, BW, stride, cfg, stream_of(a))
+                          : spx_softmax_forward(code, compressed, device_ptr(a), out.data_ptr(), rp, ix, m, (float)T,
+                                                batch, H, W, BH, BW, stride, cfg, stream_of(a));
+            if (rc == SPX_E_CONFIG && cfg && !strict) {   // the configured variant does not take this dtype / block width
+                cfg = 0;
+                tile_cfg.store(0, std::memory_order_relaxed);
+                continue;
+            }
+            break;
+        }
+        check_rc(rc, what());
+        return out;
+    }
+    c10::SmallVector<int64_t, 3> shape() const {
+        if (compressed) return {batch, stride};
+        return {batch, H, W};
+    }
+};
+typedef std::shared_ptr<const SoftmaxPlan> SoftmaxPlanPtr;
+
+class SoftmaxKernel {
+public:
+    void bind(bool backward, int compressed, int batch, int H, int W, int BH, int BW, int64_t stride, Tensor row_ptr, Tensor idx,
+              std::optional<Tensor> mask, int tile_cfg) {
+        auto p = std::make_shared<SoftmaxPlan>();
+        p->backward = backward; p->compressed = compressed; p->batch = batch; p->H = H; p->W = W; p->BH = BH; p->BW = BW;
+        p->stride = stride; p->row_ptr = std::move(row_ptr); p->idx = std::move(idx); p->mask = std::move(mask);
+        p->tile_cfg = tile_cfg;
+        if (p->mask.has_value()) require_numel(p->what(), "mask", *p->mask, stride);
+        plan_ = std::move(p);
+    }
+    void unbind() { plan_.reset(); }
+    void set_strict(bool strict) { if (plan_) plan_->strict = strict; }
+    const SoftmaxPlanPtr& plan() const { return plan_; }
+    static void require_bound(const SoftmaxPlanPtr& p) {
+        if (!p) throw ValueFailure("The kernel is not compiled.");
+    }
+    Tensor forward(const Tensor& x, double T) const {
+        const SoftmaxPlanPtr p = plan_;
+        require_bound(p);
+        py::gil_scoped_release nogil;
+        return p->run(x, nullptr, T, p->shape());
+    }
+    Tensor backward(const Tensor& grad, const Tensor& y, double T) const {
+        const SoftmaxPlanPtr p = plan_;
+        require_bound(p);
+        py::gil_scoped_release nogil;
+        return p->run(grad, &y, T, p->shape());
+    }
+
+private:
+    SoftmaxPlanPtr plan_;
+};
+
+struct SoftmaxBackward : public Node {
+    SoftmaxPlanPtr bwd;
+    bool have;
+    double T;
+    SavedVariable y;
+    std::vector<int64_t> x_shape;
+
+    variable_list apply(variable_list&& grads) override {
+        return with_python_errors([&]() -> variable_list {
+            variable_list out(1);
+            if (!grads[0].defined() || !task_should_compute_output(0)) return out;
+            if (!have) throw AttributeFailure("the operator was built without its backward kernel");
+            SoftmaxKernel::require_bound(bwd);
+            at::AutoGradMode no_grad(false);
+            const Tensor value = y.unpack(shared_from_this());
+            out[0] = bwd->run(grads[0], &value, T, x_shape);
+            return out;
+        });
+    }
+    void release_variables() override { y.reset_data(); }
+    std::string name() const override { return "SparseSoftmaxBackward"; }
+};
+
+class SoftmaxOp {
+public:
+    SoftmaxOp(std::shared_ptr<SoftmaxKernel> fwd, std::shared_ptr<SoftmaxKernel> bwd) : fwd_(std::move(fwd)), bwd_(std::move(bwd)) {}
+    Tensor call(const Tensor& x, double T) const {
+        const SoftmaxPlanPtr p = fwd_->plan(), pb = bwd_ ? bwd_->plan() : nullptr;
+        SoftmaxKernel::require_bound(p);
+        py::gil_scoped_release nogil;
+        Tensor y = p->run(x, nullptr, T, p->shape());
+        if (!records({&x})) return y;
+        auto node = std::shared_ptr<SoftmaxBackward>(new SoftmaxBackward(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(x));
+        node->bwd = pb;
+        node->have = (bool)bwd_;
+        node->T = T;
+        node->x_shape = x.sizes().vec();
+        torch::autograd::set_history(y, node);
+        node->y = SavedVariable(y, true);
+        return y;
+    }
+    std::unique_ptr<SoftmaxOp> deepcopy(const py::object& memo) const {
+        const py::object copy = py::module_::import("copy").attr("deepcopy");
+        auto kernel = [&](const std::shared_ptr<SoftmaxKernel>& k) {
+            return k ? copy(py::cast(k), memo).cast<std::shared_ptr<SoftmaxKernel>>() : nullptr;
+        };
+        return std::make_unique<SoftmaxOp>(kernel(fwd_), kernel(bwd_));
+    }
+
+private:
+    std::shared_ptr<SoftmaxKernel> fwd_, bwd_;
+};
+
+// ---- fused attention -------------------------------------------------------------------------------
+// The fused kernels over one index: launches with their operand checks and allocations.
+class AttentionKernel {
+public:
+    AttentionKernel(Tensor row_ptr, Tensor bcsr, std::optional<Tensor> col_ptr, std::optional<Tensor> bcsc,
+                    std::optional<Tensor> mask, double inv_temperature, int Nt, int Ns, int BH, int BW)
+        : row_ptr_(std::move(row_ptr)), bcsr_(std::move(bcsr)), col_ptr_(std::move(col_ptr)), bcsc_(std::move(bcsc)),
+          mask_(std::move(mask)), inv_t_((float)inv_temperature), Nt_(Nt), Ns_(Ns), BH_(BH), BW_(BW) {}
+
+    // (output, tile configuration that ran)
+    std::pair<Tensor, int> forward(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, int tile_cfg, bool strict) const {
+        py::gil_scoped_release nogil;
+        const Dims d = dims("spx_attention_forward", q_in, k_in, v_in);
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        const Tensor q = q_in.contiguous(), k = k_in.contiguous(), v = v_in.contiguous();
+        Tensor out = at::empty(q.sizes(), q.options());
+        int rc;
+        while (true) {
+            rc = spx_attention_forward(d.code, device_ptr(q), device_ptr(k), device_ptr(v), out.data_ptr(), rows(), entries(),
+                                       (const uint8_t*)device_ptr(mask_), inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_, tile_cfg, stream_of(q));
+            if (rc == SPX_E_CONFIG && tile_cfg && !strict) {   // a tuned variant that does not take these shapes
+                tile_cfg = 0;
+                continue;
+            }
+            break;
+        }
+        check_rc(rc, "spx_attention_forward");
+        return {out, tile_cfg};
+    }
+    // (output, log-sum-exp of every score row)
+    std::pair<Tensor, Tensor> forward_lse(const Tensor& q, const Tensor& k, const Tensor& v) const {
+        py::gil_scoped_release nogil;
+        const Dims d = dims("spx_attention_forward_lse", q, k, v);
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        Tensor out = at::empty(q.sizes(), q.options()), lse = at::empty({d.batch, Nt_}, q.options().dtype(at::kFloat));
+        check_rc(spx_attention_forward_lse(d.code, contig(q), contig(k), contig(v), out.data_ptr(), (float*)lse.data_ptr(),
+                                           rows(), entries(), nullptr, inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_, stream_of(q)),
+                 "spx_attention_forward_lse");
+        return {out, lse};
+    }
+    // (query gradient, row constants)
+    std::pair<Tensor, Tensor> backward_q(const Tensor& grad, const Tensor& out, const Tensor& q, const Tensor& k, const Tensor& v,
+                                         const Tensor& lse) const {
+        py::gil_scoped_release nogil;
+        const char* what = "spx_attention_backward_q";
+        const Dims d = dims(what, q, k, v);
+        require_like(what, "grad_out", grad, q);
+        require_like(what, "out", out, q);
+        require_numel(what, "row_lse", lse, (int64_t)d.batch * Nt_);
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        Tensor grad_q = at::empty(q.sizes(), q.options()), dot = at::empty({d.batch, Nt_}, q.options().dtype(at::kFloat));
+        check_rc(spx_attention_backward_q(d.code, contig(grad), contig(out), contig(q), contig(k), contig(v), (const float*)contig(lse),
+                                          grad_q.data_ptr(), (float*)dot.data_ptr(), rows(), entries(), inv_t_, d.batch, Nt_, Ns_,
+                                          d.E, BH_, BW_, stream_of(q)), what);
+        return {grad_q, dot};
+    }
+    // (key gradient, value gradient)
+    std::pair<Tensor, Tensor> backward_kv(const Tensor& grad, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& lse,
+                                          const Tensor& dot) const {
+        py::gil_scoped_release nogil;
+        const char* what = "spx_attention_backward_kv_recompute";
+        const Dims d = dims(what, q, k, v);
+        require_like(what, "grad_out", grad, q);
+        require_numel(what, "row_lse", lse, (int64_t)d.batch * Nt_);
+        require_numel(what, "row_dot", dot, (int64_t)d.batch * Nt_);
+        if (!col_ptr_.has_value() || !bcsc_.has_value()) throw ValueFailure("the column-side kernel needs the BCSC index");
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        Tensor grad_k = at::empty(k.sizes(), k.options()), grad_v = at::empty(k.sizes(), k.options());
+        check_rc(spx_attention_backward_kv_recompute(
+                     d.code, contig(grad), contig(q), contig(k), contig(v), (const float*)contig(lse), (const float*)contig(dot),
+                     grad_k.data_ptr(), grad_v.data_ptr(), (const int32_t*)device_ptr(col_ptr_), device_ptr(bcsc_),
+                     bcsc_->scalar_type() == at::kLong ? SPX_IDX_BCSC_I64 : SPX_IDX_BCSC_I32, inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_,
+                     stream_of(q)), what);
+        return {grad_k, grad_v};
+    }
+
+private:
+    struct Dims {
+        int code, batch, E;
+    };
+    // the tensors behind the pointers against what a kernel walks; AssertionError before any launch
+    Dims dims(const char* what, const Tensor& q, const Tensor& k, const Tensor& v) const {
+        if (q.dim() < 2) assertion(what, ": query of shape ", q.sizes());
+        const int64_t E = q.size(-1);
+        const int64_t per = (int64_t)Nt_ * E;
+        int64_t batch = 1;
+        for (int64_t i = 0; i < q.dim() - 2; ++i) batch *= q.size(i);
+        require_numel(what, "q", q, batch * per);
+        require_numel(what, "k", k, batch * Ns_ * E);
+        require_numel(what, "v", v, batch * Ns_ * E);
+        if (k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type())
+            assertion(what, ": operand dtypes differ: ", q.dtype(), ", ", k.dtype(), ", ", v.dtype());
+        return {dtype_code(q), (int)batch, (int)E};
+    }
+    static void require_like(const char* what, const char* name, const Tensor& t, const Tensor& q) {
+        require_numel(what, name, t, q.numel());
+        if (t.scalar_type() != q.scalar_type()) assertion(what, ": operand dtypes differ: ", name, " is ", t.dtype());
+    }
+    static void* contig(const Tensor& t) {
+        if (!t.is_contiguous()) throw ValueFailure("sparta_amd kernels need contiguous tensors");
+        return device_ptr(t);
+    }
+    const int32_t* rows() const { return (const int32_t*)device_ptr(row_ptr_); }
+    const int32_t* entries() const { return (const int32_t*)device_ptr(bcsr_); }
+
+    Tensor row_ptr_, bcsr_;
+    std::optional<Tensor> col_ptr_, bcsc_, mask_;
+    float inv_t_;
+    int Nt_, Ns_, BH_, BW_;
+};
+
+Tensor seqlen_attention(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& lens_in) {
+    py::gil_scoped_release nogil;
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    const Tensor q = q_in.contiguous(), k = k_in.contiguous(), v = v_in.contiguous(), lens = lens_in.contiguous();
+    Tensor out = at::empty(q.sizes(), q.options());
+    check_rc(spx_attention_seqlen_forward(dtype_code(q), device_ptr(q), device_ptr(k), device_ptr(v), out.data_ptr(),
+                                          (const int32_t*)device_ptr(lens), 1.0f, (int)q.size(0), (int)q.size(1), (int)q.size(2),
+                                          (int)q.size(3), 0, stream_of(q)), "spx_attention_seqlen_forward");
+    return out;
+}
+
+// ---- mixture of experts ----------------------------------------------------------------------------
+// Token index and gathered product of one call: (output, tile configuration that ran).  The caller
+// has checked the sizes.
+std::pair<Tensor, int> moe_forward(const Tensor& tokens_in, const Tensor& ids_in, const Tensor& weight_in, const Tensor& count, const Tensor& offset,
+                   const Tensor& perm, const Tensor& workspace, int tile_cfg, bool strict) {
+    py::gil_scoped_release nogil;
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    const Tensor tokens = tokens_in.contiguous(), ids = ids_in.to(at::kInt).contiguous();
+    const Tensor weight = weight_in.to(tokens.scalar_type()).contiguous();
+    const int n_tok = (int)tokens.size(0), E = (int)weight.size(0), in = (int)weight.size(1), out_dim = (int)weight.size(2);
+    const int32_t *off = (const int32_t*)device_ptr(offset), *pm = (const int32_t*)device_ptr(perm);
+    check_rc(spx_moe_index((const int32_t*)device_ptr(ids), n_tok, E, (int32_t*)device_ptr(count), (int32_t*)off, (int32_t*)pm,
+                           device_ptr(workspace), workspace.numel(), stream_of(tokens)), "spx_moe_index");
+    Tensor out = at::empty({n_tok, out_dim}, tokens.options());
+    int rc;
+    while (true) {
+        rc = spx_moe_forward(dtype_code(tokens), device_ptr(tokens), device_ptr(weight), 0, out.data_ptr(), off, pm, n_tok, in, out_dim, E,
+                             tile_cfg, stream_of(tokens));
+        if (rc == SPX_E_CONFIG && tile_cfg && !strict) {   // a tuned variant that does not take this dtype
+            tile_cfg = 0;
+            continue;
+        }
+        break;
+    }
+    check_rc(rc, "spx_moe_forward");
+    return {out, tile_cfg};
+}
+
+// ---- index build -------------------------------------------------------------------------------------
+// Buffers of several index builds and the launches that fill them.  A request: (mask as contiguous bytes,
+// block height, block width, BCSR wanted, BCSC wanted, capacity or -1, scratch bytes).  An answer:
+// (row_ptr, bcsr, row_order, col_ptr, bcsc, col_order, nnz), None where a format is not wanted.
+typedef std::tuple<Tensor, int, int, bool, bool, int64_t, int64_t> IndexRequest;
+
+std::vector<py::tuple> build_indexes(const std::vector<IndexRequest>& requests) {
+    struct Built {
+        std::optional<Tensor> row_ptr, bcsr, row_order, col_ptr, bcsc, col_order;
+        Tensor nnz, scratch;
+    };
+    std::vector<Built> built(requests.size());
+    if (!requests.empty()) {
+        py::gil_scoped_release nogil;
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        const Tensor& first = std::get<0>(requests[0]);
+        device_ptr(first);   // refuses CPU tensors
+        c10::DeviceGuard guard(first.device());
+        std::vector<spx_bcs_index_job> jobs(requests.size());
+        for (size_t i = 0; i < requests.size(); ++i) {
+            const auto& [mask, BH, BW, want_r, want_c, cap_in, ws_bytes] = requests[i];
+            const int H = (int)mask.size(0), W = (int)mask.size(1), R = H / BH, C = W / BW;
+            const int64_t cap = cap_in < 0 ? (int64_t)R * C : cap_in;
+            const auto i32 = mask.options().dtype(at::kInt);
+            Built& b = built[i];
+            spx_bcs_index_job& job = jobs[i];
+            job = spx_bcs_index_job();
+            b.nnz = at::empty({1}, i32);
+            b.scratch = at::empty({ws_bytes}, mask.options().dtype(at::kByte));
+            if (want_r) {
+                b.row_ptr = at::empty({R + 1}, i32);
+                b.bcsr = at::empty({cap}, i32);
+                b.row_order = at::empty({R}, i32);   // the launch orders of the matmul kernels
+                job.row_ptr = (int32_t*)b.row_ptr->data_ptr();
+                job.bcsr_idx = (int32_t*)b.bcsr->data_ptr();
+                job.row_order = (int32_t*)b.row_order->data_ptr();
+            }
+            if (want_c) {
+                b.col_ptr = at::empty({C + 1}, i32);
+                b.bcsc = at::empty({cap}, want_r ? i32.dtype(at::kLong) : i32);
+                b.col_order = at::empty({C}, i32);   // come out of the same launch
+                job.col_ptr = (int32_t*)b.col_ptr->data_ptr();
+                job.bcsc_idx = b.bcsc->data_ptr();
+                job.col_order = (int32_t*)b.col_order->data_ptr();
+            }
+            job.mask = (const uint8_t*)device_ptr(mask);
+            job.H = H; job.W = W; job.BH = BH; job.BW = BW;
+            job.bcsc_i64 = want_r && want_c;
+            job.nnz_dev = (int32_t*)b.nnz.data_ptr();
+            job.cap = (int)cap;
+            job.workspace = b.scratch.data_ptr();
+            job.workspace_bytes = (size_t)ws_bytes;
+        }
+        check_rc(spx_bcs_index_batch(jobs.data(), (int)jobs.size(), stream_of(first)), "spx_bcs_index_batch");
+    }
+    std::vector<py::tuple> out;
+    for (Built& b : built) out.push_back(py::make_tuple(b.row_ptr, b.bcsr, b.row_order, b.col_ptr, b.bcsc, b.col_order, b.nnz));
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
@@ -365,4 +714,26 @@ PYBIND11_MODULE(_native, m) {
         .def(py::init<std::shared_ptr<MatmulKernel>, std::shared_ptr<MatmulKernel>, std::shared_ptr<MatmulKernel>, bool, bool, bool, bool>())
         .def("__call__", &MatmulOp::call, py::arg("A"), py::arg("B"), py::arg("bias") = py::none())
         .def("__deepcopy__", &MatmulOp::deepcopy);
+    py::class_<SoftmaxKernel, std::shared_ptr<SoftmaxKernel>>(m, "SoftmaxKernel")
+        .def(py::init<>())
+        .def("bind", &SoftmaxKernel::bind)
+        .def("unbind", &SoftmaxKernel::unbind)
+        .def("set_strict", &SoftmaxKernel::set_strict)
+        .def("__deepcopy__", [](const SoftmaxKernel& k, const py::object&) { return std::make_shared<SoftmaxKernel>(k); })
+        .def("__call__", &SoftmaxKernel::forward, py::arg("x"), py::arg("T"))
+        .def("__call__", &SoftmaxKernel::backward, py::arg("grad_y"), py::arg("y"), py::arg("T"));
+    py::class_<SoftmaxOp>(m, "SoftmaxOp")
+        .def(py::init<std::shared_ptr<SoftmaxKernel>, std::shared_ptr<SoftmaxKernel>>())
+        .def("__call__", &SoftmaxOp::call, py::arg("x"), py::arg("T"))
+        .def("__deepcopy__", &SoftmaxOp::deepcopy);
+    py::class_<AttentionKernel, std::shared_ptr<AttentionKernel>>(m, "AttentionKernel")
+        .def(py::init<Tensor, Tensor, std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>, double, int, int, int, int>())
+        .def("forward", &AttentionKernel::forward)
+        .def("forward_lse", &AttentionKernel::forward_lse)
+        .def("backward_q", &AttentionKernel::backward_q)
+        .def("backward_kv", &AttentionKernel::backward_kv)
+        .def("__deepcopy__", [](const AttentionKernel& k, const py::object&) { return std::make_shared<AttentionKernel>(k); });
+    m.def("seqlen_attention", &seqlen_attention);
+    m.def("moe_forward", &moe_forward);
+    m.def("build_indexes", &build_indexes);
 }

@@ -7,6 +7,7 @@ from typing import Any, Dict, List, Optional
 import numpy as np
 import torch
 
+from sparta_amd import _lib
 from sparta_amd.specializer.kernels import (
     SparTASparseSoftmaxForwardKernel, SparTASparseSoftmaxBackwardKernel,
 )
@@ -46,6 +47,12 @@ class SparseBatchSoftmaxCtx(SparseCtxBase):
         bwd = self._kernels['backward:x'].active_kernel()
         if bwd is not None:
             self.backward = lambda grad, output: bwd(grad, output, self._T)
+        if fwd is not None:
+            # the launch objects and the autograd node that connects them
+            self._operator = _lib.native().SoftmaxOp(fwd._func, None if bwd is None else bwd._func)
+
+    def apply(self, x: torch.Tensor) -> torch.Tensor:
+        return self._operator(x, self._T)
 
     def set_sample_inputs(self, sample_inputs: List[torch.Tensor],
                           sample_grads: Optional[List[torch.Tensor]] = None):
@@ -69,16 +76,10 @@ class SparseBatchSoftmaxCtx(SparseCtxBase):
         return self._kernels['forward:y'].dense_func(*args, self._T)
 
 
-class SparseBatchSoftmaxFunc(torch.autograd.Function):
+class SparseBatchSoftmaxFunc:
+    """y = masked softmax of x with its gradient: the autograd node is part of the native operator
+    object that the context holds once it is built."""
 
     @staticmethod
-    def forward(ctx, sparta_ctx: SparseBatchSoftmaxCtx, x: torch.Tensor):
-        ctx.sparta_ctx = sparta_ctx
-        y = sparta_ctx.forward(x.detach())
-        ctx.save_for_backward(y)
-        return y
-
-    @staticmethod
-    def backward(ctx, grad: torch.Tensor):
-        y, = ctx.saved_tensors
-        return None, ctx.sparta_ctx.backward(grad.detach().contiguous(), y.detach())
+    def apply(sparta_ctx: SparseBatchSoftmaxCtx, x: torch.Tensor) -> torch.Tensor:
+        return sparta_ctx.apply(x)

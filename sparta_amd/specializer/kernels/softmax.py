@@ -11,7 +11,6 @@ import torch
 from sparta_amd import _lib
 from sparta_amd.common.tuning import TunableItemCfg
 from sparta_amd.specializer.kernels.kernel_base import KernelBase, PortConfig
-from sparta_amd.specializer.kernels.operand_sizes import require_numel
 from sparta_amd.testing import sparse_softmax_forward_reference, sparse_softmax_backward_reference
 
 
@@ -24,6 +23,7 @@ class SparseSoftmaxKernel(KernelBase):
         self._compressed = compressed
         self._dtype = dtype
         super().__init__()
+        self._func = _lib.native().SoftmaxKernel()
 
     def _add_parameters(self):
         for name in ('BATCH_SIZE', 'GLOBAL_H_VALUE', 'GLOBAL_W_VALUE'):
@@ -53,8 +53,8 @@ class SparseSoftmaxKernel(KernelBase):
     def sparse_block_shape(self):
         return self.ports['y'], self.get_block_shape()
 
-    def _launch_state(self):
-        """Everything a launch closure needs, resolved once per update_func()."""
+    def update_func(self):
+        """Bind the native launch object to the current shape, index and element mask."""
         batch_size, H, W = self.get_shape()
         BH, BW = self.get_block_shape()
         indexes = self.ports['y'].indexes
@@ -76,7 +76,8 @@ class SparseSoftmaxKernel(KernelBase):
             # short rows (known from the live block count): sixteen lanes per row
             if indexes.block_nnz * BW <= 410 * max(indexes.row_num, 1):
                 tile_cfg = 3
-        return batch_size, H, W, BH, BW, indexes, mask, shape, stride, tile_cfg
+        self._func.bind(self.__direction__ == 'backward', self._compressed, batch_size, H, W, BH, BW, stride,
+                        indexes.row_ptr, indexes._bcsr_buf, mask, tile_cfg)
 
     def _mask_and_compress(self, tensors: List[torch.Tensor], positions: List[int]):
         mask = self.ports['y'].mask
@@ -94,38 +95,6 @@ class SparseSoftmaxForwardKernel(SparseSoftmaxKernel):
         self.ports['x'] = PortConfig(name='x', is_input=True, is_sparse=True, BCSR=True)
         self.ports['y'] = PortConfig(name='y', is_input=False, is_sparse=True, BCSR=True)
         self.ports['x'].connect(self, 'y')
-
-    def update_func(self):
-        batch_size, H, W, BH, BW, indexes, mask, shape, stride, tile_cfg = self._launch_state()
-        compressed = int(self._compressed)
-        alloc = torch.empty if self._compressed else torch.zeros
-        row_ptr, idx = indexes.row_ptr, indexes._bcsr_buf
-        lib = _lib.load()
-
-        numel = batch_size * stride
-        tile = [tile_cfg]
-        if mask is not None:
-            require_numel('spx_softmax_forward', 'mask', mask, stride)
-
-        def softmax_forward_func(x: torch.Tensor, T: np.float32):
-            require_numel('spx_softmax_forward', 'x', x, numel)
-            y = alloc(shape, dtype=x.dtype, device=x.device)
-            if y.numel() == 0:  # no live block: nothing to compute
-                return y
-            x = x.contiguous()
-            while True:
-                rc = lib.spx_softmax_forward(
-                    _lib.dtype_code(x.dtype), compressed, _lib.dev_ptr(x), _lib.dev_ptr(y),
-                    _lib.dev_ptr(row_ptr), _lib.dev_ptr(idx), _lib.dev_ptr(mask), float(T),
-                    batch_size, H, W, BH, BW, stride, tile[0], _lib.current_stream(x.device))
-                if rc == _lib.E_CONFIG and tile[0] and not self._tile_strict:
-                    tile[0] = 0   # the configured variant does not take this dtype / block width
-                    continue
-                break
-            _lib.check(rc, 'spx_softmax_forward')
-            return y
-
-        self._func = softmax_forward_func
 
     def _convert_data(self, inputs, outputs):
         self._mask_and_compress(inputs, [0])
@@ -146,40 +115,6 @@ class SparseSoftmaxBackwardKernel(SparseSoftmaxKernel):
         self.ports['grad_x'] = PortConfig(name='grad_x', is_input=False, is_sparse=True, BCSR=True)
         self.ports['grad_y'].connect(self, 'y')
         self.ports['grad_y'].connect(self, 'grad_x')
-
-    def update_func(self):
-        batch_size, H, W, BH, BW, indexes, mask, shape, stride, tile_cfg = self._launch_state()
-        compressed = int(self._compressed)
-        alloc = torch.empty if self._compressed else torch.zeros
-        row_ptr, idx = indexes.row_ptr, indexes._bcsr_buf
-        lib = _lib.load()
-
-        numel = batch_size * stride
-        tile = [tile_cfg]
-        if mask is not None:
-            require_numel('spx_softmax_backward', 'mask', mask, stride)
-
-        def softmax_backward_func(grad_y: torch.Tensor, y: torch.Tensor, T: np.float32):
-            require_numel('spx_softmax_backward', 'grad_y', grad_y, numel)
-            require_numel('spx_softmax_backward', 'y', y, numel)
-            assert grad_y.dtype == y.dtype, f'operand dtypes differ: {grad_y.dtype} vs {y.dtype}'
-            grad_x = alloc(shape, dtype=grad_y.dtype, device=grad_y.device)
-            if grad_x.numel() == 0:
-                return grad_x
-            grad_y, y = grad_y.contiguous(), y.contiguous()
-            while True:
-                rc = lib.spx_softmax_backward(
-                    _lib.dtype_code(grad_y.dtype), compressed, _lib.dev_ptr(grad_y), _lib.dev_ptr(y), _lib.dev_ptr(grad_x),
-                    _lib.dev_ptr(row_ptr), _lib.dev_ptr(idx), _lib.dev_ptr(mask), float(T),
-                    batch_size, H, W, BH, BW, stride, tile[0], _lib.current_stream(grad_y.device))
-                if rc == _lib.E_CONFIG and tile[0] and not self._tile_strict:
-                    tile[0] = 0
-                    continue
-                break
-            _lib.check(rc, 'spx_softmax_backward')
-            return grad_x
-
-        self._func = softmax_backward_func
 
     def _convert_data(self, inputs, outputs):
         self._mask_and_compress(inputs, [0, 1])

@@ -44,7 +44,6 @@ class SeqlenDynamicSparseAttention(torch.nn.Module):
 
     def forward(self, Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor,
                 seqlens: Optional[torch.Tensor] = None) -> torch.Tensor:
-        Q, K, V = Q.contiguous(), K.contiguous(), V.contiguous()
         if self.global_mode:
             seqlens = SeqlenDynamicSparseAttention.global_seqlen
         assert seqlens is not None, 'no sequence lengths: pass seqlens or call set_global_seqlens'
@@ -54,9 +53,4 @@ class SeqlenDynamicSparseAttention(torch.nn.Module):
         assert B == seqlens.size(0)
         assert N % 32 == 0, 'max sequence length should be divisible by 32'
         assert E % 32 == 0, 'embed dimension size should be divisible by 32'
-        out = torch.empty_like(Q)
-        rc = _lib.load().spx_attention_seqlen_forward(
-            _lib.dtype_code(Q.dtype), _lib.dev_ptr(Q), _lib.dev_ptr(K), _lib.dev_ptr(V), _lib.dev_ptr(out),
-            _lib.dev_ptr(seqlens.contiguous()), 1.0, B, H, N, E, 0, _lib.current_stream(Q.device))
-        _lib.check(rc, 'spx_attention_seqlen_forward')
-        return out
+        return _lib.native().seqlen_attention(Q, K, V, seqlens)

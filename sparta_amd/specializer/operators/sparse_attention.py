@@ -129,6 +129,8 @@ class SparseAttention(OperatorBase):
         self._fused_tile_cfg = int(fused_tile_cfg)
         self._fused_mask_key = None   # index object the cached element mask belongs to
         self._fused_mask = None
+        self._launch_key = None       # row pointers of the index the launch object below is bound to
+        self._launch = None
         self._inv_temperature = 1.0
         self._warned_unfused = False
         self._tile_strict = False   # True while tune_tile_config times a variant: a refusal must show
@@ -195,57 +197,33 @@ class SparseAttention(OperatorBase):
                 if tensor is not None:
                     require_numel(what, name, tensor, numel)
 
+    def _launcher(self, indexes=None):
+        """The native launches over `indexes` (the operator's current index by default)."""
+        if indexes is None:
+            indexes = self._sparse_port.indexes
+        if self._launch_key is indexes.row_ptr:
+            return self._launch
+        check_index_matches('the fused attention kernels', indexes, self._Nt, self._Ns)
+        current = indexes is self._sparse_port.indexes
+        launch = _lib.native().AttentionKernel(
+            indexes.row_ptr, indexes._bcsr_buf, getattr(indexes, 'col_ptr', None), getattr(indexes, '_bcsc_buf', None),
+            self._element_mask() if current else None, self._inv_temperature, self._Nt, self._Ns,
+            indexes.block_H, indexes.block_W)
+        if current:
+            self._launch_key, self._launch = indexes.row_ptr, launch
+        return launch
+
     def _fused_forward_lse(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
         """(output, log-sum-exp per query) from spx_attention_forward_lse."""
-        indexes = self._sparse_port.indexes
-        batch, _, E = q.shape
-        out = torch.empty_like(q)
-        row_lse = torch.empty((batch, self._Nt), dtype=torch.float32, device=q.device)
-        self._check_operands('spx_attention_forward_lse', indexes, batch, E, q_like=[('q', q)],
-                             kv_like=[('k', k), ('v', v)], nnz=0)
-        rc = _lib.load().spx_attention_forward_lse(
-            _lib.dtype_code(q.dtype), _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v), _lib.dev_ptr(out),
-            _lib.dev_ptr(row_lse), _lib.dev_ptr(indexes.row_ptr), _lib.dev_ptr(indexes._bcsr_buf), None,
-            float(self._inv_temperature), batch, self._Nt, self._Ns, E, indexes.block_H, indexes.block_W,
-            _lib.current_stream(q.device))
-        _lib.check(rc, 'spx_attention_forward_lse')
-        return out, row_lse
+        return self._launcher().forward_lse(q, k, v)
 
     def _recompute_backward_q(self, grad_out, out, q, k, v, row_lse, indexes=None):
         """(query gradient, row constants) from spx_attention_backward_q."""
-        indexes = self._sparse_port.indexes if indexes is None else indexes
-        batch, _, E = grad_out.shape
-        grad_q = torch.empty_like(q)
-        row_dot = torch.empty((batch, self._Nt), dtype=torch.float32, device=q.device)
-        self._check_operands('spx_attention_backward_q', indexes, batch, E,
-                             q_like=[('grad_out', grad_out), ('out', out), ('q', q)],
-                             kv_like=[('k', k), ('v', v)], rows=[('row_lse', row_lse)], nnz=0)
-        rc = _lib.load().spx_attention_backward_q(
-            _lib.dtype_code(q.dtype), _lib.dev_ptr(grad_out), _lib.dev_ptr(out), _lib.dev_ptr(q), _lib.dev_ptr(k),
-            _lib.dev_ptr(v), _lib.dev_ptr(row_lse), _lib.dev_ptr(grad_q), _lib.dev_ptr(row_dot),
-            _lib.dev_ptr(indexes.row_ptr), _lib.dev_ptr(indexes._bcsr_buf), float(self._inv_temperature),
-            batch, self._Nt, self._Ns, E, indexes.block_H, indexes.block_W, _lib.current_stream(q.device))
-        _lib.check(rc, 'spx_attention_backward_q')
-        return grad_q, row_dot
+        return self._launcher(indexes).backward_q(grad_out, out, q, k, v, row_lse)
 
     def _recompute_backward_kv(self, grad_out, q, k, v, row_lse, row_dot, indexes=None):
         """(key gradient, value gradient) from spx_attention_backward_kv_recompute."""
-        indexes = self._sparse_port.indexes if indexes is None else indexes
-        batch, _, E = grad_out.shape
-        grad_k = torch.empty_like(k)
-        grad_v = torch.empty_like(v)
-        idx = indexes._bcsc_buf
-        kind = _lib.IDX_BCSC_I64 if idx.dtype == torch.int64 else _lib.IDX_BCSC_I32
-        self._check_operands('spx_attention_backward_kv_recompute', indexes, batch, E,
-                             q_like=[('grad_out', grad_out), ('q', q)], kv_like=[('k', k), ('v', v)],
-                             rows=[('row_lse', row_lse), ('row_dot', row_dot)], nnz=0)
-        rc = _lib.load().spx_attention_backward_kv_recompute(
-            _lib.dtype_code(q.dtype), _lib.dev_ptr(grad_out), _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v),
-            _lib.dev_ptr(row_lse), _lib.dev_ptr(row_dot), _lib.dev_ptr(grad_k), _lib.dev_ptr(grad_v),
-            _lib.dev_ptr(indexes.col_ptr), _lib.dev_ptr(idx), kind, float(self._inv_temperature),
-            batch, self._Nt, self._Ns, E, indexes.block_H, indexes.block_W, _lib.current_stream(q.device))
-        _lib.check(rc, 'spx_attention_backward_kv_recompute')
-        return grad_k, grad_v
+        return self._launcher(indexes).backward_kv(grad_out, q, k, v, row_lse, row_dot)
 
     def _element_mask(self):
         indexes = self._sparse_port.indexes
@@ -332,26 +310,8 @@ class SparseAttention(OperatorBase):
                 and indexes.block_H in (16, 32, 64, 128) and indexes.block_W in (16, 32, 64, 128))
 
     def _fused_forward(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor):
-        indexes = self._sparse_port.indexes
-        self._element_mask()
-        lead = query.shape[:-2]
-        E = query.shape[-1]
-        batch = int(np.prod(lead)) if len(lead) else 1
-        q, k, v = query.contiguous(), key.contiguous(), value.contiguous()
-        out = torch.empty_like(q)
-        self._check_operands('spx_attention_forward', indexes, batch, E, q_like=[('q', q)],
-                             kv_like=[('k', k), ('v', v)], nnz=0)
-        while True:
-            rc = _lib.load().spx_attention_forward(
-                _lib.dtype_code(q.dtype), _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v), _lib.dev_ptr(out),
-                _lib.dev_ptr(indexes.row_ptr), _lib.dev_ptr(indexes._bcsr_buf), _lib.dev_ptr(self._fused_mask),
-                float(self._inv_temperature), batch, self._Nt, self._Ns, E,
-                indexes.block_H, indexes.block_W, self._fused_tile_cfg, _lib.current_stream(q.device))
-            if rc == _lib.E_CONFIG and self._fused_tile_cfg and not self._tile_strict:
-                self._fused_tile_cfg = 0   # a tuned variant that does not take these shapes: the library's choice
-                continue
-            break
-        _lib.check(rc, 'spx_attention_forward')
+        # a tuned variant that does not take these shapes gives way to the library's choice
+        out, self._fused_tile_cfg = self._launcher().forward(query, key, value, self._fused_tile_cfg, self._tile_strict)
         return out
 
     # ---- masks -----------------------------------------------------------------------
@@ -381,6 +341,7 @@ class SparseAttention(OperatorBase):
     def _set_temperature(self, E: int):
         self._softmax.set_temperature(np.sqrt(E))
         self._inv_temperature = 1.0 / float(np.sqrt(E))
+        self._launch_key = self._launch = None
 
     def build(self, config: Dict[str, Any], sample_inputs: List[torch.Tensor]):
         query, key, value = sample_inputs

@@ -50,38 +50,17 @@ class DynamicSparseMoE(torch.nn.Module):
         # the kernel walks num_exps matrices of in_hidden x out_hidden behind the weight pointer
         assert self.weight.numel() == self.num_exps * self.in_hidden * self.out_hidden, \
             f'the weight has shape {tuple(self.weight.shape)}, expected ({self.num_exps}, {self.in_hidden}, {self.out_hidden})'
-        if exp_ids.dtype != torch.int32:
-            exp_ids = exp_ids.to(torch.int32)
         if self.sparse_index.numel() < n_tok:
             self.sparse_index = torch.empty(n_tok, dtype=torch.int32, device=tokens.device)
-        lib = _lib.load()
-        ws_bytes = lib.spx_moe_index_workspace_bytes(n_tok, self.num_exps)
+        ws_bytes = _lib.load().spx_moe_index_workspace_bytes(n_tok, self.num_exps)
         if self._workspace.numel() < ws_bytes:
             self._workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=tokens.device)
-        stream = _lib.current_stream(tokens.device)
-        rc = lib.spx_moe_index(_lib.dev_ptr(exp_ids.contiguous()), n_tok, self.num_exps,
-                               _lib.dev_ptr(self.expert_count), _lib.dev_ptr(self.expert_offset),
-                               _lib.dev_ptr(self.sparse_index), _lib.dev_ptr(self._workspace),
-                               self._workspace.numel(), stream)
-        _lib.check(rc, 'spx_moe_index')
-        tokens = tokens.contiguous()
-        out = torch.empty((n_tok, self.out_hidden), dtype=tokens.dtype, device=tokens.device)
         # the stacked [n_exp, in, out] parameter is what the kernel reads (weight layout 0):
-        # there is no second copy that could go stale when the parameter is written to
-        weight = self.weight.detach()
-        if weight.dtype != tokens.dtype:
-            weight = weight.to(tokens.dtype)
-        weight = weight.contiguous()
-        while True:
-            rc = lib.spx_moe_forward(_lib.dtype_code(tokens.dtype), _lib.dev_ptr(tokens),
-                                     _lib.dev_ptr(weight), 0, _lib.dev_ptr(out),
-                                     _lib.dev_ptr(self.expert_offset), _lib.dev_ptr(self.sparse_index),
-                                     n_tok, self.in_hidden, self.out_hidden, self.num_exps, self.tile_cfg, stream)
-            if rc == _lib.E_CONFIG and self.tile_cfg and not self._tile_strict:
-                self.tile_cfg = 0   # a tuned variant that does not take this dtype: the library's choice
-                continue
-            break
-        _lib.check(rc, 'spx_moe_forward')
+        # there is no second copy that could go stale when the parameter is written to.  A tuned
+        # variant that does not take this dtype gives way to the library's choice.
+        out, self.tile_cfg = _lib.native().moe_forward(
+            tokens, exp_ids, self.weight, self.expert_count, self.expert_offset, self.sparse_index, self._workspace,
+            self.tile_cfg, self._tile_strict)
         return out
 
     # ---- tile configuration (sparta.nn.tune(..., tile_configs=...)) ---------------------

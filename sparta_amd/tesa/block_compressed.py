@@ -201,9 +201,9 @@ class BCSFunctionContext(TeSAFunctionContext):
         self._workspaces: Dict[Tuple[int, int], int] = {}
 
     # ---- index build ------------------------------------------------------------
-    def _workspace(self, H: int, W: int, device) -> torch.Tensor:
-        """Scratch of one index build.  Taken from torch's caching allocator at every
-        build (only the byte count is cached): the allocator hands a block back out
+    def _scratch_bytes(self, H: int, W: int) -> int:
+        """Scratch of one index build (only the byte count is cached).  The scratch itself is taken
+        from torch's caching allocator at every build: the allocator hands a block back out
         only in stream order, so two operators - or two streams - that rebuild masks
         of one shape at the same time never share the liveness / prefix buffers."""
         key = (H, W)
@@ -212,11 +212,10 @@ class BCSFunctionContext(TeSAFunctionContext):
             nbytes = _lib.load().spx_bcs_index_workspace_bytes(H, W, self._block_H, self._block_W)
             assert nbytes > 0, f'mask shape ({H}, {W}) does not fit block ({self._block_H}, {self._block_W})'
             self._workspaces[key] = nbytes
-        return torch.empty((nbytes,), dtype=torch.uint8, device=device)
+        return nbytes
 
-    def _prepare(self, mask: torch.Tensor, capacity: Optional[int] = None) -> dict:
-        """Output buffers and workspace of one index build (everything
-        spx_bcs_index_scheduled takes), allocated but not yet filled."""
+    def _request(self, mask: torch.Tensor, capacity: Optional[int] = None) -> tuple:
+        """What the native builder is asked for one mask."""
         assert mask.dim() == 2, 'only 2D mask is supported'
         if mask.dtype != torch.uint8:
             mask = (mask != 0).to(torch.uint8)
@@ -224,51 +223,26 @@ class BCSFunctionContext(TeSAFunctionContext):
         H, W = mask.shape
         BH, BW = self._block_H, self._block_W
         assert H % BH == 0 and W % BW == 0, f'mask shape ({H}, {W}) does not fit block ({BH}, {BW})'
-        R, Cn = H // BH, W // BW
-        cap = R * Cn if capacity is None else int(capacity)
-        dev = mask.device
-        i32 = dict(dtype=torch.int32, device=dev)
-        job = dict(mask=mask, H=H, W=W, cap=cap, nnz_dev=torch.empty((1,), **i32),
-                   row_ptr=None, bcsr=None, col_ptr=None, bcsc=None, row_order=None, col_order=None)
-        if self._BCSR:
-            job['row_ptr'] = torch.empty((R + 1,), **i32)
-            job['bcsr'] = torch.empty((cap,), **i32)
-            job['row_order'] = torch.empty((R,), **i32)   # the launch orders of the matmul kernels
-        both = self._BCSR and self._BCSC
-        if self._BCSC:
-            job['col_ptr'] = torch.empty((Cn + 1,), **i32)
-            job['bcsc'] = torch.empty((cap,), dtype=torch.int64 if both else torch.int32, device=dev)
-            job['col_order'] = torch.empty((Cn,), **i32)  # come out of the same launch
-        job['ws'] = self._workspace(H, W, dev)
-        return job
+        return mask, BH, BW, self._BCSR, self._BCSC, -1 if capacity is None else int(capacity), self._scratch_bytes(H, W)
 
-    def _wrap(self, job: dict) -> BCSIndexes:
+    def _wrap(self, mask: torch.Tensor, built: tuple) -> BCSIndexes:
+        row_ptr, bcsr, row_order, col_ptr, bcsc, col_order, nnz_dev = built
         BH, BW = self._block_H, self._block_W
         if self._BCSR and self._BCSC:
-            indexes = BCSRCIndexes(self, job['mask'], job['row_ptr'], job['col_ptr'], job['bcsr'], job['bcsc'],
-                                   job['nnz_dev'], BH, BW)
+            indexes = BCSRCIndexes(self, mask, row_ptr, col_ptr, bcsr, bcsc, nnz_dev, BH, BW)
+            indexes.__dict__['_launch_order'] = {'row': row_order, 'col': col_order}
         elif self._BCSR:
-            indexes = BCSRIndexes(self, job['mask'], job['row_ptr'], job['bcsr'], job['nnz_dev'], BH, BW)
+            indexes = BCSRIndexes(self, mask, row_ptr, bcsr, nnz_dev, BH, BW)
+            indexes.__dict__['_launch_order'] = {'row': row_order}
         else:
-            indexes = BCSCIndexes(self, job['mask'], job['col_ptr'], job['bcsc'], job['nnz_dev'], BH, BW)
-        indexes.__dict__['_launch_order'] = {k: v for k, v in (('row', job['row_order']), ('col', job['col_order']))
-                                             if v is not None}
+            indexes = BCSCIndexes(self, mask, col_ptr, bcsc, nnz_dev, BH, BW)
+            indexes.__dict__['_launch_order'] = {'col': col_order}
         return indexes
 
     def build_indexes(self, mask: torch.Tensor, capacity: Optional[int] = None) -> BCSIndexes:
         """mask: uint8 (or any 1-byte dtype) [H, W] on the GPU.  `capacity` bounds the
         number of index entries kept (default: every block)."""
-        job = self._prepare(mask, capacity)
-        dev = job['mask'].device
-        with torch.cuda.device(dev):
-            rc = _lib.load().spx_bcs_index_scheduled(
-                _lib.dev_ptr(job['mask']), job['H'], job['W'], self._block_H, self._block_W,
-                _lib.dev_ptr(job['row_ptr']), _lib.dev_ptr(job['bcsr']), _lib.dev_ptr(job['col_ptr']),
-                _lib.dev_ptr(job['bcsc']), 1 if (self._BCSR and self._BCSC) else 0, _lib.dev_ptr(job['nnz_dev']),
-                job['cap'], _lib.dev_ptr(job['row_order']), _lib.dev_ptr(job['col_order']),
-                _lib.dev_ptr(job['ws']), job['ws'].numel(), _lib.current_stream(dev))
-        _lib.check(rc, 'spx_bcs_index_scheduled')
-        return self._wrap(job)
+        return build_indexes_batch([(self, mask, capacity)])[0]
 
     # ---- values ------------------------------------------------------------------
     def convert(self, dense: torch.Tensor, index: torch.Tensor, block_nnz: int, H: int, W: int,
@@ -334,27 +308,13 @@ def build_indexes_batch(requests) -> List[BCSIndexes]:
     qualify share one pair of launches).  `requests` is a sequence of
     (BCSFunctionContext, mask) or (BCSFunctionContext, mask, capacity); all masks on one GPU.
     The results equal those of `context.build_indexes(mask, capacity)` one by one."""
-    requests = [tuple(r) + (None,) * (3 - len(r)) for r in requests]
-    if not requests:
-        return []
-    jobs = [ctx._prepare(mask, cap) for ctx, mask, cap in requests]
-    dev = jobs[0]['mask'].device
-    assert all(j['mask'].device == dev for j in jobs), 'the masks of one batch must be on one device'
-    array = (_lib.BcsIndexJob * len(jobs))()
-    addr = lambda t: None if t is None else t.data_ptr()
-    for slot, (ctx, _, _), job in zip(array, requests, jobs):
-        slot.mask = addr(job['mask'])
-        slot.H, slot.W, slot.BH, slot.BW = job['H'], job['W'], ctx._block_H, ctx._block_W
-        slot.row_ptr, slot.bcsr_idx = addr(job['row_ptr']), addr(job['bcsr'])
-        slot.col_ptr, slot.bcsc_idx = addr(job['col_ptr']), addr(job['bcsc'])
-        slot.bcsc_i64 = 1 if (ctx._BCSR and ctx._BCSC) else 0
-        slot.nnz_dev, slot.cap = addr(job['nnz_dev']), job['cap']
-        slot.row_order, slot.col_order = addr(job['row_order']), addr(job['col_order'])
-        slot.workspace, slot.workspace_bytes = addr(job['ws']), job['ws'].numel()
-    with torch.cuda.device(dev):
-        rc = _lib.load().spx_bcs_index_batch(array, len(jobs), _lib.current_stream(dev))
-    _lib.check(rc, 'spx_bcs_index_batch')
-    return [ctx._wrap(job) for (ctx, _, _), job in zip(requests, jobs)]
+    requests = list(requests)
+    asked = [r[0]._request(*r[1:]) for r in requests]
+    if asked:
+        dev = asked[0][0].device
+        assert all(a[0].device == dev for a in asked), 'the masks of one batch must be on one device'
+    built = _lib.native().build_indexes(asked)
+    return [r[0]._wrap(a[0], answer) for r, a, answer in zip(requests, asked, built)]
 
 
 def get_bcs_function(block_H: int, block_W: int, BCSR: bool, BCSC: bool) -> BCSFunctionContext:
