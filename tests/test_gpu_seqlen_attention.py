@@ -85,6 +85,29 @@ def test_seqlen_attention_pipelined_kernel_instantiations(dtype, N, E, gpu, H=2)
         assert float(out[b, :, int(L):].abs().max() if L < N else 0.0) == 0.0
 
 
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('B,H,N,E', [(70, 3, 256, 64), (67, 2, 352, 128), (16, 8, 416, 64), (5, 16, 640, 128)])
+def test_seqlen_attention_wide_kernel(dtype, B, H, N, E, gpu):
+    """Enough work for the 128-query workgroups: more than one group of 64 ranked lengths, equal lengths,
+    lengths around every tile edge, N that ends inside a query tile and inside a key tile, and padding
+    that holds NaN (no row past a length takes part in anything)."""
+    assert N >= 256 and B * H * ((N + 127) // 128) >= 384   # the sizes at which the library takes this kernel
+    edges = [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, N - 33, N - 32, N - 1, N, N]
+    seqlens = np.array([edges[(5 * b) % len(edges)] for b in range(B)], dtype=np.int32)
+    (q, k, v), (qn, kn, vn) = rand_qkv((B, H, N, E), 13, dtype)
+    for b, L in enumerate(seqlens):
+        for t in (q, k, v):
+            t[b, :, int(L):] = float('nan')
+    att = SeqlenDynamicSparseAttention(global_mode=False)
+    out = att(q.to(gpu), k.to(gpu), v.to(gpu), torch.from_numpy(seqlens).to(gpu))
+    for b, L in enumerate(seqlens):
+        L = int(L)
+        assert float(out[b, :, L:].abs().max() if L < N else 0.0) == 0.0
+        if L:
+            s = torch.from_numpy(qn[b, :, :L] @ kn[b, :, :L].transpose(0, 2, 1))
+            assert_close(out[b, :, :L], torch.softmax(s, -1).numpy() @ vn[b, :, :L], dtype, f'wide kernel entry {b} length {L}')
+
+
 def test_seqlen_attention_rejects_bad_input(gpu):
     att = SeqlenDynamicSparseAttention(global_mode=False)
     q = torch.rand((2, 2, 48, 64), device=gpu)
