@@ -276,7 +276,7 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         const bool fill = big_tiles >= 512;
         // 128-row tiles halve the traffic of the sparse blocks and want a few rounds of workgroups to
         // even out (fp32 spends longer on a tile: more of them)
-        const int ring = tiles128 >= (sizeof(T) == 4 ? 2048 : BN == 64 ? 1024 : 768) ? 12 : 11;
+        int ring = tiles128 >= (sizeof(T) == 4 ? 2048 : BN == 64 ? 1024 : 768) ? 12 : 11;
         // The ring kernel, where it was measured ahead (rows x K x N; us of the best other kernel / ring):
         //   * operands that are not both k-contiguous: sdd 4096 x 3072 x 768 fp32 at 20 % 110 / 38, fp16 26 / 14,
         //     dsd 400 x 3072 x 768 fp32 at 15 % 38 / 10, bf16 14 / 10 - but for large fp32 problems in blocks
@@ -286,13 +286,32 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         //   * 16-bit blocks of depth 32 (two to a stage) while the result is narrow: 8192 x 1024 x 1024
         //     at 10 % 16.5 / 13.5; wide results (tiles of one or two stages) stay with the 256-row
         //     kernels: 8192 x 768 x 3072 at 10 % 23 / 28, 4096^3 at 5 % 25.5 / 31.
+        //     Up to 1024 rows the 256-row kernels have too few workgroups for long block-columns, also where
+        //     the result is wide: 1024 x 4096 x 4096 at 35 % 61 / 43, 1024^2 x 4096 at 35 % 19.8 / 14.7, at 10 %
+        //     9.8 / 9.2.  Against the column-split kernel (config 8) it is ahead from about 1100 64-row tiles on:
+        //     1500 x 1024 x 2048 15.0 / 11.9, 800 x 1024 x 3072 14.7 / 11.5, 700 x 4096 x 4096 43 / 40 at 35 %,
+        //     9.7 / 7.0, 9.3 / 6.7 and 20 / 16 at 5 - 10 %; with 640 tiles 19.0 / 22.8 (270 x 4096 x 4096), with
+        //     512 8.0 / 8.9 (1024^3).
         const bool two_blocks = p.BK * (int)sizeof(T) == 64;
+        const int64_t tiles64 = (int64_t)((p.Mc + 63) / 64) * nb * batch;
         bool use_ring = ring_ok;
         if (two_blocks && sizeof(T) == 4) use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
         else if (two_blocks && kcontig) {
-            if (fill) use_ring = ring_ok && p.Nc < 2048 && cols >= 32;
-            else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32);
+            const bool few_rows = p.Mc > 256 && p.Mc < 2048 && cols >= 32 && tiles64 >= 1100 && BN == 32;
+            if (fill) use_ring = ring_ok && cols >= 32 && (p.Nc < 2048 || (few_rows && p.Mc <= 1024));
+            else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32 || few_rows);
+            if (few_rows && tiles128 >= 640) ring = 12;   // 1200 x 3072 x 2048: 32.9 us in 64-row tiles, 24.6 in these
         }
+        // fp32 blocks of depth 16, long block-columns: four wavefronts that split a column and meet once keep
+        // more loads in flight than 256-row tiles when those are few.  256-row kernel / split columns:
+        // up to 1024 rows 512 x 4096 x 4096 at 35 % 259 / 85 us, at 5 % 45 / 20, 1024 x 2048 x 2048 74 / 45 and
+        // 16.4 / 14.4; narrow results 8192 x 2048 x 512 91 / 76 and (5 %) 28.1 / 25.9, 4096 x 2048 x 512 54 / 42,
+        // 4096 x 1024 x 512 32 / 28, 4380 x 1408 x 960 54 / 41, 4096 x 2048 x 1024 79 / 75, but 12.3 / 12.7 with four live blocks to a column and 158 / 148, 30 / 38 at
+        // 16384 rows; wide ones with more rows are mixed (2048^3 at 35 % 74 / 77, 4096 x 512 x 2048 44 / 51).
+        const int64_t live = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * p.Nc) : cols;   // stored blocks per block-column
+        const bool split_columns = sizeof(T) == 4 && two_blocks && BN == 16 && ksplit_ok && cols > 48 &&
+                                   p.Mc > 256 && (p.Mc <= 1024 || (p.Mc <= 8192 && nb <= 32 && live >= 6) ||
+                                                    (p.Mc <= 4608 && nb <= 64 && live >= 12));
         // the persistent form when its 8 * (N / BN) slots fill the device four times over, every
         // slot walks at least two 256-row tiles and the block-columns are long: 28.4 - 28.7 us
         // against 29.9 - 30.0 us for 7 on the 4096^3 problem (alternating runs on three
@@ -301,6 +320,7 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
             sizeof(T) == 2 && (BN == 16 || BN == 32 || BN == 64))
             tile_cfg = 10;
         else if (use_ring) tile_cfg = ring;
+        else if (split_columns) tile_cfg = 8;
         else if (panel_ok && p.Mc >= 512 && fill) tile_cfg = p.Mc >= 1024 ? 7 : 5;
         // few rows and short columns: no barrier and no shared block pays (64 x 768 x 3072 bf16: 3.9 us
         // against 4.4 with the columns split and 5.2 through the ring)

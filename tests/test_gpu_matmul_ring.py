@@ -34,3 +34,21 @@ def test_ring_rows_and_rounds(tile_cfg, dtype, blocks, gpu):
 def test_ring_more_block_columns_than_the_table(gpu):
     run_case(gpu, 'dsd', False, True, False, True, torch.float16, (32, 32, 16), batch=1, M=520, K=96, N=16 * 1100,
              gran=(16, 32), sparsity=0.6, seed=61, tile_cfg=11)
+
+
+@pytest.mark.parametrize('dtype,blocks,M,K,N,sparsity', [
+    # split columns: first and last row count, ragged rows, a result wide enough for 512 tiles of 256 rows
+    (torch.float32, (16, 16, 16), 257, 784, 512, 0.8), (torch.float32, (16, 16, 16), 520, 832, 2736, 0.95),
+    (torch.float32, (16, 16, 16), 1024, 1056, 2048, 0.9),
+    # ... more rows: up to 32 and up to 64 block-columns, both sides of the live-block limits
+    (torch.float32, (16, 16, 16), 1025, 1056, 512, 0.8), (torch.float32, (16, 16, 16), 1500, 1056, 1024, 0.7),
+    (torch.float32, (16, 16, 16), 1025, 800, 512, 0.95), (torch.float32, (16, 16, 16), 1025, 1056, 1040, 0.8),
+    # ring: 1100 tiles of 64 rows in tiles of 64 and of 128, and one column fewer
+    (torch.float16, (32, 32, 32), 257, 1024, 7040, 0.95), (torch.float16, (32, 32, 32), 257, 1024, 7008, 0.95),
+    (torch.bfloat16, (32, 32, 32), 1024, 1056, 2208, 0.9), (torch.bfloat16, (32, 32, 32), 1200, 1024, 1888, 0.9)])
+def test_dispatch_of_few_rows_and_long_columns(dtype, blocks, M, K, N, sparsity, gpu):
+    """The sizes at which the library's own choice changes, compressed (where it knows the number of live
+    blocks) and not, with bias and with every other call's activation fused."""
+    for compressed in (True, False):
+        run_case(gpu, 'dsd', False, True, True, compressed, dtype, blocks, batch=1, M=M, K=K, N=N, gran=(blocks[2], blocks[1]),
+                 sparsity=sparsity, seed=71, tile_cfg=0, activation='relu' if compressed else None)
