@@ -208,6 +208,7 @@ struct MoeParams {
     int w_kcontig;  // weight [E, N, K] if set, else [E, K, N]
     int split;      // 0: one launch; 1 / 2: first / second launch of a split (see moe_find_tile)
     int round_rows; // split: 256-row tiles that one round of the big-tile launch covers
+    int col_groups; // direct kernel: 0: tile (x, y) is workgroup (x, y); else see moe_tile_of_workgroup
 };
 
 // Which (expert, row tile) belongs to tile index y: one wavefront scans the per-expert
@@ -597,6 +598,23 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(MoeParams p) {
     }
 }
 
+// Workgroup L (column tiles fastest) runs on XCD L % 8.  With a multiple of eight column tiles every XCD
+// keeps the same columns for all row tiles, and its weight panels stay in its L2.  With other
+// counts the columns of an XCD would change from row tile to row tile, and every XCD would read all weights:
+// there the column tiles are cut into col_groups = 4, 2 or 1 groups, an XCD stays in one of them, and the row
+// tiles go round the 8 / col_groups XCDs of a group.  fp16, before / after: 16384 x 2048 -> 768 over 32 experts
+// 94.5 / 73.8 us (6 column tiles), 10007 x 768 -> 3072 over 32 bf16 82 / 76 us (12), 8192 x 768 -> 768 over 16 22.8 / 20.1 us,
+// 16384 x 768 -> 768 over 8 29.3 / 28.2 us (3); 16384 x 1024 -> 768 and -> 3072 the same.  With a multiple of eight
+// columns (16384 x 1024 -> 4096) no cut measured a difference.
+__device__ __forceinline__ void moe_tile_of_workgroup(const MoeParams& p, int& x, int& y) {
+    if (p.col_groups == 0) { x = blockIdx.x; y = blockIdx.y; return; }
+    const int L = blockIdx.y * gridDim.x + blockIdx.x;
+    const int xcd = L & 7, j = L >> 3;
+    const int cols = gridDim.x / p.col_groups;
+    x = (xcd % p.col_groups) * cols + j % cols;
+    y = (j / cols) * (8 / p.col_groups) + xcd / p.col_groups;
+}
+
 // ---- gathered GEMM with LDS-direct loads ------------------------------------------------
 // Same tile lookup and LDS layout as moe_gemm_kernel (k-contiguous weights only); the
 // workgroup tile is TM x TN with WAVES wavefronts (WGM of them along the rows), and the
@@ -632,17 +650,19 @@ __global__ __launch_bounds__(64 * WAVES, (TM + TN) * NBUF * KTB > 80 * 1024 ? 1 
     extern __shared__ __align__(16) char smem[];
     __shared__ int s_expert, s_row0, s_rows;
 
+    int tile_x, tile_y;
+    moe_tile_of_workgroup(p, tile_x, tile_y);
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
         int found_e, found_row0, found_rows;
-        moe_find_tile<TM>(p, blockIdx.y, lane, found_e, found_row0, found_rows);
+        moe_find_tile<TM>(p, tile_y, lane, found_e, found_row0, found_rows);
         if (lane == 0) { s_expert = found_e; s_row0 = found_row0; s_rows = found_rows; }
     }
     __syncthreads();
     const int expert = s_expert;
     if (expert < 0) return;
     const int row0 = s_row0, rows = s_rows;
-    const int n0 = blockIdx.x * TN;
+    const int n0 = tile_x * TN;
     if (expert == p.n_exp) {  // tokens without a valid expert id: zero rows
         moe_zero_tile<T>(p, row0, rows, n0, TN, NTH);
         return;
@@ -971,13 +991,16 @@ __global__ __launch_bounds__(64 * WAVES, (TM + TN) * NBUF * KTB > 80 * 1024 ? 1 
 template <typename T, int TM, int TN, int WAVES, int WGM, int NBUF, int KTB, bool BKN, bool XS>
 static int launch_moe_direct_inst(const MoeParams& p, hipStream_t st) {
     // split 2 covers at most one round of 256-row tiles, as 128-row halves
-    const int tiles = p.split == 2 ? 2 * p.round_rows : (p.n_tok + TM - 1) / TM + p.n_exp + 1;
-    if (tiles > 65535) return fail(SPX_E_SHAPE, "too many row tiles for one launch");
+    int tiles = p.split == 2 ? 2 * p.round_rows : (p.n_tok + TM - 1) / TM + p.n_exp + 1;
+    const int ntn = (p.N + TN - 1) / TN;
+    MoeParams q = p;
+    q.col_groups = ntn % 8 == 0 ? 0 : ntn % 4 == 0 ? 4 : ntn % 2 == 0 ? 2 : 1;
+    if (q.col_groups) tiles = (int)round_up(tiles, 8 / q.col_groups);
     // the epilogue stages every wavefront's (TM / WGM) x 64 output tile as rows of 128 bytes
     const int epi = sizeof(T) == 2 ? WAVES * (TM / WGM) * 128 : 0;
     const int smem = NBUF * (TM + TN) * KTB > epi ? NBUF * (TM + TN) * KTB : epi;
     SPX_GRANT_LDS((moe_gemm_direct_kernel<T, TM, TN, WAVES, WGM, NBUF, KTB, BKN, XS>), smem, "moe_gemm_direct_kernel");
-    hipLaunchKernelGGL((moe_gemm_direct_kernel<T, TM, TN, WAVES, WGM, NBUF, KTB, BKN, XS>), dim3((p.N + TN - 1) / TN, tiles, 1), dim3(64 * WAVES), smem, st, p);
+    hipLaunchKernelGGL((moe_gemm_direct_kernel<T, TM, TN, WAVES, WGM, NBUF, KTB, BKN, XS>), dim3(ntn, tiles, 1), dim3(64 * WAVES), smem, st, q);
     SPX_LAUNCH_CHECK("moe_gemm_direct_kernel");
     return 0;
 }
@@ -1088,7 +1111,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     p.expert_offset = expert_offset; p.token_perm = token_perm;
     p.n_tok = n_tok; p.K = in_dim; p.N = out_dim; p.n_exp = n_exp;
     p.w_kcontig = weight_layout == 1;
-    p.split = 0; p.round_rows = 1;
+    p.split = 0; p.round_rows = 1; p.col_groups = 0;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // tile_cfg 1: 128x128 tiles staged through registers (any dtype and weight layout);
     // 2 / 3 / 4: tiles filled by LDS-direct loads - 128x128 with four wavefronts (two
