@@ -24,6 +24,9 @@ namespace spx {
 
 constexpr int MOE_CHUNK = 1024;   // most tokens per workgroup in the index kernels (a multiple of 256)
 constexpr int MOE_FUSED_TABLE = 1024;  // (chunk, expert) counts a placement workgroup scans itself
+// Tokens up to which the placement workgroups count the experts themselves, a launch less: a call of 333 tokens
+// 29.7 -> 28.6 us, of 64 24.5 -> 23.1; at 2000 the launch is the cheaper one (82.4 / 83.2 us).
+constexpr int MOE_SELF_COUNT = 1024;
 constexpr int MOE_MAX_EXP = 2048; // LDS table capacity of the placement kernel
 
 // ---- index -------------------------------------------------------------------
@@ -77,7 +80,8 @@ __global__ __launch_bounds__(256) void moe_zero_index_kernel(int n_exp, int32_t*
 
 // Stable placement of one chunk.  Waves take 64 tokens at a time; inside a wave the
 // rank among equal experts comes from ballots, between waves from a small table.
-// FUSED: `counts` holds the raw per-chunk histograms (at most MOE_FUSED_TABLE of them);
+// FUSED: `counts` holds the raw per-chunk histograms (at most MOE_FUSED_TABLE of them), or is null
+// (at most MOE_SELF_COUNT tokens: counting them again in every workgroup is cheaper than the launch that would);
 // every workgroup scans them in (expert, chunk) order itself and workgroup 0 also writes
 // expert_offset and expert_count.  Otherwise `counts` holds every expert's prefix over the
 // chunks (moe_colscan_kernel) and `totals` the experts' token counts, which every workgroup
@@ -99,6 +103,23 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* exp_ids, 
         // entries 4 tid .. 4 tid + 3 of the (expert, chunk) order
         const int n_chunk = gridDim.x;
         const int n = n_chunk * n_exp;
+        if (counts == nullptr) {   // few tokens: every workgroup counts all of them itself
+            for (int i = threadIdx.x; i < n; i += 256) tab[i] = 0;
+            __syncthreads();
+            int id[MOE_SELF_COUNT / 256];
+#pragma unroll
+            for (int j = 0; j < MOE_SELF_COUNT / 256; ++j) {
+                const int t = j * 256 + threadIdx.x;
+                id[j] = t < n_tok ? exp_ids[t] : -1;
+            }
+#pragma unroll
+            for (int j = 0; j < MOE_SELF_COUNT / 256; ++j) {
+                const int t = j * 256 + threadIdx.x;
+                const int e = id[j] < 0 || id[j] >= n_exp - 1 ? n_exp - 1 : id[j];
+                if (t < n_tok) atomicAdd(&tab[e * n_chunk + t / chunk], 1);
+            }
+            __syncthreads();
+        }
         int v[4], sum = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -106,7 +127,7 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* exp_ids, 
             v[j] = 0;
             if (i < n) {
                 const int e = i / n_chunk, c = i - e * n_chunk;
-                v[j] = counts[c * n_exp + e];
+                v[j] = counts ? counts[c * n_exp + e] : tab[i];
             }
             sum += v[j];
         }
@@ -605,7 +626,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(MoeParams p) {
 // tiles go round the 8 / col_groups XCDs of a group.  fp16, before / after: 16384 x 2048 -> 768 over 32 experts
 // 94.5 / 73.8 us (6 column tiles), 10007 x 768 -> 3072 over 32 bf16 82 / 76 us (12), 8192 x 768 -> 768 over 16 22.8 / 20.1 us,
 // 16384 x 768 -> 768 over 8 29.3 / 28.2 us (3); 16384 x 1024 -> 768 and -> 3072 the same.  With a multiple of eight
-// columns (16384 x 1024 -> 4096) no cut measured a difference.
+// columns (16384 x 1024 -> 4096) no cut measured a difference, and with fewer than 256 rows per expert there is
+// little to share (4096 x 2048 -> 768 over 32, whole call: 51.0 in launch order, 52.8 cut).
 __device__ __forceinline__ void moe_tile_of_workgroup(const MoeParams& p, int& x, int& y) {
     if (p.col_groups == 0) { x = blockIdx.x; y = blockIdx.y; return; }
     const int L = blockIdx.y * gridDim.x + blockIdx.x;
@@ -994,7 +1016,7 @@ static int launch_moe_direct_inst(const MoeParams& p, hipStream_t st) {
     int tiles = p.split == 2 ? 2 * p.round_rows : (p.n_tok + TM - 1) / TM + p.n_exp + 1;
     const int ntn = (p.N + TN - 1) / TN;
     MoeParams q = p;
-    q.col_groups = ntn % 8 == 0 ? 0 : ntn % 4 == 0 ? 4 : ntn % 2 == 0 ? 2 : 1;
+    q.col_groups = ntn % 8 == 0 || p.n_tok < (int64_t)256 * p.n_exp ? 0 : ntn % 4 == 0 ? 4 : ntn % 2 == 0 ? 2 : 1;
     if (q.col_groups) tiles = (int)round_up(tiles, 8 / q.col_groups);
     // the epilogue stages every wavefront's (TM / WGM) x 64 output tile as rows of 128 bytes
     const int epi = sizeof(T) == 2 ? WAVES * (TM / WGM) * 128 : 0;
@@ -1014,6 +1036,138 @@ static int launch_moe_direct(const MoeParams& p, hipStream_t st) {
         if constexpr (sizeof(T) == 2) return launch_moe_direct_inst<T, TM, TN, WAVES, WGM, NBUF, KTB, true, XS>(p, st);
         else return fail(SPX_E_CONFIG, "fp32 weights stored [E, in, out] run through tile config 1");
     }
+}
+
+// ---- few rows per expert --------------------------------------------------------------------
+// With a handful of tokens to an expert the product is the reading of the weights, and a 128-row tile reads
+// them in one serial chain per (expert, 128 columns): 8 experts of 2048 x 768 kept 48 of 256 CUs busy for 22 us.
+// Here a workgroup takes 32 rows x 128 columns and each of its four wavefronts a quarter of k, through a ring of
+// its own (two stages of 32 k, filled global -> LDS directly: 8 KB of weights, 2 KB of tokens), so that no
+// barrier stands between a load and its use; the wavefronts add up through LDS once.  22.8 -> 11.5 us there (25 MB
+// of weights: 2.2 TB/s, bound by the loads a CU keeps in flight on 48 CUs); ranges of k over several
+// workgroups, added up by a second kernel, cost more than they gave (2 ranges 10.3 us, but 16.0 -> 19.5 for
+// 1000 x 2048 -> 768, 8.0 -> 11.1 for 64 x 1024 -> 4096 over 4).  [E, in, out] weights, 16-bit types.
+constexpr int MOE_ROWS_TM = 32, MOE_ROWS_TN = 128, MOE_ROWS_KT = 32;
+constexpr int MOE_ROWS_STAGE = (MOE_ROWS_TM + MOE_ROWS_TN) * MOE_ROWS_KT * 2;   // bytes
+constexpr int MOE_ROWS_PITCH = MOE_ROWS_TN + 4;                                // floats per row of a wavefront's partial tile
+constexpr int MOE_ROWS_WAVE = 2 * MOE_ROWS_STAGE;                              // LDS of a wavefront
+static_assert(MOE_ROWS_TM * MOE_ROWS_PITCH * 4 <= MOE_ROWS_WAVE, "the partial tile reuses the ring");
+
+template <typename T>
+__global__ __launch_bounds__(256, 2) void moe_rows_kernel(MoeParams p) {
+    constexpr int TM = MOE_ROWS_TM, TN = MOE_ROWS_TN, KT = MOE_ROWS_KT, NT = TN / 32;
+    constexpr int W_BYTES = KT * TN * 2;
+    constexpr int W_LOADS = W_BYTES / 1024, LOADS = MOE_ROWS_STAGE / 1024;
+    typedef typename MmaW<T>::frag Frag;
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    extern __shared__ __align__(16) char smem[];
+
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int expert, row0, rows;
+    moe_find_tile<TM>(p, blockIdx.y, lane, expert, row0, rows);
+    expert = __builtin_amdgcn_readfirstlane(expert);
+    row0 = __builtin_amdgcn_readfirstlane(row0);
+    rows = __builtin_amdgcn_readfirstlane(rows);
+    if (expert < 0) return;
+    const int n0 = blockIdx.x * TN;
+
+    f32x16 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[t][j] = 0.f;
+    char* ring = smem + wave * MOE_ROWS_WAVE;
+    if (expert < p.n_exp) {   // the pseudo expert's rows stay zero
+        const int n_st = p.K / KT;
+        const int s_begin = n_st * wave / 4, s_end = n_st * (wave + 1) / 4;
+        const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * MOE_ROWS_WAVE;
+        // weights: a load instruction fills four k-rows of 256 bytes, their 32-byte units XORed by twice the
+        // low two bits of the row (as in moe_gemm_direct_kernel); columns past the end re-read valid ones
+        const int kr = lane >> 4, c = lane & 15;
+        int n = n0 + ((((c >> 1) ^ (kr << 1)) << 1) | (c & 1)) * 8;
+        if (n + 8 > p.N) n = p.N - 8;
+        const T* w_src = reinterpret_cast<const T*>(p.weight) + (int64_t)expert * p.K * p.N + (int64_t)kr * p.N + n;
+        // tokens: sixteen rows of 64 bytes, chunks XORed by bits 2 and 3 of the row; rows past the end re-read the last one
+        const T* a_src[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int r = q * 16 + (lane >> 2);
+            a_src[q] = reinterpret_cast<const T*>(p.tokens) + (int64_t)p.token_perm[row0 + (r < rows ? r : rows - 1)] * p.K +
+                       ((lane & 3) ^ ((r >> 2) & 3)) * 8;
+        }
+        auto issue = [&](int s) {
+            const uint32_t to = lds + (uint32_t)((s - s_begin) & 1) * MOE_ROWS_STAGE;
+#pragma unroll
+            for (int q = 0; q < W_LOADS; ++q) lds_direct_load16(w_src + (int64_t)(s * KT + q * 4) * p.N, to + q * 1024);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) lds_direct_load16(a_src[q] + s * KT, to + W_BYTES + q * 1024);
+        };
+        const int l32 = lane & 31, h2 = lane >> 5, r16 = lane & 15;
+        if (s_begin < s_end) issue(s_begin);
+        if (s_begin + 1 < s_end) issue(s_begin + 1);
+        for (int s = s_begin; s < s_end; ++s) {
+            if (s + 1 < s_end) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            const char* W = ring + ((s - s_begin) & 1) * MOE_ROWS_STAGE;
+            const char* A = W + W_BYTES;
+            Frag af[KT / 16], wf[KT / 16][NT];
+#pragma unroll
+            for (int k = 0; k < KT / 16; ++k) {
+                af[k] = *reinterpret_cast<const Frag*>(A + l32 * 64 + (((k * 2 + h2) ^ ((l32 >> 2) & 3)) << 4));
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const int row = k * 16 + 8 * h2 + (r16 >> 2);   // and row + 4: the same low two bits
+                    const int unit = t * 2 + ((lane >> 4) & 1);
+                    const char* at = W + row * (TN * 2) + ((unit ^ ((row & 3) << 1)) << 5) + ((r16 & 3) << 3);
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at));
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * TN * 2));
+                    wf[k][t] = __builtin_bit_cast(Frag, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the fragments are out of the buffer that is refilled now
+            if (s + 2 < s_end) issue(s + 2);
+#pragma unroll
+            for (int k = 0; k < KT / 16; ++k)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[t] = MmaW<T>::mma(wf[k][t], af[k], acc[t]);
+        }
+    }
+
+    // lane holds D[n = t*32 + 8*jj + 4*(lane/32) + q][m = lane % 32] in acc[t][4*jj + q]
+    float* mine = reinterpret_cast<float*>(ring);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+            *reinterpret_cast<f32x4*>(mine + (lane & 31) * MOE_ROWS_PITCH + t * 32 + 8 * jj + 4 * (lane >> 5)) =
+                f32x4{acc[t][4 * jj], acc[t][4 * jj + 1], acc[t][4 * jj + 2], acc[t][4 * jj + 3]};
+    __syncthreads();
+    for (int i = threadIdx.x; i < rows * (TN / 4); i += 256) {
+        const int row = i / (TN / 4), col = (i % (TN / 4)) * 4;
+        if (n0 + col >= p.N) continue;
+        f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+            sum += *reinterpret_cast<const f32x4*>(smem + w * MOE_ROWS_WAVE + (row * MOE_ROWS_PITCH + col) * 4);
+        const int tok = p.token_perm[row0 + row];
+        T vals[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) vals[q] = Elem<T>::from_float(sum[q]);
+        *reinterpret_cast<uint64_t*>(reinterpret_cast<T*>(p.out) + (int64_t)tok * p.N + n0 + col) = *reinterpret_cast<const uint64_t*>(vals);
+    }
+}
+
+template <typename T>
+static int launch_moe_rows(const MoeParams& p, hipStream_t st) {
+    const int tiles = (p.n_tok + MOE_ROWS_TM - 1) / MOE_ROWS_TM + p.n_exp + 1;
+    if (tiles > 65535) return fail(SPX_E_SHAPE, "too many row tiles for one launch");
+    constexpr int smem = 4 * MOE_ROWS_WAVE;
+    SPX_GRANT_LDS((moe_rows_kernel<T>), smem, "moe_rows_kernel");
+    hipLaunchKernelGGL((moe_rows_kernel<T>), dim3((p.N + MOE_ROWS_TN - 1) / MOE_ROWS_TN, tiles, 1), dim3(256), smem, st, p);
+    SPX_LAUNCH_CHECK("moe_rows_kernel");
+    return 0;
 }
 
 // Tokens per workgroup of the index kernels: the smallest multiple of 256 (up to MOE_CHUNK)
@@ -1066,7 +1220,8 @@ extern "C" int spx_moe_index(const int32_t* exp_ids, int n_tok, int n_exp,
     bool fused;
     const int chunk = moe_index_chunk(n_tok, n_exp, &fused);
     const int n_chunk = (n_tok + chunk - 1) / chunk;
-    if (n_chunk > 0) {
+    const bool self_count = fused && n_tok <= MOE_SELF_COUNT;
+    if (n_chunk > 0 && !self_count) {
         hipLaunchKernelGGL(moe_hist_kernel, dim3(n_chunk), dim3(256), (n_exp + 1) * sizeof(int), st, exp_ids, n_tok, n_exp + 1, chunk, partial);
         SPX_LAUNCH_CHECK("moe_hist_kernel");
     }
@@ -1082,7 +1237,8 @@ extern "C" int spx_moe_index(const int32_t* exp_ids, int n_tok, int n_exp,
     }
     const size_t smem = 6 * (n_exp + 1) * sizeof(int);
     if (fused)
-        hipLaunchKernelGGL(moe_place_kernel<true>, dim3(n_chunk), dim3(256), smem, st, exp_ids, n_tok, n_exp + 1, chunk, partial,
+        hipLaunchKernelGGL(moe_place_kernel<true>, dim3(n_chunk), dim3(256), smem, st, exp_ids, n_tok, n_exp + 1, chunk,
+                           self_count ? nullptr : partial,
                            totals, token_perm, expert_count, expert_offset);
     else
         hipLaunchKernelGGL(moe_place_kernel<false>, dim3(n_chunk), dim3(256), smem, st, exp_ids, n_tok, n_exp + 1, chunk, partial,
@@ -1096,7 +1252,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
                                int n_tok, int in_dim, int out_dim, int n_exp,
                                int tile_cfg, spx_stream_t stream) {
     using namespace spx;
-    SPX_REQUIRE(tile_cfg >= 0 && tile_cfg <= 6, SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
+    SPX_REQUIRE(tile_cfg >= 0 && tile_cfg <= 7, SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
     SPX_REQUIRE(dtype == SPX_F32 || dtype == SPX_F16 || dtype == SPX_BF16, SPX_E_DTYPE, "unknown dtype %d", dtype);
     SPX_REQUIRE(n_tok >= 0 && in_dim > 0 && out_dim > 0 && n_exp > 0, SPX_E_SHAPE, "bad sizes");
     SPX_REQUIRE(weight_layout == 0 || weight_layout == 1, SPX_E_CONFIG, "weight_layout must be 0 ([E,in,out]) or 1 ([E,out,in])");
@@ -1119,8 +1275,9 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     // wavefronts of 64x64 - for 16-bit types in either weight layout and fp32 with
     // k-contiguous weights.  256x256 tiles move half the bytes from L2 to the CUs, which is
     // what bounds the 128x128 kernel.  5 = 4 for the whole rounds of 256-row tiles plus 2 for
-    // the row tiles of a thinly filled last round (two launches, see moe_find_tile).  0 picks
-    // between 5, 4 and 2 by the number of 256x256 tiles (below); fp32 [E, in, out] weights take 1.
+    // the row tiles of a thinly filled last round (two launches, see moe_find_tile).  7: 32-row
+    // tiles for few rows per expert (16-bit, [E, in, out] weights).  0 picks
+    // between 7, 5, 4 and 2 by the number of tiles (below); fp32 [E, in, out] weights take 1.
     const bool direct_ok = p.w_kcontig || es == 2;
     static int n_cu = 0;
     if (n_cu == 0) {
@@ -1136,10 +1293,23 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         // tiles there, and behind them as soon as a second round starts); else 128x128
         const int64_t row_tiles = (n_tok + 255) / 256, col_tiles = (out_dim + 255) / 256;
         const int64_t big_tiles = row_tiles * col_tiles;
+        // 32-row tiles whose wavefronts split k, while tiles of 128 rows (one at least to every expert with tokens) leave
+        // CUs idle and hold few rows each.  fp16 us, 128-row tiles / these: 64 x 1024 -> 4096 over 4 13.5 / 8.0,
+        // 100 x 2048 -> 3072 over 8 26.5 / 18.8, 333 x 1024 -> 768 over 16 14.8 / 9.0, 1000 x 2048 -> 768 over 8 26 / 16,
+        // 39 x 2048 -> 768 over 32 27 / 12.6, 1000 x 768 -> 768 over 32 (240 tiles) 14.4 / 12.7; with 384 - 446 tiles
+        // 16.0 / 16.2 (500 x 768 -> 4096 over 8), 21.0 / 24.5 (333 x 1024 -> 3072 over 16), at 256 rows per expert
+        // 15.7 / 15.9 (2048 x 1024 -> 768 over 8).
+        const int64_t tiles128 = ((n_tok + 127) / 128 + (int64_t)(n_tok < n_exp ? n_tok : n_exp)) * ((out_dim + 127) / 128);
+        const bool few_rows = es == 2 && !p.w_kcontig && tiles128 <= 256 && n_tok <= (int64_t)128 * n_exp;
         if (!direct_ok) tile_cfg = 1;
+        else if (few_rows) tile_cfg = 7;
         else if (es == 2 && big_tiles >= 256) tile_cfg = 5;
         else if (es == 2 && big_tiles >= 128 && (row_tiles + n_exp) * col_tiles <= n_cu) tile_cfg = 4;
         else tile_cfg = 2;
+    }
+    if (tile_cfg == 7) {
+        SPX_REQUIRE(es == 2 && !p.w_kcontig, SPX_E_CONFIG, "tile config 7 takes 16-bit types and weights stored [E, in, out]");
+        return dtype == SPX_F16 ? launch_moe_rows<_Float16>(p, st) : launch_moe_rows<bf16_t>(p, st);
     }
     if (tile_cfg >= 2) {
         SPX_REQUIRE(direct_ok, SPX_E_CONFIG, "tile config %d takes fp32 weights in layout 1 only", tile_cfg);

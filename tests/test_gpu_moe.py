@@ -228,3 +228,47 @@ def test_moe_tile_configs(layout, tile_cfg, dtype, n_tok, in_dims, out_dims, gpu
     _lib.check(rc, 'spx_moe_forward')
     want = ops.moe_reference(x.to(torch.float64).numpy(), w, ids_np)
     assert_close(out, want, dtype, f'moe tile config {tile_cfg} layout {layout} {dtype}')
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('n_tok,in_dims,out_dims', [(1, 64, 8), (5, 64, 520), (33, 192, 136), (64, 128, 128), (300, 2048, 264)])
+def test_moe_few_rows_kernel(dtype, n_tok, in_dims, out_dims, gpu):
+    """Tile config 7 through the C ABI: fewer k-stages than wavefronts and more, rows that end inside a tile,
+    several row tiles to an expert, columns that end inside a tile, tokens without an expert, and a
+    token of NaN that reaches no other row."""
+    from sparta_amd import _lib
+    n_exp = 5
+    moe, w = make_moe(n_exp, in_dims, out_dims, dtype, gpu)
+    rng = np.random.default_rng(n_tok)
+    ids_np = rng.choice([0, 1, 2, 4, 7], size=n_tok, p=[0.6, 0.2, 0.1, 0.05, 0.05]).astype(np.int32)
+    x = torch.from_numpy(rng.random((n_tok, in_dims), dtype=np.float32)).to(dtype)
+    bad = n_tok - 1 if n_tok > 1 else None
+    if bad is not None:
+        ids_np[bad] = 0
+    xg = x.to(gpu)
+    if bad is not None:
+        xg[bad] = float('nan')
+    moe(xg, torch.from_numpy(ids_np).to(gpu))  # builds the index
+    out = torch.full((n_tok, out_dims), float('nan'), dtype=dtype, device=gpu)
+    rc = _lib.load().spx_moe_forward(_lib.dtype_code(dtype), _lib.dev_ptr(xg), _lib.dev_ptr(moe.weight.detach()), 0,
+                                     _lib.dev_ptr(out), _lib.dev_ptr(moe.expert_offset), _lib.dev_ptr(moe.sparse_index),
+                                     n_tok, in_dims, out_dims, n_exp, 7, _lib.current_stream(gpu))
+    _lib.check(rc, 'spx_moe_forward')
+    valid = ids_np < n_exp
+    want = np.zeros((n_tok, out_dims))
+    if valid.any():
+        want[valid] = ops.moe_reference(x.to(torch.float64).numpy()[valid], w, ids_np[valid])
+    rows = np.arange(n_tok) != (-1 if bad is None else bad)
+    assert_close(out[torch.from_numpy(rows).to(gpu)], want[rows], dtype, f'moe few-row kernel {dtype} {(n_tok, in_dims, out_dims)}')
+    if bad is not None:
+        assert bool(torch.isnan(out[bad]).all())
+    rc = _lib.load().spx_moe_forward(_lib.dtype_code(dtype), _lib.dev_ptr(xg), _lib.dev_ptr(moe.weight.detach()), 1,
+                                     _lib.dev_ptr(out), _lib.dev_ptr(moe.expert_offset), _lib.dev_ptr(moe.sparse_index),
+                                     n_tok, in_dims, out_dims, n_exp, 7, _lib.current_stream(gpu))
+    assert rc != 0   # [E, out, in] weights are refused
+
+
+@pytest.mark.parametrize('n_tok,n_exp', [(1, 3), (255, 1000), (1024, 8), (1024, 200), (1025, 8)])
+def test_moe_index_of_few_tokens(n_tok, n_exp, gpu):
+    """Around the token count up to which the placement workgroups count the experts themselves."""
+    test_moe_index_launch_paths(n_tok, n_exp, gpu)
