@@ -293,6 +293,8 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         //     9.7 / 7.0, 9.3 / 6.7 and 20 / 16 at 5 - 10 %; with 640 tiles 19.0 / 22.8 (270 x 4096 x 4096), with
         //     512 8.0 / 8.9 (1024^3).
         const bool two_blocks = p.BK * (int)sizeof(T) == 64;
+        // stored blocks in all block-columns together (all places where it is not known)
+        const int64_t stored = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * BN) : (int64_t)cols * nb;
         const int64_t tiles64 = (int64_t)((p.Mc + 63) / 64) * nb * batch;
         bool use_ring = ring_ok;
         if (two_blocks && sizeof(T) == 4) use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
@@ -308,10 +310,15 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         // 16.4 / 14.4; narrow results 8192 x 2048 x 512 91 / 76 and (5 %) 28.1 / 25.9, 4096 x 2048 x 512 54 / 42,
         // 4096 x 1024 x 512 32 / 28, 4380 x 1408 x 960 54 / 41, 4096 x 2048 x 1024 79 / 75, but 12.3 / 12.7 with four live blocks to a column and 158 / 148, 30 / 38 at
         // 16384 rows; wide ones with more rows are mixed (2048^3 at 35 % 74 / 77, 4096 x 512 x 2048 44 / 51).
-        const int64_t live = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * p.Nc) : cols;   // stored blocks per block-column
         const bool split_columns = sizeof(T) == 4 && two_blocks && BN == 16 && ksplit_ok && cols > 48 &&
-                                   p.Mc > 256 && (p.Mc <= 1024 || (p.Mc <= 8192 && nb <= 32 && live >= 6) ||
-                                                    (p.Mc <= 4608 && nb <= 64 && live >= 12));
+                                   p.Mc > 256 && (p.Mc <= 1024 || (p.Mc <= 8192 && nb <= 32 && stored >= 6 * nb) ||
+                                                    (p.Mc <= 4608 && nb <= 64 && stored >= 12 * nb));
+        // 16-bit blocks of depth 64, a block or less to a block-column: next to no walk, the time is the output's, and the
+        // 256-row kernels write it faster.  Ring / 256-row: 32 x 64 blocks 16384 x 512 x 2048 at 5 % 27.7 / 15.4 us, 8192 x
+        // 768 x 3072 at 10 % 20.8 / 18.5 and at 5 % 19.0 / 14.2, 4096 x 1024 x 4096 at 5 % 14.4 / 12.3; 64 x 64 blocks at 10 %
+        // 29.0 / 24.5 and 23.2 / 20.9.  With 1.6 blocks to a column 16.1 / 17.4 (4096 x 1024 x 4096), with three 29 / 36
+        // (8192 x 768 x 3072); at 2048 rows 6.9 / 7.3.
+        const bool short_columns = sizeof(T) == 2 && panel_ok && !two_blocks && p.Mc >= 4096 && fill && stored * 4 <= (int64_t)nb * 5;
         // the persistent form when its 8 * (N / BN) slots fill the device four times over, every
         // slot walks at least two 256-row tiles and the block-columns are long: 28.4 - 28.7 us
         // against 29.9 - 30.0 us for 7 on the 4096^3 problem (alternating runs on three
@@ -319,6 +326,7 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         if (stream_ok && panel_ok && batch == 1 && 8 * nb >= 1024 && p.Mc >= 16 * 256 && cols >= 32 && two_blocks &&
             sizeof(T) == 2 && (BN == 16 || BN == 32 || BN == 64))
             tile_cfg = 10;
+        else if (short_columns) tile_cfg = BN == 64 ? 7 : 5;
         else if (use_ring) tile_cfg = ring;
         else if (split_columns) tile_cfg = 8;
         else if (panel_ok && p.Mc >= 512 && fill) tile_cfg = p.Mc >= 1024 ? 7 : 5;

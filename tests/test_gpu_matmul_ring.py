@@ -45,6 +45,9 @@ def test_ring_more_block_columns_than_the_table(gpu):
     (torch.float32, (16, 16, 16), 1025, 800, 512, 0.95), (torch.float32, (16, 16, 16), 1025, 1056, 1040, 0.8),
     # ring: 1100 tiles of 64 rows in tiles of 64 and of 128, and one column fewer
     (torch.float16, (32, 32, 32), 257, 1024, 7040, 0.95), (torch.float16, (32, 32, 32), 257, 1024, 7008, 0.95),
+    # 256-row tiles: a block or less to a block-column, and one side of each limit
+    (torch.float16, (32, 32, 64), 4100, 512, 1024, 0.9), (torch.bfloat16, (64, 64, 64), 4096, 256, 2048, 0.8),
+    (torch.float16, (32, 32, 64), 4100, 512, 1024, 0.8), (torch.float16, (32, 32, 64), 4095, 512, 1024, 0.9),
     (torch.bfloat16, (32, 32, 32), 1024, 1056, 2208, 0.9), (torch.bfloat16, (32, 32, 32), 1200, 1024, 1888, 0.9)])
 def test_dispatch_of_few_rows_and_long_columns(dtype, blocks, M, K, N, sparsity, gpu):
     """The sizes at which the library's own choice changes, compressed (where it knows the number of live
