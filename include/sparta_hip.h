@@ -331,9 +331,12 @@ int spx_attention_backward_kv(int dtype, const void* grad_out, const void* q, co
  * spx_attention_backward_kv_recompute gives grad_k and grad_v (as spx_attention_backward_kv).
  * Against the reference's backward chain (sparse_attention.py:76-80 run in reverse: five
  * launches, probabilities and score gradients written and re-read) the whole step reads and
- * writes only q, k, v, out, grad_out and the three gradients.  Block-level masks only (every
- * element of a live block attends): element masks go through spx_attention_forward_train.
- * 16-bit types; block shapes as spx_attention_forward_train, the column side also BH <= 2 * BW. */
+ * writes only q, k, v, out, grad_out and the three gradients.  spx_attention_backward_q and
+ * spx_attention_backward_kv_recompute take block-level masks (every element of a live block
+ * attends); the *_masked forms also the element mask that the forward pass was given (bytes
+ * [Nt, Ns], 16-byte aligned, NULL: none), with head dim 64 and query and key blocks of 32 / 64.
+ * 16-bit types; block shapes as spx_attention_forward_train, the column side without an element
+ * mask also BH <= 2 * BW. */
 int spx_attention_forward_lse(int dtype, const void* q, const void* k, const void* v, void* out,
                               float* row_lse, const int32_t* row_ptr, const int32_t* bcsr_idx,
                               const uint8_t* mask, float inv_temperature,
@@ -349,6 +352,18 @@ int spx_attention_backward_kv_recompute(int dtype, const void* grad_out, const v
                                         const int32_t* col_ptr, const void* bcsc_idx, int idx_kind,
                                         float inv_temperature,
                                         int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream);
+int spx_attention_backward_q_masked(int dtype, const void* grad_out, const void* out, const void* q,
+                                    const void* k, const void* v, const float* row_lse,
+                                    void* grad_q, float* row_dot,
+                                    const int32_t* row_ptr, const int32_t* bcsr_idx,
+                                    const uint8_t* mask, float inv_temperature,
+                                    int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream);
+int spx_attention_backward_kv_masked(int dtype, const void* grad_out, const void* q, const void* k,
+                                     const void* v, const float* row_lse, const float* row_dot,
+                                     void* grad_k, void* grad_v,
+                                     const int32_t* col_ptr, const void* bcsc_idx, int idx_kind,
+                                     const uint8_t* mask, float inv_temperature,
+                                     int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream);
 
 /* ------------------------------------------------------------------------ *
  * Sequence-length attention: q, k, v, out are [batch, heads, N, E]; batch b

@@ -2128,12 +2128,27 @@ extern "C" int spx_attention_backward_kv(int dtype, const void* grad_out, const 
     return launch_attention_bwd_col<bf16_t>(p, batch, BW, E, st);
 }
 
-extern "C" int spx_attention_backward_q(int dtype, const void* grad_out, const void* out, const void* q,
-                                        const void* k, const void* v, const float* row_lse,
-                                        void* grad_q, float* row_dot,
-                                        const int32_t* row_ptr, const int32_t* bcsr_idx, float inv_temperature,
-                                        int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
-    using namespace spx;
+namespace spx {
+// The kernels with 32 queries (keys) per wavefront, over 64-high (64-wide) blocks of head dim 64: ahead of the ones with 16 once
+// there are three workgroups for every CU.  Row side / column side, old and wide: 96 x 4096 positions fp16 (6144 workgroups) 87 / 111
+// and 77 / 93 us, 24 x 2048 (768) 15.3 / 18.7 and 15.0 / 16.7, 12 x 4096 (768) 16.9 / 19.6 and 15.6 / 17.2; 16 x 2048 (512) 10.3 / 13.0
+// and 12.1 / 13.7, 12 x 512 (96) 5.0 / 6.9 and 6.0 / 6.9.  32 x 32 blocks: level at 12288 workgroups (70 / 84 and 69 / 81), behind at
+// 768 (9.2 / 10.1 and 9.6 / 11.4).
+static bool attention_bwd_wide_wins(int edge, int E, int64_t workgroups) { return edge == 64 && E == 64 && workgroups >= 768; }
+
+static int attention_bwd_check_mask(const uint8_t* mask, int Ns, int E, int BH, int BW) {
+    if (!mask) return 0;
+    SPX_REQUIRE(E == 64 && (BH == 32 || BH == 64) && (BW == 32 || BW == 64), SPX_E_CONFIG,
+                "the backward kernels take an element mask with head dim 64 and query and key blocks of 32 / 64 (got %d, %d, %d)", E, BH, BW);
+    SPX_REQUIRE(Ns % 16 == 0 && aligned(mask, 16), SPX_E_ALIGN, "mask rows must be 16-byte aligned");
+    return 0;
+}
+
+static int attention_backward_q_impl(int dtype, const void* grad_out, const void* out, const void* q,
+                                     const void* k, const void* v, const float* row_lse,
+                                     void* grad_q, float* row_dot,
+                                     const int32_t* row_ptr, const int32_t* bcsr_idx, const uint8_t* mask, float inv_temperature,
+                                     int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
     SPX_REQUIRE(dtype == SPX_F16 || dtype == SPX_BF16, SPX_E_DTYPE,
                 "fused attention runs in float16 / bfloat16 (fp32 accumulate); got dtype %d", dtype);
     SPX_REQUIRE(grad_out && out && q && k && v && row_lse && grad_q && row_ptr && bcsr_idx, SPX_E_NULL,
@@ -2146,25 +2161,26 @@ extern "C" int spx_attention_backward_q(int dtype, const void* grad_out, const v
     SPX_REQUIRE(aligned(grad_out, 16) && aligned(out, 16) && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) &&
                 aligned(grad_q, 16) && aligned(row_lse, 4) && aligned(row_dot, 4), SPX_E_ALIGN,
                 "buffers must be 16-byte aligned");
+    if (const int rc = attention_bwd_check_mask(mask, Ns, E, BH, BW)) return rc;
     if (batch == 0) return 0;
     AttnParams p = {};
     p.q = q; p.k = k; p.v = v; p.out = const_cast<void*>(out);
-    p.row_ptr = row_ptr; p.bcsr_idx = bcsr_idx;
+    p.row_ptr = row_ptr; p.bcsr_idx = bcsr_idx; p.mask = mask;
     p.inv_t = inv_temperature;
     p.Nt = Nt; p.Ns = Ns; p.BH = BH;
     p.grad_out = grad_out; p.grad_q = grad_q; p.row_dot = row_dot; p.row_lse = const_cast<float*>(row_lse);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (mask || attention_bwd_wide_wins(BH, E, (int64_t)batch * (Nt / BH))) return launch_attention_bwd_row_wide(dtype, p, batch, BW, st);
     if (dtype == SPX_F16) return launch_attention_bwd_row_rc<_Float16>(p, batch, BW, E, st);
     return launch_attention_bwd_row_rc<bf16_t>(p, batch, BW, E, st);
 }
 
-extern "C" int spx_attention_backward_kv_recompute(int dtype, const void* grad_out, const void* q, const void* k,
-                                                   const void* v, const float* row_lse, const float* row_dot,
-                                                   void* grad_k, void* grad_v,
-                                                   const int32_t* col_ptr, const void* bcsc_idx, int idx_kind,
-                                                   float inv_temperature,
-                                                   int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
-    using namespace spx;
+static int attention_backward_kv_impl(int dtype, const void* grad_out, const void* q, const void* k,
+                                      const void* v, const float* row_lse, const float* row_dot,
+                                      void* grad_k, void* grad_v,
+                                      const int32_t* col_ptr, const void* bcsc_idx, int idx_kind,
+                                      const uint8_t* mask, float inv_temperature,
+                                      int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
     SPX_REQUIRE(dtype == SPX_F16 || dtype == SPX_BF16, SPX_E_DTYPE,
                 "fused attention runs in float16 / bfloat16 (fp32 accumulate); got dtype %d", dtype);
     SPX_REQUIRE(grad_out && q && k && v && row_lse && row_dot && grad_k && grad_v && col_ptr && bcsc_idx, SPX_E_NULL,
@@ -2173,22 +2189,65 @@ extern "C" int spx_attention_backward_kv_recompute(int dtype, const void* grad_o
                 "the key / value gradient kernel walks a BCSC index (got index kind %d)", idx_kind);
     SPX_REQUIRE(Nt > 0 && Ns > 0 && BH > 0 && BW > 0 && Nt % BH == 0 && Ns % BW == 0, SPX_E_SHAPE,
                 "mask shape (%d,%d) is not a multiple of the block (%d,%d)", Nt, Ns, BH, BW);
-    SPX_REQUIRE(attention_bwd_col_rc_supported(BH, BW, E), SPX_E_CONFIG,
+    SPX_REQUIRE(mask || attention_bwd_col_rc_supported(BH, BW, E), SPX_E_CONFIG,
                 "the recomputing key / value gradient kernel covers query blocks 32/64/128, key blocks 32/64/128 and head dims 64/128 with BH * E >= 32 * BW and BH <= 2 * BW (got %d, %d, %d)", BH, BW, E);
     SPX_REQUIRE(batch >= 0 && batch <= 65535, SPX_E_SHAPE, "batch %d out of range", batch);
     SPX_REQUIRE(aligned(grad_out, 16) && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(row_lse, 4) &&
                 aligned(row_dot, 4) && aligned(grad_k, 16) && aligned(grad_v, 16), SPX_E_ALIGN, "buffers must be 16-byte aligned");
+    if (const int rc = attention_bwd_check_mask(mask, Ns, E, BH, BW)) return rc;
     if (batch == 0) return 0;
     AttnParams p = {};
     p.q = q; p.k = k; p.v = v;
     p.inv_t = inv_temperature;
     p.Nt = Nt; p.Ns = Ns; p.BH = BH;
     p.grad_out = grad_out; p.row_dot = const_cast<float*>(row_dot); p.row_lse = const_cast<float*>(row_lse);
+    p.mask = mask;
     p.col_ptr = col_ptr; p.bcsc_idx = bcsc_idx; p.bcsc_wide = idx_kind == SPX_IDX_BCSC_I64;
     p.grad_k = grad_k; p.grad_v = grad_v;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (mask || attention_bwd_wide_wins(BW, E, (int64_t)batch * (Ns / BW))) return launch_attention_bwd_col_wide(dtype, p, batch, BW, st);
     if (dtype == SPX_F16) return launch_attention_bwd_col_rc<_Float16>(p, batch, BW, E, st);
     return launch_attention_bwd_col_rc<bf16_t>(p, batch, BW, E, st);
+}
+
+}  // namespace spx
+
+extern "C" int spx_attention_backward_q(int dtype, const void* grad_out, const void* out, const void* q,
+                                        const void* k, const void* v, const float* row_lse,
+                                        void* grad_q, float* row_dot,
+                                        const int32_t* row_ptr, const int32_t* bcsr_idx, float inv_temperature,
+                                        int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
+    return spx::attention_backward_q_impl(dtype, grad_out, out, q, k, v, row_lse, grad_q, row_dot, row_ptr, bcsr_idx, nullptr,
+                                          inv_temperature, batch, Nt, Ns, E, BH, BW, stream);
+}
+
+extern "C" int spx_attention_backward_q_masked(int dtype, const void* grad_out, const void* out, const void* q,
+                                               const void* k, const void* v, const float* row_lse,
+                                               void* grad_q, float* row_dot,
+                                               const int32_t* row_ptr, const int32_t* bcsr_idx, const uint8_t* mask, float inv_temperature,
+                                               int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
+    return spx::attention_backward_q_impl(dtype, grad_out, out, q, k, v, row_lse, grad_q, row_dot, row_ptr, bcsr_idx, mask,
+                                          inv_temperature, batch, Nt, Ns, E, BH, BW, stream);
+}
+
+extern "C" int spx_attention_backward_kv_recompute(int dtype, const void* grad_out, const void* q, const void* k,
+                                                   const void* v, const float* row_lse, const float* row_dot,
+                                                   void* grad_k, void* grad_v,
+                                                   const int32_t* col_ptr, const void* bcsc_idx, int idx_kind,
+                                                   float inv_temperature,
+                                                   int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
+    return spx::attention_backward_kv_impl(dtype, grad_out, q, k, v, row_lse, row_dot, grad_k, grad_v, col_ptr, bcsc_idx, idx_kind,
+                                           nullptr, inv_temperature, batch, Nt, Ns, E, BH, BW, stream);
+}
+
+extern "C" int spx_attention_backward_kv_masked(int dtype, const void* grad_out, const void* q, const void* k,
+                                                const void* v, const float* row_lse, const float* row_dot,
+                                                void* grad_k, void* grad_v,
+                                                const int32_t* col_ptr, const void* bcsc_idx, int idx_kind,
+                                                const uint8_t* mask, float inv_temperature,
+                                                int batch, int Nt, int Ns, int E, int BH, int BW, spx_stream_t stream) {
+    return spx::attention_backward_kv_impl(dtype, grad_out, q, k, v, row_lse, row_dot, grad_k, grad_v, col_ptr, bcsc_idx, idx_kind,
+                                           mask, inv_temperature, batch, Nt, Ns, E, BH, BW, stream);
 }
 
 extern "C" int spx_attention_seqlen_forward(int dtype, const void* q, const void* k, const void* v, void* out,

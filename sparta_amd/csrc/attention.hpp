@@ -70,4 +70,9 @@ template <> struct AttnPack<bf16_t> {
 int launch_attention_wide(int dtype, const AttnParams& p, int batch, int BW, int E, hipStream_t st);
 int launch_attention_wide_seq(int dtype, const AttnParams& p, int batch, int E, hipStream_t st);
 
+// attention_bwd_wide.hip: backward kernels that recompute the probabilities, 32 queries or keys per wavefront, with
+// element masks; query and key blocks of 32 / 64, head dim 64
+int launch_attention_bwd_row_wide(int dtype, const AttnParams& p, int batch, int BW, hipStream_t st);
+int launch_attention_bwd_col_wide(int dtype, const AttnParams& p, int batch, int BW, hipStream_t st);
+
 }  // namespace spx

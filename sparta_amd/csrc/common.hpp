@@ -212,6 +212,11 @@ __device__ __forceinline__ void lds_direct_load16_at(const void* base, uint32_t 
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_wave_base), "v"(offset), "s"(s) : "memory", "m0");
 }
 
+// One global_load_lds_dword: four bytes per lane, 64 x 4 bytes at consecutive LDS addresses.
+__device__ __forceinline__ void lds_direct_load4(const void* g, uint32_t lds_wave_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_wave_base), "v"(g) : "memory", "m0");
+}
+
 // 16-byte accesses for data that is streamed once: the non-temporal hint keeps it from
 // displacing operands that other workgroups re-read from L2.
 __device__ __forceinline__ vec16 load16_stream(const void* p) {

@@ -582,45 +582,49 @@ public:
         at::AutoDispatchBelowADInplaceOrView below_autograd;
         Tensor out = at::empty(q.sizes(), q.options()), lse = at::empty({d.batch, Nt_}, q.options().dtype(at::kFloat));
         check_rc(spx_attention_forward_lse(d.code, contig(q), contig(k), contig(v), out.data_ptr(), (float*)lse.data_ptr(),
-                                           rows(), entries(), nullptr, inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_, stream_of(q)),
+                                           rows(), entries(), (const uint8_t*)device_ptr(mask_), inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_,
+                                           stream_of(q)),
                  "spx_attention_forward_lse");
         return {out, lse};
     }
-    // (query gradient, row constants)
+    // (query gradient, row constants); `mask`: the element mask of the forward pass
     std::pair<Tensor, Tensor> backward_q(const Tensor& grad, const Tensor& out, const Tensor& q, const Tensor& k, const Tensor& v,
-                                         const Tensor& lse) const {
+                                         const Tensor& lse, const std::optional<Tensor>& mask) const {
         py::gil_scoped_release nogil;
         const char* what = "spx_attention_backward_q";
         const Dims d = dims(what, q, k, v);
         require_like(what, "grad_out", grad, q);
         require_like(what, "out", out, q);
         require_numel(what, "row_lse", lse, (int64_t)d.batch * Nt_);
+        require_mask(what, mask);
         device_ptr(q);
         at::AutoDispatchBelowADInplaceOrView below_autograd;
         Tensor grad_q = at::empty(q.sizes(), q.options()), dot = at::empty({d.batch, Nt_}, q.options().dtype(at::kFloat));
-        check_rc(spx_attention_backward_q(d.code, contig(grad), contig(out), contig(q), contig(k), contig(v), (const float*)contig(lse),
-                                          grad_q.data_ptr(), (float*)dot.data_ptr(), rows(), entries(), inv_t_, d.batch, Nt_, Ns_,
-                                          d.E, BH_, BW_, stream_of(q)), what);
+        check_rc(spx_attention_backward_q_masked(
+                     d.code, contig(grad), contig(out), contig(q), contig(k), contig(v), (const float*)contig(lse), grad_q.data_ptr(),
+                     (float*)dot.data_ptr(), rows(), entries(), (const uint8_t*)(mask ? contig(*mask) : nullptr), inv_t_, d.batch, Nt_, Ns_,
+                     d.E, BH_, BW_, stream_of(q)), what);
         return {grad_q, dot};
     }
     // (key gradient, value gradient)
     std::pair<Tensor, Tensor> backward_kv(const Tensor& grad, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& lse,
-                                          const Tensor& dot) const {
+                                          const Tensor& dot, const std::optional<Tensor>& mask) const {
         py::gil_scoped_release nogil;
         const char* what = "spx_attention_backward_kv_recompute";
         const Dims d = dims(what, q, k, v);
         require_like(what, "grad_out", grad, q);
         require_numel(what, "row_lse", lse, (int64_t)d.batch * Nt_);
         require_numel(what, "row_dot", dot, (int64_t)d.batch * Nt_);
+        require_mask(what, mask);
         if (!col_ptr_.has_value() || !bcsc_.has_value()) throw ValueFailure("the column-side kernel needs the BCSC index");
         device_ptr(q);
         at::AutoDispatchBelowADInplaceOrView below_autograd;
         Tensor grad_k = at::empty(k.sizes(), k.options()), grad_v = at::empty(k.sizes(), k.options());
-        check_rc(spx_attention_backward_kv_recompute(
+        check_rc(spx_attention_backward_kv_masked(
                      d.code, contig(grad), contig(q), contig(k), contig(v), (const float*)contig(lse), (const float*)contig(dot),
                      grad_k.data_ptr(), grad_v.data_ptr(), (const int32_t*)device_ptr(col_ptr_), device_ptr(bcsc_),
-                     bcsc_->scalar_type() == at::kLong ? SPX_IDX_BCSC_I64 : SPX_IDX_BCSC_I32, inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_,
-                     stream_of(q)), what);
+                     bcsc_->scalar_type() == at::kLong ? SPX_IDX_BCSC_I64 : SPX_IDX_BCSC_I32, (const uint8_t*)(mask ? contig(*mask) : nullptr),
+                     inv_t_, d.batch, Nt_, Ns_, d.E, BH_, BW_, stream_of(q)), what);
         return {grad_k, grad_v};
     }
 
@@ -645,6 +649,11 @@ private:
     static void require_like(const char* what, const char* name, const Tensor& t, const Tensor& q) {
         require_numel(what, name, t, q.numel());
         if (t.scalar_type() != q.scalar_type()) assertion(what, ": operand dtypes differ: ", name, " is ", t.dtype());
+    }
+    void require_mask(const char* what, const std::optional<Tensor>& mask) const {
+        if (!mask) return;
+        require_numel(what, "mask", *mask, (int64_t)Nt_ * Ns_);
+        if (mask->element_size() != 1) assertion(what, ": the element mask holds ", mask->dtype(), ", bytes are expected");
     }
     static void* contig(const Tensor& t) {
         if (!t.is_contiguous()) throw ValueFailure("sparta_amd kernels need contiguous tensors");
@@ -824,8 +833,10 @@ PYBIND11_MODULE(_native, m) {
         .def(py::init<Tensor, Tensor, std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>, double, int, int, int, int>())
         .def("forward", &AttentionKernel::forward)
         .def("forward_lse", &AttentionKernel::forward_lse)
-        .def("backward_q", &AttentionKernel::backward_q)
-        .def("backward_kv", &AttentionKernel::backward_kv)
+        .def("backward_q", &AttentionKernel::backward_q, py::arg("grad_out"), py::arg("out"), py::arg("q"), py::arg("k"), py::arg("v"),
+             py::arg("row_lse"), py::arg("mask") = py::none())
+        .def("backward_kv", &AttentionKernel::backward_kv, py::arg("grad_out"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("row_lse"),
+             py::arg("row_dot"), py::arg("mask") = py::none())
         .def("__deepcopy__", [](const AttentionKernel& k, const py::object&) { return std::make_shared<AttentionKernel>(k); });
     m.def("seqlen_attention", &seqlen_attention);
     m.def("moe_forward", &moe_forward);

@@ -71,6 +71,12 @@ class _FusedAttentionFunc(torch.autograd.Function):
         return None, grad_q if need_q else None, grad_k if need_k else None, grad_v if need_v else None
 
 
+# Training steps with an element mask recompute the probabilities from this many queries (batch x N_target) on:
+# 12 x 512 queries bf16 143 us a step with stored probabilities, 97 without (the host's part is smaller), 96 x 4096 fp16
+# 292 and 226.  Nothing smaller was in need of it.
+_MASKED_RECOMPUTE_QUERIES = 2048
+
+
 class _RecomputeAttentionFunc(torch.autograd.Function):
     """Training path that keeps no probabilities: the forward kernel records one number per
     query (the log-sum-exp of its score row), and the row-side and column-side backward
@@ -83,20 +89,23 @@ class _RecomputeAttentionFunc(torch.autograd.Function):
         # the backward kernels walk the same index even if the mask has been updated since
         ctx.indexes = op._sparse_port.indexes
         out, row_lse = op._fused_forward_lse(q, k, v)
-        ctx.save_for_backward(q, k, v, out, row_lse)
+        # the element mask of this forward pass: the backward kernels read it again, and the caller's tensor
+        # may hold the next mask by then
+        mask = op._element_mask()
+        ctx.save_for_backward(q, k, v, out, row_lse, None if mask is None else mask.clone())
         ctx.op = op
         return out
 
     @staticmethod
     def backward(ctx, grad_out: torch.Tensor):
-        q, k, v, out, row_lse = ctx.saved_tensors
+        q, k, v, out, row_lse, mask = ctx.saved_tensors
         op = ctx.op
         grad_out = grad_out.detach().contiguous()
         need_q, need_k, need_v = ctx.needs_input_grad[1:4]
-        grad_q, row_dot = op._recompute_backward_q(grad_out, out, q, k, v, row_lse, ctx.indexes)
+        grad_q, row_dot = op._recompute_backward_q(grad_out, out, q, k, v, row_lse, ctx.indexes, mask)
         grad_k = grad_v = None
         if need_k or need_v:
-            grad_k, grad_v = op._recompute_backward_kv(grad_out, q, k, v, row_lse, row_dot, ctx.indexes)
+            grad_k, grad_v = op._recompute_backward_kv(grad_out, q, k, v, row_lse, row_dot, ctx.indexes, mask)
         return None, grad_q if need_q else None, grad_k if need_k else None, grad_v if need_v else None
 
 
@@ -106,10 +115,10 @@ class SparseAttention(OperatorBase):
         fused: run the single fused forward kernel when autograd is not recording
             (default True).  The three-operator pipeline is always built as well and
             is used whenever gradients are needed.
-        recompute: with a mask that is uniform inside its blocks, train without storing
-            the probabilities (default True): the backward kernels recompute them from
-            q, k and one number per query.  Masks with partly live blocks, and
-            `recompute=False`, keep the probabilities of the live blocks for the backward pass.
+        recompute: with a mask that is uniform inside its blocks, or with head dim 64, train
+            without storing the probabilities (default True): the backward kernels recompute
+            them from q, k and one number per query.  Masks with partly live blocks and other
+            head dims, and `recompute=False`, keep the probabilities of the live blocks for the backward pass.
         fused_tile_cfg: tile configuration of the fused kernel (0 = the library's choice;
             see spx_tile_cfg_info for the others).
 
@@ -177,14 +186,15 @@ class SparseAttention(OperatorBase):
         return all(hasattr(c, 'backward_B') for c in ctxs)
 
     def _recompute_supported(self, query: torch.Tensor) -> bool:
-        """The kernels that recompute the probabilities cover block-level masks, 3-D 16-bit
-        inputs and the block shapes of both backward kernels, and walk both indexes."""
+        """The kernels that recompute the probabilities cover 3-D 16-bit inputs and the block
+        shapes of both backward kernels, with head dim 64 element masks as well, and walk both indexes."""
         indexes = self._sparse_port.indexes
         BH, BW, E = indexes.block_H, indexes.block_W, query.shape[-1]
         return (query.dim() == 3 and BH in (32, 64, 128) and BW in (32, 64, 128) and E in (64, 128)
                 and BW * E // 8 >= BH * 4 and BH * E >= 32 * BW and BH <= 2 * BW
                 and getattr(indexes, 'col_ptr', None) is not None and getattr(indexes, 'row_ptr', None) is not None
-                and self._element_mask() is None)
+                and (self._element_mask() is None
+                     or (E == 64 and max(BH, BW) <= 64 and query.shape[0] * self._Nt >= _MASKED_RECOMPUTE_QUERIES)))
 
     def _check_operands(self, what: str, indexes, batch: int, E: int, q_like=(), kv_like=(), rows=(),
                         probs=(), nnz=None):
@@ -219,13 +229,13 @@ class SparseAttention(OperatorBase):
         """(output, log-sum-exp per query) from spx_attention_forward_lse."""
         return self._launcher().forward_lse(q, k, v)
 
-    def _recompute_backward_q(self, grad_out, out, q, k, v, row_lse, indexes=None):
-        """(query gradient, row constants) from spx_attention_backward_q."""
-        return self._launcher(indexes).backward_q(grad_out, out, q, k, v, row_lse)
+    def _recompute_backward_q(self, grad_out, out, q, k, v, row_lse, indexes=None, mask=None):
+        """(query gradient, row constants) from spx_attention_backward_q, or its form with an element mask."""
+        return self._launcher(indexes).backward_q(grad_out, out, q, k, v, row_lse, mask)
 
-    def _recompute_backward_kv(self, grad_out, q, k, v, row_lse, row_dot, indexes=None):
-        """(key gradient, value gradient) from spx_attention_backward_kv_recompute."""
-        return self._launcher(indexes).backward_kv(grad_out, q, k, v, row_lse, row_dot)
+    def _recompute_backward_kv(self, grad_out, q, k, v, row_lse, row_dot, indexes=None, mask=None):
+        """(key gradient, value gradient) from spx_attention_backward_kv_recompute, or its form with an element mask."""
+        return self._launcher(indexes).backward_kv(grad_out, q, k, v, row_lse, row_dot, mask)
 
     def _element_mask(self):
         indexes = self._sparse_port.indexes
