@@ -17,7 +17,7 @@ namespace spx {
 // registers, so the 32-query accumulators fit 128 registers at head dim 64 and four wavefronts
 // share a SIMD.  Per wavefront and 32 x 64 scores: 16 MFMAs of 32 clocks (+ 8 small ones), 32 quarter-rate
 // exponentials of 16 clocks and about 85 other vector instructions of 4: vector issue bounds the kernel
-// (850 against 580 clocks), 26 us at 32 x 12 x 1024 x 64 with mixed lengths, which takes 63 - 65 us (530 TFLOP/s).
+// (850 against 580 clocks), 26 us at 32 x 12 x 1024 x 64 with mixed lengths, which takes 56 us (64 before the work was ordered; 610 TFLOP/s).
 // Measured and left out: one 32-key tile at a time, exponentials under the next tile's MFMAs (+3 %).  Both tiles keep rows of E elements without padding; the 16-byte chunks of a row
 // are XORed by a function of the row (k_swizzle, v_swizzle) for which the 16 lanes of a
 // fragment read and the 32 lanes of a transpose read cover all 64 banks.
@@ -30,20 +30,58 @@ constexpr int attn_wide_smem(int BW, int E, int waves) {
     return tiles > rows ? tiles : rows;
 }
 
-// The batch entry that workgroup entry `rank` works on when the entries are taken longest
-// first, within groups of 64 (the lengths of a group sit in the lanes of the wavefront).
-__device__ __forceinline__ int seqlen_ranked_entry(const int32_t* seqlens, int entries, int rank) {
-    const int first = rank & ~63;
+// Sequence-length mode: what work item `slot` of XCD `xcd` is.  The (entry, head) pairs are dealt out to the XCDs longest
+// entry first, and an XCD walks the query blocks that hold positions of its pairs before the ones that only get zeros:
+// those are over in no time, and between the others they kept a third of the slots from work (32 x 12 x 1024 with mixed
+// lengths: 2300 of 3650 wavefronts were at it half way through the launch).  Groups of 64 entries at a time, their
+// lengths in the lanes of the wavefront.
+struct SeqWork {
+    int64_t b;      // entry * heads + head
+    int br, len;    // query block; br * ROWS >= len: rows of zeros
+};
+template <int ROWS>
+__device__ __forceinline__ bool seqlen_work(const AttnParams& p, int entries, int nbr, int slot, int xcd, SeqWork& w) {
+    const int per_group = 8 * p.heads * nbr;   // 64 entries: 64 * heads / 8 pairs on an XCD
+    const int first = slot / per_group * 64;
+    int t = slot % per_group;
     const int n = entries - first < 64 ? entries - first : 64;
     const int lane = lane_id();
-    const int mine = lane < n ? seqlens[first + lane] : 0;
-    int ahead = 0;
+    int mine = -1;
+    if (lane < n) {
+        mine = p.seqlens[first + lane];
+        mine = mine < 0 ? 0 : mine > p.Ns ? p.Ns : mine;
+    }
+    int rank = 0;   // lanes without an entry stay behind all others
     for (int j = 0; j < n; ++j) {
         const int other = __builtin_amdgcn_readlane(mine, j);
-        ahead += (other > mine || (other == mine && j < lane)) ? 1 : 0;
+        rank += (other > mine || (other == mine && j < lane)) ? 1 : 0;
     }
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < n && ahead == (rank & 63));
-    return first + __builtin_ctzll(hit);
+    if (lane >= n) rank = lane;
+    // from here on lane r holds the r-th longest entry
+    const int len = __builtin_amdgcn_ds_permute(rank * 4, mine), id = __builtin_amdgcn_ds_permute(rank * 4, lane);
+    const int busy = len > 0 ? (len + ROWS - 1) / ROWS : 0;
+    const int pair0 = (first + lane) * p.heads;
+    const int lo = (pair0 - xcd + 7) >> 3, hi = (pair0 + p.heads - xcd + 7) >> 3;   // its pairs 8 k + xcd
+    const int pairs = lane < n ? hi - lo : 0;
+    int share = pairs * busy, upto = wave_inclusive_scan(share), blocks = busy, skip = 0;
+    const int total = __builtin_amdgcn_readlane(upto, 63);
+    if (t >= total) {
+        t -= total;
+        blocks = nbr - busy;
+        skip = busy;
+        share = pairs * blocks;
+        upto = wave_inclusive_scan(share);
+    }
+    const uint64_t past = __builtin_amdgcn_ballot_w64(upto > t);
+    if (past == 0) return false;
+    const int r = __builtin_ctzll(past);
+    t -= __builtin_amdgcn_readlane(upto - share, r);
+    const int of = __builtin_amdgcn_readlane(blocks, r);
+    const int pair = 8 * (__builtin_amdgcn_readlane(lo, r) + t / of) + xcd;
+    w.b = (int64_t)(first + __builtin_amdgcn_readlane(id, r)) * p.heads + pair % p.heads;
+    w.br = __builtin_amdgcn_readlane(skip, r) + t % of;
+    w.len = __builtin_amdgcn_readlane(len, r);
+    return true;
 }
 
 template <typename T, int BW, int E, int WAVES, bool HAS_MASK, bool SEQ = false>
@@ -69,21 +107,30 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 && BW <= 64 ? (HAS_MASK ? 3 : 4
     // workgroup L runs on XCD L % 8: give each XCD whole batch*head entries
     const int L = blockIdx.x;
     const int slot = L >> 3;
-    int64_t b = (slot / nbr) * 8 + (L & 7);
-    const int br = slot % nbr;
-    if (b >= batch) return;
+    int64_t b;
+    int br, seq_len = 0;
+    if constexpr (SEQ) {
+        SeqWork w;
+        if (!seqlen_work<32 * WAVES>(p, batch / p.heads, nbr, slot, L & 7, w)) return;
+        b = w.b;
+        br = w.br;
+        seq_len = w.len;
+        if (br * (32 * WAVES) >= seq_len) {   // rows of zeros
+            const int rows = p.Nt - br * (32 * WAVES) < 32 * WAVES ? p.Nt - br * (32 * WAVES) : 32 * WAVES;
+            char* dst = reinterpret_cast<char*>(reinterpret_cast<T*>(p.out) + (b * p.Nt + br * (32 * WAVES)) * E);
+            for (int v = threadIdx.x; v < rows * VPR; v += NT)
+                __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4*>(dst + v * 16));
+            return;
+        }
+    } else {
+        b = (slot / nbr) * 8 + (L & 7);
+        br = slot % nbr;
+        if (b >= batch) return;
+    }
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, h2 = lane >> 5;
-
-    int seq_len = 0;
-    if constexpr (SEQ) {
-        const int entry = seqlen_ranked_entry(p.seqlens, batch / p.heads, (int)b / p.heads);
-        b = (int64_t)entry * p.heads + (int)b % p.heads;
-        seq_len = p.seqlens[entry];
-        seq_len = seq_len < 0 ? 0 : (seq_len > p.Ns ? p.Ns : seq_len);
-    }
 
     const T* Q = reinterpret_cast<const T*>(p.q) + b * (int64_t)p.Nt * E;
     const T* Kg = reinterpret_cast<const T*>(p.k) + b * (int64_t)p.Ns * E;
@@ -133,7 +180,8 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 && BW <= 64 ? (HAS_MASK ? 3 : 4
     const int v_src = VT + v_key * ROW + (lane & 1) * 8;
 
     const int e_begin = SEQ ? 0 : p.row_ptr[br];
-    const int n_blk = (SEQ ? (br * (32 * WAVES) < seq_len ? (seq_len + BW - 1) / BW : 0) : p.row_ptr[br + 1]) - e_begin;
+    const int n_blk = (SEQ ? (seq_len + BW - 1) / BW : p.row_ptr[br + 1]) - e_begin;
+    const bool idle = SEQ && row0 >= seq_len;   // this wavefront only brings tiles: its rows are zeros
     int bc_vec = 0;
     if constexpr (!SEQ) {
         if (lane < n_blk) bc_vec = p.bcsr_idx[e_begin + lane] & 0xffff;
@@ -181,6 +229,7 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 && BW <= 64 ? (HAS_MASK ? 3 : 4
             __syncthreads();
         }
 
+        if (idle) continue;
         // ---- S^T tiles: 32 keys x this wave's 32 queries ------------------------------------
         f32x16 s[KT];
 #pragma unroll

@@ -1,0 +1,41 @@
+"""Sequence-length attention where its work is dealt out longest entry first: entries in groups of 64,
+pairs of (entry, head) over eight XCDs, query blocks without a position at the end."""
+import numpy as np
+import pytest
+import torch
+
+from sparta_amd.nn import SeqlenDynamicSparseAttention
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('E', [64, 128])
+@pytest.mark.parametrize('batch,heads,N,lens', [
+    (65, 3, 256, 'mixed'),      # a second group with one entry
+    (70, 5, 288, 'mixed'),      # N is no multiple of the 128 queries of a workgroup
+    (64, 6, 256, 'none'),       # nothing but zeros
+    (64, 6, 256, 'full'),
+    (48, 8, 256, 'one'),        # one position each, one entry that is full
+    (3, 16, 992, 'mixed'),
+    (130, 3, 256, 'clamped'),   # lengths below 0 and above N
+])
+def test_longest_first(batch, heads, N, lens, E, gpu):
+    assert batch * heads * ((N + 127) // 128) >= 384   # the wide kernel takes it
+    rng = np.random.default_rng(11)
+    n = {'mixed': rng.integers(0, N + 1, batch), 'none': np.zeros(batch, int), 'full': np.full(batch, N),
+         'one': np.ones(batch, int), 'clamped': rng.integers(-N, 2 * N, batch)}[lens]
+    if lens == 'one':
+        n[5] = N
+    g = torch.Generator(device=gpu).manual_seed(3)
+    q, k, v = (torch.randn((batch, heads, N, E), generator=g, device=gpu).half() for _ in range(3))
+    q = q / E ** 0.5
+    got = SeqlenDynamicSparseAttention(global_mode=False)(q, k, v, torch.from_numpy(n.astype(np.int32)).to(gpu)).float()
+    for b in range(batch):
+        m = int(min(max(n[b], 0), N))
+        assert float(got[b, :, m:].abs().max()) == 0.0 if m < N else True
+        if m:
+            s = torch.matmul(q[b, :, :m].float(), k[b, :, :m].float().transpose(1, 2).contiguous())
+            want = torch.matmul(torch.softmax(s, -1), v[b, :, :m].float())
+            # probabilities and result rounded to 11 bits, 2^-12 of the value each at most
+            rel = float((got[b, :, :m] - want).norm() / want.norm())
+            assert rel <= 1e-3, f'entry {b} of length {m}: {rel:.2e}'
