@@ -1964,12 +1964,24 @@ static int launch_attention_seqlen(const SeqlenParams& p, int batch_heads, int E
 }  // namespace spx
 
 namespace spx {
+// Wide kernel or pipelined kernel.  Pipelined / wide, us:
+//   head dim 128: 96 x 4096 fp16 130 / 112, 12 x 4096 29 / 22, 12 x 4096 bf16 37 / 28, 12 x 1024 11.6 / 10.3, 12 x 256 4.2 / 4.3;
+//   element masks: 96 x 4096 fp16 55 / 48.5, 96 x 2048 bf16 45.5 / 34, 24 x 4096 19.8 / 15.0, 32 x 32 blocks 96 x 4096 70 / 58, but
+//   12 x 2048 fp16 17.9 / 21.2, 12 x 512 5.1 / 5.3 (few workgroups: the barrier of every 32 keys shows);
+//   neither: fp16 96 x 4096 70.9 / 65.9 (32 x 32 blocks 62.6 / 56.4), 64 x 4096 43.0 / 40.6, 96 x 2048 29.3 / 29.7, 24 x 4096 18.6 / 19.9; bf16
+//   96 x 4096 72.9 / 62.8, 96 x 2048 30.2 / 28.1, 36 x 4096 32.5 / 31.0, 24 x 4096 21.3 / 21.4.
+static bool attention_wide_wins(int dtype, const uint8_t* mask, int64_t queries, int E) {
+    if (E == 128) return true;
+    if (mask) return queries >= 65536;
+    return queries >= (dtype == SPX_F16 ? 262144 : 131072);
+}
+
 static int attention_forward_impl(int dtype, const void* q, const void* k, const void* v, void* out, float* row_lse,
                                   const int32_t* row_ptr, const int32_t* bcsr_idx,
                                   const uint8_t* mask, float inv_temperature,
                                   int batch, int Nt, int Ns, int E, int BH, int BW,
                                   int tile_cfg, spx_stream_t stream) {
-    SPX_REQUIRE(tile_cfg >= 0 && tile_cfg <= 3, SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
+    SPX_REQUIRE(tile_cfg >= -1 && tile_cfg <= 3, SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
     SPX_REQUIRE(dtype == SPX_F16 || dtype == SPX_BF16, SPX_E_DTYPE,
                 "fused attention runs in float16 / bfloat16 (fp32 accumulate); got dtype %d", dtype);
     SPX_REQUIRE(q && k && v && out && row_ptr && bcsr_idx, SPX_E_NULL, "a required buffer is NULL");
@@ -1991,13 +2003,15 @@ static int attention_forward_impl(int dtype, const void* q, const void* k, const
     p.col_ptr = nullptr; p.bcsc_idx = nullptr; p.bcsc_wide = 0; p.grad_k = nullptr; p.grad_v = nullptr;
     p.seqlens = nullptr; p.heads = 1; p.row_lse = row_lse;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    // tile_cfg 0: the pipelined kernel where it applies; 1: one-buffer kernel; 2: pipelined kernel;
-    // 3: pipelined kernel on 32x32x16 MFMAs (one wavefront per 32 queries; measured within a few
-    // per cent of 2 either way, so 0 keeps 2)
-    if (tile_cfg == 0) tile_cfg = attention_v2_supported(BH, BW, E) ? 2 : 1;
-    if (tile_cfg == 3) {
-        return launch_attention_wide(dtype, p, batch, BW, E, st);
+    // tile_cfg 0: the wide or the pipelined kernel where they apply (-1: one of the two); 1: one-buffer kernel; 2: pipelined
+    // kernel; 3: wide kernel (32 queries per wavefront), which reads an element mask 16 bytes at a time
+    const bool wide_reads = !mask || (Ns % 16 == 0 && aligned(mask, 16));
+    if (tile_cfg <= 0) {
+        if (!attention_v2_supported(BH, BW, E)) tile_cfg = 1;
+        else tile_cfg = wide_reads && attention_wide_supported(BH, BW, E) && attention_wide_wins(dtype, mask, (int64_t)batch * Nt, E) ? 3 : 2;
     }
+    if (tile_cfg == 3 && !wide_reads && attention_v2_supported(BH, BW, E)) tile_cfg = 2;
+    if (tile_cfg == 3) return launch_attention_wide(dtype, p, batch, BW, E, st);
     if (tile_cfg == 2) {
         if (dtype == SPX_F16) return launch_attention_v2<_Float16>(p, batch, BW, E, st);
         return launch_attention_v2<bf16_t>(p, batch, BW, E, st);
@@ -2012,6 +2026,7 @@ extern "C" int spx_attention_forward(int dtype, const void* q, const void* k, co
                                      const uint8_t* mask, float inv_temperature,
                                      int batch, int Nt, int Ns, int E, int BH, int BW,
                                      int tile_cfg, spx_stream_t stream) {
+    SPX_REQUIRE(tile_cfg >= 0, SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
     return spx::attention_forward_impl(dtype, q, k, v, out, nullptr, row_ptr, bcsr_idx, mask, inv_temperature,
                                        batch, Nt, Ns, E, BH, BW, tile_cfg, stream);
 }
@@ -2025,7 +2040,7 @@ extern "C" int spx_attention_forward_lse(int dtype, const void* q, const void* k
     SPX_REQUIRE(attention_v2_supported(BH, BW, E), SPX_E_CONFIG,
                 "the forward kernel that records the row statistic covers query blocks 32/64/128, key blocks 32/64/128 and head dims 64/128 (got %d, %d, %d)", BH, BW, E);
     return attention_forward_impl(dtype, q, k, v, out, row_lse, row_ptr, bcsr_idx, mask, inv_temperature,
-                                  batch, Nt, Ns, E, BH, BW, 2, stream);
+                                  batch, Nt, Ns, E, BH, BW, -1, stream);
 }
 
 extern "C" int spx_attention_forward_train(int dtype, const void* q, const void* k, const void* v, void* out,
@@ -2274,7 +2289,8 @@ extern "C" int spx_attention_seqlen_forward(int dtype, const void* q, const void
         ap.Nt = N; ap.Ns = N; ap.BH = N % 64 == 0 ? 64 : 32;
         ap.seqlens = seqlens; ap.heads = heads;
         // 128 queries per workgroup read every key tile half as often, but fill the chip and cover their
-        // latencies only with enough work.  fp16 us, 64-query workgroups / wide: 32 x 12 x 1024 x 64 81 / 63,
+        // latencies only with enough work.  fp16 us, 64-query workgroups / wide (the first two since measured again at 56
+        // and 106, with the work ordered): 32 x 12 x 1024 x 64 81 / 63,
         // head dim 128 133 / 111; 16 x 12 x 512 19.5 / 14.2; 32 x 12 x 256 14.1 / 12.0; at 384 workgroups 20.2 / 15.8
         // (3 x 16 x 992) and 29.0 / 25.8 (2 x 12 x 2048); at 192 12.6 / 14.3 (2 x 12 x 1024) and 9.4 / 9.8
         // (4 x 12 x 512); short sequences 9.9 / 11.1 (32 x 16 x 192) and 6.4 / 7.7 (32 x 12 x 128).

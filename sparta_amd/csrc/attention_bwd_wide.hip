@@ -5,76 +5,6 @@
 
 namespace spx {
 
-// ---- tiles of 32 rows in LDS -------------------------------------------------------------------
-// A tile keeps the rows of 32 queries or keys as they are in memory, 2 E bytes each; the 16-byte chunks of a row
-// are XORed by `swizzle(row)`.  Both ways a tile is read then cover all 64 banks: the 16 rows of a pass of fragment
-// reads (a chunk per row) and the four rows of a pass of transpose reads (64 bytes of each).
-struct AttnTile {
-    static constexpr int E = 64, ROW = E * 2;
-    static constexpr int BYTES = 32 * ROW;
-    static constexpr int LOADS = BYTES / 1024;    // direct loads of 64 x 16 bytes
-    static constexpr int EC = E / 16, ET = E / 32;
-    __device__ static int swizzle(int row) { return ((row & 2) << 1) | ((row >> 2) & 3); }
-    int l32, h2;
-    uint32_t fill;      // source offset of load 0; load i: XORed by fill_xor(i) and 1 KB further
-    int row;            // row l32, chunk h2: fragment c (16 columns) is at row ^ (c * 32)
-    int tr[2];          // transpose reads: k-rows h2 * 4 .. + 3, and 8 further; column tile t at tr ^ (t * 64)
-    __device__ explicit AttnTile(int lane) {
-        l32 = lane & 31;
-        h2 = lane >> 5;
-        const int r = lane / (ROW / 16);
-        fill = r * ROW + (((lane % (ROW / 16)) ^ swizzle(r)) * 16);
-        row = l32 * ROW + ((h2 ^ swizzle(l32)) * 16);
-        const int k = h2 * 4 + ((lane & 15) >> 2), chunk = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
-#pragma unroll
-        for (int hi = 0; hi < 2; ++hi)
-            tr[hi] = (k + 8 * hi) * ROW + ((chunk ^ swizzle(k + 8 * hi)) * 16) + (lane & 1) * 8;
-    }
-    __device__ static constexpr uint32_t fill_xor(int i) { return (i & 1) * 32; }
-    // loads first .. first + N - 1 of the 32 rows at `rows` into the tile at LDS address `to`
-    template <int N> __device__ __forceinline__ void request(const void* rows, int first, uint32_t to) const {
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            lds_direct_load16_at(reinterpret_cast<const char*>(rows) + (first + i) * 1024, fill ^ fill_xor(first + i), to + (first + i) * 1024);
-    }
-    template <typename Frag> __device__ __forceinline__ Frag row_frag(const char* tile, int c) const {
-        return *reinterpret_cast<const Frag*>(tile + (row ^ (c * 32)));
-    }
-    template <typename Frag> __device__ __forceinline__ Frag tr_frag(const char* tile, int t, int u) const {
-        typedef short s16x8 __attribute__((ext_vector_type(8)));
-        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + (tr[0] ^ (t * 64)) + u * 16 * ROW));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + (tr[1] ^ (t * 64)) + u * 16 * ROW));
-        return __builtin_bit_cast(Frag, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    }
-};
-
-// 32 rows x 32 columns of an accumulated transpose (lane: row l32 of the result, registers: columns) to memory:
-// through LDS to whole 16-byte vectors.
-template <typename T>
-__device__ __forceinline__ void store_rows32(char* tile, T* dst, const f32x16 (&acc)[AttnTile::ET], int lane) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
-    typedef float f32x8 __attribute__((ext_vector_type(8)));
-    constexpr int E = AttnTile::E, PP = E * 2 + 16, VPR = E / 8;
-    const int l32 = lane & 31, h2 = lane >> 5;
-#pragma unroll
-    for (int t = 0; t < E / 32; ++t)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            f32x8 v = {};
-#pragma unroll
-            for (int x = 0; x < 4; ++x) v[x] = acc[t][4 * a + x];
-            *reinterpret_cast<uint64_t*>(tile + l32 * PP + (t * 32 + a * 8 + h2 * 4) * 2) = __builtin_bit_cast(u64x2, AttnPack<T>::pack(v))[0];
-        }
-#pragma unroll
-    for (int i = 0; i < 32 * VPR / 64; ++i) {
-        const int c = i * 64 + lane;
-        __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(tile + (c / VPR) * PP + (c % VPR) * 16),
-                                    reinterpret_cast<u32x4*>(reinterpret_cast<char*>(dst) + c * 16));
-    }
-}
-
 // ---- the two kernels ---------------------------------------------------------------------------------
 // One workgroup per block row (row side: dQ) or block column (column side: dK, dV) and batch entry, a wavefront per
 // 32 queries (keys).  The other side is walked in tiles of 32 rows, K and V or Q and dO, which go global -> LDS
@@ -97,19 +27,19 @@ __device__ __forceinline__ void store_rows32(char* tile, T* dst, const f32x16 (&
 // Left out, no gain: four stages, two stages, loads requested later in a stage, raised wave priority.
 constexpr int kBwdStages = 3;
 template <int WAVES, bool HAS_MASK, bool STATS> struct BwdLds {
-    static constexpr int MASK = 2 * AttnTile::BYTES;                          // 32 x 32 bytes per wavefront
+    static constexpr int MASK = 2 * AttnTile<64>::BYTES;                          // 32 x 32 bytes per wavefront
     static constexpr int STAT = MASK + (HAS_MASK ? WAVES * 1024 : 0);            // 32 + 32 floats per wavefront
     static constexpr int STAGE = STAT + (STATS ? WAVES * 256 : 0);
-    static constexpr int OUT = WAVES * 32 * (AttnTile::ROW + 16);                        // output rows, in the same space
+    static constexpr int OUT = WAVES * 32 * (AttnTile<64>::ROW + 16);                        // output rows, in the same space
     static constexpr int TOTAL = kBwdStages * STAGE > OUT ? kBwdStages * STAGE : OUT;
 };
 
 // ---- row side -----------------------------------------------------------------------------------
 template <typename T, int WAVES, bool HAS_MASK>
 __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_row_wide_kernel(AttnParams p, int nbr, int log_sub, int batch) {
-    typedef AttnTile Tile;
+    typedef AttnTile<64> Tile;
     typedef BwdLds<WAVES, HAS_MASK, false> Lds;
-    constexpr int E = Tile::E, EC = Tile::EC, ET = Tile::ET, NB = kBwdStages;
+    constexpr int E = 64, EC = Tile::EC, ET = Tile::ET, NB = kBwdStages;
     constexpr int LPT = 2 * Tile::LOADS / WAVES;             // tile loads of a wavefront and stage
     constexpr int LPW = LPT + (HAS_MASK ? 1 : 0);
     typedef typename MmaW<T>::frag Frag;
@@ -246,15 +176,15 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_ro
         if (i + 2 < n) step(i + 2, std::integral_constant<int, 2>());
     }
     __syncthreads();   // the tiles are dead: their space carries the output rows
-    store_rows32<T>(smem + wave * (32 * (E * 2 + 16)), reinterpret_cast<T*>(p.grad_q) + (b * p.Nt + row0) * E, qacc, lane);
+    store_rows32<T, E>(smem + wave * (32 * (E * 2 + 16)), reinterpret_cast<T*>(p.grad_q) + (b * p.Nt + row0) * E, qacc, lane);
 }
 
 // ---- column side --------------------------------------------------------------------------------
 template <typename T, int WAVES, bool HAS_MASK>
 __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_col_wide_kernel(AttnParams p, int nbc, int log_sub, int batch) {
-    typedef AttnTile Tile;
+    typedef AttnTile<64> Tile;
     typedef BwdLds<WAVES, HAS_MASK, true> Lds;
-    constexpr int E = Tile::E, EC = Tile::EC, ET = Tile::ET, NB = kBwdStages;
+    constexpr int E = 64, EC = Tile::EC, ET = Tile::ET, NB = kBwdStages;
     constexpr int LPT = 2 * Tile::LOADS / WAVES;
     constexpr int LPW = LPT + 1 + (HAS_MASK ? 1 : 0);
     typedef typename MmaW<T>::frag Frag;
@@ -420,8 +350,8 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_co
     __syncthreads();
     char* rows = smem + wave * (32 * (E * 2 + 16));
     const int64_t out = (b * p.Ns + key0) * E;
-    store_rows32<T>(rows, reinterpret_cast<T*>(p.grad_v) + out, vacc, lane);
-    store_rows32<T>(rows, reinterpret_cast<T*>(p.grad_k) + out, kacc, lane);
+    store_rows32<T, E>(rows, reinterpret_cast<T*>(p.grad_v) + out, vacc, lane);
+    store_rows32<T, E>(rows, reinterpret_cast<T*>(p.grad_k) + out, kacc, lane);
 }
 
 template <typename T, int WAVES, bool HAS_MASK>

@@ -106,3 +106,18 @@ def test_block_level_mask(dtype, H, N, bh, bw, gpu):
     q, k, v, g = (randn((H, N, 64), i, dtype)[1] for i in range(4))
     att, leaves = build(mask, bh, bw, q, k, v, gpu)
     check(step(att, leaves, g.to(gpu)), exact(leaves, g.to(gpu), torch.from_numpy(mask).to(gpu)), dtype, f'{H} x {N} {bh}x{bw}')
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('bh,bw', [(64, 64), (32, 32)])
+def test_element_mask_with_the_wide_forward_kernel(dtype, bh, bw, gpu, H=64, N=1024):
+    """65536 queries: the forward pass that records the row statistic is the one with 32 queries per wavefront."""
+    mask = np.tril(block_mask(N, N, bh, bw, 9, density=0.3) | np.kron(np.eye(N // bh), np.ones((bh, bw))).astype(np.uint8))
+    mask[70] = 0
+    q, k, v, g = (randn((H, N, 64), i, dtype)[1] for i in range(4))
+    att, leaves = build(mask, bh, bw, q, k, v, gpu)
+    m = torch.from_numpy(mask).to(gpu)
+    check(step(att, leaves, g.to(gpu)), exact(leaves, g.to(gpu), m), dtype, f'{dtype} {bh}x{bw}')
+    with torch.no_grad():
+        out = att(*leaves)
+    assert float(out[:, 70].abs().max()) == 0.0
