@@ -77,17 +77,20 @@ __device__ __forceinline__ Frag ring_frag(const char* part, int row0, int half, 
     }
 }
 
-// LDS layout: the ring, the output tile, then (when the launch gives it room) the launch order and the
-// column pointers.
+// LDS layout: the ring, the output tile, then the list of tiles.
 template <typename T, int TM, int BN, int NB, bool SWAP> struct RingLds {
     static constexpr int E16 = 16 / (int)sizeof(T);
     static constexpr int STAGE = (TM + BN) * 128;
     static constexpr int ROWS = SWAP ? TM : BN, COLS = SWAP ? BN : TM, LDE = COLS + E16;   // output tile
     static constexpr int TILE = ROWS * LDE * (int)sizeof(T);
-    static constexpr int TABLE = NB * STAGE + TILE;
+    static constexpr int LIST = NB * STAGE + TILE;
 };
 constexpr int kRingThreads = 320;     // four multiplying wavefronts and the loader
-constexpr int kRingTableMax = 1024;   // block-columns whose order and pointers fit the table (8 KB)
+constexpr int kRingTableMax = 1024;   // block-columns whose order and pointers fit the ring before it is filled (8 KB)
+constexpr int kRingListMax = 128;     // tiles of a workgroup that fit its list (2 KB)
+struct alignas(16) RingTile {
+    int m0, j, e0, n_blk;             // n_blk < 0: no tile
+};
 
 // The list of tiles of an XCD (workgroup L runs on XCD L % 8).  A unit is a panel of TM dense rows with
 // every `parts`-th block-column of the launch order (parts > 1: fewer panels than fill the XCDs evenly);
@@ -130,44 +133,56 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-    // launch order and column pointers in LDS: looking up a later tile takes no trip to memory
     const int n_rounds = (n_list + n_pos - 1) / n_pos;
-    const bool table = n_rounds > 1 && nb <= kRingTableMax;
-    int* const tab_ptr = reinterpret_cast<int*>(smem + Lds::TABLE);
-    int* const tab_order = tab_ptr + nb + 1;
-    if (table) {
-        for (int i = threadIdx.x; i <= nb; i += kRingThreads) tab_ptr[i] = p.ptr[i];
-        for (int i = threadIdx.x; i < nb; i += kRingThreads) tab_order[i] = p.sched ? p.sched[i] : i;
-        __syncthreads();
-    }
+    const bool listed = n_rounds > 1 && n_rounds <= kRingListMax, table = listed && nb <= kRingTableMax;
+    RingTile* const list = reinterpret_cast<RingTile*>(smem + Lds::LIST);
     struct Tile {
         int m0, j, e0, n_blk, n_st;
     };
-    // The r-th tile of this workgroup; false: none.
-    auto look_up = [&](int r, Tile& t) -> bool {
+    // launch order and column pointers while the list is made: in the ring, which is empty yet
+    int* const tab_ptr = reinterpret_cast<int*>(smem);
+    int* const tab_order = tab_ptr + nb + 1;
+    // The r-th tile of this workgroup.
+    auto look_up = [&](int r) __attribute__((always_inline)) -> RingTile {
+        const RingTile none = {0, 0, 0, -1};
         const int id = r * n_pos + (r & 1 ? n_pos - 1 - pos : pos);   // there and back along the list
-        if (id >= n_list) return false;
+        if (id >= n_list) return none;
         const int g = id / (l.group * l.cols), in = id - g * l.group * l.cols;
         const int left = n_units - g * l.group, size = left < l.group ? left : l.group;
         const int i = in / size;
         const int unit = (g * l.group + in - i * size) * 8 + xcd;
         const int mt = unit / l.parts;
         const int o = i * l.parts + unit - mt * l.parts;
-        if (o >= nb) return false;
-        t.m0 = mt * TM;
-        int e1;
+        if (o >= nb) return none;
+        const int j = table ? tab_order[o] : p.sched ? p.sched[o] : o;
+        const int* const ptr = table ? tab_ptr : p.ptr;
+        const int e0 = ptr[j];
+        return {mt * TM, j, e0, ptr[j + 1] - e0};
+    };
+    // All tiles of this workgroup at once, a thread each: what a wavefront then needs of the next one is a single read,
+    // where looking it up takes three divisions and three dependent reads between two tiles.  fp16 us before / after,
+    // 32 x 64 blocks, 64-row and 128-row tiles: 8192 x 768 -> 3072 at 10 % 28.1 / 21.3 and 22.2 / 20.3, 16384 x 512 -> 2048 at
+    // 20 % 37.1 / 29.2 and 28.4 / 27.0, 8192 x 768 -> 2304 at 20 % 24.7 / 20.4 and 20.4 / 18.5; with two tiles to a workgroup
+    // (8192 x 3072 -> 768) 17.0 / 16.5 and 14.1 / 14.6.
+    if (listed) {
         if (table) {
-            t.j = __builtin_amdgcn_readfirstlane(tab_order[o]);
-            t.e0 = __builtin_amdgcn_readfirstlane(tab_ptr[t.j]);
-            e1 = __builtin_amdgcn_readfirstlane(tab_ptr[t.j + 1]);
-        } else {
-            t.j = p.sched ? ((const_i32)p.sched)[o] : o;
-            t.e0 = ((const_i32)p.ptr)[t.j];
-            e1 = ((const_i32)p.ptr)[t.j + 1];
+            for (int i = threadIdx.x; i <= nb; i += kRingThreads) tab_ptr[i] = p.ptr[i];
+            for (int i = threadIdx.x; i < nb; i += kRingThreads) tab_order[i] = p.sched ? p.sched[i] : i;
+            __syncthreads();
         }
-        t.n_blk = e1 - t.e0;
+        for (int r = threadIdx.x; r < n_rounds; r += kRingThreads) list[r] = look_up(r);
+        __syncthreads();
+    }
+    auto tile_at = [&](int r, Tile& t) __attribute__((always_inline)) -> bool {
+        RingTile e;
+        if (listed) e = list[r];
+        else e = look_up(r);
+        t.n_blk = __builtin_amdgcn_readfirstlane(e.n_blk);
+        t.m0 = __builtin_amdgcn_readfirstlane(e.m0);
+        t.j = __builtin_amdgcn_readfirstlane(e.j);
+        t.e0 = __builtin_amdgcn_readfirstlane(e.e0);
         t.n_st = PAIR ? (t.n_blk + 1) >> 1 : t.n_blk * SPB;
-        return true;
+        return t.n_blk >= 0;
     };
 
     // Barriers, the same sequence in every wavefront: one per stage (its data has landed, and the slot
@@ -239,7 +254,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
                 if (++ld_round >= n_rounds) return;
                 const int m0 = ld.m0;
                 ld_st = 0;
-                if (!look_up(ld_round, ld)) ld.n_st = 0;
+                if (!tile_at(ld_round, ld)) ld.n_st = 0;
                 else if (ld.m0 != m0) set_rows(ld.m0);
             }
             if constexpr (PAIR) {
@@ -303,7 +318,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         uint32_t fill = (NB - 1) * STAGE;
         for (int r = 0; r < n_rounds; ++r) {
             Tile cur;
-            if (!look_up(r, cur)) continue;
+            if (!tile_at(r, cur)) continue;
             const int n_st = cur.n_st;
             for (int st = 0; st < n_st; ++st) {
                 // the stage has landed; the ones behind it may still be on their way
@@ -349,7 +364,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     uint32_t at = 0;
     for (int r = 0; r < n_rounds; ++r) {
         Tile cur;
-        if (!look_up(r, cur)) continue;
+        if (!tile_at(r, cur)) continue;
         // bias values fetched together, ahead of the walk
         float bias_m[MT][4], bias_n[NT][4];
 #pragma unroll
@@ -441,15 +456,19 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
     l.cols = (nb + l.parts - 1) / l.parts;
     const int64_t panel = (int64_t)TM * p.K * (int)sizeof(T);
     l.group = panel >= (2 << 20) ? 1 : (int)((2 << 20) / panel);
-    const int smem = Lds::TABLE + (nb <= kRingTableMax ? (2 * nb + 1) * 4 : 0);
-    constexpr int most = Lds::TABLE + (2 * kRingTableMax + 1) * 4;
-    static_assert(most <= 160 * 1024, "fits a CU");
-    int per_cu = 160 * 1024 / smem;
-    per_cu = per_cu > 4 ? 4 : per_cu;
+    constexpr int most = Lds::LIST + kRingListMax * (int)sizeof(RingTile);
+    static_assert(most <= 160 * 1024 && NB * Lds::STAGE >= (2 * kRingTableMax + 1) * 4, "fits a CU, and the tables the ring");
     // workgroups per XCD: as many as fit (the batch entries share the device)
     const int n_list = ((l.n_mtiles * l.parts + 7) / 8) * l.cols;   // the longest of the eight lists
-    int n_pos = 32 * per_cu / batch;
-    n_pos = n_pos < 1 ? 1 : n_pos > n_list ? n_list : n_pos;
+    int n_pos = 0, smem = most;
+    // (five where they fit: 64-row tiles of 2992 x 768 -> 3072 bf16 14.3 -> 11.9 us, 8192 x 3072 -> 768 fp16 16.5 -> 15.9)
+    for (int per_cu = 5; per_cu >= 1; --per_cu) {
+        n_pos = 32 * per_cu / batch;
+        n_pos = n_pos < 1 ? 1 : n_pos > n_list ? n_list : n_pos;
+        const int n_rounds = (n_list + n_pos - 1) / n_pos;
+        smem = Lds::LIST + (n_rounds > 1 && n_rounds <= kRingListMax ? n_rounds * (int)sizeof(RingTile) : 0);
+        if (per_cu * (int)round_up(smem, 1280) <= 160 * 1024) break;   // LDS is given out in pieces of 1280 bytes
+    }
     SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>), most, "spmm_ring_kernel");
     hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>), dim3(8 * n_pos, batch, 1), dim3(kRingThreads), smem, st, p, l);
     SPX_LAUNCH_CHECK("spmm_ring_kernel");

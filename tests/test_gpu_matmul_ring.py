@@ -55,3 +55,23 @@ def test_dispatch_of_few_rows_and_long_columns(dtype, blocks, M, K, N, sparsity,
     for compressed in (True, False):
         run_case(gpu, 'dsd', False, True, True, compressed, dtype, blocks, batch=1, M=M, K=K, N=N, gran=(blocks[2], blocks[1]),
                  sparsity=sparsity, seed=71, tile_cfg=0, activation='relu' if compressed else None)
+
+
+@pytest.mark.parametrize('M', [110100, 40000])
+def test_ring_more_tiles_than_the_list(M, gpu, K=64, N=1536):
+    """More than 128 tiles to a workgroup, which then looks every tile up, and 32 of them."""
+    import sparta_amd as sparta
+    g = torch.Generator(device=gpu).manual_seed(5)
+    mask = (torch.rand((N // 16, K // 32), generator=g, device=gpu) < 0.6).to(torch.uint8).repeat_interleave(16, 0).repeat_interleave(32, 1).contiguous()
+    lin = torch.nn.Linear(K, N, bias=True, device=gpu, dtype=torch.float16)
+    x = torch.randn((M, K), generator=g, device=gpu).half()
+    op = sparta.nn.SparseLinear(lin, weight_mask=mask)
+    op.build({'forward:C': {'_impl': 'sparta', 'BLOCK_SIZE_M_VALUE': 32, 'BLOCK_SIZE_K_VALUE': 32, 'BLOCK_SIZE_N_VALUE': 16, 'TILE_CFG': 11}},
+             sample_inputs=[x])
+    weight = (lin.weight.detach() * mask).float().t().contiguous()
+    with torch.no_grad():
+        y = op(x)
+        for r in range(0, M, 16384):
+            want = torch.matmul(x[r:r + 16384].float(), weight) + lin.bias.float()
+            # result rounded to 11 bits; sums of 64 products in fp32
+            assert float((y[r:r + 16384].float() - want).abs().max()) <= 2 ** -11 * float(want.abs().max()) + 1e-5
