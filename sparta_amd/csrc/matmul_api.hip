@@ -141,14 +141,18 @@ static size_t split_partial_bytes(int slices, int nnz, int batch, int BM, int BN
     return slices > 1 ? (size_t)batch * slices * nnz * BM * BN * sizeof(float) : 0;
 }
 
+static size_t split_colsum_bytes(int slices, int batch, int M, int K) {
+    return dds_colsum_whole(slices, K) ? 0 : (size_t)batch * kColsumSlices * M * sizeof(float);
+}
+
 }  // namespace spx
 
 extern "C" size_t spx_matmul_split_workspace_bytes(int dtype, int transA, int transB, int nnz, int batch, int M, int K, int N,
                                                    int BM, int BN, int slices, int with_colsum) {
     using namespace spx;
     (void)N;
-    return split_partial_bytes(split_slices(dtype, transA, transB, nnz, batch, K, BM, BN, slices), nnz, batch, BM, BN) +
-           (with_colsum ? (size_t)batch * kColsumSlices * M * sizeof(float) : 0);
+    slices = split_slices(dtype, transA, transB, nnz, batch, K, BM, BN, slices);
+    return split_partial_bytes(slices, nnz, batch, BM, BN) + (with_colsum ? split_colsum_bytes(slices, batch, M, K) : 0);
 }
 
 extern "C" int spx_matmul_split(int dtype, int transA, int transB, int compressed, const void* A, const void* B, void* C,
@@ -175,8 +179,10 @@ extern "C" int spx_matmul_split(int dtype, int transA, int transB, int compresse
     s.n_product = 0;
     const size_t part = split_partial_bytes(s.slices, nnz, batch, BM, BN);
     s.partial = reinterpret_cast<float*>(workspace);
-    s.colsum = a_colsum ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + part) : nullptr;
-    const size_t need = part + (a_colsum ? (size_t)batch * kColsumSlices * M * sizeof(float) : 0);
+    const size_t sums = a_colsum ? split_colsum_bytes(s.slices, batch, M, K) : 0;
+    s.colsum = sums ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + part) : nullptr;
+    s.colsum_out = sums ? nullptr : a_colsum;
+    const size_t need = part + sums;
     SPX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), SPX_E_WORKSPACE, "workspace of %zu bytes, %zu needed", workspace_bytes, need);
     if (batch == 0) return 0;
     DdsParams p;

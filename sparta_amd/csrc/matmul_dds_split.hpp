@@ -18,7 +18,8 @@
 //     last stage are fetched from a valid address and written to LDS as zeros.  Before, a token
 //     count that was no multiple of 128 fell to the kernel without a pipeline.
 //   * the column sums of A over k - the bias gradient - ride along: extra workgroups at the
-//     end of the launch add up 32 token ranges, and the second kernel finishes them.
+//     end of the launch add up all tokens, or where k is sliced 32 ranges of them, which the
+//     second kernel finishes.
 //
 // AT / BT: the operand is stored [K, M] / [K, N]; otherwise it is k-contiguous.  LDS layouts and
 // fragment reads: a stage keeps the rows as they are in memory; [k][m] rows give the
@@ -33,13 +34,23 @@ namespace spx {
 constexpr int kColsumSlices = 32;
 constexpr int64_t kSplitPartialBytes = (int64_t)1 << 30;   // most that a chosen split takes for its partial blocks
 
+constexpr int kColsumWholeK = 4096;
+
+// Whether a workgroup adds up its columns over all of k.  An unsliced product walks k just as far itself and hides
+// that, and the call is one launch: without column ranges, their workspace and the second kernel the weight gradient
+// with its bias gradient takes 3.1 instead of 6.2 us (115 blocks of 32 x 64 over 64 tokens fp16), 9.8 instead of 12.6
+// (1024 tokens), 42 instead of 45 (1300 blocks over 2048), 88.6 instead of 93.6 (4096).  Only a weight without a block
+// gains nothing past 2048 tokens (8.6 us against 5.2 at 4096).
+inline bool dds_colsum_whole(int slices, int K) { return slices == 1 && K <= kColsumWholeK; }
+
 struct DdsSplit {
     int slices;         // 1, 2, 4 or 8; 1: every block is one workgroup and writes C itself
     int k_slice;        // k per slice (a multiple of the stage depth)
     int nnz;            // live blocks (the bound, where nnz_dev gives the number)
     int n_product;      // workgroups of the product; the ones behind them sum columns
     float* partial;     // [batch][slices][nnz][BM * BN]
-    float* colsum;      // [batch][kColsumSlices][M], NULL: not wanted
+    float* colsum;      // [batch][kColsumSlices][M], NULL: not wanted, or:
+    void* colsum_out;   // [batch][M] of the operand type: a workgroup adds up all of k and writes the sums themselves
 };
 
 template <typename T, int BM, int BN> struct DdsSplitCfg {
@@ -48,40 +59,53 @@ template <typename T, int BM, int BN> struct DdsSplitCfg {
     static constexpr int NST = 2;
 };
 
-// Column sums of A over one of kColsumSlices ranges of k: eight lanes side by side (16 bytes of m
-// each), 32 rows of k at a time.
+// Column sums of A over one of kColsumSlices ranges of k, or over all of it: eight lanes side by side
+// (16 bytes of m each), 32 rows of k at a time.
 template <typename T>
 __device__ __forceinline__ void dds_colsum_range(const DdsParams& p, const DdsSplit& s, int id, float* lds) {
     constexpr int VE = 16 / (int)sizeof(T);
     constexpr int COLS = 8 * VE;
     const int64_t b = blockIdx.y;
-    const int sl = (id & 7) * (kColsumSlices / 8) + ((id >> 3) & (kColsumSlices / 8 - 1));  // XCD x reads what its slices read
-    const int c = (id / kColsumSlices) * COLS + (threadIdx.x & 7) * VE;
+    const bool whole = s.colsum_out != nullptr;
+    const int sl = whole ? 0 : (id & 7) * (kColsumSlices / 8) + ((id >> 3) & (kColsumSlices / 8 - 1));  // XCD x reads what its slices read
+    const int group = whole ? id : id / kColsumSlices;
+    const int c = group * COLS + (threadIdx.x & 7) * VE;
     const int rl = threadIdx.x >> 3;
-    const int k0 = (int)((int64_t)sl * p.K / kColsumSlices), k1 = (int)((int64_t)(sl + 1) * p.K / kColsumSlices);
+    const int k0 = (int)((int64_t)sl * p.K / kColsumSlices);
+    const int k1 = whole ? p.K : (int)((int64_t)(sl + 1) * p.K / kColsumSlices);
     const T* A = reinterpret_cast<const T*>(p.A) + b * p.a_batch;
     float v[VE];
 #pragma unroll
     for (int e = 0; e < VE; ++e) v[e] = 0.f;
     if (c < p.M) {
-#pragma unroll 4
-        for (int k = k0 + rl; k < k1; k += 32) {
-            union { vec16 q; T t[VE]; } u;
-            u.q = *reinterpret_cast<const vec16*>(A + (int64_t)k * p.a_ld + c);
+        // in runs of 1024 rows, 32 to a thread: the sums of all of k take no longer chains of additions than those of the ranges
+        for (int kr = k0; kr < k1; kr += 1024) {
+            const int end = kr + 1024 < k1 ? kr + 1024 : k1;
+            float run[VE];
 #pragma unroll
-            for (int e = 0; e < VE; ++e) v[e] += Elem<T>::to_float(u.t[e]);
+            for (int e = 0; e < VE; ++e) run[e] = 0.f;
+#pragma unroll 8
+            for (int k = kr + rl; k < end; k += 32) {
+                union { vec16 q; T t[VE]; } u;
+                u.q = *reinterpret_cast<const vec16*>(A + (int64_t)k * p.a_ld + c);
+#pragma unroll
+                for (int e = 0; e < VE; ++e) run[e] += Elem<T>::to_float(u.t[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < VE; ++e) v[e] += run[e];
         }
     }
     constexpr int LD = COLS + 4;
 #pragma unroll
     for (int e = 0; e < VE; ++e) lds[rl * LD + (threadIdx.x & 7) * VE + e] = v[e];
     __syncthreads();
-    const int col = (id / kColsumSlices) * COLS + threadIdx.x;
+    const int col = group * COLS + threadIdx.x;
     if (threadIdx.x < COLS && col < p.M) {
         float sum = 0.f;
 #pragma unroll
         for (int r = 0; r < 32; ++r) sum += lds[r * LD + threadIdx.x];
-        s.colsum[(b * kColsumSlices + sl) * p.M + col] = sum;
+        if (whole) reinterpret_cast<T*>(s.colsum_out)[b * p.M + col] = Elem<T>::from_float(sum);
+        else s.colsum[(b * kColsumSlices + sl) * p.M + col] = sum;
     }
 }
 
@@ -402,11 +426,12 @@ static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, i
     constexpr size_t epi = (size_t)W::KS * BM * (BN + 4) * sizeof(float);
     constexpr size_t cs = 32 * (8 * VE + 4) * sizeof(float);   // the column sums
     constexpr size_t product = epi > stages ? epi : stages, most = cs > product ? cs : product;
-    const size_t smem = s.colsum ? most : product;
+    const bool sums = s.colsum || s.colsum_out;
+    const size_t smem = sums ? most : product;
     s.k_slice = (int)round_up((p.K + s.slices - 1) / s.slices, KT);
     const int share = 8 / s.slices;
     const int64_t n_product = ((int64_t)s.nnz + share - 1) / share * 8;
-    const int64_t cs_groups = s.colsum ? (p.M + 8 * VE - 1) / (8 * VE) * kColsumSlices : 0;
+    const int64_t cs_groups = sums ? (int64_t)(p.M + 8 * VE - 1) / (8 * VE) * (s.colsum_out ? 1 : kColsumSlices) : 0;
     if (n_product + cs_groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)(n_product + cs_groups));
     if (n_product + cs_groups == 0) return 0;
     s.n_product = (int)n_product;

@@ -194,11 +194,12 @@ struct MatmulPlan {
     // `colsum` (may be null) receives the sums of op(A) over k.  Contiguous operands.
     Tensor run_split(int code, const Tensor& a, const Tensor& b, Tensor* colsum, size_t ws_bytes, at::IntArrayRef out_shape) const {
         Tensor c = compressed ? at::empty(out_shape, a.options()) : at::zeros(out_shape, a.options());
-        Tensor ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+        Tensor ws;
+        if (ws_bytes > 0) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
         check_rc(spx_matmul_split(code, trans_a, trans_b, compressed, device_ptr(a), device_ptr(b), c.data_ptr(),
                                   colsum ? device_ptr(*colsum) : nullptr, (const int32_t*)device_ptr(ptr),
                                   (const int32_t*)device_ptr(idx), nnz, sparse_stride, batch, M, K, N, BM, BN, 0,
-                                  ws.data_ptr(), ws_bytes, stream_of(a)), "spx_matmul_split");
+                                  ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(a)), "spx_matmul_split");
         return c;
     }
     // The weight gradient together with the sums of its first operand over k (the bias gradient).

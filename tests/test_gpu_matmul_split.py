@@ -46,6 +46,32 @@ def test_split_product_and_column_sums(slices, K, tA, tB, dtype, block, gpu, M=1
             assert_close(sums, op_a.sum(2), dtype, 'column sums')
 
 
+@pytest.mark.parametrize('K', [16, 1024, 1040, 4096, 4112])
+@pytest.mark.parametrize('dtype,M', [(torch.float16, 80), (torch.bfloat16, 64), (torch.float32, 48)])
+@pytest.mark.parametrize('live', [0, 3])
+def test_column_sums_of_an_unsliced_product(K, dtype, M, live, gpu, N=64, batch=2):
+    """Both sides of the depth up to which one workgroup adds up a column, ragged runs of 1024 rows and column
+    groups; without a live block only the sums are wanted.  They are fp32 sums of at most 100 additions, rounded once."""
+    a_np, a = randn((batch, K, M), 11, dtype)
+    _, b = randn((batch, K, N), 12, dtype)
+    mask = torch.zeros((M // 16, N // 16), dtype=torch.uint8)
+    mask.view(-1)[:live] = 1
+    idx = get_bcs_function(16, 16, True, False).build_indexes(mask.repeat_interleave(16, 0).repeat_interleave(16, 1).contiguous().to(gpu))
+    lib, code = _lib.load(), _lib.dtype_code(dtype)
+    a, b = a.to(gpu), b.to(gpu)
+    out = torch.empty((batch, max(live, 1) * 256), dtype=dtype, device=gpu)
+    sums = torch.full((batch, M), float('nan'), dtype=dtype, device=gpu)
+    nbytes = lib.spx_matmul_split_workspace_bytes(code, 1, 0, live, batch, M, K, N, 16, 16, 1, 1)
+    assert nbytes == (0 if K <= 4096 else batch * 32 * M * 4)
+    ws = torch.empty((max(nbytes, 16),), dtype=torch.uint8, device=gpu)
+    _lib.check(lib.spx_matmul_split(code, 1, 0, 1, _lib.dev_ptr(a), _lib.dev_ptr(b), _lib.dev_ptr(out), _lib.dev_ptr(sums),
+                                    _lib.dev_ptr(idx.row_ptr), _lib.dev_ptr(idx._bcsr_buf), live, live * 256, batch, M, K, N,
+                                    16, 16, 1, _lib.dev_ptr(ws) if nbytes else None, nbytes, _lib.current_stream(gpu)), 'spx_matmul_split')
+    want = a.double().sum(1)
+    bound = 100 * 2 ** -24 * a.double().abs().sum(1) + {torch.float16: 2 ** -11, torch.bfloat16: 2 ** -8, torch.float32: 2 ** -24}[dtype] * want.abs()
+    assert bool(((sums.double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize('M', [16, 208, 1040])
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16, torch.float32])
 def test_linear_training_step_with_ragged_token_counts(M, dtype, gpu, K=256, N=192):
