@@ -98,10 +98,11 @@ struct alignas(16) RingTile {
 // - are walked column by column, longest first, so the list falls in length group by group and
 // workgroups that take it there and back end up with equal sums.
 struct RingList {
-    int n_mtiles, parts, cols, group;   // cols: block-columns of a unit, rounded up
+    int n_mtiles, parts_log2, cols, group;   // cols: block-columns of a unit, rounded up
 };
 
-template <typename T, int TM, int BN, int BK, bool DK, bool SK, bool SWAP, int NB>
+// ONE: no workgroup has more than one tile.
+template <typename T, int TM, int BN, int BK, bool DK, bool SK, bool SWAP, int NB, bool ONE>
 __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p, RingList l) {
     typedef typename PanelMma<T>::M MMA;
     typedef typename MMA::frag Frag;
@@ -126,15 +127,15 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     const int nb = p.Nc / BN;
     // the tiles of this workgroup's XCD, and its place among the workgroups there
     const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3, n_pos = gridDim.x >> 3;
-    const int n_units = (l.n_mtiles * l.parts - xcd + 7) >> 3;
+    const int n_units = ((l.n_mtiles << l.parts_log2) - xcd + 7) >> 3;
     const int n_list = n_units * l.cols;
     if (pos >= n_list) return;
     const int64_t b = blockIdx.y;
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-    const int n_rounds = (n_list + n_pos - 1) / n_pos;
-    const bool listed = n_rounds > 1 && n_rounds <= kRingListMax, table = listed && nb <= kRingTableMax;
+    const int n_rounds = ONE ? 1 : (n_list + n_pos - 1) / n_pos;
+    const bool listed = !ONE && n_rounds > 1 && n_rounds <= kRingListMax, table = listed && nb <= kRingTableMax;
     RingTile* const list = reinterpret_cast<RingTile*>(smem + Lds::LIST);
     struct Tile {
         int m0, j, e0, n_blk, n_st;
@@ -142,18 +143,24 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     // launch order and column pointers while the list is made: in the ring, which is empty yet
     int* const tab_ptr = reinterpret_cast<int*>(smem);
     int* const tab_order = tab_ptr + nb + 1;
-    // The r-th tile of this workgroup.
-    auto look_up = [&](int r) __attribute__((always_inline)) -> RingTile {
-        const RingTile none = {0, 0, 0, -1};
+    // The place of the r-th tile of this workgroup: its row tile and its position in the launch order; false: none.
+    auto place = [&](int r, int& mt, int& o) __attribute__((always_inline)) -> bool {
         const int id = r * n_pos + (r & 1 ? n_pos - 1 - pos : pos);   // there and back along the list
-        if (id >= n_list) return none;
-        const int g = id / (l.group * l.cols), in = id - g * l.group * l.cols;
-        const int left = n_units - g * l.group, size = left < l.group ? left : l.group;
-        const int i = in / size;
-        const int unit = (g * l.group + in - i * size) * 8 + xcd;
-        const int mt = unit / l.parts;
-        const int o = i * l.parts + unit - mt * l.parts;
-        if (o >= nb) return none;
+        if (id >= n_list) return false;
+        int first = 0, size = n_units;   // (with one tile to a workgroup all of them run side by side: one group)
+        if constexpr (!ONE) {
+            first = id / (l.group * l.cols) * l.group;
+            size = n_units - first < l.group ? n_units - first : l.group;
+        }
+        const int in = id - first * l.cols, i = in / size;
+        const int unit = (first + in - i * size) * 8 + xcd;
+        mt = unit >> l.parts_log2;
+        o = (i << l.parts_log2) + unit - (mt << l.parts_log2);
+        return o < nb;
+    };
+    auto look_up = [&](int r) __attribute__((always_inline)) -> RingTile {
+        int mt, o;
+        if (!place(r, mt, o)) return {0, 0, 0, -1};
         const int j = table ? tab_order[o] : p.sched ? p.sched[o] : o;
         const int* const ptr = table ? tab_ptr : p.ptr;
         const int e0 = ptr[j];
@@ -174,9 +181,16 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         __syncthreads();
     }
     auto tile_at = [&](int r, Tile& t) __attribute__((always_inline)) -> bool {
-        RingTile e;
-        if (listed) e = list[r];
-        else e = look_up(r);
+        RingTile e = {0, 0, 0, -1};
+        int mt, o;
+        if (listed) {
+            e = list[r];
+        } else if (place(r, mt, o)) {   // (through the scalar cache)
+            e.m0 = mt * TM;
+            e.j = p.sched ? ((const_i32)p.sched)[o] : o;
+            e.e0 = ((const_i32)p.ptr)[e.j];
+            e.n_blk = ((const_i32)p.ptr)[e.j + 1] - e.e0;
+        }
         t.n_blk = __builtin_amdgcn_readfirstlane(e.n_blk);
         t.m0 = __builtin_amdgcn_readfirstlane(e.m0);
         t.j = __builtin_amdgcn_readfirstlane(e.j);
@@ -447,19 +461,20 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
     RingList l;
     l.n_mtiles = (p.Mc + TM - 1) / TM;
     if ((int64_t)l.n_mtiles * nb > 0x7fffff00) return fail(SPX_E_SHAPE, "problem too large for one launch");
-    l.parts = 1;
+    int parts = 1;
     // panels that do not deal out evenly are cut by columns, unless the copies of the dense operand that
     // every further XCD then reads cost more than the idle ones (64 MB: about 10 us)
     if (l.n_mtiles < 64)
-        while (l.parts < 8 && (int64_t)l.n_mtiles * l.parts % 8 != 0 &&
-               (int64_t)p.Mc * p.K * (int)sizeof(T) * 2 * l.parts <= (64 << 20)) l.parts *= 2;
-    l.cols = (nb + l.parts - 1) / l.parts;
+        while (parts < 8 && (int64_t)l.n_mtiles * parts % 8 != 0 &&
+               (int64_t)p.Mc * p.K * (int)sizeof(T) * 2 * parts <= (64 << 20)) parts *= 2;
+    l.parts_log2 = parts == 8 ? 3 : parts >> 1;
+    l.cols = (nb + parts - 1) / parts;
     const int64_t panel = (int64_t)TM * p.K * (int)sizeof(T);
     l.group = panel >= (2 << 20) ? 1 : (int)((2 << 20) / panel);
     constexpr int most = Lds::LIST + kRingListMax * (int)sizeof(RingTile);
     static_assert(most <= 160 * 1024 && NB * Lds::STAGE >= (2 * kRingTableMax + 1) * 4, "fits a CU, and the tables the ring");
     // workgroups per XCD: as many as fit (the batch entries share the device)
-    const int n_list = ((l.n_mtiles * l.parts + 7) / 8) * l.cols;   // the longest of the eight lists
+    const int n_list = ((l.n_mtiles * parts + 7) / 8) * l.cols;   // the longest of the eight lists
     int n_pos = 0, smem = most;
     // (five where they fit: 64-row tiles of 2992 x 768 -> 3072 bf16 14.3 -> 11.9 us, 8192 x 3072 -> 768 fp16 16.5 -> 15.9)
     for (int per_cu = 5; per_cu >= 1; --per_cu) {
@@ -469,8 +484,21 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
         smem = Lds::LIST + (n_rounds > 1 && n_rounds <= kRingListMax ? n_rounds * (int)sizeof(RingTile) : 0);
         if (per_cu * (int)round_up(smem, 1280) <= 160 * 1024) break;   // LDS is given out in pieces of 1280 bytes
     }
-    SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>), most, "spmm_ring_kernel");
-    hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB>), dim3(8 * n_pos, batch, 1), dim3(kRingThreads), smem, st, p, l);
+    // One tile to a workgroup, where 64-row tiles belong: an instance without the code for more of them, which is mostly
+    // start-up (32 x 64 blocks: 9 x 768 -> 1920 bf16 4.0 -> 3.55 us, 375 x 1152 -> 896 fp16 3.5 -> 3.0, 52 x 576 -> 768 fp32 with
+    // 16 x 16 blocks 6.1 -> 5.2; the general code's list of tiles alone cost these 0.2).
+    if constexpr (TM == 64) {
+        if (n_pos == n_list) {
+            SpmmParams q = p;
+            if (n_pos * batch <= 32) q.sched = nullptr;   // one to a CU: the order is of no account, a trip to memory less
+            SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB, true>), most, "spmm_ring_kernel");
+            hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB, true>), dim3(8 * n_pos, batch, 1), dim3(kRingThreads), smem, st, q, l);
+            SPX_LAUNCH_CHECK("spmm_ring_kernel");
+            return 0;
+        }
+    }
+    SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB, false>), most, "spmm_ring_kernel");
+    hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, NB, false>), dim3(8 * n_pos, batch, 1), dim3(kRingThreads), smem, st, p, l);
     SPX_LAUNCH_CHECK("spmm_ring_kernel");
     return 0;
 }

@@ -31,6 +31,15 @@ def test_ring_rows_and_rounds(tile_cfg, dtype, blocks, gpu):
                  sparsity=0.8, seed=M, tile_cfg=tile_cfg, activation='relu' if M % 2 else None)
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('M,N,batch', [(512, 1024, 1), (512, 1056, 1), (480, 512, 2), (480, 544, 2), (2000, 96, 1), (65, 5120, 1), (320, 5152, 1)])
+def test_ring_one_tile_to_a_workgroup(M, N, batch, dtype, gpu, K=4096):
+    """Both sides of one workgroup to a CU, where the launch order is left out, and of one tile to a workgroup; more
+    panels than the L2 of an XCD holds, and block-columns cut in parts."""
+    run_case(gpu, 'dsd', False, True, True, True, dtype, (32, 32, 32), batch=batch, M=M, K=K, N=N, gran=(32, 32),
+             sparsity=0.97, seed=M + N, tile_cfg=11)
+
+
 def test_ring_more_block_columns_than_the_table(gpu):
     run_case(gpu, 'dsd', False, True, False, True, torch.float16, (32, 32, 16), batch=1, M=520, K=96, N=16 * 1100,
              gran=(16, 32), sparsity=0.6, seed=61, tile_cfg=11)
