@@ -475,15 +475,20 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
     static_assert(most <= 160 * 1024 && NB * Lds::STAGE >= (2 * kRingTableMax + 1) * 4, "fits a CU, and the tables the ring");
     // workgroups per XCD: as many as fit (the batch entries share the device)
     const int n_list = ((l.n_mtiles * parts + 7) / 8) * l.cols;   // the longest of the eight lists
-    int n_pos = 0, smem = most;
-    // (five where they fit: 64-row tiles of 2992 x 768 -> 3072 bf16 14.3 -> 11.9 us, 8192 x 3072 -> 768 fp16 16.5 -> 15.9)
-    for (int per_cu = 5; per_cu >= 1; --per_cu) {
-        n_pos = 32 * per_cu / batch;
-        n_pos = n_pos < 1 ? 1 : n_pos > n_list ? n_list : n_pos;
-        const int n_rounds = (n_list + n_pos - 1) / n_pos;
-        smem = Lds::LIST + (n_rounds > 1 && n_rounds <= kRingListMax ? n_rounds * (int)sizeof(RingTile) : 0);
-        if (per_cu * (int)round_up(smem, 1280) <= 160 * 1024) break;   // LDS is given out in pieces of 1280 bytes
-    }
+    auto rounds_of = [&](int per_cu) {
+        const int fit = 32 * per_cu / batch, n = fit < 1 ? 1 : fit > n_list ? n_list : fit;
+        return n_list == 0 ? 0 : (n_list + n - 1) / n;
+    };
+    auto smem_of = [&](int n_rounds) { return Lds::LIST + (n_rounds > 1 && n_rounds <= kRingListMax ? n_rounds * (int)sizeof(RingTile) : 0); };
+    // At most four, and a fifth where it saves a round: 64-row tiles of 2992 x 768 -> 3072 bf16 13.4 -> 11.6 us with it, of
+    // 5000 x 2048 -> 1024 fp16 20.9 -> 18.1, of 3713 x 1280 -> 640 bf16 11.9 -> 9.1; but of 3699 x 3328 -> 832 bf16 20.0 -> 22.7, two
+    // rounds either way.
+    int per_cu = rounds_of(5) < rounds_of(4) ? 5 : 4;
+    for (; per_cu > 1; --per_cu)   // LDS is given out in pieces of 1280 bytes
+        if (per_cu * (int)round_up(smem_of(rounds_of(per_cu)), 1280) <= 160 * 1024) break;
+    const int n_rounds = rounds_of(per_cu), smem = smem_of(n_rounds);
+    int n_pos = 32 * per_cu / batch;
+    n_pos = n_pos < 1 ? 1 : n_pos > n_list ? n_list : n_pos;
     // One tile to a workgroup, where 64-row tiles belong: an instance without the code for more of them, which is mostly
     // start-up (32 x 64 blocks: 9 x 768 -> 1920 bf16 4.0 -> 3.55 us, 375 x 1152 -> 896 fp16 3.5 -> 3.0, 52 x 576 -> 768 fp32 with
     // 16 x 16 blocks 6.1 -> 5.2; the general code's list of tiles alone cost these 0.2).
