@@ -302,14 +302,14 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
     const float l_run = xor32_sum(lacc[0]);
     int out_lane = lane;   // made anew: what the stores derive from the lane would be kept through the walk, in scratch
     if constexpr (SEQ) asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(out_lane));
-    const bool dead = !(l_run > 0.f) || (SEQ && row0 + (out_lane & 31) >= seq_len);
-    const float inv_l = dead ? 0.f : 1.f / l_run;
+    const bool past = SEQ && row0 + (out_lane & 31) >= seq_len;
+    const float inv_l = l_run > 0.f ? 1.f / l_run : 0.f;
     if (!SEQ && p.row_lse && h2 == 0)
         p.row_lse[b * p.Nt + row0 + l32] = l_run > 0.f ? __builtin_fmaf(m_run, c2, __builtin_amdgcn_logf(l_run)) : __builtin_inff();
 #pragma unroll
     for (int t = 0; t < ET; ++t)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) oacc[t][j] = SEQ && dead ? 0.f : oacc[t][j] * inv_l;
+        for (int j = 0; j < 16; ++j) oacc[t][j] = past ? 0.f : oacc[t][j] * inv_l;
     __syncthreads();   // the K / V tiles are dead: their space carries the output rows
     if (rows_exist)
         store_rows32<T, E>(smem + wave * (32 * (E * 2 + 16)), reinterpret_cast<T*>(p.out) + (b * p.Nt + row0) * E, oacc, out_lane);

@@ -39,3 +39,22 @@ def test_longest_first(batch, heads, N, lens, E, gpu):
             # probabilities and result rounded to 11 bits, 2^-12 of the value each at most
             rel = float((got[b, :, :m] - want).norm() / want.norm())
             assert rel <= 1e-3, f'entry {b} of length {m}: {rel:.2e}'
+
+
+@pytest.mark.parametrize('E', [64, 128])
+def test_nan_stays_in_its_rows(E, gpu, batch=32, heads=12, N=320, n=200):
+    """A query or key that is NaN makes its own row or all rows of its head NaN; past the length it makes nothing."""
+    g = torch.Generator(device=gpu).manual_seed(4)
+    q, k, v = (torch.randn((batch, heads, N, E), generator=g, device=gpu).half() for _ in range(3))
+    q = q / E ** 0.5
+    op = SeqlenDynamicSparseAttention(global_mode=False)
+    lens = torch.full((batch,), n, dtype=torch.int32, device=gpu)
+    want = op(q, k, v, lens)
+    q[0, 1, 7] = q[0, 1, n] = k[1, 2, 150] = k[1, 3, n] = v[1, 4, n + 7] = float('nan')
+    got = op(q, k, v, lens)
+    bad = torch.zeros((batch, heads, N), dtype=torch.bool, device=gpu)
+    bad[0, 1, 7] = True
+    bad[1, 2, :n] = True
+    assert bool(got[bad].isnan().all())
+    # other rows of its wavefront may move their reference point with it: probabilities and result rounded to 11 bits, twice
+    assert float((got[~bad].float() - want[~bad].float()).abs().max()) <= 2 ** -9 * float(v.nan_to_num().abs().max())
