@@ -2288,14 +2288,9 @@ extern "C" int spx_attention_seqlen_forward(int dtype, const void* q, const void
         ap.inv_t = inv_temperature;
         ap.Nt = N; ap.Ns = N; ap.BH = N % 64 == 0 ? 64 : 32;
         ap.seqlens = seqlens; ap.heads = heads;
-        // 128 queries per workgroup read every key tile half as often, but fill the chip and cover their
-        // latencies only with enough work.  fp16 us, 64-query workgroups / wide (the first two since measured again at 56
-        // and 106, with the work ordered): 32 x 12 x 1024 x 64 81 / 63,
-        // head dim 128 133 / 111; 16 x 12 x 512 19.5 / 14.2; 32 x 12 x 256 14.1 / 12.0; at 384 workgroups 20.2 / 15.8
-        // (3 x 16 x 992) and 29.0 / 25.8 (2 x 12 x 2048); at 192 12.6 / 14.3 (2 x 12 x 1024) and 9.4 / 9.8
-        // (4 x 12 x 512); short sequences 9.9 / 11.1 (32 x 16 x 192) and 6.4 / 7.7 (32 x 12 x 128).
+        // 32 queries per wavefront, or 16 where there is little to do
         // (inv_t > 0: the wide kernel takes the maximum before it scales)
-        if (N >= 256 && (int64_t)batch * heads * ((N + 127) / 128) >= 384 && inv_temperature > 0.f)
+        if (attention_wide_seq_wins((int64_t)batch * heads, N, E) && inv_temperature > 0.f)
             return launch_attention_wide_seq(dtype, ap, batch * heads, E, st);
         if (dtype == SPX_F16) return launch_attention_v2_seq<_Float16>(ap, batch * heads, E, st);
         return launch_attention_v2_seq<bf16_t>(ap, batch * heads, E, st);

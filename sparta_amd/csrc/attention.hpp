@@ -141,6 +141,7 @@ __device__ __forceinline__ void store_rows32(char* tile, T* dst, const f32x16 (&
 // or over sequence lengths (128 queries per workgroup)
 bool attention_wide_supported(int BH, int BW, int E);
 int launch_attention_wide(int dtype, const AttnParams& p, int batch, int BW, int E, hipStream_t st);
+bool attention_wide_seq_wins(int64_t entries, int N, int E);
 int launch_attention_wide_seq(int dtype, const AttnParams& p, int batch, int E, hipStream_t st);
 
 // attention_bwd_wide.hip: backward kernels that recompute the probabilities, 32 queries or keys per wavefront, with

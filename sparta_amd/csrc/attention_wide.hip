@@ -95,22 +95,27 @@ __device__ __forceinline__ bool seqlen_work(const AttnParams& p, int entries, in
 }
 
 constexpr int kWideStages = 2;
-template <int E, int KT, int WAVES, bool HAS_MASK> struct WideLds {
+template <int E, int KT, int WAVES, bool HAS_MASK, int SPLIT = 1> struct WideLds {
     static constexpr int V = KT * AttnTile<E>::BYTES;
     static constexpr int MASK = 2 * V;                  // 32 x 32 bytes per wavefront
     static constexpr int STAGE = MASK + (HAS_MASK ? WAVES * 1024 : 0);
-    static constexpr int OUT = WAVES * 32 * (E * 2 + 16);                // output rows, in the same space
-    static constexpr int TOTAL = kWideStages * STAGE > OUT ? kWideStages * STAGE : OUT;
+    // in the same space afterwards: what the wavefronts but those of the first share of the keys hold, and the output rows
+    static constexpr int PART = E / 32 * 4096 + 512, OUT = (WAVES - WAVES / SPLIT) * PART;
+    static constexpr int END = OUT + WAVES / SPLIT * 32 * (E * 2 + 16);
+    static constexpr int TOTAL = kWideStages * STAGE > END ? kWideStages * STAGE : END;
 };
 
-template <typename T, int E, int KT, int WAVES, bool HAS_MASK, bool SEQ>
-__global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void attention_wide_kernel(AttnParams p, int nbr, int log_sub, int batch) {
+// SPLIT: wavefronts to 32 queries; each takes KT / SPLIT of a stage's tiles, and the first one adds up what they hold.
+template <typename T, int E, int KT, int WAVES, bool HAS_MASK, bool SEQ, int SPLIT>
+__global__ __launch_bounds__(64 * WAVES, SPLIT > 1 ? 2 : E == 64 ? 4 : KT == 1 ? 3 : 2) void attention_wide_kernel(AttnParams p, int nbr, int log_sub, int batch) {
     static_assert(KT == 1 || (SEQ && !HAS_MASK), "an index is walked in tiles of 32 keys, and sequence-length mode has no mask bytes");
+    static_assert(SPLIT == 1 || SEQ, "the keys of an index are not shared out");
     typedef AttnTile<E> Tile;
-    typedef WideLds<E, KT, WAVES, HAS_MASK> Lds;
+    typedef WideLds<E, KT, WAVES, HAS_MASK, SPLIT> Lds;
     constexpr int EC = Tile::EC, ET = Tile::ET, NB = kWideStages;
     constexpr int LPT = 2 * Tile::LOADS / WAVES;   // loads of a wavefront and 32 keys
-    constexpr int ROWS = 32 * WAVES, KEYS = 32 * KT;
+    constexpr int QW = WAVES / SPLIT, KW = KT / SPLIT;   // wavefronts with queries of their own; tiles of a wavefront and stage
+    constexpr int ROWS = 32 * QW, KEYS = 32 * KT;
     typedef typename MmaW<T>::frag Frag;
     typedef float f32x8 __attribute__((ext_vector_type(8)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -148,7 +153,8 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
     const int l32 = tile.l32, h2 = tile.h2;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 
-    const int row0 = br * ROWS + wave * 32;       // first query of this wavefront
+    const int qw = SPLIT > 1 ? wave % QW : wave, kw = SPLIT > 1 ? wave / QW : 0;   // its queries, its share of the keys
+    const int row0 = br * ROWS + qw * 32;         // first query of this wavefront
     // sequence lengths: Nt is a multiple of 32, so a wavefront is inside or outside; one whose rows are all past the
     // length only brings tiles
     const bool rows_exist = !SEQ || row0 < p.Nt, idle = SEQ && row0 >= seq_len;
@@ -175,7 +181,7 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
             int key0 = SEQ ? i * KEYS + kt * 32 : key0_at(i);
-            if (kt > 0 && key0 >= p.Ns) key0 -= 32;   // past the tensor and the length: any rows
+            if (kt > 0 && key0 >= p.Ns) key0 = p.Ns - 32;   // past the tensor and the length: any rows
             const uint32_t to = lds0 + at + kt * Tile::BYTES;
             if constexpr (WAVES == 1) {
                 tile.template request<LPT / 2>(Kg + (int64_t)key0 * E, 0, to);
@@ -224,13 +230,14 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
                 *reinterpret_cast<u32x4*>(smem + at + Lds::V + left * Tile::ROW + v * 16) = u32x4{0u, 0u, 0u, 0u};
             __syncthreads();
         }
-        if (idle) return;
-        const char* ks = smem + at;
+        const int mine = left - kw * KW * 32;               // of the ones that are this wavefront's
+        if (idle || (SPLIT > 1 && mine <= 0)) return;
+        const char* ks = smem + at + kw * KW * Tile::BYTES;
         const char* vs = ks + Lds::V;
         // ---- S^T: 32 keys x this wavefront's 32 queries at a time ----------------------------
-        f32x16 s[KT];
+        f32x16 s[KW];
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < KW; ++kt) {
 #pragma unroll
             for (int j = 0; j < 16; ++j) s[kt][j] = 0.f;
 #pragma unroll
@@ -246,16 +253,16 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
                 for (int j = 0; j < 16; ++j) s[0][j] = ((live[j >> 2] >> (8 * (j & 3))) & 0xffu) ? s[0][j] : DEAD;
             }
         }
-        if (SEQ && left < KEYS) {
+        if (SEQ && mine < 32 * KW) {
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt)
+            for (int kt = 0; kt < KW; ++kt)
 #pragma unroll
-                for (int j = 0; j < 16; ++j) s[kt][j] = kt * 32 + 8 * (j >> 2) + 4 * h2 + (j & 3) < left ? s[kt][j] : DEAD;
+                for (int j = 0; j < 16; ++j) s[kt][j] = kt * 32 + 8 * (j >> 2) + 4 * h2 + (j & 3) < mine ? s[kt][j] : DEAD;
         }
         // three-way maxima, two chains to 32 keys
         float tmax = DEAD;
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
+        for (int kt = 0; kt < KW; ++kt) {
             const f32x16& x = s[kt];
             const float a0 = max3f(max3f(max3f(x[0], x[1], x[2]), x[3], x[4]), x[5], x[6]);
             const float a1 = max3f(max3f(max3f(x[8], x[9], x[10]), x[11], x[12]), x[13], x[14]);
@@ -273,9 +280,9 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
         }
         fresh = fresh && !any_live;
         const float mc = -m_run * c2;
-        Frag pf[KT][2];
+        Frag pf[KW][2];
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
+        for (int kt = 0; kt < KW; ++kt)
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 f32x8 pv;
@@ -286,7 +293,7 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
             }
         // ---- O^T[e][query] += V^T P^T ------------------------------------------------------
 #pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
+        for (int kt = 0; kt < KW; ++kt)
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -299,7 +306,52 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
     }
 
     // lane holds O^T[e = t*32 + 8a + 4*h2 + q][query l32]; rows with no live entry give 0
-    const float l_run = xor32_sum(lacc[0]);
+    float l_run = xor32_sum(lacc[0]);
+    if constexpr (SPLIT > 1) {
+        __syncthreads();   // the K / V tiles are dead
+        if (kw > 0) {
+            char* to = smem + (wave - QW) * Lds::PART;
+#pragma unroll
+            for (int t = 0; t < ET; ++t)
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+                    *reinterpret_cast<f32x4*>(to + ((t * 4 + a) * 64 + lane) * 16) =
+                        f32x4{oacc[t][4 * a], oacc[t][4 * a + 1], oacc[t][4 * a + 2], oacc[t][4 * a + 3]};
+            reinterpret_cast<float*>(to + ET * 4096)[lane] = h2 ? l_run : m_run;
+        }
+        __syncthreads();
+        if (kw > 0) return;
+        // their reference points differ; one that has seen no live key has a sum of 0 and none (a NaN counts as a sum)
+        float m[SPLIT], l[SPLIT];
+        m[0] = m_run;
+        l[0] = l_run;
+#pragma unroll
+        for (int g = 1; g < SPLIT; ++g) {
+            const float* from = reinterpret_cast<const float*>(smem + ((g - 1) * QW + qw) * Lds::PART + ET * 4096);
+            m[g] = from[l32];
+            l[g] = from[32 + l32];
+        }
+        float top = DEAD;
+#pragma unroll
+        for (int g = 0; g < SPLIT; ++g) top = l[g] == 0.f ? top : fmaxf(top, m[g]);
+        l_run = 0.f;
+#pragma unroll
+        for (int g = 0; g < SPLIT; ++g) {
+            const float weight = l[g] == 0.f ? 0.f : __builtin_amdgcn_exp2f((m[g] - top) * c2);
+            l_run = __builtin_fmaf(weight, l[g], l_run);
+            const char* from = smem + ((g - 1) * QW + qw) * Lds::PART;
+#pragma unroll
+            for (int t = 0; t < ET; ++t)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    f32x4 part;
+                    if (g > 0) part = *reinterpret_cast<const f32x4*>(from + ((t * 4 + a) * 64 + lane) * 16);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        oacc[t][4 * a + x] = g == 0 ? oacc[t][4 * a + x] * weight : __builtin_fmaf(weight, part[x], oacc[t][4 * a + x]);
+                }
+        }
+    }
     int out_lane = lane;   // made anew: what the stores derive from the lane would be kept through the walk, in scratch
     if constexpr (SEQ) asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(out_lane));
     const bool past = SEQ && row0 + (out_lane & 31) >= seq_len;
@@ -310,31 +362,57 @@ __global__ __launch_bounds__(64 * WAVES, E == 64 ? 4 : KT == 1 ? 3 : 2) void att
     for (int t = 0; t < ET; ++t)
 #pragma unroll
         for (int j = 0; j < 16; ++j) oacc[t][j] = past ? 0.f : oacc[t][j] * inv_l;
-    __syncthreads();   // the K / V tiles are dead: their space carries the output rows
+    if constexpr (SPLIT == 1) __syncthreads();   // the K / V tiles are dead: their space carries the output rows
     if (rows_exist)
-        store_rows32<T, E>(smem + wave * (32 * (E * 2 + 16)), reinterpret_cast<T*>(p.out) + (b * p.Nt + row0) * E, oacc, out_lane);
+        store_rows32<T, E>(smem + Lds::OUT + qw * (32 * (E * 2 + 16)), reinterpret_cast<T*>(p.out) + (b * p.Nt + row0) * E, oacc, out_lane);
 }
 
-template <typename T, int E, int KT, int WAVES, bool HAS_MASK, bool SEQ>
+template <typename T, int E, int KT, int WAVES, bool HAS_MASK, bool SEQ, int SPLIT = 1>
 static int launch_attention_wide_inst(const AttnParams& p, int nbr, int batch, int BW, hipStream_t st) {
-    constexpr int smem = WideLds<E, KT, WAVES, HAS_MASK>::TOTAL;
+    constexpr int smem = WideLds<E, KT, WAVES, HAS_MASK, SPLIT>::TOTAL;
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    SPX_GRANT_LDS((attention_wide_kernel<T, E, KT, WAVES, HAS_MASK, SEQ>), smem, "attention_wide_kernel");
-    hipLaunchKernelGGL((attention_wide_kernel<T, E, KT, WAVES, HAS_MASK, SEQ>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, ilog2(BW / 32), batch);
+    SPX_GRANT_LDS((attention_wide_kernel<T, E, KT, WAVES, HAS_MASK, SEQ, SPLIT>), smem, "attention_wide_kernel");
+    hipLaunchKernelGGL((attention_wide_kernel<T, E, KT, WAVES, HAS_MASK, SEQ, SPLIT>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, ilog2(BW / 32), batch);
     SPX_LAUNCH_CHECK("attention_wide_kernel");
     return 0;
 }
 
-// Sequence-length mode: 128 queries per workgroup, any N that is a multiple of 32.
+// Sequence-length mode, any N that is a multiple of 32.  With enough work 128 queries per workgroup.
 // (64 queries per workgroup: 63 -> 84 us at 32 x 12 x 1024 x 64 fp16, the L1s fetch every tile twice as
-// often; 256 queries: 72 us, eight wavefronts meet at a barrier.)
+// often; 256 queries: 72 us, eight wavefronts meet at a barrier.)  Below that a launch is as long as the walk over the
+// longest sequence: 64 queries, and two wavefronts to 32 of them that share the keys out, stages of 128 keys for as long as
+// all workgroups are on the chip at once (64 KB of LDS each, head dim 64).  fp16 us, 128 queries / shared keys and stages of
+// 64 / and of 128:
+//   head dim 64   3 x 16 x 640 12.3 / 9.7 / 9.4, 1 x 16 x 2048 18.6 / 13.5 / 11.9, 6 x 8 x 1024 18.0 / 13.4 / 12.6,
+//                 5 x 12 x 1152 19.8 / 17.6 / 19.3, 8 x 12 x 1024 18.9 / 17.6 / 22.9, 9 x 16 x 1024 23.4 / 27.3 / 30.1
+//   head dim 128  2 x 12 x 1024 19.8 / 15.0, 8 x 8 x 768 20.5 / 16.7, 4 x 16 x 1024 23.4 / 20.8, 11 x 16 x 448 16.6 / 21.6
+static bool seqlen_shares_keys(int64_t entries, int N, int E) { return entries * ((N + 127) / 128) <= (E == 64 ? 768 : 512); }
+
+// Whether this kernel takes the call and not the 16-query one, whose wavefronts start sooner: N from 192 on; with few
+// workgroups long sequences or 384 of 64 queries.  fp16 us, 16-query kernel / shared keys: 2 x 12 x 512 x 64 6.8 / 7.0,
+// 4 x 12 x 512 9.3 / 8.1, 8 x 12 x 256 6.7 / 6.4, 6 x 12 x 320 6.6 / 7.3, 1 x 8 x 640 6.0 / 7.0, 1 x 12 x 768 6.8 / 6.9,
+// 1 x 16 x 1024 8.4 / 8.0, 2 x 8 x 2048 19.5 / 15.5; head dim 128 2 x 16 x 256 6.5 / 7.6, 8 x 16 x 256 9.7 / 9.6,
+// 14 x 12 x 192 8.3 / 9.5, 1 x 8 x 800 10.5 / 10.9, 1 x 8 x 1024 12.0 / 11.7.  16-query kernel / 128 queries: 32 x 16 x 192 x 64 9.6 / 9.0, 24 x 12 x 160 x
+// 64 6.6 / 6.9, 20 x 16 x 192 x 128 11.6 / 11.2.
+bool attention_wide_seq_wins(int64_t entries, int N, int E) {
+    if (N < 192) return false;
+    if (!seqlen_shares_keys(entries, N, E)) return true;
+    return N >= (E == 64 ? 768 : 896) || (entries * ((N + 63) / 64) >= 384 && N >= (E == 64 ? 192 : 256));
+}
+
 template <typename T>
 static int launch_attention_wide_seq_typed(const AttnParams& p, int batch, int E, hipStream_t st) {
+    if (E != 64 && E != 128) return fail(SPX_E_CONFIG, "the wide sequence-length kernel takes head dims 64 / 128 (got %d)", E);
+    if (seqlen_shares_keys(batch, p.Nt, E)) {
+        const int nbr = (p.Nt + 63) / 64;
+        if (E == 128) return launch_attention_wide_inst<T, 128, 2, 4, false, true, 2>(p, nbr, batch, 32, st);
+        return (int64_t)batch * nbr <= 512 ? launch_attention_wide_inst<T, 64, 4, 4, false, true, 2>(p, nbr, batch, 32, st)
+                                           : launch_attention_wide_inst<T, 64, 2, 4, false, true, 2>(p, nbr, batch, 32, st);
+    }
     const int nbr = (p.Nt + 127) / 128;
-    if (E == 64) return launch_attention_wide_inst<T, 64, 2, 4, false, true>(p, nbr, batch, 32, st);
-    if (E == 128) return launch_attention_wide_inst<T, 128, 2, 4, false, true>(p, nbr, batch, 32, st);
-    return fail(SPX_E_CONFIG, "the wide sequence-length kernel takes head dims 64 / 128 (got %d)", E);
+    return E == 64 ? launch_attention_wide_inst<T, 64, 2, 4, false, true>(p, nbr, batch, 32, st)
+                   : launch_attention_wide_inst<T, 128, 2, 4, false, true>(p, nbr, batch, 32, st);
 }
 
 // The wide-MFMA kernel covers query blocks of 32 / 64 / 128 (one wavefront per 32 queries),

@@ -20,10 +20,27 @@ pytestmark = pytest.mark.gpu
     (130, 3, 256, 'clamped'),   # lengths below 0 and above N
 ])
 def test_longest_first(batch, heads, N, lens, E, gpu):
-    assert batch * heads * ((N + 127) // 128) >= 384   # the wide kernel takes it
+    assert batch * heads * ((N + 127) // 128) >= 384   # the kernel with 32 queries to a wavefront takes it
+    check(batch, heads, N, lens, E, gpu)
+
+
+@pytest.mark.parametrize('E', [64, 128])
+@pytest.mark.parametrize('batch,heads,N,lens', [
+    (2, 16, 992, 'mixed'), (1, 3, 928, 'full'),   # stages of 128 keys with head dim 64; N no multiple of a stage
+    (7, 12, 320, 'edges'), (24, 8, 256, 'edges'), # and of 64; lengths that end in the first or second share of a stage, or leave one out
+    (8, 16, 192, 'mixed'), (48, 8, 192, 'edges'),
+    (3, 8, 1056, 'clamped'), (33, 5, 288, 'one'),
+    (768, 1, 96, 'mixed'), (767, 1, 224, 'mixed')])
+def test_shared_keys(batch, heads, N, lens, E, gpu):
+    """Both sides of the sizes at which two wavefronts share the keys of their queries out."""
+    check(batch, heads, N, lens, E, gpu)
+
+
+def check(batch, heads, N, lens, E, gpu):
     rng = np.random.default_rng(11)
     n = {'mixed': rng.integers(0, N + 1, batch), 'none': np.zeros(batch, int), 'full': np.full(batch, N),
-         'one': np.ones(batch, int), 'clamped': rng.integers(-N, 2 * N, batch)}[lens]
+         'one': np.ones(batch, int), 'clamped': rng.integers(-N, 2 * N, batch),
+         'edges': np.resize([1, 31, 32, 33, 63, 64, 65, 96, 127, 128, 129, 160, 192], batch)}[lens]
     if lens == 'one':
         n[5] = N
     g = torch.Generator(device=gpu).manual_seed(3)
@@ -42,7 +59,8 @@ def test_longest_first(batch, heads, N, lens, E, gpu):
 
 
 @pytest.mark.parametrize('E', [64, 128])
-def test_nan_stays_in_its_rows(E, gpu, batch=32, heads=12, N=320, n=200):
+@pytest.mark.parametrize('batch', [8, 11, 32])   # shared keys, stages of 128 (head dim 64) and of 64; not shared
+def test_nan_stays_in_its_rows(batch, E, gpu, heads=12, N=320, n=200):
     """A query or key that is NaN makes its own row or all rows of its head NaN; past the length it makes nothing."""
     g = torch.Generator(device=gpu).manual_seed(4)
     q, k, v = (torch.randn((batch, heads, N, E), generator=g, device=gpu).half() for _ in range(3))
