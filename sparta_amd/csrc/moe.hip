@@ -1274,7 +1274,9 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // tile_cfg 1: 128x128 tiles staged through registers (any dtype and weight layout);
     // 2 / 3 / 4: tiles filled by LDS-direct loads - 128x128 with four wavefronts (two
-    // workgroups per CU), 256x256 with eight wavefronts of 128x64, 256x256 with sixteen
+    // workgroups per CU; eight for 16-bit [E, in, out] weights: 700 x 2048 -> 2048 over 16 bf16 40.4 -> 37.8 us,
+    // 2113 x 2048 -> 2048 over 8 fp16 44.5 -> 38.7, 1342 x 1024 -> 4096 over 8 30.1 -> 27.5; behind a round of 256-row tiles 171.9 against
+    // 173.7 and 163.3 against 159.5, so there it is four), 256x256 with eight wavefronts of 128x64, 256x256 with sixteen
     // wavefronts of 64x64 - for 16-bit types in either weight layout and fp32 with
     // k-contiguous weights.  256x256 tiles move half the bytes from L2 to the CUs, which is
     // what bounds the 128x128 kernel.  5 = 4 for the whole rounds of 256-row tiles plus 2 for
@@ -1289,6 +1291,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) n_cu = prop.multiProcessorCount;
         if (n_cu <= 0) n_cu = 256;
     }
+    int stages64 = 0;   // 64 x 128 tiles with that many stages
     if (tile_cfg == 0) {
         // 16-bit types: 256x256 tiles from 256 of them on (split launch, 5); from 128 on when
         // all of them, the partly filled ones at the expert boundaries included, run in a
@@ -1308,7 +1311,22 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         else if (few_rows) tile_cfg = 7;
         else if (es == 2 && big_tiles >= 256) tile_cfg = 5;
         else if (es == 2 && big_tiles >= 128 && (row_tiles + n_exp) * col_tiles <= n_cu) tile_cfg = 4;
-        else tile_cfg = 2;
+        // experts of more than a 256-row tile leave half a tile unused each, give or take: also where that many fit a round
+        // (16108 x 768 -> 768 over 32 fp16 47.0 / 40.3 us with 128- and 256-row tiles, 4718 x 768 -> 2048 over 16 40.9 / 36.8;
+        // 1592 x 1024 -> 4096 over 16, fewer rows, 42.4 / 46.1; 10421 x 768 -> 768 over 8, 123 tiles, 26.0 / 31.2)
+        else if (es == 2 && big_tiles >= 150 && n_tok >= (int64_t)256 * n_exp && (row_tiles + n_exp * 5 / 8) * col_tiles <= n_cu) tile_cfg = 4;
+        else {
+            tile_cfg = 2;
+            // 64-row tiles, three stages deep where the workgroups are few (51 x 2048 -> 2048 over 16 bf16 33.1 / 23.4 us,
+            // 1976 x 768 -> 768 over 8 21.8 / 18.0, 3821 x 2048 -> 768 over 4 35.9 / 31.3; 375 x 2048 -> 2048 over 16, 304 tiles,
+            // 31.9 with two / 35.9), two where the experts have few rows (375 x 2048 -> 2048 over 16 40.3 / 31.9,
+            // 1130 x 1024 -> 2048 over 32 44.2 / 36.0, 68 x 768 -> 3072 over 32 34.9 / 26.9; 2110 x 1024 -> 4096 over 32, 65 rows
+            // each, 76 / 80; 139 x 768 -> 4096 over 32, 1088 tiles, 38.6 / 40.6)
+            if (es == 2 && !p.w_kcontig) {
+                if (tiles128 <= (n_tok <= (int64_t)64 * n_exp ? 288 : 224)) stages64 = 3;
+                else if (n_tok <= (int64_t)48 * n_exp && tiles128 <= 1024) stages64 = 2;
+            }
+        }
     }
     if (tile_cfg == 7) {
         SPX_REQUIRE(es == 2 && !p.w_kcontig, SPX_E_CONFIG, "tile config 7 takes 16-bit types and weights stored [E, in, out]");
@@ -1329,6 +1347,11 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
             return launch_moe_direct<T, 128, 128, 4, 2, 2, 128>(p, st);                    \
         }                                                                                  \
         if (tile_cfg == 6) return launch_moe_direct<T, 256, 256, 16, 4, 4, 64, true>(p, st); \
+        if constexpr (sizeof(T) == 2) {                                                    \
+            if (stages64 == 2) return launch_moe_direct_inst<T, 64, 128, 4, 2, 2, 128, true, false>(p, st); \
+            if (stages64 == 3) return launch_moe_direct_inst<T, 64, 128, 4, 2, 3, 128, true, false>(p, st); \
+            if (tile_cfg == 2 && !p.w_kcontig) return launch_moe_direct_inst<T, 128, 128, 8, 4, 2, 128, true, false>(p, st); \
+        }                                                                                  \
         if (tile_cfg == 2) return launch_moe_direct<T, 128, 128, 4, 2, 2, 128>(p, st);     \
         if (tile_cfg == 3) return launch_moe_direct<T, 256, 256, 8, 2, 2, 128>(p, st);     \
         return launch_moe_direct<T, 256, 256, 16, 4, 2, 128>(p, st);

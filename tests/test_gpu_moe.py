@@ -231,6 +231,23 @@ def test_moe_tile_configs(layout, tile_cfg, dtype, n_tok, in_dims, out_dims, gpu
 
 
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('n_tok,in_dims,out_dims,n_exp', [
+    (1, 64, 4616, 8), (512, 64, 3000, 8),             # 64-row tiles in three stages: one stage of k; ragged columns
+    (520, 192, 776, 4), (1600, 256, 776, 4),          # ... with more than 128 rows to an expert; 224 tiles and more
+    (767, 128, 4096, 16), (769, 320, 4096, 16),       # both sides of 48 rows to an expert: two stages, 128-row tiles
+    (13000, 64, 768, 8), (4200, 128, 2056, 16)])      # 256-row tiles whose unused halves fit a round, and do not
+def test_moe_dispatch(dtype, n_tok, in_dims, out_dims, n_exp, gpu):
+    """The sizes at which the library's own choice of tiles changes, with an empty expert and a crowded one."""
+    moe, w = make_moe(n_exp, in_dims, out_dims, dtype, gpu)
+    p = np.ones(n_exp)
+    p[0], p[1] = 0.0, 3.0
+    ids_np = np.random.default_rng(n_tok).choice(n_exp, size=n_tok, p=p / p.sum()).astype(np.int32)
+    x = torch.from_numpy(np.random.default_rng(1).random((n_tok, in_dims), dtype=np.float32)).to(dtype)
+    got = moe(x.to(gpu), torch.from_numpy(ids_np).to(gpu))
+    assert_close(got, ops.moe_reference(x.to(torch.float64).numpy(), w, ids_np), dtype, f'moe {n_tok} x {in_dims} -> {out_dims} over {n_exp}')
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('n_tok,in_dims,out_dims', [(1, 64, 8), (5, 64, 520), (33, 192, 136), (64, 128, 128), (300, 2048, 264)])
 def test_moe_few_rows_kernel(dtype, n_tok, in_dims, out_dims, gpu):
     """Tile config 7 through the C ABI: fewer k-stages than wavefronts and more, rows that end inside a tile,
