@@ -24,9 +24,9 @@ namespace spx {
 
 constexpr int MOE_CHUNK = 1024;   // most tokens per workgroup in the index kernels (a multiple of 256)
 constexpr int MOE_FUSED_TABLE = 1024;  // (chunk, expert) counts a placement workgroup scans itself
-// Tokens up to which the placement workgroups count the experts themselves, a launch less: a call of 333 tokens
-// 29.7 -> 28.6 us, of 64 24.5 -> 23.1; at 2000 the launch is the cheaper one (82.4 / 83.2 us).
-constexpr int MOE_SELF_COUNT = 1024;
+// Tokens up to which the placement workgroups count the experts themselves, a launch less: 1100 tokens 4.5 -> 3.5 us,
+// 4000 5.1 -> 4.8; 6000 5.0 against 5.5, 8000 5.0 against 7.5.
+constexpr int MOE_SELF_COUNT = 4096;
 constexpr int MOE_MAX_EXP = 2048; // LDS table capacity of the placement kernel
 constexpr int MOE_MAX_ROW_TILES = 65535;   // the y extent of a grid
 
@@ -107,17 +107,17 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* exp_ids, 
         if (counts == nullptr) {   // few tokens: every workgroup counts all of them itself
             for (int i = threadIdx.x; i < n; i += 256) tab[i] = 0;
             __syncthreads();
-            int id[MOE_SELF_COUNT / 256];
+            constexpr int BATCH = 8;   // loads in flight to a thread
+            for (int t0 = threadIdx.x; t0 < n_tok; t0 += 256 * BATCH) {
+                int id[BATCH];
 #pragma unroll
-            for (int j = 0; j < MOE_SELF_COUNT / 256; ++j) {
-                const int t = j * 256 + threadIdx.x;
-                id[j] = t < n_tok ? exp_ids[t] : -1;
-            }
+                for (int j = 0; j < BATCH; ++j) id[j] = t0 + j * 256 < n_tok ? exp_ids[t0 + j * 256] : -1;
 #pragma unroll
-            for (int j = 0; j < MOE_SELF_COUNT / 256; ++j) {
-                const int t = j * 256 + threadIdx.x;
-                const int e = id[j] < 0 || id[j] >= n_exp - 1 ? n_exp - 1 : id[j];
-                if (t < n_tok) atomicAdd(&tab[e * n_chunk + t / chunk], 1);
+                for (int j = 0; j < BATCH; ++j) {
+                    const int t = t0 + j * 256, c = __builtin_amdgcn_readfirstlane(t >> 8) / (chunk >> 8);   // chunks are whole 256s
+                    const int e = id[j] < 0 || id[j] >= n_exp - 1 ? n_exp - 1 : id[j];
+                    if (t < n_tok) atomicAdd(&tab[e * n_chunk + c], 1);
+                }
             }
             __syncthreads();
         }
@@ -188,20 +188,15 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* exp_ids, 
             if (e < 0 || e >= n_exp - 1) e = n_exp - 1;  // out of range: the pseudo expert
         }
         // intra-wave rank and per-wave count of my expert
-        int rank = 0, cnt = 0;
-        bool leader = false;
-        unsigned long long todo = __ballot(e >= 0);
-        while (todo) {
-            const int src = __ffsll((long long)todo) - 1;
-            const int e0 = __shfl(e, src, 64);
-            const unsigned long long same = __ballot(e == e0);
-            if (e == e0) {
-                rank = __popcll(same & lt_mask);
-                cnt = __popcll(same);
-                leader = lane == src;
-            }
-            todo &= ~same;
+        // (a ballot per bit of the expert; with one per expert in the wavefront 700 tokens over 32 experts took 5.6 and not
+        // 3.6 us, 16384 over 32 13.4 and not 6.9, over 4 5.3 and 5.1)
+        unsigned long long same = __ballot(e >= 0);
+        for (int bit = 31 - __builtin_clz(n_exp | 1); bit >= 0; --bit) {
+            const unsigned long long ones = __ballot((e >> bit) & 1);
+            same &= (e >> bit) & 1 ? ones : ~ones;
         }
+        const int rank = __popcll(same & lt_mask), cnt = __popcll(same);
+        const bool leader = e >= 0 && rank == 0;
         if (leader) wavecnt[wave * n_exp + e] = cnt;
         __syncthreads();
         if (e >= 0) {

@@ -230,6 +230,27 @@ def test_moe_tile_configs(layout, tile_cfg, dtype, n_tok, in_dims, out_dims, gpu
     assert_close(out, want, dtype, f'moe tile config {tile_cfg} layout {layout} {dtype}')
 
 
+@pytest.mark.parametrize('n_exp', [1, 2, 7, 8, 63, 64, 900])
+@pytest.mark.parametrize('n_tok', [1, 255, 1025, 2049, 4095, 4096, 4097, 20000])
+def test_moe_index_orders_tokens(n_tok, n_exp, gpu):
+    """Counted by the placement workgroups and by a launch of their own, every number of bits to an expert, with ids that
+    are out of range on both sides: what a stable sort by expert gives, to the last token."""
+    from sparta_amd import _lib
+    lib = _lib.load()
+    ids = np.random.default_rng(n_tok + n_exp).integers(-1, n_exp + 2, n_tok).astype(np.int32)
+    key = np.where((ids < 0) | (ids >= n_exp), n_exp, ids)
+    on = lambda n: torch.full((n,), -1, dtype=torch.int32, device=gpu)
+    dev_ids, count, offset, perm = torch.from_numpy(ids).to(gpu), on(n_exp), on(n_exp + 1), on(n_tok)
+    nbytes = lib.spx_moe_index_workspace_bytes(n_tok, n_exp)
+    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=gpu)
+    _lib.check(lib.spx_moe_index(_lib.dev_ptr(dev_ids), n_tok, n_exp, _lib.dev_ptr(count), _lib.dev_ptr(offset), _lib.dev_ptr(perm),
+                                 _lib.dev_ptr(ws), nbytes, _lib.current_stream(gpu)), 'spx_moe_index')
+    want = np.bincount(key, minlength=n_exp + 1)
+    assert np.array_equal(perm.cpu().numpy(), np.argsort(key, kind='stable'))
+    assert np.array_equal(count.cpu().numpy(), want[:n_exp])
+    assert np.array_equal(offset.cpu().numpy(), np.cumsum(want) - want)
+
+
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('n_tok,in_dims,out_dims,n_exp', [
     (1, 64, 4616, 8), (512, 64, 3000, 8),             # 64-row tiles in three stages: one stage of k; ragged columns
