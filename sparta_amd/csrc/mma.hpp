@@ -57,8 +57,8 @@ template <> struct Mma32<bf16_t> {
 };
 // 32 x 32 x 16 MFMA (2-byte types): lane l holds k = (l/32)*8 .. +7 of row (column) l % 32
 // of the A (B) operand; accumulator register j of lane l is D[8*(j/4) + 4*(l/32) + j%4][l % 32].
-// On gfx950 this shape sustains about twice the FLOP rate of the 16 x 16 x 32 one (both
-// issue every ~32 cycles per SIMD), so MFMA-bound loops should be built from it.
+// One issues every 32 clocks per SIMD (16 x 16 x 32: every 16), so the rate is the same; per
+// fragment read from LDS it does twice the work, with half of the instructions.
 template <typename T> struct MmaW;
 template <> struct MmaW<_Float16> {
     typedef f16x8 frag;

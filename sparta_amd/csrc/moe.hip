@@ -749,7 +749,7 @@ __global__ __launch_bounds__(64 * WAVES, (TM + TN) * NBUF * KTB > 80 * 1024 ? 1 
         for (int q = 0; q < A_LOADS + B_LOADS; ++q) issue_one(s, q);
     };
 
-    // 2-byte types: 32 x 32 x 16 MFMAs (twice the sustained rate of the 16 x 16 x 32 ones)
+    // 2-byte types: 32 x 32 x 16 MFMAs (half of the fragment reads of the 16 x 16 x 32 ones, at the same rate)
     constexpr bool WIDE = HasMma32<T>::value;
     constexpr int MTW = TM / WGM / 32, NTW = TN / WGN / 32;
     const int l32 = lane & 31, h2 = lane >> 5;
