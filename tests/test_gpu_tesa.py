@@ -175,6 +175,14 @@ def test_index_bench_shapes(shape, block, gran, sparsity, gpu):
     _check_indexes(ops.block_mask(shape, gran, sparsity, seed=2022), block[0], block[1], gpu)
 
 
+@pytest.mark.parametrize('R,C', [(1, 1), (16, 16), (1, 257), (257, 1), (60, 64), (61, 63), (130, 2047)])
+@pytest.mark.parametrize('sparsity', [0.0, 0.7])
+def test_index_slices(R, C, sparsity, gpu):
+    """Grids of 256 blocks and one more, and around the most slices: entries, pointers and launch order come from
+    different workgroups."""
+    _check_indexes(ops.block_mask((R * 4, C * 16), (4, 16), sparsity, seed=R + C), 4, 16, gpu)
+
+
 @pytest.mark.parametrize('fill', [0, 1])
 def test_index_all_or_nothing(fill, gpu):
     mask_np = np.full((256, 512), fill, dtype=np.uint8)
