@@ -274,9 +274,20 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         const int64_t big_tiles = (int64_t)((p.Mc + 255) / 256) * nb * batch;
         const int64_t tiles128 = (int64_t)((p.Mc + 127) / 128) * nb * batch;
         const bool fill = big_tiles >= 512;
-        // 128-row tiles halve the traffic of the sparse blocks and want a few rounds of workgroups to
-        // even out (fp32 spends longer on a tile: more of them)
-        int ring = tiles128 >= (sizeof(T) == 4 ? 2048 : BN == 64 ? 1024 : 768) ? 12 : 11;
+        const int64_t tiles64 = (int64_t)((p.Mc + 63) / 64) * nb * batch;
+        // 128-row tiles halve the traffic of the sparse blocks.  fp32 spends long on a tile and wants many of them; 16-bit
+        // types take the tiles that need fewer rounds of the workgroups that fit the chip (64 / 128 rows, us): 32 x 64 blocks
+        // 6993 x 768 -> 704 (2 rounds each) 7.4 / 10.6, 5639 x 704 -> 1152 (3) 10.4 / 15.8, 1036 x 2688 -> 2560 (2 and 1) 20.9 / 15.9,
+        // 1911 x 1600 -> 3648 (3) 15.9 / 17.1, 4674 x 2432 -> 2496 (5 and 4) 47.9 / 43.9, 15667 x 896 -> 2304 (14 and 12) 34.3 / 31.1; blocks of depth 32
+        // have shorter walks: 3917 x 2880 -> 704 (2 and 1) 20.7 / 18.2, but 6319 x 1792 -> 1792 (5 and 4) 13.9 / 17.2, 5350 x 3008 -> 1728
+        // (4 and 3) 33.4 / 38.4; 64 x 64 blocks 3870 x 576 -> 896 (2 and 1) 9.7 / 7.6, 2748 x 1728 -> 1280 (2 and 1) 7.0 / 5.6
+        int ring = tiles128 >= (sizeof(T) == 4 ? 2048 : 1024) ? 12 : 11;
+        const int slots64 = BN == 64 ? 768 : 1280, slots128 = BN == 64 ? 512 : 768;   // (16-bit types)
+        const int64_t rounds64 = (tiles64 + slots64 - 1) / slots64, rounds128 = (tiles128 + slots128 - 1) / slots128;
+        if (sizeof(T) == 2) {
+            if (BN != 64) ring = rounds128 < rounds64 && (p.BK == 64 || rounds64 <= 2) ? 12 : 11;
+            else if (rounds64 == 2 && rounds128 == 1) ring = 12;
+        }
         // The ring kernel, where it was measured ahead (rows x K x N; us of the best other kernel / ring):
         //   * operands that are not both k-contiguous: sdd 4096 x 3072 x 768 fp32 at 20 % 110 / 38, fp16 26 / 14,
         //     dsd 400 x 3072 x 768 fp32 at 15 % 38 / 10, bf16 14 / 10 - but for large fp32 problems in blocks
@@ -288,21 +299,25 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         //     kernels: 8192 x 768 x 3072 at 10 % 23 / 28, 4096^3 at 5 % 25.5 / 31.
         //     Up to 1024 rows the 256-row kernels have too few workgroups for long block-columns, also where
         //     the result is wide: 1024 x 4096 x 4096 at 35 % 61 / 43, 1024^2 x 4096 at 35 % 19.8 / 14.7, at 10 %
-        //     9.8 / 9.2.  Against the column-split kernel (config 8) it is ahead from about 1100 64-row tiles on:
-        //     1500 x 1024 x 2048 15.0 / 11.9, 800 x 1024 x 3072 14.7 / 11.5, 700 x 4096 x 4096 43 / 40 at 35 %,
-        //     9.7 / 7.0, 9.3 / 6.7 and 20 / 16 at 5 - 10 %; with 640 tiles 19.0 / 22.8 (270 x 4096 x 4096), with
-        //     512 8.0 / 8.9 (1024^3).
+        //     9.8 / 9.2.  Against the column-split kernel (config 8) it is ahead from about 700 64-row tiles on:
+        //     634 x 1152 x 3008 at 38 % 17.0 / 10.0, 580 x 3840 x 2496 at 37 % 30.8 / 23.5, 549 x 2176 x 4096 42 / 17, 1500 x 1024 x 2048 15.0 / 11.9; with 512 to
+        //     700 tiles up to 20 live blocks to a column: 693 x 1280 x 1792 at 27 % 12.3 / 8.9, 605 x 1920 x 1792 at 28 % 13.9 / 10.4, 1151 x
+        //     1856 x 1152 at 31 % 13.3 / 11.1, 944 x 1024 x 1152 at 2 % 5.7 / 4.0, but with more 13.5 / 18.7 (935 x 2880 x 1152 at 35 %),
+        //     15.0 / 17.5 (392 x 3072 x 3072 at 37 %), 16.3 / 18.5 (1163 x 3072 x 1024 at 32 %).
         const bool two_blocks = p.BK * (int)sizeof(T) == 64;
         // stored blocks in all block-columns together (all places where it is not known)
         const int64_t stored = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * BN) : (int64_t)cols * nb;
-        const int64_t tiles64 = (int64_t)((p.Mc + 63) / 64) * nb * batch;
         bool use_ring = ring_ok;
         if (two_blocks && sizeof(T) == 4) use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
         else if (two_blocks && kcontig) {
-            const bool few_rows = p.Mc > 256 && p.Mc < 2048 && cols >= 32 && tiles64 >= 1100 && BN == 32;
-            if (fill) use_ring = ring_ok && cols >= 32 && (p.Nc < 2048 || (few_rows && p.Mc <= 1024));
+            const bool few_rows = p.Mc > 256 && p.Mc < 2048 && cols >= 32 && BN == 32 &&
+                                  (tiles64 >= 700 || (tiles64 >= 512 && stored <= 20 * (int64_t)nb));
+            // wide results of 2048 to 3072 rows: 256-row tiles do not come out even (256-row kernel / ring 2474 x
+            // 1408 x 3328 at 28 % 31.0 / 23.3, 2518 x 1088 x 3776 28.7 / 21.9, 2579 x 2624 x 2048 37.9 / 30.4, 2520 x 2112 x 2240 at 13 % 18.9 / 15.7)
+            const bool mid_rows = sizeof(T) == 2 && BN == 32 && p.Mc > 2048 && p.Mc <= 3072 && p.Nc >= 2048;
+            if (mid_rows) ring = rounds128 < rounds64 ? 12 : 11;   // (4 and 3 rounds 29.3 / 23.3; 3 each 41 / 51, 2626 x 3584 x 2688 at 24 %)
+            if (fill) use_ring = ring_ok && cols >= 32 && (p.Nc < 2048 || mid_rows || (few_rows && p.Mc <= 1024));
             else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32 || few_rows);
-            if (few_rows && tiles128 >= 640) ring = 12;   // 1200 x 3072 x 2048: 32.9 us in 64-row tiles, 24.6 in these
         }
         // fp32 blocks of depth 16, long block-columns: four wavefronts that split a column and meet once keep
         // more loads in flight than 256-row tiles when those are few.  256-row kernel / split columns:

@@ -84,3 +84,19 @@ def test_ring_more_tiles_than_the_list(M, gpu, K=64, N=1536):
             want = torch.matmul(x[r:r + 16384].float(), weight) + lin.bias.float()
             # result rounded to 11 bits; sums of 64 products in fp32
             assert float((y[r:r + 16384].float() - want).abs().max()) <= 2 ** -11 * float(want.abs().max()) + 1e-5
+
+
+@pytest.mark.parametrize('dtype,blocks,M,K,N,sparsity', [
+    # 64-row tiles in one round and in two, 128-row tiles in one; and both in two
+    (torch.float16, (32, 32, 32), 2560, 64, 1024, 0.5), (torch.float16, (32, 32, 32), 2561, 64, 1024, 0.5),
+    (torch.bfloat16, (32, 64, 32), 2500, 128, 2048, 0.6), (torch.bfloat16, (64, 64, 64), 4096, 128, 832, 0.6),
+    # few rows, long columns: both sides of 700 tiles, and of 512 with few and with many blocks to a column
+    (torch.float16, (32, 32, 32), 770, 1024, 1696, 0.7), (torch.float16, (32, 32, 32), 770, 1024, 1728, 0.7),
+    # wide results of 2048 to 3072 rows
+    (torch.float16, (32, 32, 32), 2049, 1024, 2048, 0.9), (torch.float16, (32, 32, 32), 3073, 1024, 2048, 0.9),
+    (torch.bfloat16, (32, 32, 32), 1000, 1056, 1024, 0.9), (torch.bfloat16, (32, 32, 32), 1000, 1056, 1024, 0.6),
+    (torch.bfloat16, (32, 32, 32), 1000, 1056, 992, 0.9)])
+def test_dispatch_of_rows_to_a_tile(dtype, blocks, M, K, N, sparsity, gpu):
+    for compressed in (True, False):
+        run_case(gpu, 'dsd', False, True, True, compressed, dtype, blocks, batch=1, M=M, K=K, N=N, gran=(blocks[2], blocks[1]),
+                 sparsity=sparsity, seed=81, tile_cfg=0)
