@@ -386,8 +386,12 @@ static int launch_attention_wide_inst(const AttnParams& p, int nbr, int batch, i
 // 64 / and of 128:
 //   head dim 64   3 x 16 x 640 12.3 / 9.7 / 9.4, 1 x 16 x 2048 18.6 / 13.5 / 11.9, 6 x 8 x 1024 18.0 / 13.4 / 12.6,
 //                 5 x 12 x 1152 19.8 / 17.6 / 19.3, 8 x 12 x 1024 18.9 / 17.6 / 22.9, 9 x 16 x 1024 23.4 / 27.3 / 30.1
+//                 (up to 1024 workgroups of 128 queries where N is 768 and more: 8 x 16 x 1024 22.3 / 20.8, 4 x 16 x 1984 33.6 / 33.0,
+//                 but 32 x 16 x 256 11.1 / 13.2)
 //   head dim 128  2 x 12 x 1024 19.8 / 15.0, 8 x 8 x 768 20.5 / 16.7, 4 x 16 x 1024 23.4 / 20.8, 11 x 16 x 448 16.6 / 21.6
-static bool seqlen_shares_keys(int64_t entries, int N, int E) { return entries * ((N + 127) / 128) <= (E == 64 ? 768 : 512); }
+static bool seqlen_shares_keys(int64_t entries, int N, int E) {
+    return entries * ((N + 127) / 128) <= (E == 64 ? (N >= 768 ? 1024 : 768) : 512);
+}
 
 // Whether this kernel takes the call and not the 16-query one, whose wavefronts start sooner: N from 192 on; with few
 // workgroups long sequences or 384 of 64 queries.  fp16 us, 16-query kernel / shared keys: 2 x 12 x 512 x 64 6.8 / 7.0,

@@ -30,7 +30,8 @@ def test_longest_first(batch, heads, N, lens, E, gpu):
     (7, 12, 320, 'edges'), (24, 8, 256, 'edges'), # and of 64; lengths that end in the first or second share of a stage, or leave one out
     (8, 16, 192, 'mixed'), (48, 8, 192, 'edges'),
     (3, 8, 1056, 'clamped'), (33, 5, 288, 'one'),
-    (768, 1, 96, 'mixed'), (767, 1, 224, 'mixed')])
+    (768, 1, 96, 'mixed'), (767, 1, 224, 'mixed'),
+    (16, 8, 1024, 'mixed'), (19, 9, 768, 'mixed')])   # 1024 workgroups of 128 queries, and 1026
 def test_shared_keys(batch, heads, N, lens, E, gpu):
     """Both sides of the sizes at which two wavefronts share the keys of their queries out."""
     check(batch, heads, N, lens, E, gpu)
