@@ -8,8 +8,8 @@
 //                  1024 (chunk, expert) counts is scanned by every placement
 //                  workgroup itself (two launches); larger ones get a scan
 //                  launch of their own.
-//  spx_moe_forward one gathered GEMM over a flattened (expert, 128-row tile) list:
-//                  a workgroup looks its tile up in the prefix of per-expert tile
+//  spx_moe_forward one gathered GEMM over a flattened (expert, row tile) list (moe_persist.hip: large
+//                  problems): a workgroup looks its tile up in the prefix of per-expert tile
 //                  counts, gathers its token rows through token_perm, and walks
 //                  K in 64-wide stages through LDS ([row][k], XOR-swizzled 16-byte
 //                  chunks) into 16x16 MFMAs; rows are scattered back on store.
@@ -17,8 +17,7 @@
 // reference (csrc/moe_sparse_forward_kernel.cu.j2:58-71,120-325,363-483), whose
 // grid is sized by the largest expert and whose fp16 path accumulates in fp16.
 #include <type_traits>
-#include "common.hpp"
-#include "mma.hpp"
+#include "moe.hpp"
 
 namespace spx {
 
@@ -215,188 +214,6 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* exp_ids, 
 }
 
 // ---- gathered GEMM -------------------------------------------------------------
-struct MoeParams {
-    const void* tokens;
-    const void* weight;
-    void* out;
-    const int32_t* expert_offset;
-    const int32_t* token_perm;
-    int n_tok, K, N, n_exp;
-    int w_kcontig;  // weight [E, N, K] if set, else [E, K, N]
-    int split;      // 0: one launch; 1 / 2: first / second launch of a split (see moe_find_tile)
-    int round_rows; // split: 256-row tiles that one round of the big-tile launch covers
-    int col_groups; // direct kernel: 0: tile (x, y) is workgroup (x, y); else see moe_tile_of_workgroup
-};
-
-// Which (expert, row tile) belongs to tile index y: one wavefront scans the per-expert
-// tile counts.  Expert n_exp is the pseudo expert of the tokens whose id was out of
-// range (token_perm[expert_offset[n_exp] .. n_tok)): its tiles are zero-filled instead
-// of multiplied.  found_e = -1 when y is past the last tile.
-//
-// split (MoeParams::split): a launch of big (256-row) tiles leaves most CUs idle during
-// its last round when the number of row tiles is a little over a multiple of the row
-// tiles one round takes (round_rows).  The work can therefore go out as two launches:
-// split 1 = the 256-row tiles below the last multiple of round_rows (whole rounds),
-// split 2 = the remaining row tiles cut into 128-row halves for the small-tile kernel,
-// which fills the device with them.  Both launches derive the same boundary from the
-// device-side expert counts.
-// Single launch (split == 0): the row tiles are numbered with every expert's full tiles first
-// and the partly filled last tiles of the experts behind them (longest first).  Workgroups start in the order
-// of their tile numbers, so the short tiles (a partly filled tile skips the work of its empty
-// 64-row groups) fill the end of the launch, where the long ones would leave most CUs idle.
-template <int TM>
-__device__ __forceinline__ void moe_find_tile_sorted(const MoeParams& p, int y, int lane,
-                                                     int& found_e, int& found_row0, int& found_rows) {
-    int total_full = 0;
-    for (int e0 = 0; e0 <= p.n_exp; e0 += 64) {
-        const int e = e0 + lane;
-        int cnt = 0;
-        if (e <= p.n_exp) cnt = (e < p.n_exp ? p.expert_offset[e + 1] : p.n_tok) - p.expert_offset[e];
-        total_full += __shfl(wave_inclusive_scan(cnt / TM), 63, 64);
-    }
-    const bool part = y >= total_full;   // looking for a partly filled tile
-    const int want = part ? y - total_full : y;
-    int before = 0;
-    found_e = -1; found_row0 = 0; found_rows = 0;
-    if (part && p.n_exp < 64) {
-        // at most 64 candidates: the partly filled tiles go out longest first (rank = number of
-        // experts whose last tile holds more rows, ties in expert order)
-        int cnt = 0, off = 0;
-        if (lane <= p.n_exp) {
-            off = p.expert_offset[lane];
-            cnt = (lane < p.n_exp ? p.expert_offset[lane + 1] : p.n_tok) - off;
-        }
-        const int full = cnt / TM, rest = cnt - full * TM;
-        int rank = 0;
-        for (int o = 0; o <= p.n_exp; ++o) {
-            const int r = __shfl(rest, o, 64);
-            rank += (r > rest || (r == rest && o < lane)) ? 1 : 0;
-        }
-        const unsigned long long hit = __ballot(rest > 0 && rank == want);
-        if (hit) {
-            const int src = __ffsll((long long)hit) - 1;
-            found_e = src;
-            found_row0 = __shfl(off, src, 64) + __shfl(full, src, 64) * TM;
-            found_rows = __shfl(rest, src, 64);
-        }
-        return;
-    }
-    for (int e0 = 0; e0 <= p.n_exp; e0 += 64) {
-        const int e = e0 + lane;
-        int cnt = 0, off = 0;
-        if (e <= p.n_exp) {
-            off = p.expert_offset[e];
-            cnt = (e < p.n_exp ? p.expert_offset[e + 1] : p.n_tok) - off;
-        }
-        const int full = cnt / TM, rest = cnt - full * TM;
-        const int tiles = part ? (rest ? 1 : 0) : full;
-        const int inc = wave_inclusive_scan(tiles);
-        const int excl = before + inc - tiles;
-        const unsigned long long hit = __ballot(want >= excl && want < excl + tiles);
-        if (hit) {
-            const int src = __ffsll((long long)hit) - 1;
-            const int lt = want - __shfl(excl, src, 64);
-            found_e = e0 + src;
-            found_row0 = __shfl(off, src, 64) + (part ? __shfl(full, src, 64) : lt) * TM;
-            found_rows = part ? __shfl(rest, src, 64) : TM;
-            return;
-        }
-        before += __shfl(inc, 63, 64);
-    }
-}
-
-template <int TM>
-__device__ __forceinline__ void moe_find_tile(const MoeParams& p, int y, int lane,
-                                              int& found_e, int& found_row0, int& found_rows) {
-    if (p.split == 0) {
-        moe_find_tile_sorted<TM>(p, y, lane, found_e, found_row0, found_rows);
-        return;
-    }
-    const int TS = p.split ? 256 : TM;      // tile height the row tiles are counted in
-    int half = 0;
-    if (p.split == 2) { half = y & 1; y >>= 1; }
-    int tiles_before = 0;
-    int fe = -1, frow0 = 0, frows = 0, fy = -1;
-    for (int e0 = 0; e0 <= p.n_exp && (fe < 0 || p.split); e0 += 64) {
-        const int e = e0 + lane;
-        int cnt = 0, off = 0;
-        if (e <= p.n_exp) {
-            off = p.expert_offset[e];
-            cnt = (e < p.n_exp ? p.expert_offset[e + 1] : p.n_tok) - off;
-        }
-        const int tiles = (cnt + TS - 1) / TS;
-        const int inc = wave_inclusive_scan(tiles);
-        const int excl = tiles_before + inc - tiles;
-        // split 2 counts y from the boundary, which is only known after the whole scan:
-        // remember every expert's range and pick afterwards (n_exp <= 64 in one pass)
-        if (p.split != 2) {
-            const bool mine = y >= excl && y < excl + tiles;
-            const unsigned long long hit = __ballot(mine);
-            if (hit && fe < 0) {
-                const int src = __ffsll((long long)hit) - 1;
-                const int lt = y - __shfl(excl, src, 64);
-                fe = e0 + src; fy = y;
-                frow0 = __shfl(off, src, 64) + lt * TS;
-                frows = min(TS, __shfl(cnt, src, 64) - lt * TS);
-            }
-        }
-        tiles_before += __shfl(inc, 63, 64);
-    }
-    int boundary = tiles_before;  // first row tile of the second launch
-    if (p.split) {
-        const int rem = tiles_before % p.round_rows;
-        // a last round that is mostly full stays with the big tiles
-        if (rem * 10 <= p.round_rows * 6) boundary = tiles_before - rem;
-    }
-    if (p.split == 1 && fy >= boundary) fe = -1;
-    if (p.split == 2) {
-        const int yb = boundary + y;
-        fe = -1;
-        int before = 0;
-        for (int e0 = 0; e0 <= p.n_exp && fe < 0 && yb < tiles_before; e0 += 64) {
-            const int e = e0 + lane;
-            int cnt = 0, off = 0;
-            if (e <= p.n_exp) {
-                off = p.expert_offset[e];
-                cnt = (e < p.n_exp ? p.expert_offset[e + 1] : p.n_tok) - off;
-            }
-            const int tiles = (cnt + 255) / 256;
-            const int inc = wave_inclusive_scan(tiles);
-            const int excl = before + inc - tiles;
-            const unsigned long long hit = __ballot(yb >= excl && yb < excl + tiles);
-            if (hit) {
-                const int src = __ffsll((long long)hit) - 1;
-                const int lt = yb - __shfl(excl, src, 64);
-                const int r0 = lt * 256 + half * 128;
-                const int left = __shfl(cnt, src, 64) - r0;
-                if (left > 0) {
-                    fe = e0 + src;
-                    frow0 = __shfl(off, src, 64) + r0;
-                    frows = min(128, left);
-                } else {
-                    break;  // the upper half of a row tile with at most 128 rows
-                }
-            }
-            before += __shfl(inc, 63, 64);
-        }
-    }
-    found_e = fe; found_row0 = frow0; found_rows = frows;
-}
-
-// Zero rows token_perm[row0 .. row0 + rows) of `out`, columns n0 .. n0 + TN (16-byte stores).
-template <typename T>
-__device__ __forceinline__ void moe_zero_tile(const MoeParams& p, int row0, int rows, int n0, int TN, int nthreads) {
-    constexpr int VE = 16 / (int)sizeof(T);
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    T* out = reinterpret_cast<T*>(p.out);
-    const int ncol = (min(n0 + TN, p.N) - n0) / VE;  // N is a multiple of VE
-    for (int v = threadIdx.x; v < rows * ncol; v += nthreads) {
-        const int r = v / ncol, c = v - r * ncol;
-        const int tok = p.token_perm[row0 + r];
-        *reinterpret_cast<u32x4*>(out + (int64_t)tok * p.N + n0 + c * VE) = u32x4{0u, 0u, 0u, 0u};
-    }
-}
-
 constexpr int MOE_TM = 128, MOE_TN = 128;
 // k per LDS stage: 128 bytes per row for every element type
 template <typename T> struct MoeKt { static constexpr int value = 128 / (int)sizeof(T); };
@@ -1008,8 +825,7 @@ __global__ __launch_bounds__(64 * WAVES, (TM + TN) * NBUF * KTB > 80 * 1024 ? 1 
 
 template <typename T, int TM, int TN, int WAVES, int WGM, int NBUF, int KTB, bool BKN, bool XS>
 static int launch_moe_direct_inst(const MoeParams& p, hipStream_t st) {
-    // split 2 covers at most one round of 256-row tiles, as 128-row halves
-    int tiles = p.split == 2 ? 2 * p.round_rows : (p.n_tok + TM - 1) / TM + p.n_exp + 1;
+    int tiles = (p.n_tok + TM - 1) / TM + p.n_exp + 1;
     if (tiles > MOE_MAX_ROW_TILES) return fail(SPX_E_SHAPE, "too many row tiles for one launch");
     const int ntn = (p.N + TN - 1) / TN;
     MoeParams q = p;
@@ -1265,17 +1081,16 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     p.expert_offset = expert_offset; p.token_perm = token_perm;
     p.n_tok = n_tok; p.K = in_dim; p.N = out_dim; p.n_exp = n_exp;
     p.w_kcontig = weight_layout == 1;
-    p.split = 0; p.round_rows = 1; p.col_groups = 0;
+    p.col_groups = 0;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // tile_cfg 1: 128x128 tiles staged through registers (any dtype and weight layout);
     // 2 / 3 / 4: tiles filled by LDS-direct loads - 128x128 with four wavefronts (two
     // workgroups per CU; eight for 16-bit [E, in, out] weights: 700 x 2048 -> 2048 over 16 bf16 40.4 -> 37.8 us,
-    // 2113 x 2048 -> 2048 over 8 fp16 44.5 -> 38.7, 1342 x 1024 -> 4096 over 8 30.1 -> 27.5; behind a round of 256-row tiles 171.9 against
-    // 173.7 and 163.3 against 159.5, so there it is four), 256x256 with eight wavefronts of 128x64, 256x256 with sixteen
-    // wavefronts of 64x64 - for 16-bit types in either weight layout and fp32 with
+    // 2113 x 2048 -> 2048 over 8 fp16 44.5 -> 38.7, 1342 x 1024 -> 4096 over 8 30.1 -> 27.5), 256x256 with eight wavefronts of
+    // 128x64, 256x256 with sixteen wavefronts of 64x64 - for 16-bit types in either weight layout and fp32 with
     // k-contiguous weights.  256x256 tiles move half the bytes from L2 to the CUs, which is
-    // what bounds the 128x128 kernel.  5 = 4 for the whole rounds of 256-row tiles plus 2 for
-    // the row tiles of a thinly filled last round (two launches, see moe_find_tile).  7: 32-row
+    // what bounds the 128x128 kernel.  5: 256x256 tiles by workgroups that stay on their CU (moe_persist.hip; 4 where it
+    // does not take the type or the sizes).  7: 32-row
     // tiles for few rows per expert (16-bit, [E, in, out] weights).  0 picks between 7, 5, 4, 2 and, for 16-bit
     // [E, in, out] weights, 64 x 128 tiles of two or three stages that have no number of their own, by the number of
     // tiles and of rows per expert (below); fp32 [E, in, out] weights take 1.
@@ -1289,9 +1104,15 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     }
     int stages64 = 0;   // 64 x 128 tiles with that many stages
     if (tile_cfg == 0) {
-        // 16-bit types: 256x256 tiles from 256 of them on (split launch, 5); from 128 on when
+        // 16-bit types: 256x256 tiles by persistent workgroups (5) from 224 of them on; with experts of many rows, whose last
+        // tiles waste little, from fewer on, and the fewer the longer the walk over k.  us of the best other choice below /
+        // persistent: 3346 x 1024 -> 4096 over 16 (224 tiles) 62.5 / 53.1, 2670 x 768 -> 4096 over 16 (176, 166 rows each) 45.4 / 41.0,
+        // 3569 x 768 -> 3072 over 8 (168) 34.0 / 31.4, 4564 x 1024 -> 2048 over 4 (144) 35.7 / 34.2, 9889 x 2048 -> 768 over 4 (117)
+        // 46.1 / 41.0, 6673 x 2048 -> 768 over 8 (81) 42.7 / 38.4; but 3640 x 2048 -> 2048 over 4 (120) 45.8 / 49.3, 10529 x 768 -> 768 over 4 (126) 27.3 / 28.5, 2911 x 1024 -> 3072
+        // over 16 (144, 181 rows each) 41.6 / 46.7, 3254 x 1024 -> 3072 over 32 (156, 101 rows each) level, 1994 x 2048 -> 768 over 8
+        // (24) 25.3 / 29.5.  256x256 tiles of one workgroup each (4) where k is too short for the pipeline: from 128 on when
         // all of them, the partly filled ones at the expert boundaries included, run in a
-        // single round (4: ten mid-size problems measured 10 - 25 % ahead of the 128x128
+        // single round (ten mid-size problems measured 10 - 25 % ahead of the 128x128
         // tiles there, and behind them as soon as a second round starts); else 128x128
         const int64_t row_tiles = (n_tok + 255) / 256, col_tiles = (out_dim + 255) / 256;
         const int64_t big_tiles = row_tiles * col_tiles;
@@ -1303,9 +1124,19 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         // 15.7 / 15.9 (2048 x 1024 -> 768 over 8).
         const int64_t tiles128 = ((n_tok + 127) / 128 + (int64_t)(n_tok < n_exp ? n_tok : n_exp)) * ((out_dim + 127) / 128);
         const bool few_rows = es == 2 && !p.w_kcontig && tiles128 <= 256 && n_tok <= (int64_t)128 * n_exp;
+        const bool many_rows = n_tok >= (int64_t)256 * n_exp;
+        // long walks: where tiles of 256 rows go out as halves, or tiles of 128 rows are more than two to a CU (half a tile
+        // of every expert is unused, give or take)
+        const bool long_walk = in_dim >= 2048 && big_tiles >= 64 &&
+                               ((row_tiles + n_exp / 2) * col_tiles <= n_cu / 2 ||
+                                ((n_tok + 127) / 128 + n_exp / 2) * ((out_dim + 127) / 128) > 2 * n_cu);
+        const bool persist = es == 2 && moe_persist_supported(p) &&
+                             (big_tiles >= 224 || (big_tiles >= 160 && n_tok >= (int64_t)128 * n_exp) ||
+                              (many_rows && (big_tiles >= 130 || long_walk)));
         if (!direct_ok) tile_cfg = 1;
         else if (few_rows) tile_cfg = 7;
-        else if (es == 2 && big_tiles >= 256) tile_cfg = 5;
+        else if (persist) tile_cfg = 5;
+        else if (es == 2 && big_tiles >= 256) tile_cfg = 4;
         else if (es == 2 && big_tiles >= 128 && (row_tiles + n_exp) * col_tiles <= n_cu) tile_cfg = 4;
         // experts of more than a 256-row tile leave half a tile unused each, give or take: also where that many fit a round
         // (16108 x 768 -> 768 over 32 fp16 47.0 / 40.3 us with 128- and 256-row tiles, 4718 x 768 -> 2048 over 16 40.9 / 36.8;
@@ -1330,18 +1161,10 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     }
     if (tile_cfg >= 2) {
         SPX_REQUIRE(direct_ok, SPX_E_CONFIG, "tile config %d takes fp32 weights in layout 1 only", tile_cfg);
-        if (tile_cfg == 5) {
-            const int ntn = (out_dim + 255) / 256;
-            p.round_rows = n_cu / ntn > 0 ? n_cu / ntn : 1;
-        }
+        if (tile_cfg == 5 && !(es == 2 && moe_persist_supported(p))) tile_cfg = 4;
 #define SPX_MOE_DIRECT(T)                                                                  \
-        if (tile_cfg == 5) {                                                               \
-            p.split = 1;                                                                   \
-            const int rc = launch_moe_direct<T, 256, 256, 16, 4, 2, 128>(p, st);           \
-            if (rc) return rc;                                                             \
-            p.split = 2;                                                                   \
-            return launch_moe_direct<T, 128, 128, 4, 2, 2, 128>(p, st);                    \
-        }                                                                                  \
+        if constexpr (sizeof(T) == 2)                                                      \
+            if (tile_cfg == 5) return launch_moe_persist<T>(p, n_cu, st);                  \
         if (tile_cfg == 6) return launch_moe_direct<T, 256, 256, 16, 4, 4, 64, true>(p, st); \
         if constexpr (sizeof(T) == 2) {                                                    \
             if (stages64 == 2) return launch_moe_direct_inst<T, 64, 128, 4, 2, 2, 128, true, false>(p, st); \

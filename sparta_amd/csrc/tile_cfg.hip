@@ -49,7 +49,7 @@ static const spx_tile_cfg kMoeCfgs[] = {
     {2, 128, 128, 4, 2, 0, 7, "gather-128x128-lds-direct"},
     {3, 256, 256, 8, 2, 0, 7, "gather-256x256-lds-direct"},
     {4, 256, 256, 16, 2, 0, 7, "gather-256x256-direct-16-waves"},
-    {5, 256, 256, 16, 2, 0, 7, "gather-256x256-plus-128-tail"},
+    {5, 256, 256, 8, 2, 0, 7, "gather-256x256-persistent"},
     {6, 256, 256, 16, 4, 0, 6, "gather-256x256-cross-stage"},
     {7, 32, 128, 4, 2, 0, 6, "gather-32x128-k-split"},
 };

@@ -230,6 +230,42 @@ def test_moe_tile_configs(layout, tile_cfg, dtype, n_tok, in_dims, out_dims, gpu
     assert_close(out, want, dtype, f'moe tile config {tile_cfg} layout {layout} {dtype}')
 
 
+@pytest.mark.parametrize('layout', [0, 1])
+@pytest.mark.parametrize('dtype,n_tok,in_dims,out_dims,n_exp', [
+    # 256 workgroups.  No whole round: quarters of a tile, halves (15 tiles to an XCD), whole ones; the shortest k (four stages)
+    (torch.float16, 300, 256, 264, 3), (torch.bfloat16, 5000, 320, 1032, 5), (torch.float16, 9000, 256, 1288, 3),
+    # whole rounds and a rest; more experts than lanes; a strip that is not full
+    (torch.bfloat16, 20000, 576, 1544, 4), (torch.float16, 17000, 256, 1032, 70), (torch.float16, 1, 256, 8, 2)])
+def test_moe_persistent_tiles(layout, dtype, n_tok, in_dims, out_dims, n_exp, gpu):
+    """Tile config 5 through the C ABI: every cut of the last round, experts that end inside a tile and inside a half of one, an
+    empty expert, tokens without one, and a token of NaN that reaches no other row."""
+    from sparta_amd import _lib
+    moe, w = make_moe(n_exp, in_dims, out_dims, dtype, gpu)
+    rng = np.random.default_rng(n_tok)
+    share = np.r_[np.arange(1, n_exp + 1, dtype=np.float64) ** -0.8, 0.05]   # id n_exp: no expert
+    share[n_exp // 2] = 0.0
+    ids_np = rng.choice(n_exp + 1, size=n_tok, p=share / share.sum()).astype(np.int32)
+    x = torch.from_numpy(rng.random((n_tok, in_dims), dtype=np.float32)).to(dtype)
+    xg, bad = x.to(gpu), n_tok - 1
+    ids_np[bad] = 0
+    xg[bad] = float('nan')
+    moe(xg, torch.from_numpy(ids_np).to(gpu))  # builds the index
+    weight = moe.weight.detach() if layout == 0 else moe.weight.detach().transpose(1, 2).contiguous()
+    out = torch.full((n_tok, out_dims), float('nan'), dtype=dtype, device=gpu)
+
+    def call():
+        _lib.check(_lib.load().spx_moe_forward(_lib.dtype_code(dtype), _lib.dev_ptr(xg), _lib.dev_ptr(weight), layout, _lib.dev_ptr(out),
+                                               _lib.dev_ptr(moe.expert_offset), _lib.dev_ptr(moe.sparse_index), n_tok, in_dims, out_dims,
+                                               n_exp, 5, _lib.current_stream(gpu)), 'spx_moe_forward')
+
+    _, names = launched_kernels(call)
+    assert any('moe_persist_kernel' in n for n in names), names
+    assert bool(torch.isnan(out[bad]).all())
+    rows = np.arange(n_tok) != bad
+    want = ops.moe_reference(x.to(torch.float64).numpy(), np.concatenate([w, np.zeros_like(w[:1])]), ids_np)
+    assert_close(out[torch.from_numpy(rows).to(gpu)], want[rows], dtype, f'persistent moe {n_tok} x {in_dims} -> {out_dims} over {n_exp}')
+
+
 @pytest.mark.parametrize('n_exp', [1, 2, 7, 8, 63, 64, 900])
 @pytest.mark.parametrize('n_tok', [1, 255, 1025, 2049, 4095, 4096, 4097, 20000])
 def test_moe_index_orders_tokens(n_tok, n_exp, gpu):
