@@ -135,7 +135,9 @@ extern "C" int spx_matmul(int mode, int dtype, int transA, int transB, int compr
 namespace spx {
 
 static int split_slices(int dtype, int transA, int transB, int nnz, int batch, int K, int BM, int BN, int slices) {
-    return slices ? slices : dds_split_slices(dtype_bytes(dtype), !transA && transB, nnz, batch, K, BM, BN);
+    if (slices) return slices;
+    const DdsShare share = dds_share_plan(dtype_bytes(dtype), !transA, transB, nnz, batch, K, BM, BN);
+    return share.blocks ? share.slices : dds_split_slices(dtype_bytes(dtype), !transA && transB, nnz, batch, K, BM, BN);
 }
 static size_t split_partial_bytes(int slices, int nnz, int batch, int BM, int BN) {
     return slices > 1 ? (size_t)batch * slices * nnz * BM * BN * sizeof(float) : 0;
@@ -174,6 +176,7 @@ extern "C" int spx_matmul_split(int dtype, int transA, int transB, int compresse
     DdsSplit s;
     SPX_REQUIRE(slices == 0 || slices == 1 || slices == 2 || slices == 4 || slices == 8, SPX_E_CONFIG, "slices=%d not in {0,1,2,4,8}", slices);
     s.slices = split_slices(dtype, transA, transB, nnz, batch, K, BM, BN, slices);
+    s.share = slices ? 0 : dds_share_plan(es, !transA, transB, nnz, batch, K, BM, BN).blocks;
     s.k_slice = 0;
     s.nnz = nnz;
     s.n_product = 0;

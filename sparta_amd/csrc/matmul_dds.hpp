@@ -683,7 +683,9 @@ static int launch_dds_inst(const DdsParams& p, int nnz_bound, int batch, hipStre
 }
 
 template <typename T>
-int launch_dds_unsliced(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, hipStream_t st);
+int launch_dds_unsliced(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, bool share, hipStream_t st);
+template <typename T>
+bool dds_shares_rows(const DdsParams& p, int BM, int BN, int nnz_bound, int batch);
 
 // tile_cfg: 0 = by layout and depth; 1 = one LDS buffer, no prefetch;
 //           2 = pipelined (register ring + two LDS buffers); 3 / 4 = the short-K kernels above.
@@ -692,7 +694,7 @@ int launch_dds_impl(const DdsParams& p, int BM, int BN, int nnz_bound, int batch
     if (tile_cfg < 0 || tile_cfg > 4) return fail(SPX_E_CONFIG, "unknown tile config %d", tile_cfg);
     const bool row = dds_row_ok<T>(p, BM, BN);
     const bool rowq = dds_rowq_ok<T>(p, BM, BN);
-    if (tile_cfg == 0) tile_cfg = rowq ? 4 : (row ? 3 : 2);
+    if (tile_cfg == 0 && (rowq || row)) tile_cfg = rowq ? 4 : 3;
     if (tile_cfg == 4) {
         if (!rowq) return fail(SPX_E_CONFIG, "tile config 4 needs a 16-bit type, row_ptr, k-contiguous operands, compressed output, 32/64-wide blocks and K of 64 or 128");
         return launch_dds_rowq<T>(p, BM, BN, batch, st);
@@ -701,7 +703,10 @@ int launch_dds_impl(const DdsParams& p, int BM, int BN, int nnz_bound, int batch
         if (!row) return fail(SPX_E_CONFIG, "tile config 3 needs row_ptr, k-contiguous operands, 32/64-wide blocks and K of 128 or 256 bytes");
         return launch_dds_row<T>(p, BM, BN, batch, st);
     }
-    if (tile_cfg == 2 && !dds_pipe_ok<T>(p, BM, BN)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, st);
+    // many fp32 blocks of 32 x 32: two to a workgroup, which share their rows of A (matmul_dds_share.hpp)
+    if (tile_cfg == 0 && dds_shares_rows<T>(p, BM, BN, nnz_bound, batch)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, true, st);
+    if (tile_cfg == 0) tile_cfg = 2;
+    if (tile_cfg == 2 && !dds_pipe_ok<T>(p, BM, BN)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, false, st);
 #define SPX_DDS_CASE(bm, bn) \
     if (BM == bm && BN == bn) \
         return tile_cfg == 2 ? launch_dds_pipe_inst<T, bm, bn>(p, nnz_bound, batch, st) : launch_dds_inst<T, bm, bn>(p, nnz_bound, batch, st);

@@ -55,6 +55,7 @@ struct DdsSplit {
     float* partial;     // [batch][slices][nnz][BM * BN]
     float* colsum;      // [batch][kColsumSlices][M], NULL: not wanted, or:
     void* colsum_out;   // [batch][M] of the operand type: a workgroup adds up all of k and writes the sums themselves
+    int share;          // blocks of a block-row to a workgroup (matmul_dds_share.hpp), 0: one each
 };
 
 template <typename T, int BM, int BN> struct DdsSplitCfg {
@@ -419,6 +420,18 @@ inline int dds_split_slices(int elem_bytes, bool kcontig, int nnz, int batch, in
     return best;
 }
 
+// The second launch: partial blocks and ranges of the column sums, where there are any.
+template <typename T>
+static int launch_dds_split_reduce(const DdsParams& p, const DdsSplit& s, void* colsum, int BM, int BN, int batch, hipStream_t st) {
+    const int n_blocks = s.slices > 1 ? (int)(((int64_t)s.nnz * BM * BN / 4 + 255) / 256) : 0;
+    const int n_cols = s.colsum ? (p.M + 255) / 256 : 0;
+    if (n_blocks + n_cols == 0) return 0;
+    hipLaunchKernelGGL((dds_split_reduce_kernel<T>), dim3(n_blocks + n_cols, batch, 1), dim3(256), 0, st, p, s,
+                       reinterpret_cast<T*>(colsum), BM, BN, n_blocks);
+    SPX_LAUNCH_CHECK("dds_split_reduce_kernel");
+    return 0;
+}
+
 template <typename T, int BM, int BN, bool AT, bool BT>
 static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, int batch, hipStream_t st) {
     constexpr int VE = 16 / (int)sizeof(T);
@@ -442,17 +455,60 @@ static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, i
     SPX_GRANT_LDS((dds_split_kernel<T, BM, BN, AT, BT>), most, "dds_split_kernel");
     hipLaunchKernelGGL((dds_split_kernel<T, BM, BN, AT, BT>), dim3((unsigned)(n_product + cs_groups), batch, 1), dim3(256), smem, st, p, s);
     SPX_LAUNCH_CHECK("dds_split_kernel");
-    const int n_blocks = s.slices > 1 ? (int)(((int64_t)s.nnz * BM * BN / 4 + 255) / 256) : 0;
-    const int n_cols = s.colsum ? (p.M + 255) / 256 : 0;
-    if (n_blocks + n_cols == 0) return 0;
-    hipLaunchKernelGGL((dds_split_reduce_kernel<T>), dim3(n_blocks + n_cols, batch, 1), dim3(256), 0, st, p, s,
-                       reinterpret_cast<T*>(colsum), BM, BN, n_blocks);
-    SPX_LAUNCH_CHECK("dds_split_reduce_kernel");
-    return 0;
+    return launch_dds_split_reduce<T>(p, s, colsum, BM, BN, batch, st);
+}
+
+// Blocks of a block-row to a workgroup, which then share their rows of A, and slices for them; 0: one block to a workgroup.
+// Weight gradients (both operands k-major): from so many blocks times tokens on that the fewer workgroups still fill the chip
+// evenly; below, the many short chains of one block each are ahead.  Product and second kernel, us, one block / shared:
+//   fp32 16 x 16  1270 blocks over 5328 tokens 80.8 / 59.4, 1980 over 1856 50.0 / 38.2, 3074 over 336 (unsliced) 16.6 / 14.6,
+//                 but 1229 over 768 14.9 / 16.4, 31 over 4000 9.1 / 13.2
+//   fp32 32 x 32  461 over 4096 60.6 / 49.7, 898 over 4144 125 / 96, 612 over 1792 41.5 / 35.1, but 253 over 2096 25.0 / 26.5,
+//                 306 over 352 8.9 / 9.5; two blocks to a workgroup or four: 612 over 1792 35.1 / 35.9, 898 over 4144 103 / 92
+//   fp32 32 x 64  210 over 2544 39.9 / 36.3, 1371 over 4512 301 / 249, but 110 over 1056 17.4 / 20.5; 64 x 64: 583 over 4592 228 / 221, 745
+//                 over 432 31.2 / 36.9
+//   16-bit 32 x 32  450 over 2416 21.1 / 15.7, 706 over 2128 22.2 / 20.3, 305 over 1504 15.7 / 14.1, but 116 over 1248 10.2 / 9.6,
+//                 437 over 592 7.4 / 8.5;  32 x 64  410 over 4096 33.6 / 28.5, 187 over 5072 23.5 / 21.9, but 93 over 1152 10.2 / 12.4;
+//                 64 x 64  309 over 2848 29.4 / 24.6, 1021 over 784 (unsliced) 20.3 / 18.1, but 349 over 736 level, 46 over 3664 13.3 / 15.3
+// Scores (both k-contiguous, unsliced): fp32 32 x 32, two blocks, from 1000 of them on (2458 over 768 51 / 43.5 us, 1229 over 256
+// 14.9 / 13.1, 1229 over 128 9.9 / 9.6; 388 over 768 14.5 / 15.7; 64 x 64: 396 over 768 34.3 / 33.2).
+struct DdsShare {
+    int blocks, slices;
+};
+inline DdsShare dds_share_plan(int elem_bytes, bool a_kcontig, bool b_kcontig, int nnz, int batch, int K, int BM, int BN) {
+    const int64_t blocks = (int64_t)nnz * batch;
+    if (a_kcontig != b_kcontig) return {0, 1};
+    if (a_kcontig) return {elem_bytes == 4 && BM == 32 && BN == 32 && blocks >= 1000 ? 2 : 0, 1};
+    const int64_t work = blocks * K;
+    DdsShare plan = {0, K < 1024 ? 1 : 4};
+    if (elem_bytes == 4 && BM == 16 && BN == 16 && work >= 1000000) plan = {4, K < 1024 ? 1 : blocks <= 2048 ? 8 : 4};
+    else if (elem_bytes == 4 && BM == 32 && BN == 32 && K >= 1024 && work >= 800000) plan = work < 1500000 ? DdsShare{2, 4} : DdsShare{4, 8};
+    else if (elem_bytes == 4 && BM == 32 && BN == 64 && K >= 1024 && work >= 500000) plan.blocks = 2;
+    else if (elem_bytes == 2 && BM == 32 && BN == 32 && K >= 1024 && work >= 400000) plan.blocks = 4;
+    else if (elem_bytes == 2 && BM == 32 && BN == 64 && K >= 1024 && work >= 800000) plan.blocks = 2;
+    else if (elem_bytes == 2 && BM == 64 && BN == 64 && work >= 600000) plan.blocks = 2;
+    if (elem_bytes == 4 && plan.blocks) {   // no longer chains of fp32 additions than one block to a workgroup has
+        const int whole = dds_split_slices(elem_bytes, false, nnz, batch, K, BM, BN);
+        if (whole > plan.slices) plan.slices = whole;
+    }
+    while (plan.slices > 1 && plan.slices * (double)blocks * BM * BN * sizeof(float) > (double)kSplitPartialBytes) plan.slices /= 2;
+    return plan;
+}
+
+template <typename T>
+int launch_dds_share(const DdsParams& p, const DdsSplit& s, void* colsum, int BM, int BN, int batch, hipStream_t st);
+template <typename T>
+bool dds_share_takes(const DdsParams& p) {   // (byte offsets of 64 rows in 32 bits)
+    return p.row_ptr && !p.bias && p.a_ld < (1 << 23) && p.b_ld < (1 << 23);
+}
+template <typename T>
+bool dds_shares_rows(const DdsParams& p, int BM, int BN, int nnz_bound, int batch) {
+    return p.a_kcontig && dds_share_takes<T>(p) && dds_share_plan((int)sizeof(T), true, p.b_kcontig != 0, nnz_bound, batch, p.K, BM, BN).blocks > 0;
 }
 
 template <typename T>
 int launch_dds_split_impl(const DdsParams& p, const DdsSplit& s, void* colsum, int BM, int BN, int batch, hipStream_t st) {
+    if (s.share && dds_share_takes<T>(p)) return launch_dds_share<T>(p, s, colsum, BM, BN, batch, st);
 #define SPX_DDS_SPLIT_CASE(bm, bn)                                                                                  \
     if (BM == bm && BN == bn)                                                                                       \
         return !p.a_kcontig && !p.b_kcontig ? launch_dds_split_inst<T, bm, bn, true, true>(p, s, colsum, batch, st) \
