@@ -310,8 +310,22 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         // stored blocks in all block-columns together (all places where it is not known)
         const int64_t stored = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * BN) : (int64_t)cols * nb;
         bool use_ring = ring_ok;
-        if (two_blocks && sizeof(T) == 4) use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
-        else if (two_blocks && kcontig) {
+        if (two_blocks && sizeof(T) == 4) {
+            use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
+            // k-contiguous blocks of 16 x 16 (us, column-split or 256-row kernel / ring).  Block-columns of medium length over 700 to
+            // 2047 rows, up to 23 live blocks to a column, 16 where the result is wide: 1024^3 at 35 % 15.9 / 14.8, at 20 % 11.3 / 9.7,
+            // 774 x 784 x 3584 at 25 % 28.6 / 23.8, 877 x 896 x 1728 at 20 % 16.2 / 13.7, 1777 x 1088 x 832 at 11 % 13.6 / 10.6, but 512 x 1024 x
+            // 1024 at 35 % 9.8 / 12.3, 820 x 1152 x 2048 at 35 % 26.9 / 30.3, 1024 x 1024 x 2048 at 35 % 25.6 / 26.6.  Short ones over up to 6000
+            // rows, eight live blocks to a column: 2256 x 576 x 1088 15.6 / 12.0, 2425 x 576 x 1408 20.9 / 16.0, 5192 x 640 x 1024 16.7 / 14.9, but
+            // 3704 x 704 x 1280 at 22 % 27.8 / 32.1, 11824 x 576 x 832 24.8 / 27.2.
+            if (kcontig && BN == 16 && ring_ok) {
+                if (p.Mc >= 700 && p.Mc < 2048 && cols > 48 && cols <= 88 && stored <= (nb <= 96 ? 23 : 16) * (int64_t)nb) use_ring = true;
+                if (p.Mc >= 2048 && p.Mc <= 6000 && cols <= 48 && nb <= 96 && stored <= 8 * (int64_t)nb) {
+                    use_ring = true;
+                    ring = 11;   // (5192 x 640 x 1024 with 128-row tiles 18.4)
+                }
+            }
+        } else if (two_blocks && kcontig) {
             const bool few_rows = p.Mc > 256 && p.Mc < 2048 && cols >= 32 && BN == 32 &&
                                   (tiles64 >= 700 || (tiles64 >= 512 && stored <= 20 * (int64_t)nb));
             // wide results of 2048 to 3072 rows: 256-row tiles do not come out even (256-row kernel / ring 2474 x

@@ -54,6 +54,10 @@ def test_ring_more_block_columns_than_the_table(gpu):
     # ... more rows: up to 32 and up to 64 block-columns, both sides of the live-block limits
     (torch.float32, (16, 16, 16), 1025, 1056, 512, 0.8), (torch.float32, (16, 16, 16), 1500, 1056, 1024, 0.7),
     (torch.float32, (16, 16, 16), 1025, 800, 512, 0.95), (torch.float32, (16, 16, 16), 1025, 1056, 1040, 0.8),
+    # fp32 16 x 16 through the ring: medium block-columns, first row count and the one before, wide results, too many live blocks;
+    # short ones over many rows, and one row too many
+    (torch.float32, (16, 16, 16), 700, 784, 1040, 0.7), (torch.float32, (16, 16, 16), 699, 784, 1040, 0.7), (torch.float32, (16, 16, 16), 900, 1408, 1552, 0.84),
+    (torch.float32, (16, 16, 16), 900, 1408, 1536, 0.7), (torch.float32, (16, 16, 16), 2049, 768, 1536, 0.86), (torch.float32, (16, 16, 16), 6001, 512, 512, 0.9),
     # ring: 1100 tiles of 64 rows in tiles of 64 and of 128, and one column fewer
     (torch.float16, (32, 32, 32), 257, 1024, 7040, 0.95), (torch.float16, (32, 32, 32), 257, 1024, 7008, 0.95),
     # 256-row tiles: a block or less to a block-column, and one side of each limit
