@@ -7,7 +7,8 @@
 //                  ascending order behind its scanned base.  A table of at most
 //                  1024 (chunk, expert) counts is scanned by every placement
 //                  workgroup itself (two launches); larger ones get a scan
-//                  launch of their own.
+//                  launch of their own.  Up to 20480 tokens over 63 experts
+//                  one launch does all three.
 //  spx_moe_forward one gathered GEMM over a flattened (expert, row tile) list (moe_persist.hip: large
 //                  problems): a workgroup looks its tile up in the prefix of per-expert tile
 //                  counts, gathers its token rows through token_perm, and walks
@@ -24,7 +25,7 @@ namespace spx {
 constexpr int MOE_CHUNK = 1024;   // most tokens per workgroup in the index kernels (a multiple of 256)
 constexpr int MOE_FUSED_TABLE = 1024;  // (chunk, expert) counts a placement workgroup scans itself
 // Tokens up to which the placement workgroups count the experts themselves, a launch less: 1100 tokens 4.5 -> 3.5 us,
-// 4000 5.1 -> 4.8; 6000 5.0 against 5.5, 8000 5.0 against 7.5.
+// 4000 5.1 -> 4.8; 6000 5.0 against 5.5, 8000 5.0 against 7.5 (with up to 63 experts moe_index_kernel takes over).
 constexpr int MOE_SELF_COUNT = 4096;
 constexpr int MOE_MAX_EXP = 2048; // LDS table capacity of the placement kernel
 constexpr int MOE_MAX_ROW_TILES = 65535;   // the y extent of a grid
@@ -210,6 +211,76 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int32_t* exp_ids, 
             wavecnt[wave * n_exp + e] = 0;
         }
         __syncthreads();
+    }
+}
+
+// The whole index in one launch, from 4097 to 20480 tokens over at most 63 experts: a workgroup places 1024 tokens, 64 to a
+// wavefront, and counts all of them itself before, those ahead of its own apart.  The counters of an expert are sixteen
+// copies side by side, one for every sixteenth lane, so that a crowded expert does not queue up a wavefront's additions.
+// What bounds it: the launch and the additions (a 64 KB list of 16384 tokens is counted in a microsecond).  Counting and placing
+// launch against this one (kernels alone): 4100 tokens over 8 6.1 -> 3.9 us, 8192 over 32 8.7 -> 4.7, 16384 over 8 8.4 -> 5.5;
+// whole passes 5000 x 256 -> 512 over 4 13.6 -> 12.1, 8192 x 768 -> 768 over 8 24.6 -> 23.6.  A workgroup's count grows with
+// the tokens: 24000 over 4 6.2 against 6.1 us, 32768 over 4 6.2 against 7.0 (over 32 10.1 against 7.2): 20480 is the line.
+constexpr int MOE_ONE_TOKENS = 20480, MOE_ONE_EXPERTS = 63, MOE_ONE_THREADS = 1024;
+__global__ __launch_bounds__(MOE_ONE_THREADS) void moe_index_kernel(const int32_t* exp_ids, int n_tok, int n_exp, int32_t* token_perm,
+                                                                    int32_t* expert_count, int32_t* expert_offset) {
+    constexpr int COPIES = 16, MOST = MOE_ONE_EXPERTS + 1, WAVES = MOE_ONE_THREADS / 64;
+    __shared__ int counts[2][MOST * COPIES];   // [ahead of this workgroup's tokens / from them on][expert, copy]
+    __shared__ int base[MOST], wave_count[WAVES][MOST];
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
+    const int own = blockIdx.x * MOE_ONE_THREADS;
+    for (int i = threadIdx.x; i < 2 * MOST * COPIES; i += MOE_ONE_THREADS) (&counts[0][0])[i] = 0;
+    for (int i = threadIdx.x; i < WAVES * MOST; i += MOE_ONE_THREADS) (&wave_count[0][0])[i] = 0;
+    auto expert_of = [&](int t) {   // n_exp counts the pseudo expert of ids that are out of range, the last one
+        const int e = t < n_tok ? exp_ids[t] : 0;
+        return e < 0 || e >= n_exp - 1 ? n_exp - 1 : e;
+    };
+    const int mine = own + threadIdx.x;
+    const int e = mine < n_tok ? expert_of(mine) : -1;
+    __syncthreads();
+    constexpr int BATCH = 8;   // loads in flight to a thread
+    for (int t0 = threadIdx.x; t0 < n_tok; t0 += MOE_ONE_THREADS * BATCH) {
+        int id[BATCH];
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) id[j] = expert_of(t0 + j * MOE_ONE_THREADS);
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+            const int t = t0 + j * MOE_ONE_THREADS;   // (the own tokens are one j of the loop)
+            if (t < n_tok) atomicAdd(&counts[t < own ? 0 : 1][id[j] * COPIES + (lane & (COPIES - 1))], 1);
+        }
+    }
+    // intra-wave rank and count of my expert, as in moe_place_kernel
+    unsigned long long same = __ballot(e >= 0);
+    for (int bit = 31 - __builtin_clz(n_exp | 1); bit >= 0; --bit) {
+        const unsigned long long ones = __ballot((e >> bit) & 1);
+        same &= (e >> bit) & 1 ? ones : ~ones;
+    }
+    const int rank = __popcll(same & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
+    if (e >= 0 && rank == 0) wave_count[wave][e] = __popcll(same);
+    __syncthreads();
+    if (wave == 0) {   // a lane to an expert
+        int ahead = 0, total = 0;
+        if (lane < n_exp)
+            for (int c = 0; c < COPIES; ++c) {   // (the copies in turn: lanes are sixteen words apart)
+                const int at = lane * COPIES + ((c + lane) & (COPIES - 1));
+                ahead += counts[0][at];
+                total += counts[1][at];
+            }
+        total += ahead;
+        const int first = wave_inclusive_scan(total) - total;
+        if (lane < n_exp) {
+            base[lane] = first + ahead;
+            if (blockIdx.x == 0) {
+                expert_offset[lane] = first;
+                if (lane + 1 < n_exp) expert_count[lane] = total;
+            }
+        }
+    }
+    __syncthreads();
+    if (e >= 0) {
+        int at = base[e] + rank;
+        for (int w = 0; w < wave; ++w) at += wave_count[w][e];
+        token_perm[at] = mine;
     }
 }
 
@@ -1031,6 +1102,12 @@ extern "C" int spx_moe_index(const int32_t* exp_ids, int n_tok, int n_exp,
     SPX_REQUIRE(aligned(workspace, 256), SPX_E_ALIGN, "workspace must be 256-byte aligned");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     int32_t* partial = reinterpret_cast<int32_t*>(workspace);
+    if (n_tok > MOE_SELF_COUNT && n_tok <= MOE_ONE_TOKENS && n_exp <= MOE_ONE_EXPERTS) {
+        hipLaunchKernelGGL(moe_index_kernel, dim3((n_tok + MOE_ONE_THREADS - 1) / MOE_ONE_THREADS), dim3(MOE_ONE_THREADS), 0, st, exp_ids, n_tok,
+                           n_exp + 1, token_perm, expert_count, expert_offset);
+        SPX_LAUNCH_CHECK("moe_index_kernel");
+        return 0;
+    }
     bool fused;
     const int chunk = moe_index_chunk(n_tok, n_exp, &fused);
     const int n_chunk = (n_tok + chunk - 1) / chunk;

@@ -287,6 +287,29 @@ def test_moe_index_orders_tokens(n_tok, n_exp, gpu):
     assert np.array_equal(offset.cpu().numpy(), np.cumsum(want) - want)
 
 
+@pytest.mark.parametrize('n_tok,n_exp,single', [(4097, 5, True), (12289, 63, True), (20480, 8, True), (20480, 64, False), (20481, 8, False)])
+def test_moe_index_in_one_launch(n_tok, n_exp, single, gpu):
+    """Both sides of the lines up to which one launch counts and places the tokens, nearly all of them with one expert (whose
+    counters every lane of a wavefront adds to), ids out of range among them: a stable sort, to the last token."""
+    from sparta_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(n_tok + n_exp)
+    ids = np.where(rng.random(n_tok) < 0.95, n_exp - 1, rng.integers(-2, n_exp + 2, n_tok)).astype(np.int32)
+    on = lambda n: torch.full((n,), -1, dtype=torch.int32, device=gpu)
+    dev_ids, count, offset, perm = torch.from_numpy(ids).to(gpu), on(n_exp), on(n_exp + 1), on(n_tok)
+    nbytes = lib.spx_moe_index_workspace_bytes(n_tok, n_exp)
+    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=gpu)
+    _, names = launched_kernels(lambda: _lib.check(lib.spx_moe_index(
+        _lib.dev_ptr(dev_ids), n_tok, n_exp, _lib.dev_ptr(count), _lib.dev_ptr(offset), _lib.dev_ptr(perm), _lib.dev_ptr(ws),
+        nbytes, _lib.current_stream(gpu)), 'spx_moe_index'))
+    assert any('moe_index_kernel' in n for n in names) == single, names
+    key = np.where((ids < 0) | (ids >= n_exp), n_exp, ids)
+    want = np.bincount(key, minlength=n_exp + 1)
+    assert np.array_equal(perm.cpu().numpy(), np.argsort(key, kind='stable'))
+    assert np.array_equal(count.cpu().numpy(), want[:n_exp])
+    assert np.array_equal(offset.cpu().numpy(), np.cumsum(want) - want)
+
+
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize('n_tok,in_dims,out_dims,n_exp,rows,stages', [
     # behind the 32-row tiles (256 of 128 x 128): 64-row tiles in three stages, up to 288 of 128 x 128; one stage of k, ragged columns
