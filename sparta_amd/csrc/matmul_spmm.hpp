@@ -227,6 +227,10 @@ bool spmm_ring_supported(const SpmmParams& p, int BN) {
            (p.d_kcontig || (p.Mc % VE == 0 && p.d_ld % VE == 0)) && (p.out_ncontig || p.Mc % VE == 0) &&
            p.d_ld * 128 + p.K < (int64_t)1 << 29 && (p.compressed || p.s_ld * 64 + p.K < (int64_t)1 << 29);   // byte offsets in 32 bits
 }
+// Rows of the dense operand kept in LDS (matmul_spmm_rows.hpp), where that is ahead; kSpmmRowsNot: it is not.
+constexpr int kSpmmRowsNot = -1000;   // (no status of the interface)
+template <typename T>
+int launch_spmm_rows(const SpmmParams& p, int BN, int batch, hipStream_t st);
 template <typename T>
 bool spmm_thin_supported(const SpmmParams& p, int BN);
 template <typename T>
@@ -268,6 +272,11 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         return launch_spmm_thin<T>(p, batch, st);
     }
     const bool ring_ok = spmm_ring_supported<T>(p, BN);
+    if constexpr (sizeof(T) == 2)
+        if (tile_cfg == 0) {   // (the rule stands beside the kernel)
+            const int rc = launch_spmm_rows<T>(p, BN, batch, st);
+            if (rc != kSpmmRowsNot) return rc;
+        }
     if (tile_cfg == 0) {
         // 256-row tiles only when they still give every CU a few workgroups; small
         // problems are latency-bound and want more, shorter workgroups.
