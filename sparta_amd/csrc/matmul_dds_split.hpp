@@ -487,7 +487,7 @@ inline DdsShare dds_share_plan(int elem_bytes, bool a_kcontig, bool b_kcontig, i
     else if (elem_bytes == 2 && BM == 32 && BN == 32 && K >= 1024 && work >= 400000) plan.blocks = 4;
     else if (elem_bytes == 2 && BM == 32 && BN == 64 && K >= 1024 && work >= 800000) plan.blocks = 2;
     else if (elem_bytes == 2 && BM == 64 && BN == 64 && work >= 600000) plan.blocks = 2;
-    if (elem_bytes == 4 && plan.blocks) {   // no longer chains of fp32 additions than one block to a workgroup has
+    if (plan.blocks) {   // no longer chains of fp32 additions than one block to a workgroup has
         const int whole = dds_split_slices(elem_bytes, false, nnz, batch, K, BM, BN);
         if (whole > plan.slices) plan.slices = whole;
     }
