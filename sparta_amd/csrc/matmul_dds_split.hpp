@@ -470,15 +470,17 @@ static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, i
 //   16-bit 32 x 32  450 over 2416 21.1 / 15.7, 706 over 2128 22.2 / 20.3, 305 over 1504 15.7 / 14.1, but 116 over 1248 10.2 / 9.6,
 //                 437 over 592 7.4 / 8.5;  32 x 64  410 over 4096 33.6 / 28.5, 187 over 5072 23.5 / 21.9, but 93 over 1152 10.2 / 12.4;
 //                 64 x 64  309 over 2848 29.4 / 24.6, 1021 over 784 (unsliced) 20.3 / 18.1, but 349 over 736 level, 46 over 3664 13.3 / 15.3
-// Scores (both k-contiguous, unsliced): fp32 32 x 32, two blocks, from 1000 of them on (2458 over 768 51 / 43.5 us, 1229 over 256
-// 14.9 / 13.1, 1229 over 128 9.9 / 9.6; 388 over 768 14.5 / 15.7; 64 x 64: 396 over 768 34.3 / 33.2).
+// Scores (both k-contiguous): fp32 32 x 32, two blocks, from 1000 of them on (2458 over 768 51 / 43.5 us, 1229 over 256 14.9 / 13.1, 1229
+// over 128 9.9 / 9.6; 388 over 768 14.5 / 15.7; 64 x 64: 396 over 768 34.3 / 33.2), in the slices that one block to a workgroup
+// has: 2458 over 1536 in four 97.9 / 82.5, over 3072 in eight 186 / 153 with a relative error of 3.5e-7 (unsliced and shared 70.6 and
+// 136, but 7.0e-7 and 9.9e-7).
 struct DdsShare {
     int blocks, slices;
 };
 inline DdsShare dds_share_plan(int elem_bytes, bool a_kcontig, bool b_kcontig, int nnz, int batch, int K, int BM, int BN) {
     const int64_t blocks = (int64_t)nnz * batch;
     if (a_kcontig != b_kcontig) return {0, 1};
-    if (a_kcontig) return {elem_bytes == 4 && BM == 32 && BN == 32 && blocks >= 1000 ? 2 : 0, 1};
+    if (a_kcontig) return {elem_bytes == 4 && BM == 32 && BN == 32 && blocks >= 1000 ? 2 : 0, dds_split_slices(elem_bytes, true, nnz, batch, K, BM, BN)};
     const int64_t work = blocks * K;
     DdsShare plan = {0, K < 1024 ? 1 : 4};
     if (elem_bytes == 4 && BM == 16 && BN == 16 && work >= 1000000) plan = {4, K < 1024 ? 1 : blocks <= 2048 ? 8 : 4};

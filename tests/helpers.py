@@ -38,6 +38,13 @@ def assert_close(got: torch.Tensor, want: np.ndarray, dtype, what='', scale=1.0)
                            f'(bound there {bound.flat[err.argmax()]:.3e})')
 
 
+def chained_sum_error(additions):
+    """Relative error (2-norm) of fp32 sums of products of N(0, 1) values that are added up in chains of so many additions.
+    A rounded addition is off by 2^-23 / sqrt(12) of its sum's power of two, 0.41 * 2^-24 of the sum (rms, mantissas evenly
+    spread over 1 to 2), and the sums of a chain grow like the root of the additions before them."""
+    return 0.41 * 2.0 ** -24 * (additions / 2) ** 0.5
+
+
 def launched_kernels(call):
     """(what `call` returns, names of the kernels that it launched; they may be mangled)."""
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:

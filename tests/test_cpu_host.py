@@ -373,6 +373,15 @@ def test_split_product_bounds_its_workspace():
     assert size(52428, 16384, 8192, 8192, 32, 64, slices=8) == 8 * 52428 * 32 * 64 * 4
 
 
+@pytest.mark.parametrize('blocks,K,slices', [(1000, 2048, 4), (2458, 1536, 4), (1229, 3072, 8), (4096, 4096, 8), (1000, 1024, 1), (2458, 768, 1)])
+def test_split_product_keeps_its_slices_where_blocks_share_rows(blocks, K, slices):
+    """fp32 products of two k-contiguous operands in 32 x 32 blocks: as many slices of k with blocks that share their rows (from
+    1000 of them on) as a block to a workgroup takes, whose sums are as long.  The same work in blocks of 64 x 64 never shares."""
+    size = lambda nnz, BM, BN, want=0: _lib.load().spx_matmul_split_workspace_bytes(_lib.F32, 0, 1, nnz, 1, 4096, K, 4096, BM, BN, want, 0)
+    assert size(blocks, 32, 32) == (slices * blocks * 32 * 32 * 4 if slices > 1 else 0)
+    assert size(blocks, 32, 32, slices) == size(blocks, 32, 32)
+
+
 def test_attention_launch_object_appears_whole_to_other_threads():
     """The operator keeps the launch object of its current index.  A call from another thread that comes between any
     two of the assignments that store it gets one for the current index, never none and never the one before."""
