@@ -88,6 +88,10 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     constexpr int KC = 64 / ES;               // k per half
     constexpr int CH = BK / KC;               // halves per block
     constexpr int MT = TM / 64, NT = BN / 16; // 16 x 16 tiles of a wavefront
+    // fp32 blocks 16 wide: the sum of a tile in four chains of MFMAs, by half and by the parity of their k-step, added up at
+    // the end.  They are as long as those of four wavefronts that share a block-column (matmul_spmm_ksplit.hpp), and
+    // neighbouring MFMAs of a wavefront with one tile do not wait for each other.
+    constexpr int CHAINS = ES == 4 && NT == 1 ? 4 : 1;
     constexpr int NB = ring_stages(ES), D_BYTES = TM * 128, STAGE = LDS.stage;
     constexpr int ND = TM / 8, NS = BN / 8;   // load instructions of a stage: dense and sparse part
     constexpr int NL = ND + NS;
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     const T* biasT = p.bias ? reinterpret_cast<const T*>(p.bias) + b * p.bias_batch : nullptr;
     T* out = reinterpret_cast<T*>(p.out) + b * p.o_batch;
     T* const tileT = reinterpret_cast<T*>(smem + NB * STAGE);
-    f32x4 acc[MT][NT];
+    f32x4 acc[MT][NT][CHAINS];
     struct Half {
         Frag a[MT], b[NT];
     };
@@ -329,11 +333,23 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
 #pragma unroll
         for (int t = 0; t < NT; ++t) h.b[t] = ring_frag<T, BN, SK, Frag>(buf + D_BYTES, t * 16, half, r16, g4);
     };
-    auto multiply = [&](const Half& h) {
+    auto multiply = [&](const Half& h, auto half) {
+        if constexpr (CHAINS == 4) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int t = 0; t < NT; ++t) acc[i][t] = SWAP ? MMA::mma(h.b[t], h.a[i], acc[i][t]) : MMA::mma(h.a[i], h.b[t], acc[i][t]);
+                for (int i = 0; i < MT; ++i) {
+                    f32x4& c = acc[i][0][half * 2 + (j & 1)];
+                    c = SWAP ? __builtin_amdgcn_mfma_f32_16x16x4f32(h.b[0][j], h.a[i][j], c, 0, 0, 0)
+                             : __builtin_amdgcn_mfma_f32_16x16x4f32(h.a[i][j], h.b[0][j], c, 0, 0, 0);
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[i][t][0] = SWAP ? MMA::mma(h.b[t], h.a[i], acc[i][t][0]) : MMA::mma(h.a[i], h.b[t], acc[i][t][0]);
+        }
     };
     uint32_t at = 0;
     for (int r = 0; r < n_rounds; ++r) {
@@ -369,14 +385,16 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int t = 0; t < NT; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int c = 0; c < CHAINS; ++c) acc[i][t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int st = 0; st < cur.n_st; ++st) {
             __syncthreads();
             Half h0, h1;
             fetch(smem + at, 0, h0);
             fetch(smem + at, 1, h1);
-            multiply(h0);
-            if (!PAIR || 2 * st + 1 < cur.n_blk) multiply(h1);
+            multiply(h0, std::integral_constant<int, 0>());
+            if (!PAIR || 2 * st + 1 < cur.n_blk) multiply(h1, std::integral_constant<int, 1>());
             at = at + STAGE == NB * STAGE ? 0 : at + STAGE;
         }
         // ---- epilogue: the tile meets in LDS in the orientation of the output and leaves as whole 16-byte
@@ -389,10 +407,12 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
             for (int t = 0; t < NT; ++t) {
                 const int m = wave * (TM / 4) + i * 16 + (SWAP ? r16 : g4 * 4);
                 const int n = t * 16 + (SWAP ? g4 * 4 : r16);
+                f32x4 sum = acc[i][t][0];
+                if constexpr (CHAINS == 4) sum = (sum + acc[i][t][1]) + (acc[i][t][2] + acc[i][t][3]);
                 T vals[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    vals[q] = Elem<T>::from_float(epilogue_act(acc[i][t][q] + bias_m[i][q] + bias_n[t][q], p.relu));
+                    vals[q] = Elem<T>::from_float(epilogue_act(sum[q] + bias_m[i][q] + bias_n[t][q], p.relu));
                 T* dst = tileT + (SWAP ? m * LDE + n : n * LDE + m);
                 if constexpr (sizeof(T) == 2) *reinterpret_cast<uint64_t*>(dst) = *reinterpret_cast<const uint64_t*>(vals);
                 else *reinterpret_cast<vec16*>(dst) = *reinterpret_cast<const vec16*>(vals);

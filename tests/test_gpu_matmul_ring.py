@@ -4,6 +4,7 @@ number of blocks, several tiles per workgroup, and more block-columns than its t
 import pytest
 import torch
 
+from helpers import chained_sum_error
 from oracle import ops
 from sparta_amd.specializer.kernels import SparTASparseMatMulKernel
 from test_gpu_matmul import run_case
@@ -70,6 +71,27 @@ def test_dispatch_of_few_rows_and_long_columns(dtype, blocks, M, K, N, sparsity,
     for compressed in (True, False):
         run_case(gpu, 'dsd', False, True, True, compressed, dtype, blocks, batch=1, M=M, K=K, N=N, gran=(blocks[2], blocks[1]),
                  sparsity=sparsity, seed=71, tile_cfg=0, activation='relu' if compressed else None)
+
+
+@pytest.mark.parametrize('tile_cfg', [0, 11, 12])
+@pytest.mark.parametrize('mode,depth', [('dsd', 16), ('sdd', 16), ('dsd', 64)])
+def test_ring_sums_of_narrow_fp32_blocks(tile_cfg, mode, depth, gpu, size=1024, sparsity=0.65):
+    """fp32 blocks 16 wide: four chains to a sum, as long as where four wavefronts share a block-column (the column-split kernel,
+    which some of these sizes went through).  In one chain the error would be twice the expected one."""
+    kernel = SparTASparseMatMulKernel(mode=mode, biased=False, transpose_A=False, transpose_B=True, compressed=True)
+    port, tile = ('B', (16, depth)) if mode == 'dsd' else ('A', (16, depth))
+    mask = torch.from_numpy(ops.block_mask((size, size), tile, sparsity, seed=9)).to(gpu)
+    kernel.ports[port].set_mask(mask)
+    kernel.set_shape(1, size, size, size)
+    kernel.compile({'BLOCK_SIZE_M_VALUE': 16, 'BLOCK_SIZE_K_VALUE': depth, 'BLOCK_SIZE_N_VALUE': 16, 'TILE_CFG': tile_cfg})
+    g = torch.Generator(device=gpu).manual_seed(6)
+    A, B = (torch.randn((1, size, size), generator=g, device=gpu) for _ in range(2))
+    sparse = (B if mode == 'dsd' else A) * mask
+    A, B = (A, sparse) if mode == 'dsd' else (sparse, B)
+    packed = kernel.ports[port].indexes.convert(sparse)
+    got = kernel(A, packed) if mode == 'dsd' else kernel(packed, B)
+    want = A[0].double() @ B[0].double().t()
+    assert float((got[0].double() - want).norm() / want.norm()) <= 1.3 * chained_sum_error((1 - sparsity) * size / 4)
 
 
 @pytest.mark.parametrize('M', [110100, 40000])
