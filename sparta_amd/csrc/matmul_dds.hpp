@@ -703,7 +703,7 @@ int launch_dds_impl(const DdsParams& p, int BM, int BN, int nnz_bound, int batch
         if (!row) return fail(SPX_E_CONFIG, "tile config 3 needs row_ptr, k-contiguous operands, 32/64-wide blocks and K of 128 or 256 bytes");
         return launch_dds_row<T>(p, BM, BN, batch, st);
     }
-    // many fp32 blocks of 32 x 32: two to a workgroup, which share their rows of A (matmul_dds_share.hpp)
+    // many fp32 blocks of 32 x 32: two to a workgroup, which share their rows of A (dds_scores_share)
     if (tile_cfg == 0 && dds_shares_rows<T>(p, BM, BN, nnz_bound, batch)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, true, st);
     if (tile_cfg == 0) tile_cfg = 2;
     if (tile_cfg == 2 && !dds_pipe_ok<T>(p, BM, BN)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, false, st);

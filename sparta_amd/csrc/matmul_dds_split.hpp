@@ -470,17 +470,33 @@ static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, i
 //   16-bit 32 x 32  450 over 2416 21.1 / 15.7, 706 over 2128 22.2 / 20.3, 305 over 1504 15.7 / 14.1, but 116 over 1248 10.2 / 9.6,
 //                 437 over 592 7.4 / 8.5;  32 x 64  410 over 4096 33.6 / 28.5, 187 over 5072 23.5 / 21.9, but 93 over 1152 10.2 / 12.4;
 //                 64 x 64  309 over 2848 29.4 / 24.6, 1021 over 784 (unsliced) 20.3 / 18.1, but 349 over 736 level, 46 over 3664 13.3 / 15.3
-// Scores (both k-contiguous): fp32 32 x 32, two blocks, from 1000 of them on (2458 over 768 51 / 43.5 us, 1229 over 256 14.9 / 13.1, 1229
-// over 128 9.9 / 9.6; 388 over 768 14.5 / 15.7; 64 x 64: 396 over 768 34.3 / 33.2), in the slices that one block to a workgroup
-// has: 2458 over 1536 in four 97.9 / 82.5, over 3072 in eight 186 / 153 with a relative error of 3.5e-7 (unsliced and shared 70.6 and
-// 136, but 7.0e-7 and 9.9e-7).
 struct DdsShare {
     int blocks, slices;
 };
-inline DdsShare dds_share_plan(int elem_bytes, bool a_kcontig, bool b_kcontig, int nnz, int batch, int K, int BM, int BN) {
+
+// Scores (both operands k-contiguous), fp32 32 x 32: two blocks to a workgroup from 1000 of them on, in the slices that one block
+// to a workgroup has (2458 blocks over 1536 in four 97.9 / 82.5 us, over 3072 in eight 186 / 153 with a relative error of
+// 3.5e-7; unsliced and shared 70.6 and 136, but 7.0e-7 and 9.9e-7), where that saves rounds: the workgroups that are on a CU together
+// take as long as their number says, a pair of blocks 1.33 times a single one and a little at the start.  us over 768, one block
+// / shared: 1024 blocks (four and three rounds) 20.8 / 24.5, 1100 (five, three) 25.1 / 24.5, 1400 (six, three) 28.5 / 24.8,
+// 1536 (six, four) 28.9 / 30.5, 1700 (seven, four) 32.6 / 30.9, 2048 (eight, five) 37.3 / 36.9, 2458 51 / 43.5, 2700 (eleven, six) 49.2 / 42.0;
+// over 256 the pair is ahead sooner: 1536 14.5 / 13.5, but 1024 10.2 / 10.9.  Many short block-rows, whose last group is not full,
+// count as they are launched: 4 x 300 blocks in 96 block-rows each (five, four) 26.3 / 31.0.  Fewer blocks: 388 over 768 14.5 / 15.7.
+// 64 x 64: 396 over 768 34.3 / 33.2.
+inline bool dds_scores_share(int elem_bytes, int nnz, int batch, int M, int K, int BM, int BN, int slices) {
+    if (elem_bytes != 4 || BM != 32 || BN != 32 || (int64_t)nnz * batch < 1000) return false;
+    const int64_t rows = M / BM < nnz ? M / BM : nnz, groups = (nnz + rows) / 2;   // as launch_dds_share_inst launches them
+    const int64_t one = ((int64_t)nnz * batch * slices + 255) / 256, shared = (groups * batch * slices + 255) / 256;
+    return 4 * shared + (K > 512 ? 3 : 2) <= 3 * one;
+}
+
+inline DdsShare dds_share_plan(int elem_bytes, bool a_kcontig, bool b_kcontig, int nnz, int batch, int M, int K, int BM, int BN) {
     const int64_t blocks = (int64_t)nnz * batch;
     if (a_kcontig != b_kcontig) return {0, 1};
-    if (a_kcontig) return {elem_bytes == 4 && BM == 32 && BN == 32 && blocks >= 1000 ? 2 : 0, dds_split_slices(elem_bytes, true, nnz, batch, K, BM, BN)};
+    if (a_kcontig) {
+        const int slices = dds_split_slices(elem_bytes, true, nnz, batch, K, BM, BN);
+        return {dds_scores_share(elem_bytes, nnz, batch, M, K, BM, BN, slices) ? 2 : 0, slices};
+    }
     const int64_t work = blocks * K;
     DdsShare plan = {0, K < 1024 ? 1 : 4};
     if (elem_bytes == 4 && BM == 16 && BN == 16 && work >= 1000000) plan = {4, K < 1024 ? 1 : blocks <= 2048 ? 8 : 4};
@@ -503,9 +519,11 @@ template <typename T>
 bool dds_share_takes(const DdsParams& p) {   // (byte offsets of 64 rows in 32 bits)
     return p.row_ptr && !p.bias && p.a_ld < (1 << 23) && p.b_ld < (1 << 23);
 }
+// Unsliced products of spx_matmul.  (Several long ones outgrow the L2s side by side: 4 x 550 blocks over 2048 103 / 123 us, 4 x 450 91 / 103, but
+// 1536 of a single product 69 / 72 and 2048 of one 90 / 88.)
 template <typename T>
 bool dds_shares_rows(const DdsParams& p, int BM, int BN, int nnz_bound, int batch) {
-    return p.a_kcontig && dds_share_takes<T>(p) && dds_share_plan((int)sizeof(T), true, p.b_kcontig != 0, nnz_bound, batch, p.K, BM, BN).blocks > 0;
+    return p.a_kcontig && p.b_kcontig && (batch == 1 || p.K <= 1024) && dds_share_takes<T>(p) && dds_scores_share((int)sizeof(T), nnz_bound, batch, p.M, p.K, BM, BN, 1);
 }
 
 template <typename T>
