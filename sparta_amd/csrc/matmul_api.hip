@@ -135,9 +135,7 @@ extern "C" int spx_matmul(int mode, int dtype, int transA, int transB, int compr
 namespace spx {
 
 static int split_slices(int dtype, int transA, int transB, int nnz, int batch, int M, int K, int BM, int BN, int slices) {
-    if (slices) return slices;
-    const DdsShare share = dds_share_plan(dtype_bytes(dtype), !transA, transB, nnz, batch, M, K, BM, BN);
-    return share.blocks ? share.slices : dds_split_slices(dtype_bytes(dtype), !transA && transB, nnz, batch, K, BM, BN);
+    return slices ? slices : dds_share_plan(dtype_bytes(dtype), !transA, transB, nnz, batch, M, K, BM, BN).slices;
 }
 static size_t split_partial_bytes(int slices, int nnz, int batch, int BM, int BN) {
     return slices > 1 ? (size_t)batch * slices * nnz * BM * BN * sizeof(float) : 0;

@@ -683,9 +683,9 @@ static int launch_dds_inst(const DdsParams& p, int nnz_bound, int batch, hipStre
 }
 
 template <typename T>
-int launch_dds_unsliced(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, bool share, hipStream_t st);
+int launch_dds_unsliced(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, int share, hipStream_t st);
 template <typename T>
-bool dds_shares_rows(const DdsParams& p, int BM, int BN, int nnz_bound, int batch);
+int dds_shared_blocks(const DdsParams& p, int BM, int BN, int nnz_bound, int batch);
 
 // tile_cfg: 0 = by layout and depth; 1 = one LDS buffer, no prefetch;
 //           2 = pipelined (register ring + two LDS buffers); 3 / 4 = the short-K kernels above.
@@ -703,10 +703,11 @@ int launch_dds_impl(const DdsParams& p, int BM, int BN, int nnz_bound, int batch
         if (!row) return fail(SPX_E_CONFIG, "tile config 3 needs row_ptr, k-contiguous operands, 32/64-wide blocks and K of 128 or 256 bytes");
         return launch_dds_row<T>(p, BM, BN, batch, st);
     }
-    // many fp32 blocks of 32 x 32: two to a workgroup, which share their rows of A (dds_scores_share)
-    if (tile_cfg == 0 && dds_shares_rows<T>(p, BM, BN, nnz_bound, batch)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, true, st);
+    // several blocks to a workgroup, which share their rows of A (matmul_dds_share.hpp)
+    const int share = tile_cfg == 0 ? dds_shared_blocks<T>(p, BM, BN, nnz_bound, batch) : 0;
+    if (share) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, share, st);
     if (tile_cfg == 0) tile_cfg = 2;
-    if (tile_cfg == 2 && !dds_pipe_ok<T>(p, BM, BN)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, false, st);
+    if (tile_cfg == 2 && !dds_pipe_ok<T>(p, BM, BN)) return launch_dds_unsliced<T>(p, BM, BN, nnz_bound, batch, 0, st);
 #define SPX_DDS_CASE(bm, bn) \
     if (BM == bm && BN == bn) \
         return tile_cfg == 2 ? launch_dds_pipe_inst<T, bm, bn>(p, nnz_bound, batch, st) : launch_dds_inst<T, bm, bn>(p, nnz_bound, batch, st);

@@ -27,6 +27,7 @@
 // group addresses four entries of k-row i / 4, lane j receives column j of the four rows) or
 // four 4-byte reads (fp32).
 #pragma once
+#include <cmath>
 #include "matmul_dds.hpp"
 
 namespace spx {
@@ -458,18 +459,7 @@ static int launch_dds_split_inst(const DdsParams& p, DdsSplit s, void* colsum, i
     return launch_dds_split_reduce<T>(p, s, colsum, BM, BN, batch, st);
 }
 
-// Blocks of a block-row to a workgroup, which then share their rows of A, and slices for them; 0: one block to a workgroup.
-// Weight gradients (both operands k-major): from so many blocks times tokens on that the fewer workgroups still fill the chip
-// evenly; below, the many short chains of one block each are ahead.  Product and second kernel, us, one block / shared:
-//   fp32 16 x 16  1270 blocks over 5328 tokens 80.8 / 59.4, 1980 over 1856 50.0 / 38.2, 3074 over 336 (unsliced) 16.6 / 14.6,
-//                 but 1229 over 768 14.9 / 16.4, 31 over 4000 9.1 / 13.2
-//   fp32 32 x 32  461 over 4096 60.6 / 49.7, 898 over 4144 125 / 96, 612 over 1792 41.5 / 35.1, but 253 over 2096 25.0 / 26.5,
-//                 306 over 352 8.9 / 9.5; two blocks to a workgroup or four: 612 over 1792 35.1 / 35.9, 898 over 4144 103 / 92
-//   fp32 32 x 64  210 over 2544 39.9 / 36.3, 1371 over 4512 301 / 249, but 110 over 1056 17.4 / 20.5; 64 x 64: 583 over 4592 228 / 221, 745
-//                 over 432 31.2 / 36.9
-//   16-bit 32 x 32  450 over 2416 21.1 / 15.7, 706 over 2128 22.2 / 20.3, 305 over 1504 15.7 / 14.1, but 116 over 1248 10.2 / 9.6,
-//                 437 over 592 7.4 / 8.5;  32 x 64  410 over 4096 33.6 / 28.5, 187 over 5072 23.5 / 21.9, but 93 over 1152 10.2 / 12.4;
-//                 64 x 64  309 over 2848 29.4 / 24.6, 1021 over 784 (unsliced) 20.3 / 18.1, but 349 over 736 level, 46 over 3664 13.3 / 15.3
+// Blocks of a block-row to a workgroup, which then share their rows of A (0: one block to a workgroup), and the slices of k.
 struct DdsShare {
     int blocks, slices;
 };
@@ -490,26 +480,80 @@ inline bool dds_scores_share(int elem_bytes, int nnz, int batch, int M, int K, i
     return 4 * shared + (K > 512 ? 3 : 2) <= 3 * one;
 }
 
+// Weight gradients (both operands k-major).  Estimates in us of product and second kernel, fitted to 1000 random problems of 512 to
+// 4096 rows and columns, 256 to 8192 tokens and 2 - 40 % live blocks (root mean square off by 2 - 8 %):
+//   start + sliced ? second + partial * (bytes of the partial blocks, written and read, at 4 TB/s) : 0
+//         + thousands of tokens in a slice * (depth + rounds * ceil(W) + work * W + generation * ceil(W / fit))
+// W: workgroups to a CU, fit: that are there together.
+struct DdsEstimate {
+    int elem_bytes, BM, BN, blocks, fit;   // blocks to a workgroup
+    double start, second, partial, depth, rounds, work, generation;
+};
+inline double dds_estimate(const DdsEstimate& e, double blocks, double rows, int K, int slices) {
+    // a block-row's last group is half full, give or take
+    const double groups = (blocks + rows * (e.blocks - 1) * 0.5) / e.blocks, per_cu = groups * slices / 256;
+    const double part = slices > 1 ? e.second + e.partial * slices * blocks * e.BM * e.BN * 8 / 4e6 : 0.0;
+    return e.start + part + (double)K / slices * 1e-3 * (e.depth + e.rounds * std::ceil(per_cu) + e.work * per_cu + e.generation * std::ceil(per_cu / e.fit));
+}
+
+// From how many blocks times tokens on they are looked at (below, the many short chains of one block each are ahead), and what
+// is taken then.  us with one block to a workgroup / with four or two, at the slices that the estimates choose:
+//   16-bit 32 x 32  653 blocks over 1152 11.9 / 14.4 (in four slices, as all of them once were, 16.6), but 450 over 2416 21.1 / 15.7;
+//                   fewer than 100 level or behind (71 over 7888 13.9 / 14.8)
+//   16-bit 32 x 64  1077 over 1280 24.2 / 19.8 (four slices 30.9), 410 over 4096 33.6 / 28.5, but 64 over 2480 10.5 / 10.7
+//   16-bit 64 x 64  691 over 1360 21.6 / 19.4 (four slices 33.1), but 126 over 5552 21.9 / 24.7
+//   fp32 32 x 32    504 over 4736 70.2 / 64.9 (four blocks 84.5), 898 over 4144 125 / 96, but 253 over 2096 25.0 / 26.5
+//   fp32 32 x 64    210 over 2544 39.9 / 36.3, but 128 over 6032 43.5 / 50.4
+//   fp32 16 x 16    1270 over 5328 80.8 / 59.4, 1980 over 1856 50.0 / 38.2, 3074 over 336 (unsliced) 16.6 / 14.6, but 1229 over 768 14.9 /
+//                   16.4, 31 over 4000 9.1 / 13.2: a line, without estimates
+// Slices: for 16-bit types no fewer than one block to a workgroup has, so that no chain of fp32 additions is longer.  fp32 keeps
+// four or eight, whose sums are the more exact ones, also where one block in fewer slices would be ahead (2462 blocks over 1056 in
+// eight 92 us, in two 79).
 inline DdsShare dds_share_plan(int elem_bytes, bool a_kcontig, bool b_kcontig, int nnz, int batch, int M, int K, int BM, int BN) {
-    const int64_t blocks = (int64_t)nnz * batch;
-    if (a_kcontig != b_kcontig) return {0, 1};
+    static const DdsEstimate estimates[] = {
+        {2, 32, 32, 1, 5, 4.71, 2.42, 0.56, 0.42, 0.71, 1.10, 2.48}, {2, 32, 32, 4, 4, 7.06, 0.00, 0.72, 1.49, 1.71, 1.98, 2.57},
+        {2, 32, 64, 1, 5, 5.20, 2.15, 0.53, 1.62, 1.38, 0.93, 1.80}, {2, 32, 64, 2, 4, 4.71, 2.25, 0.65, 0.75, 1.25, 1.53, 4.19},
+        {2, 64, 64, 1, 5, 4.50, 2.09, 0.52, 2.44, 2.90, 0.51, 0.35}, {2, 64, 64, 2, 3, 5.36, 2.20, 0.65, 1.05, 0.66, 2.39, 5.35},
+        {4, 32, 32, 1, 5, 6.49, 0.00, 1.05, 3.48, 3.89, 1.55, 0.00}, {4, 32, 32, 2, 6, 7.69, 0.00, 0.76, 0.00, 6.91, 0.69, 6.08},
+        {4, 32, 32, 4, 4, 7.24, 0.00, 0.88, 0.00, 11.77, 2.38, 9.50},
+        {4, 32, 64, 1, 5, 6.06, 0.00, 0.63, 6.51, 9.38, 0.33, 0.50}, {4, 32, 64, 2, 4, 8.07, 0.00, 0.59, 0.37, 12.51, 2.33, 8.01}};
+    DdsShare plan = {0, dds_split_slices(elem_bytes, a_kcontig && b_kcontig, nnz, batch, K, BM, BN)};
+    if (a_kcontig != b_kcontig) return plan;
     if (a_kcontig) {
-        const int slices = dds_split_slices(elem_bytes, true, nnz, batch, K, BM, BN);
-        return {dds_scores_share(elem_bytes, nnz, batch, M, K, BM, BN, slices) ? 2 : 0, slices};
+        if (dds_scores_share(elem_bytes, nnz, batch, M, K, BM, BN, plan.slices)) plan.blocks = 2;
+        return plan;
     }
-    const int64_t work = blocks * K;
-    DdsShare plan = {0, K < 1024 ? 1 : 4};
-    if (elem_bytes == 4 && BM == 16 && BN == 16 && work >= 1000000) plan = {4, K < 1024 ? 1 : blocks <= 2048 ? 8 : 4};
-    else if (elem_bytes == 4 && BM == 32 && BN == 32 && K >= 1024 && work >= 800000) plan = work < 1500000 ? DdsShare{2, 4} : DdsShare{4, 8};
-    else if (elem_bytes == 4 && BM == 32 && BN == 64 && K >= 1024 && work >= 500000) plan.blocks = 2;
-    else if (elem_bytes == 2 && BM == 32 && BN == 32 && K >= 1024 && work >= 400000) plan.blocks = 4;
-    else if (elem_bytes == 2 && BM == 32 && BN == 64 && K >= 1024 && work >= 800000) plan.blocks = 2;
-    else if (elem_bytes == 2 && BM == 64 && BN == 64 && work >= 600000) plan.blocks = 2;
-    if (plan.blocks) {   // no longer chains of fp32 additions than one block to a workgroup has
-        const int whole = dds_split_slices(elem_bytes, false, nnz, batch, K, BM, BN);
-        if (whole > plan.slices) plan.slices = whole;
+    const int64_t blocks = (int64_t)nnz * batch, work = blocks * K;
+    const auto fits = [&](int slices) { return slices * (double)blocks * BM * BN * sizeof(float) <= (double)kSplitPartialBytes; };
+    int least = plan.slices;
+    if (elem_bytes == 4 && BM == 16 && BN == 16) {
+        if (work < 1000000) return plan;
+        least = K < 1024 ? 1 : blocks <= 2048 ? 8 : 4;
+    } else if (elem_bytes == 4 && BM == 32 && BN == 32) {
+        if (K < 1024 || work < 800000) return plan;
+        least = work < 1500000 ? 4 : 8;
+    } else if (elem_bytes == 4 && BM == 32 && BN == 64) {
+        if (K < 1024 || work < 500000) return plan;
+        least = 4;
+    } else if (!(elem_bytes == 2 && ((BM == 32 && BN == 32 && K >= 1024 && work >= 400000 && blocks >= 100) || (BM == 32 && BN == 64 && K >= 1024 && work >= 800000) ||
+                                     (BM == 64 && BN == 64 && work >= 600000)))) {
+        return plan;
     }
-    while (plan.slices > 1 && plan.slices * (double)blocks * BM * BN * sizeof(float) > (double)kSplitPartialBytes) plan.slices /= 2;
+    if (least < plan.slices) least = plan.slices;
+    while (least > 1 && !fits(least)) least /= 2;
+    if (BM == 16) return {4, least};
+    const double rows = (double)(M / BM < nnz ? M / BM : nnz) * batch;
+    double best = 0;
+    plan.blocks = -1;
+    for (const DdsEstimate& e : estimates)
+        if (e.elem_bytes == elem_bytes && e.BM == BM && e.BN == BN)
+            for (int slices = least; slices <= 8 && (slices == least || fits(slices)); slices *= 2) {
+                const double us = dds_estimate(e, (double)blocks, rows, K, slices);
+                if (plan.blocks < 0 || us < best) {
+                    best = us;
+                    plan = {e.blocks == 1 ? 0 : e.blocks, slices};
+                }
+            }
     return plan;
 }
 
@@ -519,11 +563,15 @@ template <typename T>
 bool dds_share_takes(const DdsParams& p) {   // (byte offsets of 64 rows in 32 bits)
     return p.row_ptr && !p.bias && p.a_ld < (1 << 23) && p.b_ld < (1 << 23);
 }
-// Unsliced products of spx_matmul.  (Several long ones outgrow the L2s side by side: 4 x 550 blocks over 2048 103 / 123 us, 4 x 450 91 / 103, but
-// 1536 of a single product 69 / 72 and 2048 of one 90 / 88.)
+// Blocks to a workgroup of an unsliced product of spx_matmul, 0: one each.  (Several long scores outgrow the L2s side by side: 4 x 550
+// blocks over 2048 103 / 123 us, 4 x 450 91 / 103, but 1536 of a single product 69 / 72 and 2048 of one 90 / 88.  Weight gradients that the
+// plan does not slice come here where no column sums are wanted: 2409 16-bit blocks of 32 x 32 over 2048 51 / 36.)
 template <typename T>
-bool dds_shares_rows(const DdsParams& p, int BM, int BN, int nnz_bound, int batch) {
-    return p.a_kcontig && p.b_kcontig && (batch == 1 || p.K <= 1024) && dds_share_takes<T>(p) && dds_scores_share((int)sizeof(T), nnz_bound, batch, p.M, p.K, BM, BN, 1);
+int dds_shared_blocks(const DdsParams& p, int BM, int BN, int nnz_bound, int batch) {
+    if (p.a_kcontig != p.b_kcontig || !dds_share_takes<T>(p)) return 0;
+    if (p.a_kcontig) return (batch == 1 || p.K <= 1024) && dds_scores_share((int)sizeof(T), nnz_bound, batch, p.M, p.K, BM, BN, 1) ? 2 : 0;
+    const DdsShare plan = dds_share_plan((int)sizeof(T), false, false, nnz_bound, batch, p.M, p.K, BM, BN);
+    return plan.slices == 1 ? plan.blocks : 0;
 }
 
 template <typename T>

@@ -6,8 +6,8 @@ int launch_dds_split<bf16_t>(const DdsParams& p, const DdsSplit& s, void* colsum
     return launch_dds_split_impl<bf16_t>(p, s, colsum, BM, BN, batch, st);
 }
 template <>
-int launch_dds_unsliced<bf16_t>(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, bool share, hipStream_t st) {
-    return launch_dds_split<bf16_t>(p, DdsSplit{1, 0, nnz_bound, 0, nullptr, nullptr, nullptr, share ? 2 : 0}, nullptr, BM, BN, batch, st);
+int launch_dds_unsliced<bf16_t>(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, int share, hipStream_t st) {
+    return launch_dds_split<bf16_t>(p, DdsSplit{1, 0, nnz_bound, 0, nullptr, nullptr, nullptr, share}, nullptr, BM, BN, batch, st);
 }
-template bool dds_shares_rows<bf16_t>(const DdsParams&, int, int, int, int);
+template int dds_shared_blocks<bf16_t>(const DdsParams&, int, int, int, int);
 }  // namespace spx

@@ -6,8 +6,8 @@ int launch_dds_split<_Float16>(const DdsParams& p, const DdsSplit& s, void* cols
     return launch_dds_split_impl<_Float16>(p, s, colsum, BM, BN, batch, st);
 }
 template <>
-int launch_dds_unsliced<_Float16>(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, bool share, hipStream_t st) {
-    return launch_dds_split<_Float16>(p, DdsSplit{1, 0, nnz_bound, 0, nullptr, nullptr, nullptr, share ? 2 : 0}, nullptr, BM, BN, batch, st);
+int launch_dds_unsliced<_Float16>(const DdsParams& p, int BM, int BN, int nnz_bound, int batch, int share, hipStream_t st) {
+    return launch_dds_split<_Float16>(p, DdsSplit{1, 0, nnz_bound, 0, nullptr, nullptr, nullptr, share}, nullptr, BM, BN, batch, st);
 }
-template bool dds_shares_rows<_Float16>(const DdsParams&, int, int, int, int);
+template int dds_shared_blocks<_Float16>(const DdsParams&, int, int, int, int);
 }  // namespace spx
