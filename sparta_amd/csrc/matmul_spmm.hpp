@@ -11,6 +11,7 @@
 // block through LDS as [row][k] and feeds 16x16 MFMAs; the tile leaves through
 // LDS so HBM sees full-width row segments.
 #pragma once
+#include <cmath>
 #include "common.hpp"
 #include "mma.hpp"
 #include "matmul_spmm_ring_plan.hpp"
@@ -236,6 +237,28 @@ bool spmm_thin_supported(const SpmmParams& p, int BN);
 template <typename T>
 int launch_spmm_thin(const SpmmParams& p, int batch, hipStream_t st);
 
+// fp32 blocks of 16 x 16, both operands k-contiguous: whether 64-row tiles of the ring kernel are ahead of split columns (`split`)
+// or of 256-row tiles.  Estimates in us, fitted to 1300 random problems of 700 to 6000 rows and 2 - 40 % live blocks (root mean square off by
+// 5 - 8 %).  What counts: the rounds of workgroups (the second one takes as long as the first, however few tiles it has), the dense
+// rows that every XCD reads anew where panels are dealt out by columns, and the panels that leave XCDs idle in the other two.
+// Other kernel / ring: 1024^3 at 35 % (one round) 17.5 / 15.0, 774 x 784 x 3584 at 25 % 28.6 / 23.8, 877 x 896 x 1728 at 20 % 16.2 / 13.7,
+// 1044 x 1328 x 3648 at 10 % 30.3 / 22.2, 2285 x 576 x 1024 at 8 % 15.2 / 10.2, 4577 x 576 x 512 at 14 % 19.8 / 13.2, but 512 x 1024 x
+// 1024 at 35 % 9.8 / 12.3, 1809 x 1056 x 704 at 31 % 18.5 / 27.4, 1966 x 784 x 576 at 14 % 10.6 / 17.3, 985 x 1120 x 768 at 40 % 14.3 / 15.7,
+// 1848 x 1040 x 1920 at 38 % 43.4 / 51.5, 2855 x 656 x 832 at 18 % 17.7 / 22.3, 5998 x 752 x 1024 at 3 % 11.2 / 14.5.
+inline bool spmm_ring_ahead_of_16(const SpmmParams& p, int64_t stored, bool split) {
+    const int nb = p.Nc / 16, panels64 = (p.Mc + 63) / 64, panels256 = (p.Mc + 255) / 256;
+    const double per = (double)stored / nb, out = (double)p.Mc * p.Nc * 1e-6;   // blocks to a column, millions of results
+    const RingLaunch l = ring_launch(4, 64, 16, p.out_ncontig != 0, p.Mc, p.K, p.Nc, 1);
+    const int rounds = ring_rounds(l.n_list, l.n_pos);
+    const double tiles = l.n_list / 32.0, dense = (double)p.Mc * p.K * 4e-6 * (1 << l.list.parts_log2);   // tiles to a CU; MB
+    const double ring = rounds == 1 ? 4.41 + per * (0.244 + 0.052 * tiles) + 0.149 * out + 0.006 * dense
+                                    : 4.09 + per * (0.195 * rounds + 0.067 * tiles) + 0.51 * out + 0.065 * dense;
+    const double tiles64 = (panels64 + 7) / 8 * nb / 32.0, tiles256 = (panels256 + 7) / 8 * nb / 32.0;   // of the XCD that has most, to a CU
+    const double other = split ? 4.85 + tiles64 * (0.409 + 0.076 * per) + 0.045 * std::ceil(tiles64 / 5) * per + 0.84 * out
+                               : 7.25 + per * (0.252 * std::ceil(tiles256) + 0.169 * std::ceil(tiles256 / 3) + 0.042 * tiles256) + 0.37 * out;
+    return ring < other;
+}
+
 // tile_cfg: 0 = pick by layout and size;
 //   1 / 2  LDS-staged kernel, 64 / 128-row workgroup tiles (any layout);
 //   3 / 4  register-direct kernel, 64 / 256-row workgroup tiles (k-contiguous operands);
@@ -318,21 +341,25 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         const bool two_blocks = p.BK * (int)sizeof(T) == 64;
         // stored blocks in all block-columns together (all places where it is not known)
         const int64_t stored = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * BN) : (int64_t)cols * nb;
+        // fp32 blocks of depth 16, long block-columns: four wavefronts that split a column and meet once keep
+        // more loads in flight than 256-row tiles when those are few.  256-row kernel / split columns:
+        // up to 1024 rows 512 x 4096 x 4096 at 35 % 259 / 85 us, at 5 % 45 / 20, 1024 x 2048 x 2048 74 / 45 and
+        // 16.4 / 14.4; narrow results 8192 x 2048 x 512 91 / 76 and (5 %) 28.1 / 25.9, 4096 x 2048 x 512 54 / 42,
+        // 4096 x 1024 x 512 32 / 28, 4380 x 1408 x 960 54 / 41, 4096 x 2048 x 1024 79 / 75, but 12.3 / 12.7 with four live blocks to a column and 158 / 148, 30 / 38 at
+        // 16384 rows; wide ones with more rows are mixed (2048^3 at 35 % 74 / 77, 4096 x 512 x 2048 44 / 51).
+        const bool split_columns = sizeof(T) == 4 && two_blocks && BN == 16 && ksplit_ok && cols > 48 &&
+                                   p.Mc > 256 && (p.Mc <= 1024 || (p.Mc <= 8192 && nb <= 32 && stored >= 6 * nb) ||
+                                                    (p.Mc <= 4608 && nb <= 64 && stored >= 12 * nb));
         bool use_ring = ring_ok;
         if (two_blocks && sizeof(T) == 4) {
             use_ring = ring_ok && (!kcontig || cols <= 48) && !(p.Mc >= 2048 && fill);
-            // k-contiguous blocks of 16 x 16 (us, column-split or 256-row kernel / ring).  Block-columns of medium length over 700 to
-            // 2047 rows, up to 23 live blocks to a column, 16 where the result is wide: 1024^3 at 35 % 15.9 / 14.8, at 20 % 11.3 / 9.7,
-            // 774 x 784 x 3584 at 25 % 28.6 / 23.8, 877 x 896 x 1728 at 20 % 16.2 / 13.7, 1777 x 1088 x 832 at 11 % 13.6 / 10.6, but 512 x 1024 x
-            // 1024 at 35 % 9.8 / 12.3, 820 x 1152 x 2048 at 35 % 26.9 / 30.3, 1024 x 1024 x 2048 at 35 % 25.6 / 26.6.  Short ones over up to 6000
-            // rows, eight live blocks to a column: 2256 x 576 x 1088 15.6 / 12.0, 2425 x 576 x 1408 20.9 / 16.0, 5192 x 640 x 1024 16.7 / 14.9, but
-            // 3704 x 704 x 1280 at 22 % 27.8 / 32.1, 11824 x 576 x 832 24.8 / 27.2.
-            if (kcontig && BN == 16 && ring_ok) {
-                if (p.Mc >= 700 && p.Mc < 2048 && cols > 48 && cols <= 88 && stored <= (nb <= 96 ? 23 : 16) * (int64_t)nb) use_ring = true;
-                if (p.Mc >= 2048 && p.Mc <= 6000 && cols <= 48 && nb <= 96 && stored <= 8 * (int64_t)nb) {
-                    use_ring = true;
-                    ring = 11;   // (5192 x 640 x 1024 with 128-row tiles 18.4)
-                }
+            // blocks of 16 x 16, where the number of blocks is known: by estimates (of wide results with more rows, 2719 x 640 x 2624, and
+            // of less than two blocks to a column, 2187 x 544 x 1984, they are too good for the ring)
+            if (kcontig && BN == 16 && ring_ok && batch == 1 && p.compressed && p.s_batch > 0 && p.Mc >= 700 && p.Mc <= 6000 &&
+                (p.Mc < 2048 ? cols > 48 && cols <= 88 : cols <= 48 && fill && nb <= 96 && stored >= 2 * (int64_t)nb && stored <= 8 * (int64_t)nb) &&
+                spmm_ring_ahead_of_16(p, stored, split_columns || !fill)) {
+                use_ring = true;
+                ring = 11;
             }
         } else if (two_blocks && kcontig) {
             const bool few_rows = p.Mc > 256 && p.Mc < 2048 && cols >= 32 && BN == 32 &&
@@ -344,15 +371,6 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
             if (fill) use_ring = ring_ok && cols >= 32 && (p.Nc < 2048 || mid_rows || (few_rows && p.Mc <= 1024));
             else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32 || few_rows);
         }
-        // fp32 blocks of depth 16, long block-columns: four wavefronts that split a column and meet once keep
-        // more loads in flight than 256-row tiles when those are few.  256-row kernel / split columns:
-        // up to 1024 rows 512 x 4096 x 4096 at 35 % 259 / 85 us, at 5 % 45 / 20, 1024 x 2048 x 2048 74 / 45 and
-        // 16.4 / 14.4; narrow results 8192 x 2048 x 512 91 / 76 and (5 %) 28.1 / 25.9, 4096 x 2048 x 512 54 / 42,
-        // 4096 x 1024 x 512 32 / 28, 4380 x 1408 x 960 54 / 41, 4096 x 2048 x 1024 79 / 75, but 12.3 / 12.7 with four live blocks to a column and 158 / 148, 30 / 38 at
-        // 16384 rows; wide ones with more rows are mixed (2048^3 at 35 % 74 / 77, 4096 x 512 x 2048 44 / 51).
-        const bool split_columns = sizeof(T) == 4 && two_blocks && BN == 16 && ksplit_ok && cols > 48 &&
-                                   p.Mc > 256 && (p.Mc <= 1024 || (p.Mc <= 8192 && nb <= 32 && stored >= 6 * nb) ||
-                                                    (p.Mc <= 4608 && nb <= 64 && stored >= 12 * nb));
         // 16-bit blocks of depth 64, a block or less to a block-column: next to no walk, the time is the output's, and the
         // 256-row kernels write it faster.  Ring / 256-row: 32 x 64 blocks 16384 x 512 x 2048 at 5 % 27.7 / 15.4 us, 8192 x
         // 768 x 3072 at 10 % 20.8 / 18.5 and at 5 % 19.0 / 14.2, 4096 x 1024 x 4096 at 5 % 14.4 / 12.3; 64 x 64 blocks at 10 %

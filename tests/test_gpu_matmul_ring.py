@@ -1,10 +1,11 @@
 """The LDS-ring kernel (tile configs 11 and 12) against the numpy oracle: all four operand layouts in
 both output orientations, rows that end inside a tile, block-columns without, with one and with an odd
 number of blocks, several tiles per workgroup, and more block-columns than its table holds."""
+import numpy as np
 import pytest
 import torch
 
-from helpers import chained_sum_error
+from helpers import assert_close, chained_sum_error, launched_kernels, template_numbers
 from oracle import ops
 from sparta_amd.specializer.kernels import SparTASparseMatMulKernel
 from test_gpu_matmul import run_case
@@ -92,6 +93,37 @@ def test_ring_sums_of_narrow_fp32_blocks(tile_cfg, mode, depth, gpu, size=1024, 
     got = kernel(A, packed) if mode == 'dsd' else kernel(packed, B)
     want = A[0].double() @ B[0].double().t()
     assert float((got[0].double() - want).norm() / want.norm()) <= 1.3 * chained_sum_error((1 - sparsity) * size / 4)
+
+
+@pytest.mark.parametrize('M,K,N,live,kernel', [
+    # split columns or ring: one round of tiles with 22 blocks to a column and with 32; two rounds, a quarter of the second, and three full ones
+    (1024, 1024, 1024, 22 * 64, 'ring'), (1024, 1024, 1024, 32 * 64, 'ksplit'), (1809, 1056, 704, 20 * 44, 'ksplit'), (774, 784, 3584, 12 * 224, 'ring'),
+    # first row count, longest columns, and the ones beside them
+    (700, 784, 1024, 12 * 64, 'ring'), (699, 784, 1024, 12 * 64, 'ksplit'), (700, 1408, 1024, 12 * 64, 'ring'), (700, 1424, 1024, 12 * 64, 'ksplit'),
+    # 256-row tiles or ring: five panels and eight
+    (1044, 1328, 3648, 8 * 228, 'ring'), (1848, 1040, 1920, 7 * 120, 'panel'),
+    # more rows: nine panels and sixteen, columns of up to 48 k-blocks, two to eight blocks to a column, up to 96 columns, last row count
+    (2049, 576, 1024, 2 * 64, 'ring'), (2049, 576, 1024, 2 * 64 - 1, 'panel'), (2199, 512, 1408, 8 * 88, 'ring'), (2199, 512, 1408, 8 * 88 + 1, 'panel'),
+    (2049, 576, 1552, 4 * 97, 'panel'), (3995, 512, 960, 2 * 60, 'panel'), (4577, 768, 512, 5 * 32, 'ring'), (4577, 784, 512, 5 * 32, 'panel'),
+    (6000, 512, 576, 3 * 36, 'ring'), (6001, 512, 576, 3 * 36, 'panel')])
+def test_dispatch_of_fp32_blocks_of_16(M, K, N, live, kernel, gpu):
+    """fp32 blocks of 16 x 16 run through the ring kernel, with 64-row tiles, where the estimates say so: both sides of what they turn
+    on, and of the sizes that they are asked for."""
+    import sparta_amd as sparta
+    grid = np.zeros(N // 16 * (K // 16), dtype=np.uint8)
+    grid[np.random.default_rng(M + live).permutation(grid.size)[:live]] = 1
+    mask_np = np.repeat(np.repeat(grid.reshape(N // 16, K // 16), 16, 0), 16, 1)
+    lin = torch.nn.Linear(K, N, bias=True, device=gpu)
+    x = torch.randn((M, K), generator=torch.Generator(device=gpu).manual_seed(7), device=gpu)
+    op = sparta.nn.SparseLinear(lin, weight_mask=torch.from_numpy(mask_np).to(gpu))
+    op.build({'forward:C': {'_impl': 'sparta', 'BLOCK_SIZE_M_VALUE': 32, 'BLOCK_SIZE_K_VALUE': 16, 'BLOCK_SIZE_N_VALUE': 16}}, sample_inputs=[x])
+    with torch.no_grad():
+        y, names = launched_kernels(lambda: op(x))
+    assert [k for k in ('ring', 'ksplit', 'panel') if any(f'spmm_{k}' in n for n in names)] == [kernel], names
+    if kernel == 'ring':
+        assert [n[0] for n in template_numbers(names, 'spmm_ring_kernel')] == [64], names
+    want = x.double().cpu().numpy() @ (lin.weight.detach().double().cpu().numpy() * mask_np).T + lin.bias.detach().double().cpu().numpy()
+    assert_close(y, want, torch.float32, f'{M} x {K} -> {N}, {live} blocks')
 
 
 @pytest.mark.parametrize('M', [110100, 40000])
