@@ -19,6 +19,7 @@
 // grid is sized by the largest expert and whose fp16 path accumulates in fp16.
 #include <type_traits>
 #include "moe.hpp"
+#include "moe_plan.hpp"
 
 namespace spx {
 
@@ -1179,6 +1180,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) n_cu = prop.multiProcessorCount;
         if (n_cu <= 0) n_cu = 256;
     }
+    const bool persist_ok = es == 2 && persist_fits(n_tok, in_dim, out_dim, n_exp, n_cu);
     int stages64 = 0;   // 64 x 128 tiles with that many stages
     if (tile_cfg == 0) {
         // 16-bit types: 256x256 tiles by persistent workgroups (5) from 224 of them on; with experts of many rows, whose last
@@ -1187,7 +1189,8 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         // 3569 x 768 -> 3072 over 8 (168) 34.0 / 31.4, 4564 x 1024 -> 2048 over 4 (144) 35.7 / 34.2, 9889 x 2048 -> 768 over 4 (117)
         // 46.1 / 41.0, 6673 x 2048 -> 768 over 8 (81) 42.7 / 38.4; but 3640 x 2048 -> 2048 over 4 (120) 45.8 / 49.3, 10529 x 768 -> 768 over 4 (126) 27.3 / 28.5, 2911 x 1024 -> 3072
         // over 16 (144, 181 rows each) 41.6 / 46.7, 3254 x 1024 -> 3072 over 32 (156, 101 rows each) level, 1994 x 2048 -> 768 over 8
-        // (24) 25.3 / 29.5.  256x256 tiles of one workgroup each (4) where k is too short for the pipeline: from 128 on when
+        // (24) 25.3 / 29.5.  256x256 tiles of one workgroup each (4) where k is too short for the pipeline (16384 x 64 -> 4096 over 8 43.3 us,
+        // with a second launch of 128-row tiles for what whole rounds leave 45.4; k of 192 64.6 / 63.8, 40000 tokens over 32 158 / 152): from 128 on when
         // all of them, the partly filled ones at the expert boundaries included, run in a
         // single round (ten mid-size problems measured 10 - 25 % ahead of the 128x128
         // tiles there, and behind them as soon as a second round starts); else 128x128
@@ -1207,7 +1210,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         const bool long_walk = in_dim >= 2048 && big_tiles >= 64 &&
                                ((row_tiles + n_exp / 2) * col_tiles <= n_cu / 2 ||
                                 ((n_tok + 127) / 128 + n_exp / 2) * ((out_dim + 127) / 128) > 2 * n_cu);
-        const bool persist = es == 2 && moe_persist_supported(p) &&
+        const bool persist = persist_ok &&
                              (big_tiles >= 224 || (big_tiles >= 160 && n_tok >= (int64_t)128 * n_exp) ||
                               (many_rows && (big_tiles >= 130 || long_walk)));
         if (!direct_ok) tile_cfg = 1;
@@ -1238,7 +1241,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
     }
     if (tile_cfg >= 2) {
         SPX_REQUIRE(direct_ok, SPX_E_CONFIG, "tile config %d takes fp32 weights in layout 1 only", tile_cfg);
-        if (tile_cfg == 5 && !(es == 2 && moe_persist_supported(p))) tile_cfg = 4;
+        if (tile_cfg == 5 && !persist_ok) tile_cfg = 4;
 #define SPX_MOE_DIRECT(T)                                                                  \
         if constexpr (sizeof(T) == 2)                                                      \
             if (tile_cfg == 5) return launch_moe_persist<T>(p, n_cu, st);                  \

@@ -100,8 +100,7 @@ __device__ __forceinline__ void moe_zero_tile(const MoeParams& p, int row0, int 
     }
 }
 
-// moe_persist.hip: 256 x 256 tiles by workgroups that stay on their CU (16-bit types)
-bool moe_persist_supported(const MoeParams& p);
+// moe_persist.hip: 256 x 256 tiles by workgroups that stay on their CU (16-bit types; what persist_fits takes)
 template <typename T> int launch_moe_persist(const MoeParams& p, int n_cu, hipStream_t st);
 
 }  // namespace spx

@@ -1,6 +1,7 @@
 // Gathered GEMM of the mixture of experts: 256 x 256 tiles by workgroups that stay on their CU.
 #include <type_traits>
 #include "moe.hpp"
+#include "moe_plan.hpp"
 
 namespace spx {
 
@@ -20,14 +21,7 @@ namespace spx {
 // whole rounds left took 166; this kernel with sixteen wavefronts of 64 x 64 156, eight 150, four of 128 x 128 157, all loads
 // in the boundary's k-step + 1; column by column over all rows, as the other kernels go, + 3 (and 13838 x 2048 -> 2048 over 32
 // bf16 186 with the two launches, 168 column by column, 158 in strips).
-constexpr int kPersistThreads = 512, kPersistSlot = 512 * 128;
-constexpr int kPersistTok = 2 * kPersistSlot;                    // token ids of two tiles
-constexpr int kPersistList = kPersistTok + 2 * 256 * 4;          // the workgroup's tiles
-constexpr int kPersistLds = 160 * 1024;
 constexpr int kStrip = 4;   // row tiles; 2 and 8: up to 2 % behind
-struct alignas(16) PersistTile {
-    int expert, row0, rows, n0;   // expert < 0: no tile
-};
 
 // A value that the compiler does not carry from place to place: what is derived from it is worked out where it is used.
 __device__ __forceinline__ int here(int v) {
@@ -343,22 +337,9 @@ __global__ __launch_bounds__(kPersistThreads, 2) void moe_persist_kernel(MoePara
     }
 }
 
-static int persist_workgroups(int n_cu) { return n_cu < 8 ? 8 : n_cu & ~7; }
-
-static int64_t persist_rounds(const MoeParams& p, int n_wg) {
-    const int64_t row_tiles = p.n_tok / 256 + (int64_t)p.n_exp + 1, col_tiles = (p.N + 255) / 256;
-    return (row_tiles * col_tiles + n_wg - 1) / n_wg + 1;
-}
-
-bool moe_persist_supported(const MoeParams& p) {
-    // four stages to a tile: the token ids of the next one arrive meanwhile; offsets of tokens and weights in 32 bits
-    return p.K >= 256 && (int64_t)p.n_tok * p.K * 2 < (int64_t)1 << 32 && (int64_t)p.N * 128 < (int64_t)1 << 32 &&
-           persist_rounds(p, 8) * (int64_t)sizeof(PersistTile) <= kPersistLds - kPersistList;
-}
-
 template <typename T, bool BKN>
 static int launch_moe_persist_inst(const MoeParams& p, int n_wg, hipStream_t st) {
-    const int smem = kPersistList + (int)persist_rounds(p, n_wg) * (int)sizeof(PersistTile);
+    const int smem = kPersistList + (int)persist_rounds(p.n_tok, p.N, p.n_exp, n_wg) * (int)sizeof(PersistTile);
     SPX_GRANT_LDS((moe_persist_kernel<T, BKN>), kPersistLds, "moe_persist_kernel");
     hipLaunchKernelGGL((moe_persist_kernel<T, BKN>), dim3(n_wg), dim3(kPersistThreads), smem, st, p);
     SPX_LAUNCH_CHECK("moe_persist_kernel");

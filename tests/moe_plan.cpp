@@ -1,0 +1,17 @@
+// Asks the plan of the persistent gathered GEMM, from the header that its launcher and its kernel share.
+// Input, a problem per line: tokens K N experts w_kcontig CUs.  Output: whether it fits, the tiles that a workgroup's list has
+// room for, and the end of that list in LDS.
+#include <cstdio>
+#include "moe_plan.hpp"
+
+using namespace spx;
+
+int main() {
+    int n_tok, K, N, n_exp, w_kcontig, n_cu;
+    while (std::scanf("%d %d %d %d %d %d", &n_tok, &K, &N, &n_exp, &w_kcontig, &n_cu) == 6) {
+        const int64_t rounds = persist_rounds(n_tok, N, n_exp, persist_workgroups(n_cu));
+        std::printf("%d %lld %lld\n", persist_fits(n_tok, K, N, n_exp, n_cu) ? 1 : 0, (long long)rounds,
+                    (long long)(kPersistList + rounds * (int64_t)sizeof(PersistTile)));
+    }
+    return 0;
+}

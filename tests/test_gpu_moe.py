@@ -266,6 +266,25 @@ def test_moe_persistent_tiles(layout, dtype, n_tok, in_dims, out_dims, n_exp, gp
     assert_close(out[torch.from_numpy(rows).to(gpu)], want[rows], dtype, f'persistent moe {n_tok} x {in_dims} -> {out_dims} over {n_exp}')
 
 
+def test_moe_persistent_tiles_of_a_large_layer(gpu, n_tok=131072, in_dims=256, out_dims=8192, n_exp=8):
+    """16640 tiles and more, 66 to a workgroup, through the library's own choice."""
+    moe, w = make_moe(n_exp, in_dims, out_dims, torch.float16, gpu)
+    rng = np.random.default_rng(5)
+    ids_np = rng.choice(n_exp, size=n_tok, p=np.arange(1, n_exp + 1) / (n_exp * (n_exp + 1) / 2)).astype(np.int32)
+    x = torch.from_numpy(rng.random((n_tok, in_dims), dtype=np.float32)).half()
+    x_dev, ids = x.to(gpu), torch.from_numpy(ids_np).to(gpu)
+    got, names = launched_kernels(lambda: moe(x_dev, ids))
+    assert any('moe_persist_kernel' in n for n in names), names
+    weight = moe.weight.detach().float()   # [E, in, out]
+    for e in range(n_exp):
+        rows = torch.nonzero(ids == e).flatten()
+        for r in range(0, rows.numel(), 8192):
+            some = rows[r:r + 8192]
+            want = torch.matmul(x_dev[some].float(), weight[e])
+            # result rounded to 11 bits; fp32 sums of 256 products in another order
+            assert float((got[some].float() - want).abs().max()) <= 2 ** -11 * float(want.abs().max()) + 1e-4
+
+
 @pytest.mark.parametrize('n_exp', [1, 2, 7, 8, 63, 64, 900])
 @pytest.mark.parametrize('n_tok', [1, 255, 1025, 2049, 4095, 4096, 4097, 20000])
 def test_moe_index_orders_tokens(n_tok, n_exp, gpu):
