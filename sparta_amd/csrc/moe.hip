@@ -1180,7 +1180,7 @@ extern "C" int spx_moe_forward(int dtype, const void* tokens, const void* weight
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) n_cu = prop.multiProcessorCount;
         if (n_cu <= 0) n_cu = 256;
     }
-    const bool persist_ok = es == 2 && persist_fits(n_tok, in_dim, out_dim, n_exp, n_cu);
+    const bool persist_ok = es == 2 && persist_fits(n_tok, in_dim, out_dim, n_exp, p.w_kcontig != 0, n_cu);
     int stages64 = 0;   // 64 x 128 tiles with that many stages
     if (tile_cfg == 0) {
         // 16-bit types: 256x256 tiles by persistent workgroups (5) from 224 of them on; with experts of many rows, whose last

@@ -23,11 +23,11 @@ constexpr int64_t persist_rounds(int n_tok, int N, int n_exp, int n_wg) {
     return (row_tiles * col_tiles + n_wg - 1) / n_wg + 1;
 }
 
-// Four stages to a tile: the token ids of the next one arrive meanwhile.  Byte offsets of tokens and weights in 32 bits.
-// The list of tiles in LDS.
-constexpr bool persist_fits(int n_tok, int K, int N, int n_exp, int n_cu) {
+// Four stages to a tile: the token ids of the next one arrive meanwhile.  Byte offsets in 32 bits: of all tokens, and of the weights of
+// a tile, 64 rows of k ([E, in, out]) or 256 rows of columns ([E, out, in]).  The list of tiles in LDS.
+constexpr bool persist_fits(int n_tok, int K, int N, int n_exp, bool w_kcontig, int n_cu) {
     const int64_t limit = (int64_t)1 << 32;
-    return K >= 256 && (int64_t)n_tok * K * 2 < limit && (int64_t)N * 128 < limit &&
+    return K >= 256 && (int64_t)n_tok * K * 2 < limit && (w_kcontig ? (int64_t)K * 512 : (int64_t)N * 128) < limit &&
            persist_rounds(n_tok, N, n_exp, persist_workgroups(n_cu)) * (int64_t)sizeof(PersistTile) <= kPersistLds - kPersistList;
 }
 
