@@ -64,14 +64,8 @@ __global__ __launch_bounds__(kRowsWaves * 64, kRowsWaves / 4) void spmm_rows_ker
     // ---- index of the share -----------------------------------------------------------------------------------------------
     const int first = p.ptr[c0], n_entry = p.ptr[c0 + n_cols] - first;
     for (int i = threadIdx.x; i <= n_cols; i += WAVES * 64) s_start[i] = p.ptr[c0 + i] - first;
-    for (int i = threadIdx.x; i < n_entry; i += WAVES * 64) {
-        if (p.idx_kind == SPX_IDX_BCSC_I64) {
-            const unsigned long long v = reinterpret_cast<const unsigned long long*>(p.idx)[first + i];
-            s_entry[i] = make_uint2((uint32_t)(v & 0xffff), (uint32_t)(v >> 32));
-        } else {
-            s_entry[i] = make_uint2((uint32_t)reinterpret_cast<const int32_t*>(p.idx)[first + i] & 0xffffu, (uint32_t)(first + i));
-        }
-    }
+    for (int i = threadIdx.x; i < n_entry; i += WAVES * 64)   // (k-contiguous blocks of a dsd product come with a BCSR index)
+        s_entry[i] = make_uint2((uint32_t)reinterpret_cast<const int32_t*>(p.idx)[first + i] & 0xffffu, (uint32_t)(first + i));
     if (bias)
         for (int i = threadIdx.x; i < n_cols * BN; i += WAVES * 64) s_bias[i] = bias[i];
     if (threadIdx.x == 0) *s_next = 0;
@@ -232,7 +226,7 @@ inline bool spmm_rows_plan(const SpmmParams& p, int BN, int batch, RowsPlan* pla
 
 template <typename T>
 int launch_spmm_rows_impl(const SpmmParams& p, int BN, int batch, hipStream_t st) {
-    if (!(BN == 32 && p.BK == 32 && p.compressed && p.s_batch > 0 && p.d_kcontig && p.s_kcontig && p.out_ncontig && !(p.bias && p.bias_on_m) &&
+    if (!(BN == 32 && p.BK == 32 && p.compressed && p.s_batch > 0 && p.d_kcontig && p.s_kcontig && p.out_ncontig &&
           p.K % 64 == 0 && p.d_ld % 8 == 0 && p.o_ld % 8 == 0 && p.d_ld < (1 << 24) && p.Mc >= 2200 && p.Mc < (1 << 24)))
         return kSpmmRowsNot;
     // Enough live blocks to a column that its walk counts, and rounds of workgroups that at least half fill the chip.  170 problems
