@@ -238,7 +238,7 @@ def test_moe_tile_configs(layout, tile_cfg, dtype, n_tok, in_dims, out_dims, gpu
     (torch.bfloat16, 20000, 576, 1544, 4), (torch.float16, 17000, 256, 1032, 70), (torch.float16, 1, 256, 8, 2)])
 def test_moe_persistent_tiles(layout, dtype, n_tok, in_dims, out_dims, n_exp, gpu):
     """Tile config 5 through the C ABI: every cut of the last round, experts that end inside a tile and inside a half of one, an
-    empty expert, tokens without one, and a token of NaN that reaches no other row."""
+    empty expert, tokens without one, and a token of NaN that reaches no other row.  A single token is finite."""
     from sparta_amd import _lib
     moe, w = make_moe(n_exp, in_dims, out_dims, dtype, gpu)
     rng = np.random.default_rng(n_tok)
@@ -246,12 +246,13 @@ def test_moe_persistent_tiles(layout, dtype, n_tok, in_dims, out_dims, n_exp, gp
     share[n_exp // 2] = 0.0
     ids_np = rng.choice(n_exp + 1, size=n_tok, p=share / share.sum()).astype(np.int32)
     x = torch.from_numpy(rng.random((n_tok, in_dims), dtype=np.float32)).to(dtype)
-    xg, bad = x.to(gpu), n_tok - 1
-    ids_np[bad] = 0
-    xg[bad] = float('nan')
+    xg, bad = x.to(gpu), np.arange(n_tok) == (n_tok - 1 if n_tok > 1 else -1)
+    ids_np[-1] = 0
+    xg[torch.from_numpy(bad).to(gpu)] = float('nan')
     moe(xg, torch.from_numpy(ids_np).to(gpu))  # builds the index
     weight = moe.weight.detach() if layout == 0 else moe.weight.detach().transpose(1, 2).contiguous()
     out = torch.full((n_tok, out_dims), float('nan'), dtype=dtype, device=gpu)
+    out[torch.from_numpy(bad).to(gpu)] = 7.0   # (a row that nobody writes is not NaN)
 
     def call():
         _lib.check(_lib.load().spx_moe_forward(_lib.dtype_code(dtype), _lib.dev_ptr(xg), _lib.dev_ptr(weight), layout, _lib.dev_ptr(out),
@@ -260,8 +261,8 @@ def test_moe_persistent_tiles(layout, dtype, n_tok, in_dims, out_dims, n_exp, gp
 
     _, names = launched_kernels(call)
     assert any('moe_persist_kernel' in n for n in names), names
-    assert bool(torch.isnan(out[bad]).all())
-    rows = np.arange(n_tok) != bad
+    rows = ~bad
+    assert bool(torch.isnan(out[torch.from_numpy(bad).to(gpu)]).all())
     want = ops.moe_reference(x.to(torch.float64).numpy(), np.concatenate([w, np.zeros_like(w[:1])]), ids_np)
     assert_close(out[torch.from_numpy(rows).to(gpu)], want[rows], dtype, f'persistent moe {n_tok} x {in_dims} -> {out_dims} over {n_exp}')
 
