@@ -134,8 +134,10 @@ extern "C" int spx_matmul(int mode, int dtype, int transA, int transB, int compr
 
 namespace spx {
 
-static int split_slices(int dtype, int transA, int transB, int nnz, int batch, int M, int K, int BM, int BN, int slices) {
-    return slices ? slices : dds_share_plan(dtype_bytes(dtype), !transA, transB, nnz, batch, M, K, BM, BN).slices;
+// `slices`: as asked for, 0: the plan's own choice.
+static DdsShare split_plan(int dtype, int transA, int transB, int nnz, int batch, int M, int K, int BM, int BN, int slices) {
+    if (slices) return {0, slices};
+    return dds_share_plan(dtype_bytes(dtype), !transA, transB, nnz, batch, M, K, BM, BN);
 }
 static size_t split_partial_bytes(int slices, int nnz, int batch, int BM, int BN) {
     return slices > 1 ? (size_t)batch * slices * nnz * BM * BN * sizeof(float) : 0;
@@ -151,7 +153,7 @@ extern "C" size_t spx_matmul_split_workspace_bytes(int dtype, int transA, int tr
                                                    int BM, int BN, int slices, int with_colsum) {
     using namespace spx;
     (void)N;
-    slices = split_slices(dtype, transA, transB, nnz, batch, M, K, BM, BN, slices);
+    slices = split_plan(dtype, transA, transB, nnz, batch, M, K, BM, BN, slices).slices;
     return split_partial_bytes(slices, nnz, batch, BM, BN) + (with_colsum ? split_colsum_bytes(dtype, slices, nnz, batch, M, K) : 0);
 }
 
@@ -173,8 +175,9 @@ extern "C" int spx_matmul_split(int dtype, int transA, int transB, int compresse
     SPX_REQUIRE(!compressed || (sparse_batch_stride * es) % 16 == 0, SPX_E_ALIGN, "sparse batch stride must keep blocks 16-byte aligned");
     DdsSplit s;
     SPX_REQUIRE(slices == 0 || slices == 1 || slices == 2 || slices == 4 || slices == 8, SPX_E_CONFIG, "slices=%d not in {0,1,2,4,8}", slices);
-    s.slices = split_slices(dtype, transA, transB, nnz, batch, M, K, BM, BN, slices);
-    s.share = slices ? 0 : dds_share_plan(es, !transA, transB, nnz, batch, M, K, BM, BN).blocks;
+    const DdsShare plan = split_plan(dtype, transA, transB, nnz, batch, M, K, BM, BN, slices);
+    s.slices = plan.slices;
+    s.share = plan.blocks;
     s.k_slice = 0;
     s.nnz = nnz;
     s.n_product = 0;

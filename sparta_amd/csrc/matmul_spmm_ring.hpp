@@ -90,7 +90,8 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     constexpr int MT = TM / 64, NT = BN / 16; // 16 x 16 tiles of a wavefront
     // fp32 blocks 16 wide: the sum of a tile in four chains of MFMAs, by half and by the parity of their k-step, added up at
     // the end.  They are as long as those of four wavefronts that share a block-column (matmul_spmm_ksplit.hpp), and
-    // neighbouring MFMAs of a wavefront with one tile do not wait for each other.
+    // neighbouring MFMAs of a wavefront with one tile do not wait for each other.  1024^3 at 35 %: relative error 3.4e-7 in one
+    // chain, 1.8e-7 in four, 15.3 and 15.0 us (split columns 16.4).
     constexpr int CHAINS = ES == 4 && NT == 1 ? 4 : 1;
     constexpr int NB = ring_stages(ES), D_BYTES = TM * 128, STAGE = LDS.stage;
     constexpr int ND = TM / 8, NS = BN / 8;   // load instructions of a stage: dense and sparse part
