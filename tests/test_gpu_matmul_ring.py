@@ -56,8 +56,7 @@ def test_ring_more_block_columns_than_the_table(gpu):
     # ... more rows: up to 32 and up to 64 block-columns, both sides of the live-block limits
     (torch.float32, (16, 16, 16), 1025, 1056, 512, 0.8), (torch.float32, (16, 16, 16), 1500, 1056, 1024, 0.7),
     (torch.float32, (16, 16, 16), 1025, 800, 512, 0.95), (torch.float32, (16, 16, 16), 1025, 1056, 1040, 0.8),
-    # fp32 16 x 16 through the ring: medium block-columns, first row count and the one before, wide results, too many live blocks;
-    # short ones over many rows, and one row too many
+    # fp32 16 x 16 around the rows and columns that the ring kernel is looked at for (test_dispatch_of_fp32_blocks_of_16 reads the launches)
     (torch.float32, (16, 16, 16), 700, 784, 1040, 0.7), (torch.float32, (16, 16, 16), 699, 784, 1040, 0.7), (torch.float32, (16, 16, 16), 900, 1408, 1552, 0.84),
     (torch.float32, (16, 16, 16), 900, 1408, 1536, 0.7), (torch.float32, (16, 16, 16), 2049, 768, 1536, 0.86), (torch.float32, (16, 16, 16), 6001, 512, 512, 0.9),
     # ring: 1100 tiles of 64 rows in tiles of 64 and of 128, and one column fewer
