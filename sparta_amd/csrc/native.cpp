@@ -729,10 +729,33 @@ std::pair<Tensor, int> moe_forward(const Tensor& tokens_in, const Tensor& ids_in
 // (row_ptr, bcsr, row_order, col_ptr, bcsc, col_order, nnz), None where a format is not wanted.
 typedef std::tuple<Tensor, int, int, bool, bool, int64_t, int64_t> IndexRequest;
 
+// The tensors of one allocation, one after the other.  What an index consists of lives and dies together, and an
+// allocation costs the host as much as a launch does (two masks: 13.3 us with an allocation to a tensor, of which ten).
+class Slab {
+public:
+    int64_t reserve(int64_t bytes) {   // where they begin
+        const int64_t at = bytes_;
+        bytes_ += (bytes + 255) / 256 * 256;
+        return at;
+    }
+    void allocate(const Tensor& like) { base_ = at::empty({bytes_}, like.options().dtype(at::kByte)); }
+    Tensor tensor(int64_t at, int64_t numel, at::ScalarType type) const {
+        auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(base_.storage()), base_.key_set(), c10::scalarTypeToTypeMeta(type));
+        impl->set_storage_offset(at / (int64_t)c10::elementSize(type));
+        impl->set_sizes_contiguous({numel});
+        return Tensor(std::move(impl));
+    }
+    void* place(int64_t at) const { return (char*)base_.data_ptr() + at; }
+
+private:
+    int64_t bytes_ = 0;
+    Tensor base_;
+};
+
 std::vector<py::tuple> build_indexes(const std::vector<IndexRequest>& requests) {
     struct Built {
         std::optional<Tensor> row_ptr, bcsr, row_order, col_ptr, bcsc, col_order;
-        Tensor nnz, scratch;
+        Tensor nnz;
     };
     std::vector<Built> built(requests.size());
     if (!requests.empty()) {
@@ -742,38 +765,52 @@ std::vector<py::tuple> build_indexes(const std::vector<IndexRequest>& requests) 
         device_ptr(first);   // refuses CPU tensors
         c10::DeviceGuard guard(first.device());
         std::vector<spx_bcs_index_job> jobs(requests.size());
+        Slab scratch;   // of all builds; given back when the call returns, in stream order
+        std::vector<int64_t> scratch_at(requests.size());
+        for (size_t i = 0; i < requests.size(); ++i) scratch_at[i] = scratch.reserve(std::get<6>(requests[i]));
+        scratch.allocate(first);
         for (size_t i = 0; i < requests.size(); ++i) {
             const auto& [mask, BH, BW, want_r, want_c, cap_in, ws_bytes] = requests[i];
             const int H = (int)mask.size(0), W = (int)mask.size(1), R = H / BH, C = W / BW;
             const int64_t cap = cap_in < 0 ? (int64_t)R * C : cap_in;
-            const auto i32 = mask.options().dtype(at::kInt);
+            const bool wide = want_r && want_c;   // int64 entries of the BCSC index
             Built& b = built[i];
             spx_bcs_index_job& job = jobs[i];
             job = spx_bcs_index_job();
-            b.nnz = at::empty({1}, i32);
-            b.scratch = at::empty({ws_bytes}, mask.options().dtype(at::kByte));
+            Slab slab;
+            const int64_t nnz_at = slab.reserve(4);
+            int64_t ptr_at[2] = {}, idx_at[2] = {}, order_at[2] = {};
+            for (int f = 0; f < 2; ++f) {
+                if (!(f == 0 ? want_r : want_c)) continue;
+                const int64_t n = f == 0 ? R : C;
+                ptr_at[f] = slab.reserve(4 * (n + 1));
+                order_at[f] = slab.reserve(4 * n);   // the launch orders of the matmul kernels come out of the same launch
+                idx_at[f] = slab.reserve((f == 1 && wide ? 8 : 4) * cap);
+            }
+            slab.allocate(mask);
+            b.nnz = slab.tensor(nnz_at, 1, at::kInt);
             if (want_r) {
-                b.row_ptr = at::empty({R + 1}, i32);
-                b.bcsr = at::empty({cap}, i32);
-                b.row_order = at::empty({R}, i32);   // the launch orders of the matmul kernels
-                job.row_ptr = (int32_t*)b.row_ptr->data_ptr();
-                job.bcsr_idx = (int32_t*)b.bcsr->data_ptr();
-                job.row_order = (int32_t*)b.row_order->data_ptr();
+                b.row_ptr = slab.tensor(ptr_at[0], R + 1, at::kInt);
+                b.bcsr = slab.tensor(idx_at[0], cap, at::kInt);
+                b.row_order = slab.tensor(order_at[0], R, at::kInt);
+                job.row_ptr = (int32_t*)slab.place(ptr_at[0]);
+                job.bcsr_idx = (int32_t*)slab.place(idx_at[0]);
+                job.row_order = (int32_t*)slab.place(order_at[0]);
             }
             if (want_c) {
-                b.col_ptr = at::empty({C + 1}, i32);
-                b.bcsc = at::empty({cap}, want_r ? i32.dtype(at::kLong) : i32);
-                b.col_order = at::empty({C}, i32);   // come out of the same launch
-                job.col_ptr = (int32_t*)b.col_ptr->data_ptr();
-                job.bcsc_idx = b.bcsc->data_ptr();
-                job.col_order = (int32_t*)b.col_order->data_ptr();
+                b.col_ptr = slab.tensor(ptr_at[1], C + 1, at::kInt);
+                b.bcsc = slab.tensor(idx_at[1], cap, wide ? at::kLong : at::kInt);
+                b.col_order = slab.tensor(order_at[1], C, at::kInt);
+                job.col_ptr = (int32_t*)slab.place(ptr_at[1]);
+                job.bcsc_idx = slab.place(idx_at[1]);
+                job.col_order = (int32_t*)slab.place(order_at[1]);
             }
             job.mask = (const uint8_t*)device_ptr(mask);
             job.H = H; job.W = W; job.BH = BH; job.BW = BW;
-            job.bcsc_i64 = want_r && want_c;
-            job.nnz_dev = (int32_t*)b.nnz.data_ptr();
+            job.bcsc_i64 = wide;
+            job.nnz_dev = (int32_t*)slab.place(nnz_at);
             job.cap = (int)cap;
-            job.workspace = b.scratch.data_ptr();
+            job.workspace = scratch.place(scratch_at[i]);
             job.workspace_bytes = (size_t)ws_bytes;
         }
         check_rc(spx_bcs_index_batch(jobs.data(), (int)jobs.size(), stream_of(first)), "spx_bcs_index_batch");

@@ -112,11 +112,12 @@ class SparseMatMulKernel(KernelBase):
         self.set_parameter('GLOBAL_N_VALUE', N)
 
     def get_shape(self):
-        return tuple(self.get_parameter(n) for n in
-                     ('BATCH_SIZE', 'GLOBAL_M_VALUE', 'GLOBAL_K_VALUE', 'GLOBAL_N_VALUE'))
+        p = self._parameters
+        return p['BATCH_SIZE'].value, p['GLOBAL_M_VALUE'].value, p['GLOBAL_K_VALUE'].value, p['GLOBAL_N_VALUE'].value
 
     def get_block_shape(self):
-        return tuple(self.get_parameter(f'BLOCK_SIZE_{d}_VALUE') for d in 'MKN')
+        p = self._parameters
+        return p['BLOCK_SIZE_M_VALUE'].value, p['BLOCK_SIZE_K_VALUE'].value, p['BLOCK_SIZE_N_VALUE'].value
 
     def sparse_block_shape(self):
         return (self.ports[self._sparse_port],

@@ -85,18 +85,19 @@ class SparseLinear(OperatorBase):
                         weight_mask: Optional[torch.Tensor] = None,
                         output_mask: Optional[torch.Tensor] = None) -> Dict[str, torch.Tensor]:
         """Check the arguments of `update_mask`; returns {sparse port: mask}."""
-        given = {k: v for k, v in (('input', input_mask), ('weight', weight_mask), ('output', output_mask))
-                 if v is not None}
+        given = [(k, v) for k, v in (('input', input_mask), ('weight', weight_mask), ('output', output_mask))
+                 if v is not None]
         if len(given) > 1:
             raise ValueError('linear operators with multiple sparse masks are not supported')
         if not given:
             raise ValueError('expected a sparse mask on input / weight / output')
-        (kind, mask), = given.items()
-        M, K, N = self._shape['M'], self._shape['K'], self._shape['N']
-        want = {'input': (M, K), 'weight': (N, K), 'output': (M, N)}[kind]
-        ok = all(w is None or w == got for w, got in zip(want, mask.shape))
-        shown = tuple('?' if w is None else w for w in want)
-        assert ok and mask.dim() == 2, f'expected {kind} mask shape {shown}, got {tuple(mask.shape)}'
+        (kind, mask), = given
+        rows, cols = ('N', 'K') if kind == 'weight' else ('M', 'K') if kind == 'input' else ('M', 'N')
+        want, shape = (self._shape[rows], self._shape[cols]), tuple(mask.shape)
+        if shape != want:   # (a side that is not known yet takes any size)
+            ok = all(w is None or w == got for w, got in zip(want, shape))
+            shown = tuple('?' if w is None else w for w in want)
+            assert ok and len(shape) == 2, f'expected {kind} mask shape {shown}, got {shape}'
         return {self._PORT_OF[kind]: mask}
 
     def _read_sample_inputs(self, A: torch.Tensor):

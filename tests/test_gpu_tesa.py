@@ -118,6 +118,31 @@ def test_index_batch_equals_single_builds(gpu):
     assert build_indexes_batch([]) == []
 
 
+@pytest.mark.parametrize('r,c', [(True, True), (True, False), (False, True)])
+def test_index_tensors_of_a_build_lie_apart(r, c, gpu):
+    """The tensors of an index come out of one allocation: none overlaps another, each begins at a multiple of 256 bytes, the
+    values survive the other indexes of the call and the scratch that its builds shared."""
+    from sparta_amd.tesa import build_indexes_batch
+    masks = [torch.from_numpy(ops.block_mask((H, W), (32, 16), 0.6, seed=H)).to(gpu) for H, W in ((32, 16), (96, 1040), (1056, 48))]
+    ctx = get_bcs_function(32, 16, r, c)
+    indexes = build_indexes_batch([(ctx, m) for m in masks])
+    for x in indexes:
+        parts = [t for n in ('row_ptr', '_bcsr_buf', 'col_ptr', '_bcsc_buf', 'nnz_dev') if (t := getattr(x, n, None)) is not None]
+        parts += list(x.__dict__['_launch_order'].values())
+        assert len(parts) == 1 + 3 * (r + c) and all(t.is_contiguous() and t.data_ptr() % 256 == 0 for t in parts)
+        spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in parts)
+        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+    kept = indexes[1]
+    del indexes, x, parts
+    junk = [torch.full((1 << 20,), 255, dtype=torch.uint8, device=gpu) for _ in range(8)]
+    row_ptr, bcsr, col_ptr, _, nnz = bcs.build_bcsrc(masks[1].cpu().numpy(), 32, 16)
+    assert kept.block_nnz == nnz and len(junk) == 8
+    if r:
+        assert np.array_equal(kept.row_ptr.cpu().numpy(), row_ptr) and np.array_equal(kept.BCSR_idx.cpu().numpy(), bcsr)
+    if c:
+        assert np.array_equal(kept.col_ptr.cpu().numpy(), col_ptr)
+
+
 @pytest.mark.parametrize('n', [1, 2, 4, 5])
 def test_index_builds_share_launches_only_where_there_are_several(n, gpu):
     """Up to four builds of one call share a pair of launches; one on its own - a single call, or what is left over of
