@@ -166,10 +166,8 @@ __global__ __launch_bounds__(64 * WAVES, SPLIT > 1 ? 2 : E == 64 ? 4 : KT == 1 ?
     for (int c = 0; c < EC; ++c)
         qf[c] = *reinterpret_cast<const Frag*>(reinterpret_cast<const T*>(p.q) + (b * p.Nt + (rows_exist ? row0 + l32 : 0)) * E + c * 16 + h2 * 8);
 
-    typedef const __attribute__((address_space(4))) int32_t* const_i32;
-    const int e_begin = SEQ ? 0 : ((const_i32)p.row_ptr)[br];
-    const int n_ent = SEQ ? 0 : ((const_i32)p.row_ptr)[br + 1] - e_begin;
-    const int col_first = SEQ || n_ent == 0 ? 0 : ((const_i32)p.bcsr_idx)[e_begin] & 0xffff;
+    const int e_begin = SEQ ? 0 : p.row_ptr[br];
+    const int n_ent = SEQ ? 0 : p.row_ptr[br + 1] - e_begin;
     const int n = SEQ ? (seq_len + KEYS - 1) / KEYS : n_ent << log_sub;
     int bc_vec = 0;
     if constexpr (!SEQ) {
@@ -180,10 +178,10 @@ __global__ __launch_bounds__(64 * WAVES, SPLIT > 1 ? 2 : E == 64 ? 4 : KT == 1 ?
         const int col = e < 64 ? __builtin_amdgcn_readlane(bc_vec, e) : __builtin_amdgcn_readfirstlane(p.bcsr_idx[e_begin + e] & 0xffff);
         return ((col << log_sub) + (i & ((1 << log_sub) - 1))) * 32;
     };
-    auto issue = [&](int i, int at, auto first) {
+    auto issue = [&](int i, int at) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
-            int key0 = SEQ ? i * KEYS + kt * 32 : first ? (col_first << log_sub) * 32 : key0_at(i);
+            int key0 = SEQ ? i * KEYS + kt * 32 : key0_at(i);
             if (kt > 0 && key0 >= p.Ns) key0 = p.Ns - 32;   // past the tensor and the length: any rows
             const uint32_t to = lds0 + at + kt * Tile::BYTES;
             if constexpr (WAVES == 1) {
@@ -197,7 +195,7 @@ __global__ __launch_bounds__(64 * WAVES, SPLIT > 1 ? 2 : E == 64 ? 4 : KT == 1 ?
                 lds_direct_load16_at(p.mask + (int64_t)row0 * p.Ns + key0, (lane >> 1) * p.Ns + (lane & 1) * 16, to + Lds::MASK + wave * 1024);
         }
     };
-    if (n > 0) issue(0, 0, std::true_type());
+    if (n > 0) issue(0, 0);
 
     f32x16 oacc[ET];
 #pragma unroll
@@ -225,7 +223,7 @@ __global__ __launch_bounds__(64 * WAVES, SPLIT > 1 ? 2 : E == 64 ? 4 : KT == 1 ?
         constexpr int at = slot * Lds::STAGE, fill = (slot + NB - 1) % NB * Lds::STAGE;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of stage i is in LDS
         __syncthreads();                                   // everybody's is, and stage i - 1 has been read
-        if (i + 1 < n) issue(i + 1, fill, std::false_type());
+        if (i + 1 < n) issue(i + 1, fill);
         const int left = SEQ ? seq_len - i * KEYS : KEYS;   // live keys of this stage
         if (SEQ && left < KEYS) {
             // value rows past the length: their probabilities are 0, and 0 times what padding may hold is not
