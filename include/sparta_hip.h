@@ -338,7 +338,8 @@ int spx_attention_backward_kv(int dtype, const void* grad_out, const void* q, co
  * writes only q, k, v, out, grad_out and the three gradients.  spx_attention_backward_q and
  * spx_attention_backward_kv_recompute take block-level masks (every element of a live block
  * attends); the *_masked forms also the element mask that the forward pass was given (bytes
- * [Nt, Ns], 16-byte aligned, NULL: none), with head dim 64 and query and key blocks of 32 / 64;
+ * [Nt, Ns], 16-byte aligned, NULL: none), with query and key blocks of 32 / 64 and head dim 64, or
+ * 128 with key blocks no wider than query blocks;
  * the *_live_mask forms its live blocks, as spx_bcs_gather gives them (bytes [nnz, BH, BW] in
  * the order of the compressed values: BCSR with SPX_IDX_BCSC_I64, BCSC with SPX_IDX_BCSC_I32),
  * which is all that a training step has to keep of it.

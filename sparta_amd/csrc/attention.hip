@@ -1549,12 +1549,16 @@ __global__ __launch_bounds__(64 * WAVES, (BH * E <= 64 * 64 || BH == 32) ? 3 : (
 //   (dP - D) / T = dO V^T   (V scaled by 1 / T, accumulators started at -D / T),
 //   P = exp2(S - L),  dS = P o (dP - D) / T,  both already in the B-operand layout of
 //   dK^T += Q^T dS  and  dV^T += dO^T P.
-// L and D of the block's queries pass through LDS (one float per thread).  Block-level masks
-// only.
+// L and D of the block's queries pass through LDS (one float per thread).
 // F32S: S is scaled in fp32 instead of K to 16 bits, for row statistics that are (attention_fp32_scores); with head dim 64 the
 // 16-bit scaling of K is no further off with those than with the others.
-template <typename T, int BH, int E, int WAVES, bool F32S>
-__global__ __launch_bounds__(64 * WAVES, (BH * E <= 64 * 64 || BH == 32) ? 3 : (BH * E <= 128 * 64 ? 2 : 1))
+// HAS_MASK (F32S as well): an element mask as in the wide kernels, the [Nt, Ns] tensor or its live blocks in BCSR order; dP is scaled
+// in fp32 too, as it is where the probabilities are stored.  The bytes of a block pass through LDS; a wavefront looks at
+// its 16 columns of all rows at once and skips the rest where they are all 1.  A step with head dim 128 and a causal mask is 96 x 1024
+// fp16 162 -> 115 us with it, 24 x 3200 156 -> 111, 32 x 32 blocks 137 -> 94 (with stored probabilities the forward kernel alone took 86).
+// Two wavefronts to a SIMD with head dim 128 also in 32-high blocks: three spilled 28 registers under a mask (24 x 3200 36.2 -> 32.2 us without one).
+template <typename T, int BH, int E, int WAVES, bool F32S, bool HAS_MASK>
+__global__ __launch_bounds__(64 * WAVES, BH * E <= 64 * 64 ? (E == 128 ? 2 : 3) : (BH * E <= 128 * 64 ? 2 : 1))
 void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
     constexpr int BW = 16 * WAVES;
     constexpr int NT = 64 * WAVES;
@@ -1563,6 +1567,9 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
     constexpr int Q_OFF = BH * DP, S_OFF = 2 * BH * DP;   // S_OFF: BH values of L, then BH of D / T
     constexpr int VPR = E / 8;                // 16-byte vectors per row
     constexpr int NVD = BH * VPR / NT;        // vectors per thread: dO / Q tile
+    constexpr int M_OFF = S_OFF + 2 * BH * 4, MP = BW + 16;                  // mask bytes of the block, rows of MP
+    constexpr int NVM = (BH * BW / 16 + NT - 1) / NT;                        // vectors per thread: mask bytes
+    static_assert(F32S || !HAS_MASK, "scores under an element mask are scaled in fp32");
     static_assert(BH * VPR % NT == 0 && QT % 2 == 0 && 2 * BH <= NT, "tiles do not split over the workgroup");
     typedef typename Mma32<T>::frag Frag;
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -1601,7 +1608,7 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
             vs[x] = (float)v_raw[x] * p.inv_t;
             ks[x] = (float)k_raw[x] * c2;
         }
-        vf[c] = AttnPack<T>::pack(vs);
+        vf[c] = HAS_MASK ? v_raw : AttnPack<T>::pack(vs);
         kf[c] = F32S ? k_raw : AttnPack<T>::pack(ks);
     }
 
@@ -1623,9 +1630,24 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
         return p.bcsc_wide ? (int)(reinterpret_cast<const long long*>(p.bcsc_idx)[e] & 0xffff)
                            : (reinterpret_cast<const int32_t*>(p.bcsc_idx)[e] & 0xffff);
     };
-    u32x4 do_r[NVD], q_r[NVD];
+    auto mask_block = [&](int e) -> int {   // its mask bytes are the rows from BH times this on
+        if (!HAS_MASK) return 0;
+        if (!p.mask_blocks) return query_block(e);
+        return p.bcsc_wide ? (int)(reinterpret_cast<const long long*>(p.bcsc_idx)[e] >> 32) : e;
+    };
+    const int mask_ld = p.mask_blocks ? BW : p.Ns;
+    const uint8_t* const mask = HAS_MASK ? p.mask + (p.mask_blocks ? 0 : j * BW) : nullptr;
+    u32x4 do_r[NVD], q_r[NVD], m_r[NVM];
     float st_r = 0.f;
-    auto issue = [&](int qb) {
+    auto issue = [&](int qb, int mb) {
+        if constexpr (HAS_MASK) {
+            const uint8_t* const rows = mask + (int64_t)mb * BH * mask_ld;
+#pragma unroll
+            for (int i = 0; i < NVM; ++i) {
+                const int v = threadIdx.x + i * NT;
+                if (v < BH * BW / 16) m_r[i] = *reinterpret_cast<const u32x4*>(rows + (int64_t)(v / (BW / 16)) * mask_ld + v % (BW / 16) * 16);
+            }
+        }
         const int64_t off = (int64_t)qb * BH * E;
 #pragma unroll
         for (int i = 0; i < NVD; ++i) do_r[i] = *reinterpret_cast<const u32x4*>(dO + off + i * NT * 8);
@@ -1633,11 +1655,12 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
         for (int i = 0; i < NVD; ++i) q_r[i] = *reinterpret_cast<const u32x4*>(Q + off + i * NT * 8);
         if (has_stat) st_r = stat[qb * BH];
     };
-    int qb = 0, qb_next = 0;
+    int qb = 0, qb_next = 0, mb_next = 0;
     if (e_begin < e_end) {
         qb = query_block(e_begin);
         qb_next = query_block(e_begin + 1 < e_end ? e_begin + 1 : e_begin);
-        issue(qb);
+        mb_next = mask_block(e_begin + 1 < e_end ? e_begin + 1 : e_begin);
+        issue(qb, mask_block(e_begin));
     }
     for (int e = e_begin; e < e_end; ++e) {
         __syncthreads();   // everyone is done with the previous tiles
@@ -1646,10 +1669,19 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
 #pragma unroll
         for (int i = 0; i < NVD; ++i) *reinterpret_cast<u32x4*>(smem + Q_OFF + d_dst + i * D_RSTEP * DP) = q_r[i];
         if (has_stat) *reinterpret_cast<float*>(smem + S_OFF + threadIdx.x * 4) = st_r;
+        if constexpr (HAS_MASK) {
+#pragma unroll
+            for (int i = 0; i < NVM; ++i) {
+                const int v = threadIdx.x + i * NT;
+                if (v < BH * BW / 16) *reinterpret_cast<u32x4*>(smem + M_OFF + v / (BW / 16) * MP + v % (BW / 16) * 16) = m_r[i];
+            }
+        }
         // next live block of the column (the last step re-reads its own block; the copy is not used)
         qb = qb_next;
+        const int mb = mb_next;
         qb_next = query_block(e + 2 < e_end ? e + 2 : e_end - 1);
-        issue(qb);
+        mb_next = mask_block(e + 2 < e_end ? e + 2 : e_end - 1);
+        issue(qb, mb);
         __syncthreads();
 
         // ---- S - L and (dP - D) / T: 16 queries x this wave's 16 keys per tile -----------------
@@ -1658,7 +1690,8 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
         for (int t = 0; t < QT; ++t) {
             const f32x4 lse = *reinterpret_cast<const f32x4*>(smem + S_OFF + (t * 16 + g4 * 4) * 4);
             s[t] = F32S ? f32x4{0.f, 0.f, 0.f, 0.f} : -lse;
-            dp[t] = -*reinterpret_cast<const f32x4*>(smem + S_OFF + (BH + t * 16 + g4 * 4) * 4);
+            const f32x4 dot = *reinterpret_cast<const f32x4*>(smem + S_OFF + (BH + t * 16 + g4 * 4) * 4);
+            dp[t] = HAS_MASK ? f32x4{0.f, 0.f, 0.f, 0.f} : -dot;
 #pragma unroll
             for (int c = 0; c < EC; ++c) {
                 const Frag qa = *reinterpret_cast<const Frag*>(smem + Q_OFF + a_src + t * 16 * DP + c * 64);
@@ -1669,6 +1702,20 @@ void attention_bwd_col_rc_kernel(AttnParams p, int nbc, int batch) {
             if constexpr (F32S) {
 #pragma unroll
                 for (int x = 0; x < 4; ++x) s[t][x] = __builtin_fmaf(s[t][x], c2, -lse[x]);
+            }
+            if constexpr (HAS_MASK) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) dp[t][x] = __builtin_fmaf(dp[t][x], p.inv_t, -dot[x]);
+            }
+        }
+        if constexpr (HAS_MASK) {
+            const u32x4 row = *reinterpret_cast<const u32x4*>(smem + M_OFF + lane % BH * MP + wave * 16);
+            if (__builtin_amdgcn_ballot_w64((row[0] & row[1] & row[2] & row[3]) != 0x01010101u) != 0) {
+#pragma unroll
+                for (int t = 0; t < QT; ++t)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        s[t][x] = smem[M_OFF + (t * 16 + g4 * 4 + x) * MP + wave * 16 + r16] ? s[t][x] : -__builtin_inff();
             }
         }
         // ---- P = exp2(S - L), dS = P o (dP - D) / T: both as B operands ------------------------
@@ -1767,22 +1814,26 @@ static bool attention_bwd_col_rc_supported(int BH, int BW, int E) {
     return attention_bwd_col_supported(BH, BW, E) && BH <= 2 * BW;
 }
 
-template <typename T, int BH, int E, int WAVES, bool F32S>
+template <typename T, int BH, int E, int WAVES, bool F32S, bool HAS_MASK>
 static int launch_attention_bwd_col_rc_inst(const AttnParams& p, int batch, hipStream_t st) {
-    constexpr size_t smem = 2 * BH * (E * 2 + 32) + 2 * BH * 4;
+    constexpr size_t smem = 2 * BH * (E * 2 + 32) + 2 * BH * 4 + (HAS_MASK ? BH * (16 * WAVES + 16) : 0);
     const int nbc = p.Ns / (16 * WAVES);
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbc;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    SPX_GRANT_LDS((attention_bwd_col_rc_kernel<T, BH, E, WAVES, F32S>), smem, "attention_bwd_col_rc_kernel");
-    hipLaunchKernelGGL((attention_bwd_col_rc_kernel<T, BH, E, WAVES, F32S>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbc, batch);
+    SPX_GRANT_LDS((attention_bwd_col_rc_kernel<T, BH, E, WAVES, F32S, HAS_MASK>), smem, "attention_bwd_col_rc_kernel");
+    hipLaunchKernelGGL((attention_bwd_col_rc_kernel<T, BH, E, WAVES, F32S, HAS_MASK>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbc, batch);
     SPX_LAUNCH_CHECK("attention_bwd_col_rc_kernel");
     return 0;
 }
 
 template <typename T>
 static int launch_attention_bwd_col_rc(const AttnParams& p, int batch, int BW, int E, hipStream_t st) {
+#define SPX_ATTNCR_MASK_CASE(bh, bw) \
+    if (p.mask && p.BH == bh && BW == bw && E == 128) return launch_attention_bwd_col_rc_inst<T, bh, 128, bw / 16, true, true>(p, batch, st);
+    SPX_ATTNCR_MASK_CASE(32, 32) SPX_ATTNCR_MASK_CASE(64, 32) SPX_ATTNCR_MASK_CASE(64, 64)
+#undef SPX_ATTNCR_MASK_CASE
 #define SPX_ATTNCR_CASE(bh, bw, e) \
-    if (p.BH == bh && BW == bw && E == e) return launch_attention_bwd_col_rc_inst<T, bh, e, bw / 16, e == 128 && attention_wide_supported(bh, bw, e)>(p, batch, st);
+    if (!p.mask && p.BH == bh && BW == bw && E == e) return launch_attention_bwd_col_rc_inst<T, bh, e, bw / 16, e == 128 && attention_wide_supported(bh, bw, e), false>(p, batch, st);
     SPX_ATTNCR_CASE(32, 32, 64) SPX_ATTNCR_CASE(32, 64, 64)
     SPX_ATTNCR_CASE(32, 32, 128) SPX_ATTNCR_CASE(32, 64, 128) SPX_ATTNCR_CASE(32, 128, 128)
     SPX_ATTNCR_CASE(64, 32, 64) SPX_ATTNCR_CASE(64, 64, 64) SPX_ATTNCR_CASE(64, 128, 64)
@@ -2176,12 +2227,19 @@ namespace spx {
 // and 15.6 / 17.2; 16 x 2048 (512) 10.3 / 13.0 and 12.1 / 13.7, 12 x 512 (96) 5.0 / 6.9 and 6.0 / 6.9.  32 x 32 blocks: level at 12288
 // workgroups (70 / 84 and 69 / 81), behind at 768 (9.2 / 10.1 and 9.6 / 11.4).
 static bool attention_bwd_wide_wins(int edge, int E, int64_t workgroups) { return edge == 64 && E == 64 && workgroups >= 768; }
+// Row side with head dim 128 (scores scaled in fp32 by both kernels), 16 / 32 queries per wavefront: 24 x 3200 fp16 (1200 workgroups) 38.3 / 34.2,
+// 48 x 1024 bf16 (768) 28.3 / 21.4, 96 x 1024 fp16 (1536) 40.6 / 36.7; 24 x 1024 (384) 16.2 / 17.3, 12 x 1024 11.4 / 12.7.  The column side
+// stays with 16 keys (see attention_bwd_wide.hip), under an element mask as well.
+static bool attention_bwd_row_wide_wins(int BH, int BW, int E, int64_t workgroups) {
+    if (E == 128) return BH == 64 && BW <= 64 && workgroups >= 600;
+    return attention_bwd_wide_wins(BH, E, workgroups);
+}
 
 // (blocks of 32 and 64: rows of the mask and of its live blocks are multiples of 16 bytes)
 static int attention_bwd_check_mask(const uint8_t* mask, int E, int BH, int BW) {
     if (!mask) return 0;
-    SPX_REQUIRE(E == 64 && (BH == 32 || BH == 64) && (BW == 32 || BW == 64), SPX_E_CONFIG,
-                "the backward kernels take an element mask with head dim 64 and query and key blocks of 32 / 64 (got %d, %d, %d)", E, BH, BW);
+    SPX_REQUIRE((BH == 32 || BH == 64) && (BW == 32 || BW == 64) && attention_wide_supported(BH, BW, E), SPX_E_CONFIG,
+                "the backward kernels take an element mask with query and key blocks of 32 / 64 and head dim 64, or 128 with key blocks no wider than query blocks (got %d, %d, %d)", BH, BW, E);
     SPX_REQUIRE(aligned(mask, 16), SPX_E_ALIGN, "the element mask must be 16-byte aligned");
     return 0;
 }
@@ -2213,7 +2271,7 @@ static int attention_backward_q_impl(int dtype, const void* grad_out, const void
     p.grad_out = grad_out; p.grad_q = grad_q; p.row_dot = row_dot; p.row_lse = const_cast<float*>(row_lse);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const bool fp32_scores = attention_fp32_scores(dtype, mask, (int64_t)batch * Nt, BH, BW, E);
-    if (mask || attention_bwd_wide_wins(BH, E, (int64_t)batch * (Nt / BH))) return launch_attention_bwd_row_wide(dtype, p, batch, BW, fp32_scores, st);
+    if (mask || attention_bwd_row_wide_wins(BH, BW, E, (int64_t)batch * (Nt / BH))) return launch_attention_bwd_row_wide(dtype, p, batch, BW, E, fp32_scores, st);
     if (dtype == SPX_F16) return launch_attention_bwd_row_rc<_Float16>(p, batch, BW, E, fp32_scores, st);
     return launch_attention_bwd_row_rc<bf16_t>(p, batch, BW, E, fp32_scores, st);
 }
@@ -2248,7 +2306,7 @@ static int attention_backward_kv_impl(int dtype, const void* grad_out, const voi
     p.col_ptr = col_ptr; p.bcsc_idx = bcsc_idx; p.bcsc_wide = idx_kind == SPX_IDX_BCSC_I64;
     p.grad_k = grad_k; p.grad_v = grad_v;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (mask || attention_bwd_wide_wins(BW, E, (int64_t)batch * (Ns / BW))) return launch_attention_bwd_col_wide(dtype, p, batch, BW, st);
+    if ((mask && E == 64) || attention_bwd_wide_wins(BW, E, (int64_t)batch * (Ns / BW))) return launch_attention_bwd_col_wide(dtype, p, batch, BW, st);
     if (dtype == SPX_F16) return launch_attention_bwd_col_rc<_Float16>(p, batch, BW, E, st);
     return launch_attention_bwd_col_rc<bf16_t>(p, batch, BW, E, st);
 }

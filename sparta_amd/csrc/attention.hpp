@@ -150,9 +150,9 @@ bool attention_wide_seq_wins(int64_t entries, int N, int E);
 int launch_attention_wide_seq(int dtype, const AttnParams& p, int batch, int E, hipStream_t st);
 
 // attention_bwd_wide.hip: backward kernels that recompute the probabilities, 32 queries or keys per wavefront, with
-// element masks; query and key blocks of 32 / 64, head dim 64
+// element masks; query and key blocks of 32 / 64, head dim 64 (on the row side also 128)
 // (fp32_scores: what the row statistic is of, see attention.hip; always with an element mask)
-int launch_attention_bwd_row_wide(int dtype, const AttnParams& p, int batch, int BW, bool fp32_scores, hipStream_t st);
+int launch_attention_bwd_row_wide(int dtype, const AttnParams& p, int batch, int BW, int E, bool fp32_scores, hipStream_t st);
 int launch_attention_bwd_col_wide(int dtype, const AttnParams& p, int batch, int BW, hipStream_t st);
 
 }  // namespace spx

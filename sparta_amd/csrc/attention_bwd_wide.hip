@@ -27,21 +27,27 @@ namespace spx {
 // (2.2 in kernels with fewer MFMAs).  96 x 4096 x 64 fp16, 392 blocks of 64 x 64: row side 87 -> 77 us, column side 111 -> 93
 // (58 and 77 GFLOP: 750 and 830 TFLOP/s); without the tile loads 66 and 82, without exponentials 92, without LDS reads 88.
 // Left out, no gain: four stages, two stages, loads requested later in a stage, raised wave priority.
-constexpr int kBwdStages = 3;
-template <int WAVES, bool HAS_MASK, bool STATS> struct BwdLds {
-    static constexpr int MASK = 2 * AttnTile<64>::BYTES;                          // 32 x 32 bytes per wavefront
+// Head dim 128, row side only: two stages, for four workgroups of two wavefronts to a CU.  24 x 3200 positions, 202 blocks of
+// 64 x 64 to a head, fp16 38.3 (16 queries per wavefront) -> 34.2 us, with an element mask 37.8 (stored probabilities) -> 37.7.  On
+// the column side the accumulators of 32 keys and their rows of K and V are 192 registers: what is spilled is read
+// back behind the loads of the next stage (41 -> 45 us), and with one wavefront to a SIMD nothing covers it.  Two wavefronts to
+// 32 queries that share the keys out lose as well (34 -> 39 us, though 12 x 1024 12.7 -> 11.8).
+constexpr int bwd_stages(int E) { return E == 64 ? 3 : 2; }
+template <int E, int WAVES, bool HAS_MASK, bool STATS> struct BwdLds {
+    static constexpr int NB = bwd_stages(E);
+    static constexpr int MASK = 2 * AttnTile<E>::BYTES;                          // 32 x 32 bytes per wavefront
     static constexpr int STAT = MASK + (HAS_MASK ? WAVES * 1024 : 0);            // 32 + 32 floats per wavefront
     static constexpr int STAGE = STAT + (STATS ? WAVES * 256 : 0);
-    static constexpr int OUT = WAVES * 32 * (AttnTile<64>::ROW + 16);                        // output rows, in the same space
-    static constexpr int TOTAL = kBwdStages * STAGE > OUT ? kBwdStages * STAGE : OUT;
+    static constexpr int OUT = WAVES * 32 * (AttnTile<E>::ROW + 16);             // output rows, in the same space
+    static constexpr int TOTAL = NB * STAGE > OUT ? NB * STAGE : OUT;
 };
 
 // ---- row side -----------------------------------------------------------------------------------
-template <typename T, int WAVES, bool HAS_MASK, bool F32S>
-__global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_row_wide_kernel(AttnParams p, int nbr, int log_sub, int batch) {
-    typedef AttnTile<64> Tile;
-    typedef BwdLds<WAVES, HAS_MASK, false> Lds;
-    constexpr int E = 64, EC = Tile::EC, ET = Tile::ET, NB = kBwdStages;
+template <typename T, int E, int WAVES, bool HAS_MASK, bool F32S>
+__global__ __launch_bounds__(64 * WAVES, HAS_MASK || E == 128 ? 2 : 3) void attention_bwd_row_wide_kernel(AttnParams p, int nbr, int log_sub, int batch) {
+    typedef AttnTile<E> Tile;
+    typedef BwdLds<E, WAVES, HAS_MASK, false> Lds;
+    constexpr int EC = Tile::EC, ET = Tile::ET, NB = Lds::NB;
     constexpr int LPT = 2 * Tile::LOADS / WAVES;             // tile loads of a wavefront and stage
     constexpr int LPW = LPT + (HAS_MASK ? 1 : 0);
     typedef typename MmaW<T>::frag Frag;
@@ -95,11 +101,11 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_ro
         const int key0 = key0_at(i);
         const uint32_t to = lds0 + at;
         if constexpr (WAVES == 1) {
-            tile.request<LPT / 2>(Kg + (int64_t)key0 * E, 0, to);
-            tile.request<LPT / 2>(Vg + (int64_t)key0 * E, 0, to + Tile::BYTES);
+            tile.template request<LPT / 2>(Kg + (int64_t)key0 * E, 0, to);
+            tile.template request<LPT / 2>(Vg + (int64_t)key0 * E, 0, to + Tile::BYTES);
         } else {   // the first half of the wavefronts brings K, the others V
             const T* from = wave < WAVES / 2 ? Kg : Vg;
-            tile.request<LPT>(from + (int64_t)key0 * E, (wave & (WAVES / 2 - 1)) * LPT, to + (wave < WAVES / 2 ? 0 : Tile::BYTES));
+            tile.template request<LPT>(from + (int64_t)key0 * E, (wave & (WAVES / 2 - 1)) * LPT, to + (wave < WAVES / 2 ? 0 : Tile::BYTES));
         }
         if constexpr (HAS_MASK)
             lds_direct_load16_at(mask + mask_column(i, key0), (lane >> 1) * mask_ld + (lane & 1) * 16, to + Lds::MASK + wave * 1024);
@@ -139,7 +145,7 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_ro
     // the slots are constants, so the offsets of the LDS reads are too
     auto step = [&](int i, auto slot) {
         constexpr int at = slot * Lds::STAGE, fill = (slot + NB - 1) % NB * Lds::STAGE;
-        if (i + 1 < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
+        if (NB > 2 && i + 1 < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();   // stage i has landed, stage i - 1 has been read
         const char* kt = smem + at;
@@ -148,9 +154,9 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_ro
 
         f32x16 s = s0, dp = dp0;
 #pragma unroll
-        for (int c = 0; c < EC; ++c) s = MmaW<T>::mma(tile.row_frag<Frag>(kt, c), qf[c], s);
+        for (int c = 0; c < EC; ++c) s = MmaW<T>::mma(tile.template row_frag<Frag>(kt, c), qf[c], s);
 #pragma unroll
-        for (int c = 0; c < EC; ++c) dp = MmaW<T>::mma(tile.row_frag<Frag>(vt, c), gf[c], dp);
+        for (int c = 0; c < EC; ++c) dp = MmaW<T>::mma(tile.template row_frag<Frag>(vt, c), gf[c], dp);
 #pragma unroll
         for (int j = 0; j < 16; ++j) s[j] = __builtin_amdgcn_exp2f(F32S ? __builtin_fmaf(s[j], c2, -lse) : s[j]);
         if constexpr (HAS_MASK) {
@@ -174,12 +180,13 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_ro
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int t = 0; t < ET; ++t) qacc[t] = MmaW<T>::mma(tile.tr_frag<Frag>(kt, t, u), sf[u], qacc[t]);
+            for (int t = 0; t < ET; ++t) qacc[t] = MmaW<T>::mma(tile.template tr_frag<Frag>(kt, t, u), sf[u], qacc[t]);
     };
     for (int i = 0; i < n; i += NB) {
         step(i, std::integral_constant<int, 0>());
         if (i + 1 < n) step(i + 1, std::integral_constant<int, 1>());
-        if (i + 2 < n) step(i + 2, std::integral_constant<int, 2>());
+        if constexpr (NB > 2)
+            if (i + 2 < n) step(i + 2, std::integral_constant<int, 2>());
     }
     __syncthreads();   // the tiles are dead: their space carries the output rows
     store_rows32<T, E>(smem + wave * (32 * (E * 2 + 16)), reinterpret_cast<T*>(p.grad_q) + (b * p.Nt + row0) * E, qacc, lane);
@@ -189,8 +196,8 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_ro
 template <typename T, int WAVES, bool HAS_MASK>
 __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_col_wide_kernel(AttnParams p, int nbc, int log_sub, int batch) {
     typedef AttnTile<64> Tile;
-    typedef BwdLds<WAVES, HAS_MASK, true> Lds;
-    constexpr int E = 64, EC = Tile::EC, ET = Tile::ET, NB = kBwdStages;
+    typedef BwdLds<64, WAVES, HAS_MASK, true> Lds;
+    constexpr int E = 64, EC = Tile::EC, ET = Tile::ET, NB = Lds::NB;
     constexpr int LPT = 2 * Tile::LOADS / WAVES;
     constexpr int LPW = LPT + 1 + (HAS_MASK ? 1 : 0);
     typedef typename MmaW<T>::frag Frag;
@@ -378,21 +385,21 @@ __global__ __launch_bounds__(64 * WAVES, HAS_MASK ? 2 : 3) void attention_bwd_co
     store_rows32<T, E>(rows, reinterpret_cast<T*>(p.grad_k) + out, kacc, lane);
 }
 
-template <typename T, int WAVES, bool HAS_MASK, bool F32S>
+template <typename T, int E, int WAVES, bool HAS_MASK, bool F32S>
 static int launch_bwd_row_wide_inst(const AttnParams& p, int batch, int BW, hipStream_t st) {
-    constexpr int smem = BwdLds<WAVES, HAS_MASK, false>::TOTAL;
+    constexpr int smem = BwdLds<E, WAVES, HAS_MASK, false>::TOTAL;
     const int nbr = p.Nt / p.BH;
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbr;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
-    SPX_GRANT_LDS((attention_bwd_row_wide_kernel<T, WAVES, HAS_MASK, F32S>), smem, "attention_bwd_row_wide_kernel");
-    hipLaunchKernelGGL((attention_bwd_row_wide_kernel<T, WAVES, HAS_MASK, F32S>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, ilog2(BW / 32), batch);
+    SPX_GRANT_LDS((attention_bwd_row_wide_kernel<T, E, WAVES, HAS_MASK, F32S>), smem, "attention_bwd_row_wide_kernel");
+    hipLaunchKernelGGL((attention_bwd_row_wide_kernel<T, E, WAVES, HAS_MASK, F32S>), dim3((unsigned)groups), dim3(64 * WAVES), smem, st, p, nbr, ilog2(BW / 32), batch);
     SPX_LAUNCH_CHECK("attention_bwd_row_wide_kernel");
     return 0;
 }
 
 template <typename T, int WAVES, bool HAS_MASK>
 static int launch_bwd_col_wide_inst(const AttnParams& p, int batch, int BW, hipStream_t st) {
-    constexpr int smem = BwdLds<WAVES, HAS_MASK, true>::TOTAL;
+    constexpr int smem = BwdLds<64, WAVES, HAS_MASK, true>::TOTAL;
     const int nbc = p.Ns / BW;
     const int64_t groups = ((int64_t)batch + 7) / 8 * 8 * nbc;
     if (groups > 0x7fffffff) return fail(SPX_E_SHAPE, "too many workgroups (%lld)", (long long)groups);
@@ -403,15 +410,17 @@ static int launch_bwd_col_wide_inst(const AttnParams& p, int batch, int BW, hipS
 }
 
 template <typename T>
-static int launch_bwd_row_wide_typed(const AttnParams& p, int batch, int BW, bool fp32_scores, hipStream_t st) {
+static int launch_bwd_row_wide_typed(const AttnParams& p, int batch, int BW, int E, bool fp32_scores, hipStream_t st) {
 #define SPX_BWD_CASE(bh)                                                                                   \
-    if (p.BH == bh)                                                                                        \
-        return p.mask        ? launch_bwd_row_wide_inst<T, bh / 32, true, true>(p, batch, BW, st)          \
-               : fp32_scores ? launch_bwd_row_wide_inst<T, bh / 32, false, true>(p, batch, BW, st)         \
-                             : launch_bwd_row_wide_inst<T, bh / 32, false, false>(p, batch, BW, st);
+    if (p.BH == bh && E == 64)                                                                             \
+        return p.mask        ? launch_bwd_row_wide_inst<T, 64, bh / 32, true, true>(p, batch, BW, st)      \
+               : fp32_scores ? launch_bwd_row_wide_inst<T, 64, bh / 32, false, true>(p, batch, BW, st)     \
+                             : launch_bwd_row_wide_inst<T, 64, bh / 32, false, false>(p, batch, BW, st);   \
+    if (p.BH == bh && E == 128 && p.mask) return launch_bwd_row_wide_inst<T, 128, bh / 32, true, true>(p, batch, BW, st);
     SPX_BWD_CASE(32) SPX_BWD_CASE(64)
 #undef SPX_BWD_CASE
-    return fail(SPX_E_CONFIG, "the attention backward kernel does not cover query blocks of %d", p.BH);
+    if (p.BH == 64 && E == 128 && fp32_scores) return launch_bwd_row_wide_inst<T, 128, 2, false, true>(p, batch, BW, st);
+    return fail(SPX_E_CONFIG, "the attention backward kernel does not cover query blocks of %d with head dim %d", p.BH, E);
 }
 
 template <typename T>
@@ -424,9 +433,9 @@ static int launch_bwd_col_wide_typed(const AttnParams& p, int batch, int BW, hip
     return fail(SPX_E_CONFIG, "the attention backward kernel does not cover key blocks of %d", BW);
 }
 
-int launch_attention_bwd_row_wide(int dtype, const AttnParams& p, int batch, int BW, bool fp32_scores, hipStream_t st) {
-    if (dtype == SPX_F16) return launch_bwd_row_wide_typed<_Float16>(p, batch, BW, fp32_scores, st);
-    return launch_bwd_row_wide_typed<bf16_t>(p, batch, BW, fp32_scores, st);
+int launch_attention_bwd_row_wide(int dtype, const AttnParams& p, int batch, int BW, int E, bool fp32_scores, hipStream_t st) {
+    if (dtype == SPX_F16) return launch_bwd_row_wide_typed<_Float16>(p, batch, BW, E, fp32_scores, st);
+    return launch_bwd_row_wide_typed<bf16_t>(p, batch, BW, E, fp32_scores, st);
 }
 
 int launch_attention_bwd_col_wide(int dtype, const AttnParams& p, int batch, int BW, hipStream_t st) {

@@ -114,10 +114,10 @@ class SparseAttention(OperatorBase):
         fused: run the single fused forward kernel when autograd is not recording
             (default True).  The three-operator pipeline is always built as well and
             is used whenever gradients are needed.
-        recompute: with a mask that is uniform inside its blocks, or with head dim 64, train
+        recompute: with a mask that is uniform inside its blocks, or with blocks of 32 / 64, train
             without storing the probabilities (default True): the backward kernels recompute
-            them from q, k and one number per query.  Masks with partly live blocks and other
-            head dims, and `recompute=False`, keep the probabilities of the live blocks for the backward pass.
+            them from q, k and one number per query.  Masks with partly live blocks of other
+            shapes, and `recompute=False`, keep the probabilities of the live blocks for the backward pass.
         fused_tile_cfg: tile configuration of the fused kernel (0 = the library's choice;
             see spx_tile_cfg_info for the others).
 
@@ -186,14 +186,14 @@ class SparseAttention(OperatorBase):
 
     def _recompute_supported(self, query: torch.Tensor) -> bool:
         """The kernels that recompute the probabilities cover 3-D 16-bit inputs and the block
-        shapes of both backward kernels, with head dim 64 element masks as well, and walk both indexes."""
+        shapes of both backward kernels, element masks over blocks of 32 / 64 as well, and walk both indexes."""
         indexes = self._sparse_port.indexes
         BH, BW, E = indexes.block_H, indexes.block_W, query.shape[-1]
         return (query.dim() == 3 and BH in (32, 64, 128) and BW in (32, 64, 128) and E in (64, 128)
                 and BW * E // 8 >= BH * 4 and BH * E >= 32 * BW and BH <= 2 * BW
                 and getattr(indexes, 'col_ptr', None) is not None and getattr(indexes, 'row_ptr', None) is not None
                 and (self._element_mask() is None
-                     or (E == 64 and max(BH, BW) <= 64 and query.shape[0] * self._Nt >= _MASKED_RECOMPUTE_QUERIES
+                     or (max(BH, BW) <= 64 and BW * E <= 128 * BH and query.shape[0] * self._Nt >= _MASKED_RECOMPUTE_QUERIES
                          and self._element_mask().data_ptr() % 16 == 0)))   # (else its forward kernel scales the scores to 16 bits)
 
     def _check_operands(self, what: str, indexes, batch: int, E: int, q_like=(), kv_like=(), rows=(),

@@ -259,3 +259,46 @@ def test_element_mask_that_is_not_aligned(gpu, H=16, N=256):
     att.update_mask(odd)
     assert att._element_mask().data_ptr() % 16 == 4 and not att._recompute_supported(leaves[0])
     check(step(att, leaves, g.to(gpu)), exact(leaves, g.to(gpu), torch.from_numpy(mask).to(gpu)), torch.bfloat16, 'at an odd place')
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('H,Nt,Ns,bh,bw,elements', [
+    (9, 256, 512, 32, 32, True), (9, 256, 512, 64, 64, True), (8, 256, 512, 64, 32, True),   # element masks; whole groups of 8 heads and not
+    (2, 1024, 2112, 32, 32, True),                                                           # more than 64 entries to a block row
+    (75, 512, 256, 64, 64, False), (74, 512, 256, 64, 32, False)])                           # 600 workgroups on the row side, and 592
+def test_head_dim_128(dtype, H, Nt, Ns, bh, bw, elements, gpu, E=128):
+    """Element masks: row side with 32 queries per wavefront, column side with 16 keys; partly live blocks, queries and keys
+    without any, values other than one, large scores.  Block-level masks next to the size from which the row side changes."""
+    rng = np.random.default_rng(19)
+    mask = block_mask(Nt, Ns, bh, bw, 1, density=0.97 if Ns > 2048 else 0.4)
+    if elements:
+        mask *= (rng.random((Nt, Ns)) < 0.7).astype(np.uint8)
+        mask[:, 5 * bw // 4:] |= np.tril(block_mask(Nt, Ns, bh, bw, 2))[:, 5 * bw // 4:]
+        mask[bh + 3] = 0
+        mask[:, 7] = 0
+        mask[bh:, 40:60] *= 2
+    q, k, v, g = (randn(s, i, dtype)[1] for i, s in enumerate([(H, Nt, E), (H, Ns, E), (H, Ns, E), (H, Nt, E)]))
+    att, leaves = build(mask, bh, bw, q * 4, k, v, gpu)
+    assert att._recompute_supported(leaves[0]) and (att._element_mask() is not None) == elements
+    got = step(att, leaves, g.to(gpu))
+    check(got, exact(leaves, g.to(gpu), torch.from_numpy(mask).to(gpu)), dtype, f'{dtype} {bh}x{bw}')
+    if not elements:
+        return
+    assert float(got[0][:, bh + 3].abs().max()) == 0.0 and float(got[1][:, 7].abs().max()) == 0.0
+    # the mask itself, and an index by column, at the C entry points
+    from sparta_amd import _lib
+    q, k, v, g = (t.detach() for t in (*leaves, g.to(gpu)))
+    indexes, whole = att._sparse_port.indexes, att._element_mask()
+    out, lse = att._fused_forward_lse(q, k, v)
+    grad_q, dot = torch.empty_like(q), torch.empty_like(lse)
+    lib, ptr, code = _lib.load(), _lib.dev_ptr, _lib.dtype_code(dtype)
+    sizes = (float(att._inv_temperature), H, Nt, Ns, E, bh, bw, _lib.current_stream(gpu))
+    _lib.check(lib.spx_attention_backward_q_masked(code, ptr(g), ptr(out), ptr(q), ptr(k), ptr(v), ptr(lse), ptr(grad_q), ptr(dot),
+                                                   ptr(indexes.row_ptr), ptr(indexes._bcsr_buf), ptr(whole), *sizes), 'masked')
+    assert torch.equal(grad_q.double(), got[0])
+    by_column = indexes.function_context.__class__(bh, bw, False, True).build_indexes(whole)
+    for data, call in ((whole, lib.spx_attention_backward_kv_masked), (by_column.convert(whole), lib.spx_attention_backward_kv_live_mask)):
+        grad_k, grad_v = torch.empty_like(k), torch.empty_like(v)
+        _lib.check(call(code, ptr(g), ptr(q), ptr(k), ptr(v), ptr(lse), ptr(dot), ptr(grad_k), ptr(grad_v), ptr(by_column.col_ptr),
+                        ptr(by_column._bcsc_buf), _lib.IDX_BCSC_I32, ptr(data), *sizes), 'masked')
+        assert torch.equal(grad_k.double(), got[1]) and torch.equal(grad_v.double(), got[2])
