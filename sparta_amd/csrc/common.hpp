@@ -228,5 +228,11 @@ __device__ __forceinline__ void store16_stream(void* p, const vec16& v) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(p));
 }
+// Results that the next launch reads: written through the L2 at once, so that they neither wait in it for their eviction nor go
+// past the last-level cache as non-temporal ones do.  (Two wait states, for the data registers of a store of four.)
+__device__ __forceinline__ void store16_through(void* p, const vec16& v) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(u32x4{v.x, v.y, v.z, v.w}));
+}
 
 }  // namespace spx

@@ -399,7 +399,12 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
             at = at + STAGE == NB * STAGE ? 0 : at + STAGE;
         }
         // ---- epilogue: the tile meets in LDS in the orientation of the output and leaves as whole 16-byte
-        // vectors of contiguous rows
+        // vectors of contiguous rows.  16-bit rows of 64 bytes with an activation, i.e. the operand of the next product, are
+        // written through to the last-level cache, which non-temporal stores go past: dynamic feed-forward blocks of 8192 x
+        // 768 -> 3072 -> 768 fp16 21.1 + 19.1 -> 20.0 + 14.4 us, 4096 x 1024 -> 4096 17.0 + 16.6 -> 16.9 + 13.7, 2767 x 512 -> 1024 7.0 + 5.4 ->
+        // 6.7 + 4.6; not where the XCDs share out the columns of a panel in small parts, and with them the lines of a row (2314 x 704 -> 1408,
+        // eight parts, 9.6 + 8.6 -> 10.4 + 9.0).  Results without one keep the non-temporal hint, which a product alone gains 1 - 3 % from
+        // (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
         if (cur.n_st == 0) __syncthreads();
         constexpr int ROWS = LDS.rows, LDE = LDS.pitch;
 #pragma unroll
@@ -420,15 +425,20 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
             }
         __syncthreads();
         constexpr int CPR = LDS.cols / E16;   // 16-byte vectors per row
+        constexpr bool THROUGH = ES == 2 && BN == 32 && SWAP && DK && SK;
+        auto leave = [&](auto through) __attribute__((always_inline)) {
 #pragma unroll
-        for (int v0 = 0; v0 < ROWS * CPR; v0 += 256) {
-            const int v = v0 + threadIdx.x;
-            const int row = v / CPR, c = v % CPR * E16;
-            const bool in = (ROWS * CPR % 256 == 0 || v < ROWS * CPR) && cur.m0 + (SWAP ? row : c) < p.Mc;
-            T* dst = SWAP ? out + (int64_t)(cur.m0 + row) * p.o_ld + (int64_t)cur.j * BN + c
-                          : out + ((int64_t)cur.j * BN + row) * p.o_ld + cur.m0 + c;
-            if (in) store16_stream(dst, *reinterpret_cast<const vec16*>(tileT + row * LDE + c));
-        }
+            for (int v0 = 0; v0 < ROWS * CPR; v0 += 256) {
+                const int v = v0 + threadIdx.x;
+                const int row = v / CPR, c = v % CPR * E16;
+                const bool in = (ROWS * CPR % 256 == 0 || v < ROWS * CPR) && cur.m0 + (SWAP ? row : c) < p.Mc;
+                T* dst = SWAP ? out + (int64_t)(cur.m0 + row) * p.o_ld + (int64_t)cur.j * BN + c
+                              : out + ((int64_t)cur.j * BN + row) * p.o_ld + cur.m0 + c;
+                if (in) (through ? store16_through : store16_stream)(dst, *reinterpret_cast<const vec16*>(tileT + row * LDE + c));
+            }
+        };
+        if (THROUGH && p.relu && l.parts_log2 <= 1) leave(std::true_type());
+        else leave(std::false_type());
     }
 }
 

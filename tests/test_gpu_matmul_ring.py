@@ -35,6 +35,16 @@ def test_ring_rows_and_rounds(tile_cfg, dtype, blocks, gpu):
                  sparsity=0.8, seed=M, tile_cfg=tile_cfg, activation='relu' if M % 2 else None)
 
 
+@pytest.mark.parametrize('tile_cfg', [11, 12])
+@pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 32, 64))])
+def test_ring_results_with_an_activation(tile_cfg, dtype, blocks, gpu):
+    """64-byte row pieces that are written through the L2s: panels in one part, in two, in four and in eight (where they are
+    not), rows that end inside a tile."""
+    for M in (1024, 2200, 1090, 65):
+        run_case(gpu, 'dsd', False, True, True, M != 2200, dtype, blocks, batch=1, M=M, K=192, N=544, gran=(blocks[2], blocks[1]),
+                 sparsity=0.7, seed=M, tile_cfg=tile_cfg, activation='relu')
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
 @pytest.mark.parametrize('M,N,batch', [(512, 1024, 1), (512, 1056, 1), (480, 512, 2), (480, 544, 2), (2000, 96, 1), (65, 5120, 1), (320, 5152, 1)])
 def test_ring_one_tile_to_a_workgroup(M, N, batch, dtype, gpu, K=4096):
