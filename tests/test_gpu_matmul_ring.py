@@ -36,7 +36,7 @@ def test_ring_rows_and_rounds(tile_cfg, dtype, blocks, gpu):
 
 
 @pytest.mark.parametrize('tile_cfg', [11, 12])
-@pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 32, 64))])
+@pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 64, 32))])
 def test_ring_results_with_an_activation(tile_cfg, dtype, blocks, gpu):
     """64-byte row pieces that are written through the L2s: panels in one part, in two, in four and in eight (where they are
     not), rows that end inside a tile."""
