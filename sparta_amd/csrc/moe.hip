@@ -472,7 +472,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(MoeParams p) {
         for (int pass = 0; pass < 8; ++pass) {
             const int row = pass * 8 + (lane >> 3);
             const u32x4 v = *reinterpret_cast<const u32x4*>(ep + row * 128 + ((c ^ (row & 7)) << 4));
-            if (toks[pass] >= 0 && n < p.N) *reinterpret_cast<u32x4*>(out + (int64_t)toks[pass] * p.N + n) = v;
+            if (toks[pass] >= 0 && n < p.N) store16_through(out + (int64_t)toks[pass] * p.N + n, __builtin_bit_cast(vec16, v));
         }
     } else {
     int toks[4];
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(64 * WAVES, (TM + TN) * NBUF * KTB > 80 * 1024 ? 1 
         for (int pass = 0; pass < WR / 8; ++pass) {
             const int row = pass * 8 + (lane >> 3);
             const u32x4 v = *reinterpret_cast<const u32x4*>(ep + row * 128 + ((c ^ (row & 7)) << 4));
-            if (toks[pass] >= 0 && n < p.N) *reinterpret_cast<u32x4*>(out + (int64_t)toks[pass] * p.N + n) = v;
+            if (toks[pass] >= 0 && n < p.N) store16_through(out + (int64_t)toks[pass] * p.N + n, __builtin_bit_cast(vec16, v));
         }
     } else {
     int toks[MT];   // fetched together ahead of the stores, as above

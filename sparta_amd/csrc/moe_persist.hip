@@ -269,7 +269,7 @@ __global__ __launch_bounds__(kPersistThreads, 2) void moe_persist_kernel(MoePara
         stage(kind, act, std::integral_constant<int, 3>(), n_st - 1);
     };
     // lane holds out[m = i*32 + l32][n = t*32 + 8*jj + 4*h2 + q] in acc[i][t][4*jj + q]
-    auto store = [&](auto kind) __attribute__((always_inline)) {
+    auto store = [&](auto kind, auto through) __attribute__((always_inline)) {
         constexpr int TM = kind == 0 ? 256 : 128, TN = kind == 2 ? 128 : 256;
         typedef float f32x2 __attribute__((ext_vector_type(2)));
         const int lane = here(threadIdx.x) & 63, r16 = lane & 15;
@@ -310,8 +310,11 @@ __global__ __launch_bounds__(kPersistThreads, 2) void moe_persist_kernel(MoePara
                 const int n = cur.n0 + wn * (TN / 4) + t * 32 + chunk * 8;
 #pragma unroll
                 for (int x = 0; x < 2; ++x)
-                    if (row + 16 * x < cur.rows && n < p.N)
-                        *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.out) + (int64_t)tok[x] * p.N + n) = out[x];
+                    if (row + 16 * x < cur.rows && n < p.N) {
+                        T* const to = reinterpret_cast<T*>(p.out) + (int64_t)tok[x] * p.N + n;
+                        if constexpr (through) store16_through(to, __builtin_bit_cast(vec16, out[x]));
+                        else *reinterpret_cast<u32x4*>(to) = out[x];
+                    }
             }
         }
     };
@@ -319,7 +322,8 @@ __global__ __launch_bounds__(kPersistThreads, 2) void moe_persist_kernel(MoePara
         // a partly filled tile: wavefronts whose rows are all past its end bring their share of the stages only
         if (wm * ((kind == 0 ? 256 : 128) / WGM) < cur.rows) {
             walk(kind, std::true_type{});
-            store(kind);
+            if (nxt.kind < 0 && n_whole < 2) store(kind, std::true_type{});
+            else store(kind, std::false_type{});
             clear();
         } else {
             walk(kind, std::false_type{});
