@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void dds_share_kernel(DdsParams p, DdsSplit
 #pragma unroll
         for (int x = 0; x < MT; ++x)
 #pragma unroll
-            for (int y = 0; y < NT; ++y) *reinterpret_cast<f32x4*>(to + ((part * MT + x) * 16 + r16) * BN + y * 16 + g4 * 4) = acc[x][y];
+            for (int y = 0; y < NT; ++y) store16_through(to + ((part * MT + x) * 16 + r16) * BN + y * 16 + g4 * 4, __builtin_bit_cast(vec16, acc[x][y]));
         return;
     }
     T* const C = reinterpret_cast<T*>(p.C) + b * p.c_batch + (p.compressed ? (int64_t)e * (BM * BN) : (int64_t)bi * BM * p.N + (int64_t)bj * BN);

@@ -341,7 +341,7 @@ __global__ __launch_bounds__(256) void dds_split_kernel(DdsParams p, DdsSplit s)
         f32x4 sum = *reinterpret_cast<const f32x4*>(Ef + m * LDE + n);
 #pragma unroll
         for (int kp = 1; kp < W::KS; ++kp) sum += *reinterpret_cast<const f32x4*>(Ef + (kp * BM + m) * LDE + n);
-        *reinterpret_cast<f32x4*>(dstp + v * 4) = sum;
+        store16_through(dstp + v * 4, __builtin_bit_cast(vec16, sum));
     }
 }
 
