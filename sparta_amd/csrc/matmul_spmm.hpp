@@ -39,6 +39,7 @@ struct SpmmParams {
     int bias_on_m;       // bias indexed by canonical m instead of n
     int64_t d_batch, s_batch, o_batch, bias_batch;
     int relu;           // epilogue: negative results (after the bias) become zero
+    int sub_log2;       // ring kernel, one tile to a workgroup: log2 of the tiles side by side in a block-column
 };
 
 // Optional activation of the epilogue; NaN stays NaN (as torch.relu keeps it).

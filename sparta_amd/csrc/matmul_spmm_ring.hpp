@@ -152,9 +152,10 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
             e = list[r];
         } else if (place(r, mt, o)) {   // (through the scalar cache)
             e.m0 = mt * TM;
-            e.j = p.sched ? ((const_i32)p.sched)[o] : o;
-            e.e0 = ((const_i32)p.ptr)[e.j];
-            e.n_blk = ((const_i32)p.ptr)[e.j + 1] - e.e0;
+            const int sub = ONE ? p.sub_log2 : 0, j = p.sched ? ((const_i32)p.sched)[o >> sub] : o >> sub;
+            e.j = (j << sub) + (o & ((1 << sub) - 1));   // in tiles
+            e.e0 = ((const_i32)p.ptr)[j];
+            e.n_blk = ((const_i32)p.ptr)[j + 1] - e.e0;
         }
         t.n_blk = __builtin_amdgcn_readfirstlane(e.n_blk);
         t.m0 = __builtin_amdgcn_readfirstlane(e.m0);
@@ -197,7 +198,8 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
                 }
             }
         };
-        const int64_t sld = p.compressed ? (SK ? BK : BN) : p.s_ld;
+        const int sub = ONE ? p.sub_log2 : 0;
+        const int64_t sld = p.compressed ? (SK ? BK : BN << sub) : p.s_ld;
         uint32_t s_off[NS];
         int s_upper = 0;
 #pragma unroll
@@ -246,7 +248,8 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         };
         auto s_block = [&](int64_t ent, int ch) {
             const int k = (int)(ent & 0xffff) * BK + ch * KC;
-            if (p.compressed) return S + (ent >> 32) * (BK * BN) + (SK ? ch * KC : ch * KC * BN);
+            if (p.compressed)
+                return S + (ent >> 32) * (BK * BN << sub) + (ld.j & ((1 << sub) - 1)) * (SK ? BK * BN : BN) + (SK ? ch * KC : ch * KC * (BN << sub));
             return SK ? S + (int64_t)ld.j * BN * p.s_ld + k : S + (int64_t)k * p.s_ld + (int64_t)ld.j * BN;
         };
         auto issue = [&](uint32_t at) {   // the stage under the cursor into the slot at byte offset `at`
@@ -472,7 +475,13 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
 }
 
 template <typename T, int TM>
-int launch_spmm_ring_tile(const SpmmParams& p, int BN, int batch, hipStream_t st) {
+int launch_spmm_ring_tile(const SpmmParams& p0, int BN, int batch, hipStream_t st) {
+    SpmmParams p = p0;
+    p.sub_log2 = 0;
+    if constexpr (TM == 64) {
+        p.sub_log2 = ring_sub_log2((int)sizeof(T), BN, p.out_ncontig != 0, p.Mc, p.K, p.Nc, batch);
+        BN >>= p.sub_log2;
+    }
 #define SPX_RING_LAYOUT(bn, bk, dk, sk)                                                                     \
     if ((p.d_kcontig != 0) == dk && (p.s_kcontig != 0) == sk)                                               \
         return p.out_ncontig ? launch_spmm_ring_inst<T, TM, bn, bk, dk, sk, true>(p, batch, st)             \

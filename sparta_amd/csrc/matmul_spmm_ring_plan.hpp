@@ -126,4 +126,19 @@ constexpr RingLaunch ring_launch(int elem_bytes, int TM, int BN, bool swap, int 
     return ring_launch_of(l, lds, per_cu, batch);
 }
 
+// 64-row tiles, log2 of the parts that a block-column is cut into, each a tile of its own, where every tile then still has a
+// workgroup to itself.  fp32: as narrow as it gets, a tile's MFMAs are most of its time (64 x 64 blocks at 30 - 40 %, us: 52 x 1600 -> 3584
+// 20.9, in halves 13.6, in quarters 10.4; gradients of the input 64 x 2688 -> 1408 24.9 / 15.1 / 12.8, 304 x 1856 -> 1088 21.7 / 13.8 /
+// 12.8; 1024^3 at 20 % 12.4 / 10.4 / 9.9; 32 x 64 blocks 903 x 3200 -> 512 12.4 / 11.8; no size behind).  16-bit types: 64-wide blocks in
+// halves, where that fills idle CUs (1 x 1024 -> 4096 (64 tiles) 7.0 / 5.8, 109 x 2944 -> 576 9.5 / 8.4, 185 x 1536 -> 1728 (81) 6.0 / 5.4;
+// 129 x 640 -> 2688 (126) 4.1 / 4.5, 208 x 2432 -> 3264 (204) 10.2 / 11.0; 32-wide blocks lose, 304 x 896 -> 2944 7.8 / 8.3).
+constexpr int ring_sub_log2(int elem_bytes, int BN, bool swap, int Mc, int K, int Nc, int batch) {
+    int sub = elem_bytes == 4 ? (BN == 64 ? 2 : BN == 32 ? 1 : 0) : BN == 64 && (int64_t)((Mc + 63) / 64) * (Nc / BN) * batch <= 96 ? 1 : 0;
+    for (; sub > 0; --sub) {
+        const RingLaunch l = ring_launch(elem_bytes, 64, BN >> sub, swap, Mc, K, Nc, batch);
+        if (l.n_pos == l.n_list) break;
+    }
+    return sub;
+}
+
 }  // namespace spx

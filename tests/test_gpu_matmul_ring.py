@@ -35,6 +35,23 @@ def test_ring_rows_and_rounds(tile_cfg, dtype, blocks, gpu):
                  sparsity=0.8, seed=M, tile_cfg=tile_cfg, activation='relu' if M % 2 else None)
 
 
+@pytest.mark.parametrize('mode,compressed', [('dsd', True), ('dsd', False), ('sdd', True), ('sdd', False)])
+@pytest.mark.parametrize('dtype,wide,rows,columns,tile', [
+    # fp32: quarters, halves and whole block-columns as the workgroups allow (four to a CU with 16-wide tiles); one row
+    (torch.float32, 64, 1000, 16, 16), (torch.float32, 64, 1000, 17, 32), (torch.float32, 64, 1024, 65, 64),
+    (torch.float32, 32, 1000, 32, 16), (torch.float32, 32, 1000, 33, 32), (torch.float32, 64, 8, 3, 16), (torch.float32, 16, 200, 5, 16),
+    # 16-bit types: halves of 64-wide block-columns up to 96 tiles
+    (torch.float16, 64, 200, 24, 32), (torch.bfloat16, 64, 200, 25, 64), (torch.bfloat16, 64, 8, 96, 32), (torch.float16, 32, 200, 3, 32)])
+def test_ring_parts_of_a_block_column(mode, compressed, dtype, wide, rows, columns, tile, gpu):
+    """64-row tiles narrower than the blocks: both sides of the sizes from which a block-column is cut, both storages of the
+    sparse operand, either way round, with bias."""
+    blocks = (32, 64, wide) if mode == 'dsd' else (wide, 64, 32)
+    M, N = (rows, wide * columns) if mode == 'dsd' else (wide * columns, rows)
+    _, names = launched_kernels(lambda: run_case(gpu, mode, False, mode == 'dsd', True, compressed, dtype, blocks, batch=1, M=M, K=192, N=N,
+                                                 gran=(wide, 64), sparsity=0.4, seed=rows + columns, tile_cfg=11))
+    assert [n[1] for n in template_numbers(names, 'spmm_ring_kernel')] == [tile]
+
+
 @pytest.mark.parametrize('tile_cfg', [11, 12])
 @pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 64, 32))])
 def test_ring_results_with_an_activation(tile_cfg, dtype, blocks, gpu):
