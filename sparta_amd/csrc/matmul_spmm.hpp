@@ -367,7 +367,11 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
                                   (tiles64 >= 700 || (tiles64 >= 512 && stored <= 20 * (int64_t)nb));
             // wide results of 2048 to 3072 rows: 256-row tiles do not come out even (256-row kernel / ring 2474 x
             // 1408 x 3328 at 28 % 31.0 / 23.3, 2518 x 1088 x 3776 28.7 / 21.9, 2579 x 2624 x 2048 37.9 / 30.4, 2520 x 2112 x 2240 at 13 % 18.9 / 15.7)
-            const bool mid_rows = sizeof(T) == 2 && BN == 32 && p.Mc > 2048 && p.Mc <= 3072 && p.Nc >= 2048;
+            // ... and neither do five and six of them over eight XCDs (256-row kernel / ring, us: 1256 x 3200 x 3488 at 21 % 33.8 / 22.9, 1503 x 1280 x
+            // 3392 16.9 / 12.6, 1220 x 2496 x 3424 with 4.1 blocks to a column 10.6 / 8.9; seven 1606 x 2880 x 2688 15.0 / 17.3, shorter walks 1537 x
+            // 896 x 3616 7.5 / 8.1)
+            const bool mid_rows = sizeof(T) == 2 && BN == 32 && p.Nc >= 2048 &&
+                                  ((p.Mc > 2048 && p.Mc <= 3072) || (p.Mc > 1024 && p.Mc <= 1536 && stored >= 4 * (int64_t)nb));
             if (mid_rows) ring = rounds128 < rounds64 ? 12 : 11;   // (4 and 3 rounds 29.3 / 23.3; 3 each 41 / 51, 2626 x 3584 x 2688 at 24 %)
             if (fill) use_ring = ring_ok && cols >= 32 && (p.Nc < 2048 || mid_rows || (few_rows && p.Mc <= 1024));
             else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32 || few_rows);
@@ -392,6 +396,15 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         else if (use_ring) tile_cfg = ring;
         else if (split_columns) tile_cfg = 8;
         else if (panel_ok && p.Mc >= 512 && fill) tile_cfg = p.Mc >= 1024 ? 7 : 5;
+        // 16-bit blocks of 32 x 32, tiles that have a workgroup each: the ring kernel shares a walk out over more wavefronts than split
+        // columns do and brings it through LDS stages ahead.  Split columns / ring, us: 320 x 1024 -> 1472 at 16 % 6.7 / 4.5, 80 x 1792 ->
+        // 1856 5.9 / 4.4, 592 x 2880 -> 1536 at 27 % 15.0 / 10.6, 401 x 1152 -> 1344 at 26 % 7.1 / 5.9; longer walks in more tiles 368 x 2496 ->
+        // 1472 at 36 % 8.9 / 10.1, 832 x 3136 -> 896 at 40 % 12.8 / 14.9.  No split (below) / ring: 192 x 896 -> 1408 at 26 % 5.7 / 4.5, 64 x 704 -> 1856
+        // 5.3 / 4.5, but 28 x 960 -> 2816 4.2 / 4.5, 3 x 3328 -> 1728 3.9 / 5.7 and five blocks to a column 87 x 576 -> 3136 4.4 / 5.2.  Where the live blocks are not counted, up to 64 places to a column (277 x 3840 -> 960 at 24 % 8.8 / 10.0).
+        else if (sizeof(T) == 2 && ring_ok && kcontig && two_blocks && BN == 32 && !fill && p.Mc > 32 && tiles64 <= 512 &&
+                 (tiles64 <= 256 || stored <= 26 * (int64_t)nb) && (p.compressed || cols <= 64) &&
+                 (p.Mc <= 256 && cols <= 32 ? stored >= 6 * (int64_t)nb : cols >= 8 && stored >= 4 * (int64_t)nb))
+            tile_cfg = 11;
         // few rows and short columns: no barrier and no shared block pays (64 x 768 x 3072 bf16: 3.9 us
         // against 4.4 with the columns split and 5.2 through the ring)
         else if (kcontig && (p.Mc <= 16 ? cols <= 128 : p.Mc <= 256 && cols <= 32)) tile_cfg = 3;

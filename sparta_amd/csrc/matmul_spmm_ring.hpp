@@ -78,9 +78,11 @@ __device__ __forceinline__ Frag ring_frag(const char* part, int row0, int half, 
     }
 }
 
-// ONE: no workgroup has more than one tile.
-template <typename T, int TM, int BN, int BK, bool DK, bool SK, bool SWAP, bool ONE>
-__global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p, RingList l) {
+// ONE: no workgroup has more than one tile.  GROUPS (then only): so many times four multiplying wavefronts, a loader and a ring
+// share the blocks of the tile out; the first group adds up what the others hold.
+template <typename T, int TM, int BN, int BK, bool DK, bool SK, bool SWAP, bool ONE, int GROUPS = 1>
+__global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(SpmmParams p, RingList l) {
+    static_assert(GROUPS == 1 || (ONE && TM == 64), "the walk of a single 64-row tile is shared out");
     typedef typename PanelMma<T>::M MMA;
     typedef typename MMA::frag Frag;
     constexpr int ES = (int)sizeof(T), E16 = 16 / ES;
@@ -105,6 +107,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     typedef const __attribute__((address_space(4))) int32_t* const_i32;     // read through the scalar cache
     typedef const __attribute__((address_space(4))) int64_t* const_i64;
     extern __shared__ __align__(16) char smem[];
+    constexpr int TILE = GROUPS * NB * STAGE;   // the output tile, behind the rings
 
     const int nb = p.Nc / BN;
     // the tiles of this workgroup's XCD, and its place among the workgroups there
@@ -113,14 +116,17 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     if (pos >= share.n_list) return;
     const int64_t b = blockIdx.y;
     const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_of = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int group = GROUPS > 1 ? wave_of / 5 : 0, wave = GROUPS > 1 ? wave_of % 5 : wave_of;
+    char* const ring = smem + group * (NB * STAGE);
 
     const int n_rounds = ONE ? 1 : share.n_rounds;
     const bool listed = !ONE && share.listed, table = listed && nb <= kRingTableMax;
     RingTile* const list = reinterpret_cast<RingTile*>(smem + LDS.list);
     struct Tile {
-        int m0, j, e0, n_blk, n_st;
+        int m0, j, e0, n_blk, n_st, n_bar;   // n_bar: stages of the group that has most
     };
+    auto stages = [](int n_blk) { return PAIR ? (n_blk + 1) >> 1 : n_blk * SPB; };
     // launch order and column pointers while the list is made: in the ring, which is empty yet
     int* const tab_ptr = reinterpret_cast<int*>(smem);
     int* const tab_order = tab_ptr + nb + 1;
@@ -161,8 +167,17 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         t.m0 = __builtin_amdgcn_readfirstlane(e.m0);
         t.j = __builtin_amdgcn_readfirstlane(e.j);
         t.e0 = __builtin_amdgcn_readfirstlane(e.e0);
-        t.n_st = PAIR ? (t.n_blk + 1) >> 1 : t.n_blk * SPB;
-        return t.n_blk >= 0;
+        const bool exists = t.n_blk >= 0;
+        if constexpr (GROUPS > 1) {
+            const int most = (t.n_blk + GROUPS - 1) / GROUPS, first = group * most;
+            t.n_bar = stages(most);
+            t.e0 += first;
+            t.n_blk = t.n_blk - first < most ? t.n_blk - first : most;
+            if (t.n_blk < 0) t.n_blk = 0;
+        }
+        t.n_st = stages(t.n_blk);
+        if constexpr (GROUPS == 1) t.n_bar = t.n_st;
+        return exists;
     };
 
     // Barriers, the same sequence in every wavefront: one per stage (its data has landed, and the slot
@@ -173,7 +188,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         // ---- the loader --------------------------------------------------------------------------------
         const T* D = reinterpret_cast<const T*>(p.D) + b * p.d_batch;
         const T* S = reinterpret_cast<const T*>(p.S) + b * p.s_batch;
-        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
         constexpr int USH = ES == 2 ? 5 : 6;   // log2 of a unit
         // byte offsets of this lane in the load instructions of the dense part, from the tile's first row
         // (column) and the stage's k; they fit 32 bits (checked on the host)
@@ -301,8 +316,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         for (int r = 0; r < n_rounds; ++r) {
             Tile cur;
             if (!tile_at(r, cur)) continue;
-            const int n_st = cur.n_st;
-            for (int st = 0; st < n_st; ++st) {
+            for (int st = 0; st < cur.n_bar; ++st) {
                 // the stage has landed; the ones behind it may still be on their way
                 if (NB == 4 && ahead == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NL) : "memory");
                 else if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
@@ -316,7 +330,11 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
                 }
                 fill = fill + STAGE == NB * STAGE ? 0 : fill + STAGE;
             }
-            if (n_st == 0) __syncthreads();
+            if (cur.n_bar == 0) __syncthreads();
+            if constexpr (GROUPS > 1) {
+                __syncthreads();
+                __syncthreads();
+            }
             __syncthreads();
         }
         return;
@@ -326,7 +344,7 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
     const int r16 = lane & 15, g4 = lane >> 4;
     const T* biasT = p.bias ? reinterpret_cast<const T*>(p.bias) + b * p.bias_batch : nullptr;
     T* out = reinterpret_cast<T*>(p.out) + b * p.o_batch;
-    T* const tileT = reinterpret_cast<T*>(smem + NB * STAGE);
+    T* const tileT = reinterpret_cast<T*>(smem + TILE);
     f32x4 acc[MT][NT][CHAINS];
     struct Half {
         Frag a[MT], b[NT];
@@ -392,11 +410,12 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int c = 0; c < CHAINS; ++c) acc[i][t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int st = 0; st < cur.n_st; ++st) {
+        for (int st = 0; st < cur.n_bar; ++st) {
             __syncthreads();
+            if (GROUPS > 1 && st >= cur.n_st) continue;
             Half h0, h1;
-            fetch(smem + at, 0, h0);
-            fetch(smem + at, 1, h1);
+            fetch(ring + at, 0, h0);
+            fetch(ring + at, 1, h1);
             multiply(h0, std::integral_constant<int, 0>());
             if (!PAIR || 2 * st + 1 < cur.n_blk) multiply(h1, std::integral_constant<int, 1>());
             at = at + STAGE == NB * STAGE ? 0 : at + STAGE;
@@ -408,7 +427,30 @@ __global__ __launch_bounds__(kRingThreads, 3) void spmm_ring_kernel(SpmmParams p
         // 6.7 + 4.6; not where the XCDs share out the columns of a panel in small parts, and with them the lines of a row (2314 x 704 -> 1408,
         // eight parts, 9.6 + 8.6 -> 10.4 + 9.0).  Results without one keep the non-temporal hint, which a product alone gains 1 - 3 % from
         // (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
-        if (cur.n_st == 0) __syncthreads();
+        if (cur.n_bar == 0) __syncthreads();
+        if constexpr (GROUPS > 1) {
+            __syncthreads();   // the rings have been read: their space carries the sums of the other groups
+            f32x4* const part = reinterpret_cast<f32x4*>(smem) + wave * (NT * 64) + lane;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                f32x4& sum = acc[0][t][0];
+                if constexpr (CHAINS == 4) {
+                    sum = (sum + acc[0][t][1]) + (acc[0][t][2] + acc[0][t][3]);
+                    acc[0][t][1] = acc[0][t][2] = acc[0][t][3] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                if (group > 0) part[((group - 1) * 4 * NT + t) * 64] = sum;
+            }
+            __syncthreads();
+            if (group == 0) {
+#pragma unroll
+                for (int g = 0; g < GROUPS - 1; ++g)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[0][t][0] += part[(g * 4 * NT + t) * 64];
+            } else {
+                __syncthreads();
+                return;
+            }
+        }
         constexpr int ROWS = LDS.rows, LDE = LDS.pitch;
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -462,10 +504,20 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
         if (n_pos == launch.n_list) {
             SpmmParams q = p;
             if (n_pos * batch <= 32) q.sched = nullptr;   // one to a CU: the order is of no account, a trip to memory less
-            SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, true>), most, "spmm_ring_kernel");
-            hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, true>), dim3(8 * n_pos, batch, 1), dim3(kRingThreads), smem, st, q, l);
-            SPX_LAUNCH_CHECK("spmm_ring_kernel");
-            return 0;
+            // (where the live blocks are not counted, every eighth)
+            const int64_t columns = p.Nc / (BN << p.sub_log2), places = columns * (p.K / BK);
+            const int64_t blocks = p.compressed && p.s_batch > 0 ? p.s_batch / (BK * BN << p.sub_log2) : places / 8;
+            const int groups = ring_groups(ES, BN, SWAP, n_pos * batch, (double)blocks * BK * ES / (columns * 128));
+            const int lds = smem + (groups - 1) * ring_stages(ES) * LDS.stage;
+#define SPX_RING_GROUPS(n)                                                                                                                  \
+    if (groups == n) {                                                                                                                      \
+        SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, true, n>), kRingLdsOfCu, "spmm_ring_kernel");                          \
+        hipLaunchKernelGGL((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, true, n>), dim3(8 * n_pos, batch, 1), dim3(n * kRingThreads), lds, st, q, l); \
+        SPX_LAUNCH_CHECK("spmm_ring_kernel");                                                                                               \
+        return 0;                                                                                                                           \
+    }
+            SPX_RING_GROUPS(1) SPX_RING_GROUPS(2) SPX_RING_GROUPS(3)
+#undef SPX_RING_GROUPS
         }
     }
     SPX_GRANT_LDS((spmm_ring_kernel<T, TM, BN, BK, DK, SK, SWAP, false>), most, "spmm_ring_kernel");

@@ -140,5 +140,17 @@ constexpr int ring_sub_log2(int elem_bytes, int BN, bool swap, int Mc, int K, in
     }
     return sub;
 }
+// Groups of wavefronts that share the walk of a tile out, where each tile has a workgroup to itself: three where the workgroups have
+// a CU each, two where two share one (`n_pos`: workgroups of an XCD, 32 CUs).  stages: of a walk, on the average.  One, two and
+// three groups, us: fp16 64 x 64 blocks at 30 - 40 %, gradient of the input 416 x 4032 -> 1152 (126 tiles) 18.4 / 13.6 / 11.6, 416 x 1152 -> 4032 (441) 8.8 /
+// 7.0 / 11.2, 816 x 4032 -> 1472 (663) 11.4 / 12.8 / 16.5, 128 x 3392 -> 2816 12.0 / 9.0 / 8.2, 4 x 3264 -> 2112 9.5 / 7.2 / 6.6; bf16 32 x 32 blocks, gradient of
+// 304 x 2944 -> 896 15.2 / 9.8 / 8.4; fp32 46 x 4096 -> 960 at 34 % 15.4 / 12.4 / 12.0, 512 x 1408 -> 896 (448) 7.6 / 7.6 / 9.4, 304 x 1088 -> 1856 (580)
+// 10.5 / 11.4 / 13.6.  Walks of two stages: 288 x 2112 -> 2560 at 6 % 5.7 / - / 6.5.
+constexpr int ring_groups(int elem_bytes, int BN, bool swap, int n_pos, double stages) {
+    const RingLds lds = ring_lds(elem_bytes, 64, BN, swap);
+    int groups = stages < 2.5 ? 1 : n_pos <= 32 ? 3 : n_pos <= 64 ? 2 : 1;
+    while (groups > 1 && !ring_fits(lds.list + (groups - 1) * ring_stages(elem_bytes) * lds.stage, n_pos <= 32 ? 1 : 2)) --groups;
+    return groups;
+}
 
 }  // namespace spx

@@ -52,6 +52,28 @@ def test_ring_parts_of_a_block_column(mode, compressed, dtype, wide, rows, colum
     assert [n[1] for n in template_numbers(names, 'spmm_ring_kernel')] == [tile]
 
 
+@pytest.mark.parametrize('mode,transposed,compressed', [('dsd', True, True), ('dsd', False, True), ('dsd', True, False), ('sdd', False, True)])
+@pytest.mark.parametrize('dtype,wide,depth,columns,K,sparsity,groups', [
+    # eight panels of rows, a tile of every column to an XCD: 32 and 64 of them, and one more
+    (torch.float16, 32, 64, 32, 768, 0.6, 3), (torch.bfloat16, 32, 64, 33, 768, 0.6, 2), (torch.float16, 64, 64, 64, 768, 0.6, 2),
+    (torch.float16, 32, 64, 65, 768, 0.6, 1), (torch.float32, 16, 32, 32, 512, 0.6, 3), (torch.float32, 16, 64, 64, 512, 0.6, 2),
+    (torch.float32, 32, 32, 40, 512, 0.6, 1),     # halves: 80 tiles
+    # two blocks to a stage: odd walks, shares of one block, columns with fewer blocks than groups, and with none
+    (torch.float16, 32, 32, 20, 480, 0.5, 3), (torch.bfloat16, 32, 32, 50, 320, 0.4, 2), (torch.float32, 16, 16, 24, 240, 0.6, 3),
+    (torch.float16, 32, 64, 20, 640, 0.9, 1)])   # a stage or less to a walk: one group
+def test_ring_groups(mode, transposed, compressed, dtype, wide, depth, columns, K, sparsity, groups, gpu, rows=504):
+    """A walk shared out over groups of wavefronts: both sides of the sizes at which their number changes, with bias and rows
+    that end inside a tile."""
+    blocks = (32, depth, wide) if mode == 'dsd' else (wide, depth, 32)
+    M, N = (rows, wide * columns) if mode == 'dsd' else (wide * columns, rows)
+    _, names = launched_kernels(lambda: run_case(gpu, mode, False, transposed, True, compressed, dtype, blocks, batch=1, M=M, K=K, N=N,
+                                                 gran=(depth, wide) if mode == 'dsd' and not transposed else (wide, depth), sparsity=sparsity, seed=columns, tile_cfg=11))
+    numbers = template_numbers(names, 'spmm_ring_kernel')
+    assert len(numbers) == 1
+    if compressed:
+        assert numbers[0][-1] == groups, numbers
+
+
 @pytest.mark.parametrize('tile_cfg', [11, 12])
 @pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 64, 32))])
 def test_ring_results_with_an_activation(tile_cfg, dtype, blocks, gpu):
