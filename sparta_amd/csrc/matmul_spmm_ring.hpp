@@ -426,7 +426,10 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
         // written through to the last-level cache, which non-temporal stores go past: dynamic feed-forward blocks of 8192 x
         // 768 -> 3072 -> 768 fp16 21.1 + 19.1 -> 20.0 + 14.4 us, 4096 x 1024 -> 4096 17.0 + 16.6 -> 16.9 + 13.7, 2767 x 512 -> 1024 7.0 + 5.4 ->
         // 6.7 + 4.6; not where the XCDs share out the columns of a panel in small parts, and with them the lines of a row (2314 x 704 -> 1408,
-        // eight parts, 9.6 + 8.6 -> 10.4 + 9.0).  Results without one keep the non-temporal hint, which a product alone gains 1 - 3 % from
+        // eight parts, 9.6 + 8.6 -> 10.4 + 9.0).  The product itself takes up to a few percent longer where it has few rows or does not widen
+        // them (with the hint / through: 4096 x 768 -> 2304 10.8 / 11.5, 4000 x 1024 -> 4096 15.0 / 15.7, 8192 x 2048 -> 1024 19.1 / 20.1, 16384 x 1024 ->
+        // 1024 16.5 / 17.2; 8192 x 768 -> 3072 20.8 / 20.4, 8192 x 1024 -> 2048 at 15 % 17.5 / 17.7, at 35 % 28.2 / 26.9, 12345 x 1024 -> 2048 39.1 / 39.9), so
+        // these keep the hint: a first product of a feed-forward block is twice as wide as deep.  Results without one keep the non-temporal hint, which a product alone gains 1 - 3 % from
         // (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
         if (cur.n_bar == 0) __syncthreads();
         if constexpr (GROUPS > 1) {
@@ -483,7 +486,7 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
                 if (in) (through ? store16_through : store16_stream)(dst, *reinterpret_cast<const vec16*>(tileT + row * LDE + c));
             }
         };
-        if (THROUGH && p.relu && l.parts_log2 <= 1) leave(std::true_type());
+        if (THROUGH && p.relu && p.Mc > 5120 && p.Nc >= 2 * p.K && l.parts_log2 <= 1) leave(std::true_type());
         else leave(std::false_type());
     }
 }

@@ -77,9 +77,9 @@ def test_ring_groups(mode, transposed, compressed, dtype, wide, depth, columns, 
 @pytest.mark.parametrize('tile_cfg', [11, 12])
 @pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 64, 32))])
 def test_ring_results_with_an_activation(tile_cfg, dtype, blocks, gpu):
-    """64-byte row pieces that are written through the L2s: panels in one part, in two, in four and in eight (where they are
-    not), rows that end inside a tile."""
-    for M in (1024, 2200, 1090, 65):
+    """64-byte row pieces that are written through the L2s (over 5120 rows, panels in one part and in two) and that are not:
+    fewer rows, panels in four parts and in eight; rows that end inside a tile."""
+    for M in (1024, 2200, 1090, 65, 5130, 5600, 6100):
         run_case(gpu, 'dsd', False, True, True, M != 2200, dtype, blocks, batch=1, M=M, K=192, N=544, gran=(blocks[2], blocks[1]),
                  sparsity=0.7, seed=M, tile_cfg=tile_cfg, activation='relu')
 
