@@ -159,10 +159,11 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
             e = list[r];
         } else if (place(r, mt, o)) {   // (through the scalar cache)
             e.m0 = mt * TM;
-            const int sub = CUT ? p.sub_log2 : 0, j = p.sched ? ((const_i32)p.sched)[o >> sub] : o >> sub;
-            e.j = (j << sub) + (o & ((1 << sub) - 1));   // in tiles
-            e.e0 = ((const_i32)p.ptr)[j];
-            e.n_blk = ((const_i32)p.ptr)[j + 1] - e.e0;
+            const int sub = CUT ? p.sub_log2 : 0, column = o >> sub;
+            e.j = p.sched ? ((const_i32)p.sched)[column] : column;
+            e.e0 = ((const_i32)p.ptr)[e.j];
+            e.n_blk = ((const_i32)p.ptr)[e.j + 1] - e.e0;
+            if constexpr (CUT) e.j = (e.j << sub) + (o & ((1 << sub) - 1));   // in tiles
         }
         t.n_blk = __builtin_amdgcn_readfirstlane(e.n_blk);
         t.m0 = __builtin_amdgcn_readfirstlane(e.m0);
@@ -177,7 +178,6 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
             if (t.n_blk < 0) t.n_blk = 0;
         }
         t.n_st = stages(t.n_blk);
-        if constexpr (GROUPS == 1) t.n_bar = t.n_st;
         return exists;
     };
 
@@ -317,7 +317,8 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
         for (int r = 0; r < n_rounds; ++r) {
             Tile cur;
             if (!tile_at(r, cur)) continue;
-            for (int st = 0; st < cur.n_bar; ++st) {
+            const int n_bar = GROUPS > 1 ? cur.n_bar : cur.n_st;
+            for (int st = 0; st < n_bar; ++st) {
                 // the stage has landed; the ones behind it may still be on their way
                 if (NB == 4 && ahead == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NL) : "memory");
                 else if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
                 }
                 fill = fill + STAGE == NB * STAGE ? 0 : fill + STAGE;
             }
-            if (cur.n_bar == 0) __syncthreads();
+            if (n_bar == 0) __syncthreads();
             if constexpr (GROUPS > 1) {
                 __syncthreads();
                 __syncthreads();
@@ -411,7 +412,8 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int c = 0; c < CHAINS; ++c) acc[i][t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int st = 0; st < cur.n_bar; ++st) {
+        const int n_bar = GROUPS > 1 ? cur.n_bar : cur.n_st;
+        for (int st = 0; st < n_bar; ++st) {
             __syncthreads();
             if (GROUPS > 1 && st >= cur.n_st) continue;
             Half h0, h1;
@@ -429,9 +431,9 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
         // eight parts, 9.6 + 8.6 -> 10.4 + 9.0).  The product itself takes up to a few percent longer where it has few rows or does not widen
         // them (with the hint / through: 4096 x 768 -> 2304 10.8 / 11.5, 4000 x 1024 -> 4096 15.0 / 15.7, 8192 x 2048 -> 1024 19.1 / 20.1, 16384 x 1024 ->
         // 1024 16.5 / 17.2; 8192 x 768 -> 3072 20.8 / 20.4, 8192 x 1024 -> 2048 at 15 % 17.5 / 17.7, at 35 % 28.2 / 26.9, 12345 x 1024 -> 2048 39.1 / 39.9), so
-        // these keep the hint: a first product of a feed-forward block is twice as wide as deep.  Results without one keep the non-temporal hint, which a product alone gains 1 - 3 % from
-        // (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
-        if (cur.n_bar == 0) __syncthreads();
+        // these keep the hint: a first product of a feed-forward block is twice as wide as deep.  Results without an activation
+        // keep it too, a product alone gains 1 - 3 % from it (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
+        if (n_bar == 0) __syncthreads();
         if constexpr (GROUPS > 1) {
             __syncthreads();   // the rings have been read: their space carries the sums of the other groups
             f32x4* const part = reinterpret_cast<f32x4*>(smem) + wave * (NT * 64) + lane;
@@ -475,19 +477,24 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
         __syncthreads();
         constexpr int CPR = LDS.cols / E16;   // 16-byte vectors per row
         constexpr bool THROUGH = ES == 2 && BN == 32 && SWAP && DK && SK;
-        auto leave = [&](auto through) __attribute__((always_inline)) {
+        const bool through = THROUGH && p.relu && p.Mc > 5120 && p.Nc >= 2 * p.K && l.parts_log2 <= 1;
 #pragma unroll
-            for (int v0 = 0; v0 < ROWS * CPR; v0 += 256) {
-                const int v = v0 + threadIdx.x;
-                const int row = v / CPR, c = v % CPR * E16;
-                const bool in = (ROWS * CPR % 256 == 0 || v < ROWS * CPR) && cur.m0 + (SWAP ? row : c) < p.Mc;
-                T* dst = SWAP ? out + (int64_t)(cur.m0 + row) * p.o_ld + (int64_t)cur.j * BN + c
-                              : out + ((int64_t)cur.j * BN + row) * p.o_ld + cur.m0 + c;
-                if (in) (through ? store16_through : store16_stream)(dst, *reinterpret_cast<const vec16*>(tileT + row * LDE + c));
+        for (int v0 = 0; v0 < ROWS * CPR; v0 += 256) {
+            const int v = v0 + threadIdx.x;
+            const int row = v / CPR, c = v % CPR * E16;
+            const bool in = (ROWS * CPR % 256 == 0 || v < ROWS * CPR) && cur.m0 + (SWAP ? row : c) < p.Mc;
+            T* dst = SWAP ? out + (int64_t)(cur.m0 + row) * p.o_ld + (int64_t)cur.j * BN + c
+                          : out + ((int64_t)cur.j * BN + row) * p.o_ld + cur.m0 + c;
+            if (!in) continue;
+            const vec16 piece = *reinterpret_cast<const vec16*>(tileT + row * LDE + c);
+            if constexpr (THROUGH) {
+                if (through) {
+                    store16_through(dst, piece);
+                    continue;
+                }
             }
-        };
-        if (THROUGH && p.relu && p.Mc > 5120 && p.Nc >= 2 * p.K && l.parts_log2 <= 1) leave(std::true_type());
-        else leave(std::false_type());
+            store16_stream(dst, piece);
+        }
     }
 }
 
