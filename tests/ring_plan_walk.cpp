@@ -2,7 +2,9 @@
 // Input, a launch per line: elem_bytes TM BN swap M K N batch cover.  Output: slots, LDS bytes, the fewest and the most
 // tiles of a workgroup over the XCDs, the most LDS that a workgroup's list reaches to, where `cover` is set whether
 // every tile has exactly one workgroup (-1: not walked), the workgroups of the launch that are side by side on the chip
-// (over the batch), and how many the choice of a tile height counts on.
+// (over the batch), and how many the choice of a tile height counts on; then, for 64-row tiles (0 otherwise), the log2 of the
+// parts that a block-column is cut into, `cover` of that launch, whether each of its tiles has a workgroup to itself, the groups of
+// wavefronts that share a long walk there, the LDS of a workgroup with them, and how many of them a CU has to hold.
 #include <cstdio>
 #include <vector>
 #include "matmul_spmm_ring_plan.hpp"
@@ -42,8 +44,16 @@ int main() {
             const int end = ring_lds(es, TM, BN, swap != 0).list + (share.listed ? share.n_rounds * (int)sizeof(RingTile) : 0);
             if (end > reach) reach = end;
         }
-        std::printf("%d %d %d %d %d %d %d %d\n", launch.list.slots, launch.smem, fewest, most, reach,
+        const bool low = TM == 64;
+        const int sub = low ? ring_sub_log2(es, BN, swap != 0, M, K, N, batch) : 0, part = BN >> sub;
+        const RingLaunch cut = ring_launch(es, TM, part, swap != 0, M, K, N, batch);
+        const bool one = low && cut.n_pos == cut.n_list;
+        const int groups = one ? ring_groups(es, part, swap != 0, cut.n_pos * batch, 100.0) : 0;
+        const RingLds lds = ring_lds(es, TM, part, swap != 0);
+        std::printf("%d %d %d %d %d %d %d %d", launch.list.slots, launch.smem, fewest, most, reach,
                     cover ? covered(launch, N / BN) : -1, 8 * launch.n_pos * batch, ring_slots(es, TM, BN, swap != 0));
+        std::printf(" %d %d %d %d %d %d\n", sub, cover && low ? covered(cut, N / part) : -1, (int)one, groups,
+                    groups ? cut.smem + (groups - 1) * ring_stages(es) * lds.stage : 0, (cut.n_pos * batch + 31) / 32);
     }
     return 0;
 }

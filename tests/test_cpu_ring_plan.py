@@ -29,6 +29,12 @@ class Walk(NamedTuple):
     covered: int
     side_by_side: int
     counted_on: int
+    sub: int             # log2 of the parts of a block-column, 64-row tiles
+    parts_covered: int
+    alone: int           # each tile has a workgroup to itself
+    groups: int
+    groups_smem: int
+    groups_per_cu: int
 
 
 @pytest.fixture(scope='module')
@@ -88,6 +94,30 @@ def test_every_tile_has_one_workgroup(walk):
              for m in (1, 64, 65, 500, 1024, 3000, 4161, 8200, 20000, 70000)]
     for case, w in zip(cases, walk(cases, cover=True)):
         assert w.covered == 1, (case, w)
+
+
+def test_parts_of_a_block_column_and_groups_of_wavefronts(walk):
+    """A block-column is cut only into tiles that there are instances for and that have a workgroup each, each of them once; the
+    workgroups with several groups of wavefronts that share a CU fit its LDS."""
+    rng = random.Random(7)
+    cases = [(es, 64, BN, swap, rng.randint(1, 64) if rng.random() < 0.3 else int(2 ** rng.uniform(6, 13)), 64 * rng.randint(1, 64),
+              BN * int(2 ** rng.uniform(0, 7)), rng.choice([1, 1, 1, 2, 7, 40, 300]))
+             for es in (2, 4) for BN in (16, 32, 64) for swap in (0, 1) for _ in range(400)]
+    walks = walk(cases, cover=True)
+    for case, w in zip(cases, walks):
+        es, _, BN = case[:3]
+        assert w.parts_covered == 1, (case, w)
+        assert w.sub == 0 or (w.alone and BN >> w.sub >= (32 if es == 2 else 16)), (case, w)
+        assert w.groups_smem <= LDS_OF_CU, (case, w)
+        if w.groups > 1:
+            piece = 1280   # LDS is given out in pieces
+            assert w.groups <= 3 and w.groups_per_cu * (-(-w.groups_smem // piece) * piece) <= LDS_OF_CU, (case, w)
+            # the sums that the other groups leave (16 bytes to a lane and 16 columns) fit the rings that carried the operands
+            columns, stages = BN >> w.sub, 2 if es == 2 else 3
+            assert (w.groups - 1) * 4 * (columns // 16) * 64 * 16 <= w.groups * stages * (64 + columns) * 128, (case, w)
+    assert {(c[0], c[2], w.sub) for c, w in zip(cases, walks)} == {(2, 16, 0), (2, 32, 0), (2, 64, 0), (2, 64, 1), (4, 16, 0), (4, 32, 0),
+                                                                   (4, 32, 1), (4, 64, 0), (4, 64, 1), (4, 64, 2)}
+    assert {w.groups for w in walks} == {0, 1, 2, 3}
 
 
 @pytest.mark.parametrize('TM', [64, 128])
