@@ -120,8 +120,8 @@ def test_index_batch_equals_single_builds(gpu):
 
 @pytest.mark.parametrize('r,c', [(True, True), (True, False), (False, True)])
 def test_index_tensors_of_a_build_lie_apart(r, c, gpu):
-    """The tensors of an index come out of one allocation: none overlaps another, each begins at a multiple of 256 bytes, the
-    values survive the other indexes of the call and the scratch that its builds shared."""
+    """The tensors of the indexes of a call: none overlaps another, each begins at a multiple of 256 bytes, the values survive
+    the other indexes of the call and the scratch that its builds shared."""
     from sparta_amd.tesa import build_indexes_batch
     masks = [torch.from_numpy(ops.block_mask((H, W), (32, 16), 0.6, seed=H)).to(gpu) for H, W in ((32, 16), (96, 1040), (1056, 48))]
     ctx = get_bcs_function(32, 16, r, c)
@@ -141,6 +141,30 @@ def test_index_tensors_of_a_build_lie_apart(r, c, gpu):
         assert np.array_equal(kept.row_ptr.cpu().numpy(), row_ptr) and np.array_equal(kept.BCSR_idx.cpu().numpy(), bcsr)
     if c:
         assert np.array_equal(kept.col_ptr.cpu().numpy(), col_ptr)
+
+
+@pytest.mark.parametrize('r,c', [(True, True), (True, False), (False, True)])
+def test_index_tensors_of_a_build_are_saved_and_copied_one_by_one(r, c, gpu, tmp_path):
+    """Every tensor of an index owns its storage: all of them go into one file together, also int32 and int64 entries, and what is
+    written for one of them alone, or kept of it, is its own bytes and not the other tensors'."""
+    import copy
+    import io
+    mask = torch.from_numpy(ops.block_mask((1056, 1040), (32, 16), 0.6, seed=5)).to(gpu)
+    index = get_bcs_function(32, 16, r, c).build_indexes(mask)
+    tensors = {n: t for n in ('row_ptr', '_bcsr_buf', 'col_ptr', '_bcsc_buf', 'nnz_dev') if (t := getattr(index, n, None)) is not None}
+    tensors.update(index.__dict__['_launch_order'])
+    assert len(tensors) == 1 + 3 * (r + c)
+    live = {n: t[:index.block_nnz] if t.numel() == index.capacity else t for n, t in tensors.items()}   # (past them nothing is written)
+    torch.save(tensors, tmp_path / 'index.pt')
+    loaded = torch.load(tmp_path / 'index.pt', weights_only=True)
+    copied = copy.deepcopy(tensors)
+    for name, t in tensors.items():
+        for other in (loaded[name], copied[name]):
+            assert other.dtype == t.dtype and other.shape == t.shape and torch.equal(other[:live[name].numel()], live[name]), name
+        assert t.storage_offset() == 0 and t.untyped_storage().nbytes() == t.numel() * t.element_size(), name
+        alone = io.BytesIO()
+        torch.save(t, alone)
+        assert len(alone.getvalue()) <= t.numel() * t.element_size() + 4096, name
 
 
 @pytest.mark.parametrize('n', [1, 2, 4, 5])
