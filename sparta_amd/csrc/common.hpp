@@ -228,11 +228,12 @@ __device__ __forceinline__ void store16_stream(void* p, const vec16& v) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     __builtin_nontemporal_store(u32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(p));
 }
-// Results that the next launch reads: written through the L2 at once, so that they neither wait in it for their eviction nor go
-// past the last-level cache as non-temporal ones do.  (Two wait states, for the data registers of a store of four.)
+// Results that the next launch reads: written through the L2 at once (the store of agent scope, a single `sc1` instruction), so that
+// they neither wait in it for their eviction nor go past the last-level cache as non-temporal ones do.  A builtin, not inline asm: the
+// compiler puts the wait states in front that a register written by an MFMA needs, and sees what is written.
 __device__ __forceinline__ void store16_through(void* p, const vec16& v) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(u32x4{v.x, v.y, v.z, v.w}));
+    __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)p, u32x4{v.x, v.y, v.z, v.w}, "agent");
 }
 
 }  // namespace spx
