@@ -40,6 +40,7 @@ static int run_matmul(int mode, int transA, int transB, int compressed,
     p.bias = bias; p.out = C; p.ptr = ptr; p.idx = idx; p.idx_kind = idx_kind; p.sched = sched;
     p.K = K; p.BK = BK; p.log_bk = ilog2(BK);
     p.compressed = compressed;
+    p.counted = compressed && sparse_batch_stride > 0 && !nnz_dev;
     p.o_batch = (int64_t)M * N;
     p.bias_batch = N;
     int BNc;  // canonical sparse block width

@@ -30,6 +30,7 @@ struct SpmmParams {
     int Mc, K, Nc;       // canonical sizes (Mc: dense rows, Nc: sparse-side cols)
     int BK, log_bk;
     int d_kcontig;       // D[m*d_ld + k] if set, else D[k*d_ld + m]
+    int counted;         // s_batch is the size of the live blocks (compressed, and not kept at the capacity of the index)
     int64_t d_ld;
     int s_kcontig;       // block element (k, n): n*s_ld + k if set, else k*s_ld + n
     int compressed;      // S blocks at slot*BK*BN, else inside the dense matrix
@@ -340,8 +341,9 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         //     1856 x 1152 at 31 % 13.3 / 11.1, 944 x 1024 x 1152 at 2 % 5.7 / 4.0, but with more 13.5 / 18.7 (935 x 2880 x 1152 at 35 %),
         //     15.0 / 17.5 (392 x 3072 x 3072 at 37 %), 16.3 / 18.5 (1163 x 3072 x 1024 at 32 %).
         const bool two_blocks = p.BK * (int)sizeof(T) == 64;
-        // stored blocks in all block-columns together (all places where it is not known)
+        // stored blocks in all block-columns together (all places where it is not known), and the live ones as the later rules count on them
         const int64_t stored = p.compressed && p.s_batch > 0 ? p.s_batch / ((int64_t)p.BK * BN) : (int64_t)cols * nb;
+        const int64_t live = spmm_live_blocks(p.counted, stored, (int64_t)cols * nb);
         // fp32 blocks of depth 16, long block-columns: four wavefronts that split a column and meet once keep
         // more loads in flight than 256-row tiles when those are few.  256-row kernel / split columns:
         // up to 1024 rows 512 x 4096 x 4096 at 35 % 259 / 85 us, at 5 % 45 / 20, 1024 x 2048 x 2048 74 / 45 and
@@ -369,9 +371,10 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
             // 1408 x 3328 at 28 % 31.0 / 23.3, 2518 x 1088 x 3776 28.7 / 21.9, 2579 x 2624 x 2048 37.9 / 30.4, 2520 x 2112 x 2240 at 13 % 18.9 / 15.7)
             // ... and neither do five and six of them over eight XCDs (256-row kernel / ring, us: 1256 x 3200 x 3488 at 21 % 33.8 / 22.9, 1503 x 1280 x
             // 3392 16.9 / 12.6, 1220 x 2496 x 3424 with 4.1 blocks to a column 10.6 / 8.9; seven 1606 x 2880 x 2688 15.0 / 17.3, shorter walks 1537 x
-            // 896 x 3616 7.5 / 8.1)
+            // 896 x 3616 7.5 / 8.1; where the live blocks are not counted, dense storage with one, two, four and eight to a column: 1500 x 1024 x 3072
+            // 6.9 / 6.9, 7.7 / 7.3, 9.9 / 8.9, 13.6 / 12.6, 1256 x 2048 x 3424 6.6 / 6.9, 8.5 / 7.3, 11.1 / 9.5, 16.7 / 13.5)
             const bool mid_rows = sizeof(T) == 2 && BN == 32 && p.Nc >= 2048 &&
-                                  ((p.Mc > 2048 && p.Mc <= 3072) || (p.Mc > 1024 && p.Mc <= 1536 && stored >= 4 * (int64_t)nb));
+                                  ((p.Mc > 2048 && p.Mc <= 3072) || (p.Mc > 1024 && p.Mc <= 1536 && live >= 4 * (int64_t)nb));
             if (mid_rows) ring = rounds128 < rounds64 ? 12 : 11;   // (4 and 3 rounds 29.3 / 23.3; 3 each 41 / 51, 2626 x 3584 x 2688 at 24 %)
             if (fill) use_ring = ring_ok && cols >= 32 && (p.Nc < 2048 || mid_rows || (few_rows && p.Mc <= 1024));
             else use_ring = ring_ok && p.Mc > 256 && (p.Mc >= 2048 || cols < 32 || few_rows);
@@ -400,10 +403,18 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         // columns do and brings it through LDS stages ahead.  Split columns / ring, us: 320 x 1024 -> 1472 at 16 % 6.7 / 4.5, 80 x 1792 ->
         // 1856 5.9 / 4.4, 592 x 2880 -> 1536 at 27 % 15.0 / 10.6, 401 x 1152 -> 1344 at 26 % 7.1 / 5.9; longer walks in more tiles 368 x 2496 ->
         // 1472 at 36 % 8.9 / 10.1, 832 x 3136 -> 896 at 40 % 12.8 / 14.9.  No split (below) / ring: 192 x 896 -> 1408 at 26 % 5.7 / 4.5, 64 x 704 -> 1856
-        // 5.3 / 4.5, but 28 x 960 -> 2816 4.2 / 4.5, 3 x 3328 -> 1728 3.9 / 5.7 and five blocks to a column 87 x 576 -> 3136 4.4 / 5.2.  Where the live blocks are not counted, up to 64 places to a column (277 x 3840 -> 960 at 24 % 8.8 / 10.0).
+        // 5.3 / 4.5, but 28 x 960 -> 2816 4.2 / 4.5, 3 x 3328 -> 1728 3.9 / 5.7 and five blocks to a column 87 x 576 -> 3136 4.4 / 5.2.
+        // Where the live blocks are not counted: from the places on that several groups of wavefronts share a walk (five blocks, 40 places), and
+        // where the others have more tiles than CUs.  Dense storage, one, three and eight live blocks to a column, split columns / ring: 300 x 1280 -> 1024 (40
+        // places) 4.2 / 4.0, 4.4 / 4.0, 5.1 / 4.8, but 300 x 1184 -> 1024 (37) 4.2 / 4.0, 4.4 / 4.6, 5.1 / 6.5; 300 x 1088 -> 2048 (320 tiles) 4.9 / 4.1,
+        // 5.7 / 5.2, 6.8 / 6.8, 800 x 1024 -> 1024 (416) 5.2 / 4.6, 5.9 / 5.1, 7.2 / 7.4, 600 x 2048 -> 1024 (320) with 8, 16 and 26 7.3 / 5.7, 8.9 / 7.0, 11.1 / 8.7.  No
+        // split / ring: one, two, four and ten: 128 x 512 -> 1536 (96 tiles) 3.7 / 3.9, 4.2 / 4.5, 5.0 / 5.1, 7.0 / 6.7, 64 x 768 -> 3072 3.5 / 3.8, 4.2 / 4.4,
+        // 5.4 / 5.4, 7.4 / 7.2, but 256 x 768 -> 3072 (384) 4.7 / 4.6, 5.3 / 4.8, 7.3 / 5.8, 11.1 / 7.6.  Up to 64 places to a column (277 x 3840 -> 960 at 24 % 8.8 / 10.0).
         else if (sizeof(T) == 2 && ring_ok && kcontig && two_blocks && BN == 32 && !fill && p.Mc > 32 && tiles64 <= 512 &&
-                 (tiles64 <= 256 || stored <= 26 * (int64_t)nb) && (p.compressed || cols <= 64) &&
-                 (p.Mc <= 256 && cols <= 32 ? stored >= 6 * (int64_t)nb : cols >= 8 && stored >= 4 * (int64_t)nb))
+                 (tiles64 <= 256 || live <= 26 * (int64_t)nb) &&
+                 (!p.counted                     ? cols >= 8 && cols <= 64 && (tiles64 > 256 || live >= 5 * (int64_t)nb)
+                  : p.Mc <= 256 && cols <= 32    ? live >= 6 * (int64_t)nb
+                                                 : cols >= 8 && live >= 4 * (int64_t)nb))
             tile_cfg = 11;
         // few rows and short columns: no barrier and no shared block pays (64 x 768 x 3072 bf16: 3.9 us
         // against 4.4 with the columns split and 5.2 through the ring)

@@ -515,9 +515,8 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
         if (n_pos == launch.n_list) {
             SpmmParams q = p;
             if (n_pos * batch <= 32) q.sched = nullptr;   // one to a CU: the order is of no account, a trip to memory less
-            // (where the live blocks are not counted, every eighth)
-            const int64_t columns = p.Nc / (BN << p.sub_log2), places = columns * (p.K / BK);
-            const int64_t blocks = p.compressed && p.s_batch > 0 ? p.s_batch / (BK * BN << p.sub_log2) : places / 8;
+            const int64_t columns = p.Nc / (BN << p.sub_log2);
+            const int64_t blocks = spmm_live_blocks(p.counted, p.s_batch / (BK * BN << p.sub_log2), columns * (p.K / BK));
             const int groups = ring_groups(ES, BN, SWAP, n_pos * batch, (double)blocks * BK * ES / (columns * 128));
             const int lds = smem + (groups - 1) * ring_stages(ES) * LDS.stage;
             constexpr bool cut = BN < 64 && (ES == 4 || BN == 32);   // what ring_sub_log2 makes

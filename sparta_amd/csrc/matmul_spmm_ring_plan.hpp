@@ -126,6 +126,10 @@ constexpr RingLaunch ring_launch(int elem_bytes, int TM, int BN, bool swap, int 
     return ring_launch_of(l, lds, per_cu, batch);
 }
 
+// Live blocks of a sparse operand that the choice of a kernel and of its launch counts on: every eighth place where they are not
+// counted on the host (a dense operand under a mask, a compressed one kept at the capacity of its index).
+constexpr int64_t spmm_live_blocks(bool counted, int64_t stored, int64_t places) { return counted ? stored : places / 8; }
+
 // 64-row tiles, log2 of the parts that a block-column is cut into, each a tile of its own, where every tile then still has a
 // workgroup to itself.  fp32: as narrow as it gets, a tile's MFMAs are most of its time (64 x 64 blocks at 30 - 40 %, us: 52 x 1600 -> 3584
 // 20.9, in halves 13.6, in quarters 10.4; gradients of the input 64 x 2688 -> 1408 24.9 / 15.1 / 12.8, 304 x 1856 -> 1088 21.7 / 13.8 /

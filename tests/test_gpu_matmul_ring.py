@@ -122,6 +122,38 @@ def test_dispatch_of_few_rows_and_long_columns(dtype, blocks, M, K, N, sparsity,
                  sparsity=sparsity, seed=71, tile_cfg=0, activation='relu' if compressed else None)
 
 
+@pytest.mark.parametrize('storage', ['dense', 'capacity', 'counted'])
+@pytest.mark.parametrize('M,K,N,live,kernels', [
+    # few rows, up to 32 places to a column: up to 256 tiles and more
+    (128, 512, 1536, 1, ('direct', 'direct')), (128, 512, 1536, 10, ('direct', 'ring')), (256, 768, 3072, 2, ('ring', 'direct')),
+    # 39 places, 40, 64 and 65; more than 256 tiles with fewer
+    (300, 1248, 1024, 8, ('ksplit', 'ring')), (300, 1280, 1024, 3, ('ring', 'ksplit')), (300, 2048, 1024, 8, ('ring', 'ring')),
+    (300, 2080, 1024, 8, ('ksplit', 'ring')), (300, 1088, 2048, 8, ('ring', 'ring')),
+    # wide results of 1025 to 1536 rows
+    (1500, 1024, 3072, 2, ('ring', 'panel')), (1500, 1024, 3072, 5, ('ring', 'ring'))])
+def test_dispatch_where_the_live_blocks_are_not_counted(M, K, N, live, kernels, storage, gpu):
+    """16-bit blocks of 32 x 32.  A dense operand under a mask and a compressed one at the capacity of its index take the kernel
+    that fits the places (first of `kernels`), one that is counted the kernel that fits its live blocks."""
+    rng = np.random.default_rng(M + K)
+    nb, cols = N // 32, K // 32
+    grid = np.zeros(nb * cols, np.uint8)
+    grid[rng.permutation(nb * cols)[:live * nb]] = 1
+    mask = torch.from_numpy(np.kron(grid.reshape(nb, cols), np.ones((32, 32), np.uint8))).to(gpu)
+    kernel = SparTASparseMatMulKernel(mode='dsd', biased=False, transpose_A=False, transpose_B=True, compressed=storage != 'dense')
+    kernel.ports['B'].set_mask(mask)
+    kernel.ports['B'].at_capacity = storage == 'capacity'
+    kernel.set_shape(1, M, K, N)
+    kernel.compile({'BLOCK_SIZE_M_VALUE': 32, 'BLOCK_SIZE_K_VALUE': 32, 'BLOCK_SIZE_N_VALUE': 32})
+    g = torch.Generator(device=gpu).manual_seed(M)
+    A, B = (torch.randn(s, generator=g, device=gpu).half() for s in ((1, M, K), (1, N, K)))
+    B = B * mask
+    packed = B if storage == 'dense' else kernel.ports['B'].indexes.convert(B, at_capacity=storage == 'capacity')
+    C, names = launched_kernels(lambda: kernel(A, packed))
+    assert_close(C, torch.matmul(A[0].double(), B[0].double().T).cpu().numpy()[None], torch.float16, f'{M}x{K}x{N} {storage}')
+    taken = [k for k in ('direct', 'ksplit', 'ring', 'panel', 'stream') if any(f'spmm_{k}' in n for n in names)]
+    assert taken == [kernels[storage == 'counted']], names
+
+
 @pytest.mark.parametrize('tile_cfg', [0, 11, 12])
 @pytest.mark.parametrize('mode,depth', [('dsd', 16), ('sdd', 16), ('dsd', 64)])
 def test_ring_sums_of_narrow_fp32_blocks(tile_cfg, mode, depth, gpu, size=1024, sparsity=0.65):
