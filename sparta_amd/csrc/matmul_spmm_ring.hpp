@@ -530,7 +530,10 @@ static int launch_spmm_ring_inst(const SpmmParams& p, int batch, hipStream_t st)
             if (p.sub_log2 == 0) {
                 SPX_RING_GROUPS(false, 1)
             }
-            SPX_RING_GROUPS(cut, 1) SPX_RING_GROUPS(cut, 2) SPX_RING_GROUPS(cut, 3)
+            SPX_RING_GROUPS(cut, 1)
+            if constexpr (ring_most_groups(ES, BN) == 3) {
+                SPX_RING_GROUPS(cut, 2) SPX_RING_GROUPS(cut, 3)
+            }
 #undef SPX_RING_GROUPS
         }
     }

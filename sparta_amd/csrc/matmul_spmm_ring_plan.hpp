@@ -150,7 +150,11 @@ constexpr int ring_sub_log2(int elem_bytes, int BN, bool swap, int Mc, int K, in
 // 7.0 / 11.2, 816 x 4032 -> 1472 (663) 11.4 / 12.8 / 16.5, 128 x 3392 -> 2816 12.0 / 9.0 / 8.2, 4 x 3264 -> 2112 9.5 / 7.2 / 6.6; bf16 32 x 32 blocks, gradient of
 // 304 x 2944 -> 896 15.2 / 9.8 / 8.4; fp32 46 x 4096 -> 960 at 34 % 15.4 / 12.4 / 12.0, 512 x 1408 -> 896 (448) 7.6 / 7.6 / 9.4, 304 x 1088 -> 1856 (580)
 // 10.5 / 11.4 / 13.6.  Walks of two stages: 288 x 2112 -> 2560 at 6 % 5.7 / - / 6.5.
+// fp32 tiles wider than 16: one.  Block-columns are cut narrower wherever every tile then still has a workgroup, so there are
+// over 64 of these to an XCD.
+constexpr int ring_most_groups(int elem_bytes, int BN) { return elem_bytes == 4 && BN > 16 ? 1 : 3; }
 constexpr int ring_groups(int elem_bytes, int BN, bool swap, int n_pos, double stages) {
+    if (ring_most_groups(elem_bytes, BN) == 1) return 1;
     const RingLds lds = ring_lds(elem_bytes, 64, BN, swap);
     int groups = stages < 2.5 ? 1 : n_pos <= 32 ? 3 : n_pos <= 64 ? 2 : 1;
     while (groups > 1 && !ring_fits(lds.list + (groups - 1) * ring_stages(elem_bytes) * lds.stage, n_pos <= 32 ? 1 : 2)) --groups;

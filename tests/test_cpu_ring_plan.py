@@ -3,6 +3,7 @@ share: the list of a workgroup's tiles lies inside the LDS that the launch asks 
 differ in length - and every tile belongs to exactly one workgroup.  No GPU."""
 import os
 import random
+import re
 import shutil
 import subprocess
 from typing import NamedTuple
@@ -10,6 +11,7 @@ from typing import NamedTuple
 import pytest
 
 from conftest import ROOT
+from sparta_amd import _lib
 
 LIST_MAX, LDS_OF_CU = 128, 160 * 1024
 # (16-bit 32 x 64 blocks of 768 -> 3072, 128-row tiles; fp32 32 x 32; batched products) sizes at which the XCDs lie on the
@@ -18,6 +20,10 @@ STRADDLING = [(2, 128, 32, 1, 131073, 768, 3072, 1), (2, 128, 32, 1, 131968, 768
               (4, 128, 32, 1, 87936, 768, 3072, 1), (2, 128, 32, 1, 6208, 768, 4096, 16), (4, 128, 32, 1, 5504, 3072, 768, 48),
               # what the GPU tests run
               (2, 64, 16, 1, 109100, 64, 1536, 1), (2, 128, 16, 1, 131200, 64, 1536, 1), (2, 64, 16, 1, 4160, 64, 240, 128)]
+
+
+# (element bytes, width of a tile, groups of wavefronts) that launches of 64-row tiles make
+GROUPS = {(2, w, g) for w in (16, 32, 64) for g in (1, 2, 3)} | {(4, 16, g) for g in (1, 2, 3)} | {(4, 32, 1), (4, 64, 1)}
 
 
 class Walk(NamedTuple):
@@ -117,7 +123,17 @@ def test_parts_of_a_block_column_and_groups_of_wavefronts(walk):
             assert (w.groups - 1) * 4 * (columns // 16) * 64 * 16 <= w.groups * stages * (64 + columns) * 128, (case, w)
     assert {(c[0], c[2], w.sub) for c, w in zip(cases, walks)} == {(2, 16, 0), (2, 32, 0), (2, 64, 0), (2, 64, 1), (4, 16, 0), (4, 32, 0),
                                                                    (4, 32, 1), (4, 64, 0), (4, 64, 1), (4, 64, 2)}
-    assert {w.groups for w in walks} == {0, 1, 2, 3}
+    assert {(c[0], c[2] >> w.sub, w.groups) for c, w in zip(cases, walks) if w.groups} == GROUPS
+
+
+def test_the_library_has_the_groups_that_launches_make():
+    """... and none that no launch reaches: a width and a number of groups are 24 kernels or more."""
+    if shutil.which('nm') is None or not os.path.exists(_lib.LIB_PATH):
+        pytest.skip('no nm, or nothing is built')
+    names = subprocess.run(['nm', '-D', '--defined-only', _lib.LIB_PATH], capture_output=True, text=True, check=True).stdout
+    kernels = re.findall(r'spmm_ring_kernelI(f|DF16_|NS_\w+?)Li(\d+)ELi(\d+)ELi(\d+)E((?:Lb[01]E)+)Li(\d)E', names)
+    assert len(kernels) > 100
+    assert {(4 if t == 'f' else 2, int(width), int(groups)) for t, _, width, _, _, groups in kernels} == GROUPS
 
 
 @pytest.mark.parametrize('TM', [64, 128])
