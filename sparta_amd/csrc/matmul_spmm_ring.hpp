@@ -424,15 +424,7 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
             at = at + STAGE == NB * STAGE ? 0 : at + STAGE;
         }
         // ---- epilogue: the tile meets in LDS in the orientation of the output and leaves as whole 16-byte
-        // vectors of contiguous rows.  16-bit rows of 64 bytes with an activation, i.e. the operand of the next product, are
-        // written through to the last-level cache, which non-temporal stores go past: dynamic feed-forward blocks of 8192 x
-        // 768 -> 3072 -> 768 fp16 21.1 + 19.1 -> 20.0 + 14.4 us, 4096 x 1024 -> 4096 17.0 + 16.6 -> 16.9 + 13.7, 2767 x 512 -> 1024 7.0 + 5.4 ->
-        // 6.7 + 4.6; not where the XCDs share out the columns of a panel in small parts, and with them the lines of a row (2314 x 704 -> 1408,
-        // eight parts, 9.6 + 8.6 -> 10.4 + 9.0).  The product itself takes up to a few percent longer where it has few rows or does not widen
-        // them (with the hint / through: 4096 x 768 -> 2304 10.8 / 11.5, 4000 x 1024 -> 4096 15.0 / 15.7, 8192 x 2048 -> 1024 19.1 / 20.1, 16384 x 1024 ->
-        // 1024 16.5 / 17.2; 8192 x 768 -> 3072 20.8 / 20.4, 8192 x 1024 -> 2048 at 15 % 17.5 / 17.7, at 35 % 28.2 / 26.9, 12345 x 1024 -> 2048 39.1 / 39.9), so
-        // these keep the hint: a first product of a feed-forward block is twice as wide as deep.  Results without an activation
-        // keep it too, a product alone gains 1 - 3 % from it (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
+        // vectors of contiguous rows, past the last-level cache or (ring_results_through) through to it
         if (n_bar == 0) __syncthreads();
         if constexpr (GROUPS > 1) {
             __syncthreads();   // the rings have been read: their space carries the sums of the other groups
@@ -477,7 +469,7 @@ __global__ __launch_bounds__(kRingThreads * GROUPS, 3) void spmm_ring_kernel(Spm
         __syncthreads();
         constexpr int CPR = LDS.cols / E16;   // 16-byte vectors per row
         constexpr bool THROUGH = ES == 2 && BN == 32 && SWAP && DK && SK;
-        const bool through = THROUGH && p.relu && p.Mc > 5120 && p.Nc >= 2 * p.K && l.parts_log2 <= 1;
+        const bool through = THROUGH && p.relu && ring_results_through(p.Mc, p.K, p.Nc, l.parts_log2);
 #pragma unroll
         for (int v0 = 0; v0 < ROWS * CPR; v0 += 256) {
             const int v = v0 + threadIdx.x;

@@ -161,4 +161,16 @@ constexpr int ring_groups(int elem_bytes, int BN, bool swap, int n_pos, double s
     return groups;
 }
 
+// 16-bit results in rows of 64 bytes, k-contiguous operands, with an activation: whether they are written through to the last-level
+// cache, which non-temporal stores go past.  The next product then reads them from there.  Feed-forward blocks K -> N -> K, fp16, both products
+// with the hint / with this, us: 8192 x 768 -> 3072 38.4 / 33.4, 8192 x 1024 -> 2048 38.3 / 35.5, 8192 x 512 -> 2048 32.7 / 30.1, 12345 x 1024 -> 2048
+// 55.0 / 50.3; between 5121 and 8192 rows level (5200 x 768 -> 3072 32.5 / 32.6, 6000 rows 32.9 / 33.3, 7000 rows 35.8 / 35.4, 6500 x 1024 -> 2048 37.4 / 37.8,
+// 5700 x 1024 -> 4096 42.1 / 41.7), with blocks of depth 32 too (8192 x 768 -> 3072 49.1 / 49.0).
+// Refused, as a product on its own takes up to 7 % longer: fewer rows (4096 x 768 -> 2304 10.8 / 11.5, 4000 x 1024 -> 4096 15.0 / 15.7, though
+// some pairs would gain, 4096 x 1024 -> 4096 33.6 / 30.6 and 2767 x 512 -> 1024 12.4 / 11.3) and results that are no wider than twice the depth
+// (8192 x 2048 -> 1024 19.1 / 20.1, 16384 x 1024 -> 1024 16.5 / 17.2); and panels whose columns, and with them the lines of a row, several
+// XCDs share out (2314 x 704 -> 1408 in eight parts, the pair 18.2 / 19.4).  Results without an activation keep the hint, from which a product
+// on its own gains 1 - 3 % (9235 x 1024 -> 2176 24.0 / 24.4, 2423 x 2176 -> 2624 20.1 / 20.7); plain stores take 0.4 - 2 us longer than either.
+constexpr bool ring_results_through(int Mc, int K, int Nc, int parts_log2) { return Mc > 5120 && Nc >= 2 * K && parts_log2 <= 1; }
+
 }  // namespace spx

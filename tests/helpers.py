@@ -45,6 +45,13 @@ def chained_sum_error(additions):
     return 0.41 * 2.0 ** -24 * (additions / 2) ** 0.5
 
 
+# Ring kernel: (rows of a tile, M) of products K -> N with an activation, and whether their results are written through: more rows
+# and fewer, panels in one part, in two and in eight
+RESULTS_K_N = (192, 544)
+RESULTS_THROUGH = {(64, 1024): 0, (64, 2200): 0, (64, 1090): 0, (64, 65): 0, (64, 5120): 0, (64, 5130): 1, (64, 6100): 1,
+                   (128, 1024): 0, (128, 2200): 0, (128, 65): 0, (128, 5130): 0, (128, 5600): 1, (128, 6100): 1}
+
+
 def launched_kernels(call):
     """(what `call` returns, names of the kernels that it launched; they may be mangled)."""
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:

@@ -4,7 +4,8 @@
 // every tile has exactly one workgroup (-1: not walked), the workgroups of the launch that are side by side on the chip
 // (over the batch), and how many the choice of a tile height counts on; then, for 64-row tiles (0 otherwise), the log2 of the
 // parts that a block-column is cut into, `cover` of that launch, whether each of its tiles has a workgroup to itself, the groups of
-// wavefronts that share a long walk there, the LDS of a workgroup with them, and how many of them a CU has to hold.
+// wavefronts that share a long walk there, the LDS of a workgroup with them, and how many of them a CU has to hold; last, whether results with an
+// activation are written through (16-bit rows of 64 bytes).
 #include <cstdio>
 #include <vector>
 #include "matmul_spmm_ring_plan.hpp"
@@ -52,8 +53,9 @@ int main() {
         const RingLds lds = ring_lds(es, TM, part, swap != 0);
         std::printf("%d %d %d %d %d %d %d %d", launch.list.slots, launch.smem, fewest, most, reach,
                     cover ? covered(launch, N / BN) : -1, 8 * launch.n_pos * batch, ring_slots(es, TM, BN, swap != 0));
-        std::printf(" %d %d %d %d %d %d\n", sub, cover && low ? covered(cut, N / part) : -1, (int)one, groups,
-                    groups ? cut.smem + (groups - 1) * ring_stages(es) * lds.stage : 0, (cut.n_pos * batch + 31) / 32);
+        std::printf(" %d %d %d %d %d %d %d\n", sub, cover && low ? covered(cut, N / part) : -1, (int)one, groups,
+                    groups ? cut.smem + (groups - 1) * ring_stages(es) * lds.stage : 0, (cut.n_pos * batch + 31) / 32,
+                    (int)ring_results_through(M, K, N, launch.list.parts_log2));
     }
     return 0;
 }

@@ -11,6 +11,7 @@ from typing import NamedTuple
 import pytest
 
 from conftest import ROOT
+from helpers import RESULTS_K_N, RESULTS_THROUGH
 from sparta_amd import _lib
 
 LIST_MAX, LDS_OF_CU = 128, 160 * 1024
@@ -41,6 +42,7 @@ class Walk(NamedTuple):
     groups: int
     groups_smem: int
     groups_per_cu: int
+    through: int         # results with an activation go through to the last-level cache
 
 
 @pytest.fixture(scope='module')
@@ -134,6 +136,16 @@ def test_the_library_has_the_groups_that_launches_make():
     kernels = re.findall(r'spmm_ring_kernelI(f|DF16_|NS_\w+?)Li(\d+)ELi(\d+)ELi(\d+)E((?:Lb[01]E)+)Li(\d)E', names)
     assert len(kernels) > 100
     assert {(4 if t == 'f' else 2, int(width), int(groups)) for t, _, width, _, _, groups in kernels} == GROUPS
+
+
+def test_results_with_an_activation_that_are_written_through(walk):
+    """Both sides of each line, and the sizes that the GPU test of the stores runs (their values are the same either way)."""
+    sizes = [(8192, 768, 3072, 1), (5121, 768, 1536, 1), (5120, 768, 3072, 0), (8192, 768, 1504, 0), (16384, 1024, 1024, 0), (8192, 1024, 2048, 1)]
+    for M, K, N, through in sizes:
+        assert walk([(2, 64, 32, 1, M, K, N, 1)])[0].through == through, (M, K, N)
+    for (TM, M), through in RESULTS_THROUGH.items():
+        assert walk([(2, TM, 32, 1, M, *RESULTS_K_N, 1)])[0].through == through, (TM, M)
+    assert set(RESULTS_THROUGH.values()) == {0, 1}
 
 
 @pytest.mark.parametrize('TM', [64, 128])

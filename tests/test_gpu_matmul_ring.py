@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_close, chained_sum_error, launched_kernels, template_numbers
+from helpers import RESULTS_K_N, RESULTS_THROUGH, assert_close, chained_sum_error, launched_kernels, template_numbers
 from oracle import ops
 from sparta_amd.specializer.kernels import SparTASparseMatMulKernel
 from test_gpu_matmul import run_case
@@ -70,17 +70,38 @@ def test_ring_groups(mode, transposed, compressed, dtype, wide, depth, columns, 
                                                  gran=(depth, wide) if mode == 'dsd' and not transposed else (wide, depth), sparsity=sparsity, seed=columns, tile_cfg=11))
     numbers = template_numbers(names, 'spmm_ring_kernel')
     assert len(numbers) == 1
-    if compressed:
-        assert numbers[0][-1] == groups, numbers
+    # (where the blocks are not counted, an eighth of the places: two stages or less here)
+    assert numbers[0][-1] == (groups if compressed else 1), numbers
+
+
+@pytest.mark.parametrize('mode,transposed,compressed', [('dsd', True, True), ('dsd', False, True), ('dsd', True, False), ('dsd', False, False),
+                                                        ('sdd', False, True), ('sdd', False, False)])
+@pytest.mark.parametrize('dtype,wide,depth,rows,columns,batch,K,tile,groups', [
+    # 16-bit block-columns 64 wide cut in halves whose walks are shared: 96 of them, few rows, a tile to a batch entry and XCD
+    (torch.float16, 64, 64, 504, 12, 1, 1280, 32, 3), (torch.bfloat16, 64, 32, 8, 44, 1, 3392, 32, 3), (torch.float16, 64, 64, 40, 2, 40, 1280, 32, 2),
+    # as many stages as the estimate of uncounted blocks has to reach
+    (torch.float16, 32, 32, 504, 20, 1, 1280, 32, 3), (torch.bfloat16, 32, 64, 504, 40, 1, 1280, 32, 2), (torch.float32, 64, 16, 200, 10, 1, 640, 16, 3),
+    (torch.float32, 16, 64, 504, 40, 1, 640, 16, 2)])
+def test_ring_groups_of_cut_and_of_uncounted_block_columns(mode, transposed, compressed, dtype, wide, depth, rows, columns, batch, K, tile, groups, gpu):
+    """Walks shared out over groups of wavefronts where a tile is half of a block-column, and where the sparse operand is a dense
+    tensor under a mask, i.e. the groups follow from its places."""
+    blocks = (32, depth, wide) if mode == 'dsd' else (wide, depth, 32)
+    M, N = (rows, wide * columns) if mode == 'dsd' else (wide * columns, rows)
+    _, names = launched_kernels(lambda: run_case(gpu, mode, False, transposed, True, compressed, dtype, blocks, batch=batch, M=M, K=K, N=N,
+                                                 gran=(depth, wide) if mode == 'dsd' and not transposed else (wide, depth), sparsity=0.7,
+                                                 seed=columns, tile_cfg=11))
+    numbers = template_numbers(names, 'spmm_ring_kernel')
+    assert [(n[1], n[-1]) for n in numbers] == [(tile, groups)], numbers
 
 
 @pytest.mark.parametrize('tile_cfg', [11, 12])
 @pytest.mark.parametrize('dtype,blocks', [(torch.float16, (32, 32, 32)), (torch.bfloat16, (32, 64, 32))])
 def test_ring_results_with_an_activation(tile_cfg, dtype, blocks, gpu):
-    """64-byte row pieces that are written through the L2s (over 5120 rows, panels in one part and in two) and that are not:
-    fewer rows, panels in four parts and in eight; rows that end inside a tile."""
-    for M in (1024, 2200, 1090, 65, 5130, 5600, 6100):
-        run_case(gpu, 'dsd', False, True, True, M != 2200, dtype, blocks, batch=1, M=M, K=192, N=544, gran=(blocks[2], blocks[1]),
+    """64-byte row pieces that are written through the L2s and that are not, rows that end inside a tile.  Which of the sizes are
+    does not show in the values: test_cpu_ring_plan.py asks the rule that the kernel asks."""
+    K, N = RESULTS_K_N
+    for M in [m for rows, m in RESULTS_THROUGH if rows == (64 if tile_cfg == 11 else 128)]:
+        run_case(gpu, 'dsd', False, True, True, M != 2200, dtype, blocks, batch=1, M=M, K=K, N=N, gran=(blocks[2], blocks[1]),
                  sparsity=0.7, seed=M, tile_cfg=tile_cfg, activation='relu')
 
 
