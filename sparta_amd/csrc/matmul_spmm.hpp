@@ -404,6 +404,10 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         // 1856 5.9 / 4.4, 592 x 2880 -> 1536 at 27 % 15.0 / 10.6, 401 x 1152 -> 1344 at 26 % 7.1 / 5.9; longer walks in more tiles 368 x 2496 ->
         // 1472 at 36 % 8.9 / 10.1, 832 x 3136 -> 896 at 40 % 12.8 / 14.9.  No split (below) / ring: 192 x 896 -> 1408 at 26 % 5.7 / 4.5, 64 x 704 -> 1856
         // 5.3 / 4.5, but 28 x 960 -> 2816 4.2 / 4.5, 3 x 3328 -> 1728 3.9 / 5.7 and five blocks to a column 87 x 576 -> 3136 4.4 / 5.2.
+        // The lines: split columns are ahead where a walk has too few stages for several groups, four blocks to a column up to 256 tiles
+        // (ring / split 1.13 over 80 problems of 64 to 592 rows, with five 0.98, six 0.96, eight to twenty 1.00 - 1.03; above 256 tiles 0.94, 0.80, 0.81, 0.84 - 0.89).  No
+        // split is ahead up to 48 rows below twelve blocks (33 x 704 -> 1856 with six, eight and twelve 4.2 / 4.6, 4.5 / 5.0, 5.2 / 5.2; 48 rows 4.5 / 4.7,
+        // 4.7 / 5.0, 5.5 / 5.4; 64 rows 4.8 / 4.6, 5.1 / 4.7, 6.0 / 5.3).
         // Where the live blocks are not counted: from the places on that several groups of wavefronts share a walk (five blocks, 40 places), and
         // where the others have more tiles than CUs.  Dense storage, one, three and eight live blocks to a column, split columns / ring: 300 x 1280 -> 1024 (40
         // places) 4.2 / 4.0, 4.4 / 4.0, 5.1 / 4.8, but 300 x 1184 -> 1024 (37) 4.2 / 4.0, 4.4 / 4.6, 5.1 / 6.5; 300 x 1088 -> 2048 (320 tiles) 4.9 / 4.1,
@@ -413,8 +417,8 @@ int launch_spmm_impl(const SpmmParams& p, int BN, int batch, int tile_cfg, hipSt
         else if (sizeof(T) == 2 && ring_ok && kcontig && two_blocks && BN == 32 && !fill && p.Mc > 32 && tiles64 <= 512 &&
                  (tiles64 <= 256 || live <= 26 * (int64_t)nb) &&
                  (!p.counted                     ? cols >= 8 && cols <= 64 && (tiles64 > 256 || live >= 5 * (int64_t)nb)
-                  : p.Mc <= 256 && cols <= 32    ? live >= 6 * (int64_t)nb
-                                                 : cols >= 8 && live >= 4 * (int64_t)nb))
+                  : p.Mc <= 256 && cols <= 32    ? live >= (p.Mc <= 48 ? 12 : 6) * (int64_t)nb
+                                                 : cols >= 8 && live >= (tiles64 > 256 ? 4 : 5) * (int64_t)nb))
             tile_cfg = 11;
         // few rows and short columns: no barrier and no shared block pays (64 x 768 x 3072 bf16: 3.9 us
         // against 4.4 with the columns split and 5.2 through the ring)

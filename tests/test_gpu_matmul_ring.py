@@ -147,13 +147,17 @@ def test_dispatch_of_few_rows_and_long_columns(dtype, blocks, M, K, N, sparsity,
 @pytest.mark.parametrize('M,K,N,live,kernels', [
     # few rows, up to 32 places to a column: up to 256 tiles and more
     (128, 512, 1536, 1, ('direct', 'direct')), (128, 512, 1536, 10, ('direct', 'ring')), (256, 768, 3072, 2, ('ring', 'direct')),
+    # ... up to 48 rows and more
+    (48, 704, 704, 11, ('direct', 'direct')), (48, 704, 704, 12, ('direct', 'ring')), (49, 704, 704, 6, ('direct', 'ring')),
+    # four live blocks to a column and five, up to 256 tiles and more
+    (128, 1280, 1024, 4, ('ring', 'ksplit')), (128, 1280, 1024, 5, ('ring', 'ring')), (300, 1280, 1664, 4, ('ring', 'ring')),
     # 39 places, 40, 64 and 65; more than 256 tiles with fewer
     (300, 1248, 1024, 8, ('ksplit', 'ring')), (300, 1280, 1024, 3, ('ring', 'ksplit')), (300, 2048, 1024, 8, ('ring', 'ring')),
     (300, 2080, 1024, 8, ('ksplit', 'ring')), (300, 1088, 2048, 8, ('ring', 'ring')),
     # wide results of 1025 to 1536 rows
     (1500, 1024, 3072, 2, ('ring', 'panel')), (1500, 1024, 3072, 5, ('ring', 'ring'))])
-def test_dispatch_where_the_live_blocks_are_not_counted(M, K, N, live, kernels, storage, gpu):
-    """16-bit blocks of 32 x 32.  A dense operand under a mask and a compressed one at the capacity of its index take the kernel
+def test_dispatch_of_few_tiles(M, K, N, live, kernels, storage, gpu):
+    """16-bit blocks of 32 x 32, few tiles.  A dense operand under a mask and a compressed one at the capacity of its index take the kernel
     that fits the places (first of `kernels`), one that is counted the kernel that fits its live blocks."""
     rng = np.random.default_rng(M + K)
     nb, cols = N // 32, K // 32
