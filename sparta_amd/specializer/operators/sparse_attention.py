@@ -73,7 +73,8 @@ class _FusedAttentionFunc(torch.autograd.Function):
 
 # Training steps with an element mask recompute the probabilities from this many queries (batch x N_target) on:
 # 12 x 512 queries bf16 143 us a step with stored probabilities, 97 without (the host's part is smaller), 96 x 4096 fp16
-# 292 and 226.  Nothing smaller was in need of it.
+# 292 and 226.  Nothing smaller was in need of it.  Head dim 128, causal windows of two to five blocks, fp16: 4 x 512 148 and 103, the
+# kernels alone 19 and 23 to 42 and 44; 12 x 1024 148 and 103, 30 and 33 to 54 and 55; 24 x 1024 39 and 38 to 84 and 67.
 _MASKED_RECOMPUTE_QUERIES = 2048
 
 
